@@ -40,10 +40,11 @@ HBM_PEAK_GBS = 8000.0
 # Integer VALU issue of one MI355X: 256 CUs x 4 SIMDs x 2.4 GHz / 4 cycles per
 # wave64 instruction x 64 lanes = 3.93e13 lane-ops/s.
 VALU_PEAK_TOPS = 39.3
-# VALU instructions per DP cell of edr_wave_kernel<N, 16> (AMD ISA of the built
-# kernel: 2 subtractions + 2 compares for the match, the row shift, M + s,
-# min3, compare, select, the +1 add).
-EDR_VALU_PER_CELL = 10
+# VALU instructions per DP cell of edr_wave_kernel<N, 16> in a block that tests
+# no match (AMD ISA of the built kernel, four rows per lane: add, min3, compare,
+# select, and a quarter of the row shift); a block that does has five more (two
+# subtractions, two compares, the borrow), so this is the least a batch needs.
+EDR_VALU_PER_CELL = 4.25
 METRIC = "range queries/s + EDR cell-updates/s, batched vs plain; p99 latency"
 
 

@@ -2,33 +2,15 @@
 // launch.  Same recurrence as Grid::SimilarityExecuter (Grid.cpp:1222-1318);
 // no reference counterpart for the batching itself.
 //
-// Wave-systolic layout.  A wave64 runs four independent pairs, one per 16-lane
-// DPP row ("segment"), or one long pair over all 64 lanes.  Inside a segment of
-// S lanes, lane l owns DP row r = S*s + l + 1 of strip s and keeps that row's
-// point in registers; at step t it computes column c = t - l + 1, so a strip
-// sweeps its S rows across all columns in m + S - 1 steps.  The three
-// neighbours of a cell come from registers:
-//   U = D[r-1][c]   the left lane's value of the previous step (DPP shift)
-//   L = D[r][c-1]   the lane's own value of the previous step
-//   M = D[r-1][c-1] the left lane's value two steps back, i.e. the U the lane
-//                   received one step earlier
-// and the cell rule of Grid.cpp:1297-1300 reduces exactly to
-//   D = (M == L) ? U : min(M, L, U)
-// (M strictly smallest -> M; L strictly smallest -> L; every tie for the
-// minimum, and M == L < U in particular, -> U).
-// The first lane of a segment takes U + 1 from the row above the strip, kept
-// in LDS as 16-bit values of D + 1 and read once per step as a broadcast (the
-// value is the `old` operand of the shift, so lane 0 keeps it).  Each lane
-// stores its cell plus one into the same buffer at its own column; the strip's
-// last lane stores every column last, which leaves its row there for the next
-// strip, and each column is read (step c - 1) no later than its first store of
-// the strip (lane 0, same step, after the read).  Column points are read
-// straight from the NaN-padded trajectory store (64 consecutive points per
-// wave access, L1 resident across the lanes that reuse them); a NaN point
-// never matches, so lanes before their first column keep D[r][0] = r untouched
-// and lanes past the last column compute values nobody reads.  The cell
-// D[n][m] is captured by the lane that owns row n at the step it reaches
-// column m.
+// Wave-systolic layout (edr_dp.hpp).  A wave64 runs four independent pairs, one
+// per 16-lane DPP row ("segment"), or one long pair over all 64 lanes.  Inside
+// a segment of S lanes, lane l owns K consecutive DP rows of a strip of S * K
+// rows and computes them for column t - l + 1 at step t, so a strip sweeps its
+// rows across all columns in m + S - 1 steps: the row above comes from the left
+// lane's bottom row of the step before (a DPP shift), everything else from the
+// lane's own registers.  The first lane's row above the strip is kept in LDS
+// as 16-bit values, into which every lane stores its bottom row, the strip's
+// last lane last.
 //
 // Work: jobs of up to four pairs (one for 64-lane segments) with the same
 // strip count, ordered longest first, handed out by one atomic counter per
@@ -36,37 +18,18 @@
 // buckets.
 #include <cmath>
 
+#include "edr_dp.hpp"
 #include "gat_common.hpp"
 
 namespace {
 
-constexpr int kBlk = 16;   // steps per feed block
-constexpr int kPad = 16;   // NaN points before every trajectory of a padded store
+using edr::kBlk;
+using edr::kPad;
 
 struct Job {
   int32_t first, count;
 };
 static_assert(sizeof(Job) == sizeof(gat_edr_job), "job layout");
-
-// Stores of different lanes to one LDS column come from different steps'
-// store instructions, and the row left behind is the last lane's only if those
-// instructions keep program order.  Per lane their addresses differ, so the
-// scheduler may reorder them; this barrier lets every other kind of
-// instruction (ALU, global loads, LDS reads) move across it, but not LDS
-// writes.
-__device__ __forceinline__ void keep_store_order() {
-  // 0x1 ALU, 0x2 VALU, 0x4 SALU, 0x10 VMEM, 0x20 VMEM read, 0x100 DS read.
-  __builtin_amdgcn_sched_barrier(0x1 | 0x2 | 0x4 | 0x10 | 0x20 | 0x100);
-}
-
-// Lane l of a segment takes src from lane l - 1; lane 0 keeps old.  Segments
-// of 16 lanes are DPP rows (row_shr:1); a 64-lane segment is the wave
-// (wave_shr:1).
-template <int SEG>
-__device__ __forceinline__ int shift_in(int old, int src) {
-  static_assert(SEG == 16 || SEG == 64, "segments of 16 or 64 lanes");
-  return __builtin_amdgcn_update_dpp(old, src, SEG == 16 ? 0x111 : 0x138, 0xf, 0xf, false);
-}
 
 // A launch over a window of the job array: jobs [window[0], window[0] +
 // window[1]) of the njobs the array holds, the window written on the device
@@ -105,7 +68,7 @@ __global__ __launch_bounds__(64, (MAXM >= 2048 && SEG == 16) ? 2 : 4) void edr_w
                                                       int32_t* __restrict__ out) {
   constexpr int kSeg = SEG;        // lanes per pair
   constexpr int kSegs = 64 / SEG;  // pairs per wave
-  // Row above the current strip plus one, D[r0][c] + 1, at [c + kOff][segment]
+  // Row above the current strip, E[r0][c] = D[r0][c] - r0, at [c + kOff][segment]
   // for columns 2 - SEG .. MAXM + SEG + kBlk - 1 (the lanes' look-behind, the
   // columns, and the last blocks' overrun).  Segments interleave, so one
   // segment's consecutive columns are 2 * kSegs bytes apart and each step's
@@ -116,7 +79,6 @@ __global__ __launch_bounds__(64, (MAXM >= 2048 && SEG == 16) ? 2 : 4) void edr_w
   const int lane = threadIdx.x;
   const int seg = lane / kSeg;
   const int l = lane & (kSeg - 1);
-  const float2 nan2 = make_float2(__builtin_nanf(""), __builtin_nanf(""));
   jobs += take_window(window, njobs);
   for (;;) {
     int ji = 0;
@@ -156,135 +118,198 @@ __global__ __launch_bounds__(64, (MAXM >= 2048 && SEG == 16) ? 2 : 4) void edr_w
     const int n0 = __builtin_amdgcn_readlane(n, 0), n1 = __builtin_amdgcn_readlane(n, 16);
     const int n2 = __builtin_amdgcn_readlane(n, 32), n3 = __builtin_amdgcn_readlane(n, 48);
     const int nmax = max(max(n0, n1), max(n2, n3));
-    // Smallest column and row counts among the live segments: capture starts
-    // at the first strip that is some segment's last and the first column
-    // that is some segment's last.
-    int mmin = mmax, nmin = nmax;
-    if (n0 > 0) { mmin = min(mmin, m0); nmin = min(nmin, n0); }
-    if (n1 > 0) { mmin = min(mmin, m1); nmin = min(nmin, n1); }
-    if (n2 > 0) { mmin = min(mmin, m2); nmin = min(nmin, n2); }
-    if (n3 > 0) { mmin = min(mmin, m3); nmin = min(nmin, n3); }
-    const int first_last_strip = (nmin + kSeg - 1) / kSeg - 1;
-    const int strips = (nmax + kSeg - 1) / kSeg;
-    const int my_last = (n + kSeg - 1) / kSeg - 1;
-    const int steps = mmax + kSeg - 1;
-    job_priority(int64_t(strips) * steps);
-    // Row 0: D[0][c] + 1 = c + 1.  (Kept rolled: unrolled, its length grows with MAXM
-    // and so does the register count.)
+    const int strips = (nmax + kSeg * edr::kLaneRows - 1) / (kSeg * edr::kLaneRows);
+    job_priority(int64_t(strips) * (mmax + kSeg - 1) * 2);
+    // Row 0: E[0][c] = c, as far as the job's last block reads.  (Kept rolled:
+    // unrolled, its length grows with MAXM and so does the register count.)
+    const int used = min(kRows, mmax + 2 * SEG + kBlk);
 #pragma unroll 2
-    for (int i = l; i < kRows; i += kSeg) above[i][seg] = int16_t(i - kOff + 1);
-    int res = 0;
-    for (int s = 0; s < strips; ++s) {
-      // Orders the previous strip's (or the initial) writes of `above` before
-      // this strip's reads of them by other lanes.
-      __syncthreads();
-      const int r = kSeg * s + l + 1;
-      const float2 rp = r <= n ? R[r - 1] : nan2;
-      const float rx = rp.x, ry = rp.y;
-      int c1 = r + 1;  // D[r][c - 1] + 1, from D[r][0] = r
-      int u1p = r;     // D[r-1][c - 1] + 1, from D[r-1][0] + 1
-      const int tcap = (s == my_last) ? m + l - 1 : -1;  // step at which lane l holds D[r][m]
-      const bool last_strip_somewhere = s >= first_last_strip;
-      const float2* cp = C - l;  // column point of step t is cp[t]
-      // Column points of steps tb .. tb + 15.  Lanes look back up to SEG - 1
-      // points before the trajectory.  A lane whose block starts more than
-      // kPad points before it (64-lane segments, first blocks only) has all 16
-      // points before it: it takes NaN, never matching, and loads from the
-      // padding instead.
-      auto load_block = [&](float2(&dst)[kBlk], int tb) __attribute__((always_inline)) {
-        if (SEG <= kPad + 1 || tb - (kSeg - 1) >= -kPad) {
-#pragma unroll
-          for (int j = 0; j < kBlk; ++j) dst[j] = cp[tb + j];
-        } else {
-          const bool before = tb - l < -kPad;
-          const float2* bp = before ? C - kPad : cp + tb;
-#pragma unroll
-          for (int j = 0; j < kBlk; ++j) {
-            const float2 v = bp[j];
-            dst[j] = before ? nan2 : v;
-          }
-        }
-      };
-      // One feed block of kBlk steps over the column points in `src` (steps
-      // t0 .. t0 + 15) while the next block's points load into `dst`.  Two
-      // register sets alternate, so no block copies one into the other.
-      auto sweep = [&](const float2(&src)[kBlk], float2(&dst)[kBlk], int t0) __attribute__((always_inline)) {
-        // Feed: U + 1 for the segment's first lane at step t0 + j (column
-        // t0 + j + 1), read for the whole block before its first store: this
-        // strip stores column c first at step c - 1, and no earlier block of
-        // the strip stores past column t0.
-        const int16_t(*feed)[kSegs] = &above[kOff + t0 + 1];
-        int fv[kBlk];
-#pragma unroll
-        for (int j = 0; j < kBlk; ++j) fv[j] = feed[j][seg];
-        // Every lane stores its cell plus one at its column, t0 + j - l + 1.
-        // The last lane stores a column last, so after the strip the buffer
-        // holds the strip's last row (columns up to the widest segment's last);
-        // lane 0 stores column c at the step that reads its feed, after the
-        // read.
-        int16_t(*own)[kSegs] = &above[kOff + t0 - l + 1];
-        load_block(dst, t0 + kBlk);
-        const bool capture = last_strip_somewhere && t0 + kBlk - 1 >= mmin - 1;
-        if (capture) {
-#pragma unroll
-          for (int j = 0; j < kBlk; ++j) {
-            const bool match = fabsf(rx - src[j].x) < u && fabsf(ry - src[j].y) < u;
-            const int u1 = shift_in<SEG>(fv[j], c1);
-            const int mm = u1p - (match ? 1 : 0);
-            const int mn = min(min(u1, c1), mm);
-            const int d = (mm == c1) ? u1 : mn;
-            res = (t0 + j == tcap) ? d : res;
-            c1 = d + 1;
-            u1p = u1;
-            own[j][seg] = int16_t(c1);
-            keep_store_order();
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < kBlk; ++j) {
-            const bool match = fabsf(rx - src[j].x) < u && fabsf(ry - src[j].y) < u;
-            const int u1 = shift_in<SEG>(fv[j], c1);
-            const int mm = u1p - (match ? 1 : 0);
-            const int mn = min(min(u1, c1), mm);
-            const int d = (mm == c1) ? u1 : mn;
-            c1 = d + 1;
-            u1p = u1;
-            own[j][seg] = int16_t(c1);
-            keep_store_order();
-          }
-        }
-      };
-      float2 colA[kBlk], colB[kBlk];
-      load_block(colA, 0);
-      for (int t0 = 0; t0 < steps; t0 += 2 * kBlk) {
-        sweep(colA, colB, t0);
-        if (t0 + kBlk >= steps) break;
-        sweep(colB, colA, t0 + kBlk);
-      }
+    for (int i = l; i < used; i += kSeg) above[i][seg] = int16_t(i - kOff);
+    int ns[kSegs], ms[kSegs];
+    if constexpr (kSegs == 4) {
+      ns[0] = n0; ns[1] = n1; ns[2] = n2; ns[3] = n3;
+      ms[0] = m0; ms[1] = m1; ms[2] = m2; ms[3] = m3;
+    } else {
+      ns[0] = n0;
+      ms[0] = m0;
     }
+    bool mine = false;
+    const int res = edr::sweep_pairs<SEG, SEG == 64>(R, n, C, m, nmax, mmax, ns, ms, u, above, seg, l, &mine);
     __syncthreads();  // the next job re-initialises `above`
     if (live && !valid && l == 0) out[job.first + seg] = -1;
-    if (valid && l == ((n - 1) & (kSeg - 1))) out[job.first + seg] = res;
+    if (valid && mine) out[job.first + seg] = res + n;  // D = E + n
   }
 }
 
 // One pair over W waves of a workgroup (no reference counterpart): wave w
-// runs the pair's 64-row strips w, w + W, ... in lockstep with the others,
-// one block of 16 steps per iteration and a workgroup barrier between
+// runs the pair's strips w, w + W, ... of 64 * K rows in lockstep with the
+// others, one block of 16 steps per iteration and a workgroup barrier between
 // iterations, so a pair's strips overlap instead of running one after another.
 // A strip reads the row above it from the previous strip's wave: that wave's
-// last lane writes its row, D + 1 per column, into the wave's own LDS row
+// last lane writes its bottom row, E per column, into the wave's own LDS row
 // buffer at step c + 62 for column c, and the consumer reads column c at step
-// c - 1 of its own strip (the feed of the block holding that step, loaded when
-// the block starts).  So a strip starts kLag >= 5 blocks after the previous
-// one (column 16b + 16, the last a consumer block b reads, is written in the
-// producer's block b + 4), and no sooner than its wave has finished its
-// previous strip — which also keeps a wave's writes to its buffer behind the
-// next wave's reads of the previous contents (those reads start kLag blocks
-// earlier on every column).  Every wave runs the same number of iterations,
-// so the barriers always match.  The cell rule, the row/column orientation
-// and the capture of D[n][m] are edr_wave_kernel's with 64-lane segments.
+// c - 1 of its own strip; a block's feed is read one block ahead of its use.
+// So a strip starts kLag = 6 blocks after the previous one (column 16b + 32,
+// the last read during a consumer's block b, is written in the producer's
+// block b + 5), and no sooner than its wave has finished its previous strip —
+// which also keeps a wave's writes to its buffer behind the next wave's reads
+// of the previous contents (those reads start kLag blocks earlier on every
+// column).  Every wave runs the same number of iterations, so the barriers
+// always match.  The cell rule, the row/column orientation, the far-block test
+// and the capture of D[n][m] are sweep_strip's (edr_dp.hpp) with 64-lane
+// segments; K (1, 2 or 4) is the least that gives every wave at most one strip,
+// up to 4: a wave is alone on its SIMD here, so a step costs its instructions
+// (17 VALU at K = 4, 5 at K = 1) and fewer rows per lane end a pair sooner.
 constexpr int kLag = 6;
+
+template <int MAXM, int W>
+struct PipeShared {
+  // Columns -62 .. 0 sit before column 0 (lane 63's look-behind); a block's
+  // feed, read a block ahead, goes up to column 16 * nblocks + 16 <= m + 94.
+  static constexpr int kOff = 64;
+  static constexpr int kLen = kOff + MAXM + 112;
+  int16_t rows[W + 1][kLen];  // [W]: row 0, E[0][c] = c
+  // The column trajectory, columns -63 .. 16 * nblocks + 15 (<= m + 93) at
+  // [kColOff + column], NaN outside 0 .. m - 1: too few waves run here to hide
+  // a global load's latency behind a block's 16 steps.
+  static constexpr int kColOff = 64;
+  static constexpr int kColLen = kColOff + MAXM + 96;
+  float2 cols[kColLen];
+  static constexpr int kChunks = MAXM / kBlk;
+  float4 chunk[kChunks];  // boxes of columns 16 b .. 16 b + 15
+  int32_t job_slot;
+};
+
+template <int K, int MAXM, int W>
+__device__ __forceinline__ void pipe_pair(PipeShared<MAXM, W>& sh, const float2* R, int n, int m, float u, int wv,
+                                          int l, int32_t* out) {
+  using S = PipeShared<MAXM, W>;
+  constexpr int kRows = 64 * K;
+  const int strips = (n + kRows - 1) / kRows;
+  const int steps = m + 63;
+  const int nblocks = (steps + kBlk - 1) / kBlk;
+  const int nchunks = (m + kBlk - 1) / kBlk;
+  // Strip s starts at block (s / W) * P + (s % W) * kLag, P = max(nblocks,
+  // W * kLag): kLag after strip s - 1 and P >= nblocks after the same wave's
+  // previous strip.
+  const int P = max(nblocks, W * kLag);
+  const int kend = ((strips - 1) / W) * P + ((strips - 1) % W) * kLag + nblocks;
+  job_priority(int64_t(kend) * kBlk * 2);
+  edr::LaneRows<K> rows;
+  rows.start();
+  int s = wv, start = wv * kLag;
+  int tcap = -1, ic = 0, tend = -1, res = 0;
+  bool mine = false;
+  uint64_t near0 = 0, near1 = 0, near2 = 0;  // blocks of the strip that may match
+  bool loaded = false;
+  float2 src[kBlk];
+  int fv[kBlk];
+#pragma unroll
+  for (int j = 0; j < kBlk; ++j) {
+    src[j] = make_float2(0.0f, 0.0f);
+    fv[j] = 0;
+  }
+  const int16_t* above = sh.rows[W];
+  int16_t* own = sh.rows[wv];
+  auto begin_strip = [&]() __attribute__((always_inline)) {
+    rows.start();
+    const float4 box = edr::segment_box<64>(rows.load(R, n, s * kRows + l * K));
+    auto touches = [&](int c) __attribute__((always_inline)) -> uint64_t {
+      return __ballot(c < nchunks && edr::may_touch(box, sh.chunk[min(c, S::kChunks - 1)], u));
+    };
+    // A block's lanes reach back over the five chunks up to its own.
+    const uint64_t t0 = touches(l), t1 = touches(l + 64), t2 = touches(l + 128);
+    near0 = near1 = near2 = 0;
+#pragma unroll
+    for (int d = 0; d < 5; ++d) {
+      near0 |= t0 << d;
+      near1 |= t1 << d | (d ? t0 >> (64 - d) : 0);
+      near2 |= t2 << d | (d ? t1 >> (64 - d) : 0);
+    }
+    loaded = false;
+    const int loc = n - 1 - s * kRows;  // < kRows in the last strip only
+    const bool ends = loc < kRows;
+    ic = ends ? loc % K : 0;
+    tend = ends ? m + loc / K - 1 : -1;
+    const bool here = ends && l == loc / K;
+    tcap = here ? tend : -1;
+    mine = mine || here;
+    above = sh.rows[s == 0 ? W : (s - 1) % W] + S::kOff + 1;
+#pragma unroll
+    for (int j = 0; j < kBlk; ++j) fv[j] = above[j];
+  };
+  auto column = [&](int t) __attribute__((always_inline)) { return sh.cols[S::kColOff + t - l]; };
+  auto block = [&](auto near_c, auto cap_c, int t0) __attribute__((always_inline)) {
+    constexpr bool kNear = decltype(near_c)::value, kCap = decltype(cap_c)::value;
+    int bottom[kBlk];
+    const int16_t* feed = above + t0 + kBlk;
+#pragma unroll
+    for (int j = 0; j < kBlk; ++j) {
+      const int u0 = edr::shift_in<64>(fv[j], rows.e[K - 1]);
+      rows.template step<kNear>(u0, src[j], u);
+      if constexpr (kCap) {
+#pragma unroll
+        for (int i = 0; i < K; ++i) res = (t0 + j == tcap && i == ic) ? rows.e[i] : res;
+      }
+      bottom[j] = rows.e[K - 1];
+      fv[j] = feed[j];
+      if constexpr (kNear) src[j] = column(t0 + kBlk + j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // The last lane's cells after the chain of steps: a branch per step would
+    // sit in its way.
+    if (l == 63) {
+      int16_t* dst = own + S::kOff + t0 - 62;
+#pragma unroll
+      for (int j = 0; j < kBlk; ++j) dst[j] = int16_t(bottom[j]);
+    }
+  };
+  auto block_near_cap = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll 1
+    for (int t = t0; t < t0 + kBlk; ++t) {
+      const int u0 = edr::shift_in<64>(above[t], rows.e[K - 1]);
+      rows.template step<true>(u0, column(t), u);
+#pragma unroll
+      for (int i = 0; i < K; ++i) res = (t == tcap && i == ic) ? rows.e[i] : res;
+      if (l == 63) own[S::kOff + t - 62] = int16_t(rows.e[K - 1]);
+    }
+  };
+  for (int k = 0; k < kend; ++k) {
+    const int b = k - start;
+    if (b >= 0 && s < strips) {
+      if (b == 0) begin_strip();
+      const int t0 = b * kBlk;
+      const uint64_t word = b < 64 ? near0 : b < 128 ? near1 : near2;
+      const bool near = (word >> (b & 63)) & 1u;
+      const bool cap = tend >= t0 && tend < t0 + kBlk;
+      if (near) {
+        if (cap) {
+          block_near_cap(t0);
+#pragma unroll
+          for (int j = 0; j < kBlk; ++j) fv[j] = above[t0 + kBlk + j];
+          loaded = false;
+        } else {
+          if (!loaded) {
+#pragma unroll
+            for (int j = 0; j < kBlk; ++j) src[j] = column(t0 + j);
+          }
+          block(std::true_type{}, std::false_type{}, t0);
+          loaded = true;
+        }
+      } else {
+        if (cap) block(std::false_type{}, std::true_type{}, t0);
+        else block(std::false_type{}, std::false_type{}, t0);
+        loaded = false;
+      }
+      if (b == nblocks - 1) {
+        s += W;
+        start += P;
+      }
+    }
+    __syncthreads();
+  }
+  if (mine) *out = res + n;  // D = E + n
+}
 
 template <int MAXM, int W>
 __global__ __launch_bounds__(64 * W) void edr_pipe_kernel(const int2* __restrict__ pairs, int64_t npairs,
@@ -298,27 +323,16 @@ __global__ __launch_bounds__(64 * W) void edr_pipe_kernel(const int2* __restrict
                                                           const int64_t* __restrict__ coff,
                                                           const int32_t* __restrict__ clen, float u,
                                                           int32_t* __restrict__ out) {
-  // Columns -62 .. 0 sit before column 0 (lane 63's look-behind); a block's
-  // feed reads up to column 16 * nblocks <= m + 78 (the last block's overrun).
-  constexpr int kOff = 64;
-  constexpr int kLen = kOff + MAXM + 96;
-  __shared__ int16_t rows[W][kLen];
-  // The column trajectory in LDS, columns -63 .. 16 * nblocks - 1 (<= m + 77)
-  // at [kColOff + column]: a pair over W waves keeps one wave per SIMD, too
-  // few to hide a global load's latency behind a block's 16 steps, so each
-  // block's points come from LDS instead.
-  constexpr int kColOff = 64;
-  constexpr int kColLen = kColOff + MAXM + 80;
-  __shared__ float2 cols[kColLen];
-  __shared__ int32_t job_slot;
-  const int wv = threadIdx.x / 64;
+  using S = PipeShared<MAXM, W>;
+  __shared__ S sh;
+  const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / 64);
   const int l = threadIdx.x & 63;
-  const float2 nan2 = make_float2(__builtin_nanf(""), __builtin_nanf(""));
   jobs += take_window(window, njobs);
+  for (int i = threadIdx.x; i < S::kLen; i += 64 * W) sh.rows[W][i] = int16_t(i - S::kOff);
   for (;;) {
-    if (threadIdx.x == 0) job_slot = atomicAdd(counter, 1);
+    if (threadIdx.x == 0) sh.job_slot = atomicAdd(counter, 1);
     __syncthreads();
-    const int ji = job_slot;
+    const int ji = sh.job_slot;
     __syncthreads();  // every wave has read the slot before the next job overwrites it
     if (ji < 0 || ji >= njobs) break;  // a counter that was not cleared hands out nothing
     const Job job = jobs[ji];
@@ -326,7 +340,7 @@ __global__ __launch_bounds__(64 * W) void edr_pipe_kernel(const int2* __restrict
     const bool live = job.count >= 1 && job.first >= 0 && int64_t(job.first) < npairs;
     int n = 0, m = 0;
     const float2* R = cxy;
-    const float2* C = cxy + kPad;
+    const float2* C = cxy;
     bool valid = false;
     if (live) {
       const int2 pr = pairs[job.first];
@@ -345,100 +359,20 @@ __global__ __launch_bounds__(64 * W) void edr_pipe_kernel(const int2* __restrict
       if (live && threadIdx.x == 0) out[job.first] = -1;
       continue;
     }
-    const int strips = (n + 63) / 64;
-    const int steps = m + 63;
-    const int nblocks = (steps + kBlk - 1) / kBlk;
-    // Strip s starts at block (s / W) * P + (s % W) * kLag, P = max(nblocks,
-    // W * kLag): kLag after strip s - 1 and P >= nblocks after the same wave's
-    // previous strip.
-    const int P = max(nblocks, W * kLag);
-    const int kend = ((strips - 1) / W) * P + ((strips - 1) % W) * kLag + nblocks;
-    job_priority(int64_t(kend) * kBlk);
-    // Stage the columns the blocks read (lane l of block tb reads columns
-    // tb - l .. tb - l + 15); those more than kPad before the trajectory are
-    // NaN, never matching.
-    for (int i = int(threadIdx.x) - 63; i < nblocks * kBlk; i += 64 * W) cols[kColOff + i] = i < -kPad ? nan2 : C[i];
-    __syncthreads();
-    // Per-lane state of the wave's current strip.
-    int cur = -1;       // strip
-    int c1 = 0, u1p = 0, tcap = -1, res = 0;
-    float rx = 0.0f, ry = 0.0f;
-    // The row point of the wave's next strip, loaded a strip ahead.
-    float2 next_row = 64 * wv + l + 1 <= n ? R[64 * wv + l] : nan2;
-    float2 colA[kBlk], colB[kBlk];
-    auto load_block = [&](float2(&dst)[kBlk], int tb) __attribute__((always_inline)) {
-      const float2* cl = &cols[kColOff + tb - l];
-#pragma unroll
-      for (int j = 0; j < kBlk; ++j) dst[j] = cl[j];
-    };
-    // One iteration: the wave's block of its current strip, if any, with the
-    // block's column points in src and the next block's loading into dst.
-    auto step = [&](int k, float2(&src)[kBlk], float2(&dst)[kBlk]) __attribute__((always_inline)) {
-      const int d = k - wv * kLag;
-      if (d < 0) return;
-      const int i = d / P;
-      const int b = d - i * P;
-      const int s = wv + i * W;
-      if (b >= nblocks || s >= strips) return;
-      const int t0 = b * kBlk;
-      if (b == 0) {  // a new strip: row point, D[r][0] + 1, D[r-1][0] + 1
-        cur = s;
-        const int r = 64 * s + l + 1;
-        rx = next_row.x;
-        ry = next_row.y;
-        const int rn = r + 64 * W;  // the wave's next strip
-        next_row = rn <= n ? R[rn - 1] : nan2;
-        c1 = r + 1;
-        u1p = r;
-        tcap = (s == strips - 1) ? m + l - 1 : -1;
-        load_block(src, 0);
-      }
-      // Feed: D[r0][t0 + j + 1] + 1 from the previous strip's wave (row 0: c + 1).
-      int fv[kBlk];
-      if (s == 0) {
-#pragma unroll
-        for (int j = 0; j < kBlk; ++j) fv[j] = t0 + j + 2;
-      } else {
-        const int16_t* feed = &rows[(s - 1) % W][kOff + t0 + 1];
-#pragma unroll
-        for (int j = 0; j < kBlk; ++j) fv[j] = feed[j];
-      }
-      if (t0 + kBlk < steps) load_block(dst, t0 + kBlk);
-      int16_t* own = &rows[wv][kOff + t0 - 63 + 1];
-      // A wave here is often alone on its SIMD, so each step waits on its
-      // dependent chain (shift, min, select, +1).  The block's matches are
-      // tested before the chain and the last lane's cells are stored after
-      // it, so nothing else (no per-step branch for that lane's store) sits
-      // in the chain's way; the stored columns are still written within the
-      // producer block the consumers' lag allows for.
-      int mt[kBlk];  // 1 where the step's points match (values, not lane masks: those would crowd the SGPRs)
-#pragma unroll
-      for (int j = 0; j < kBlk; ++j) mt[j] = (fabsf(rx - src[j].x) < u && fabsf(ry - src[j].y) < u) ? 1 : 0;
-      int out_c[kBlk];
-#pragma unroll
-      for (int j = 0; j < kBlk; ++j) {
-        const int u1 = shift_in<64>(fv[j], c1);
-        const int mm = u1p - mt[j];
-        const int mn = min(min(u1, c1), mm);
-        const int d = (mm == c1) ? u1 : mn;
-        res = (t0 + j == tcap) ? d : res;
-        c1 = d + 1;
-        u1p = u1;
-        out_c[j] = c1;
-      }
-      if (l == 63) {
-#pragma unroll
-        for (int j = 0; j < kBlk; ++j) own[j] = int16_t(out_c[j]);
-      }
-    };
-    for (int k = 0; k < kend; k += 2) {
-      step(k, colA, colB);
-      __syncthreads();
-      step(k + 1, colB, colA);
-      __syncthreads();
+    // Stage the columns the blocks read, a box per chunk of 16.
+    for (int i = int(threadIdx.x) - 64; i < m + 96; i += 64 * W) {
+      const float2 p = i >= 0 && i < m ? C[i] : edr::nan_point();
+      sh.cols[S::kColOff + i] = p;
+      // 64 divides the stride and the start: a row of 16 lanes holds one chunk.
+      const float4 box = edr::segment_box<16>(edr::grow(edr::empty_box(), p));
+      if ((threadIdx.x & 15) == 0 && i >= 0 && i < m) sh.chunk[i / kBlk] = box;
     }
-    if (cur == strips - 1 && l == ((n - 1) & 63)) out[job.first] = res;
-    __syncthreads();  // the next job's strips reuse the row buffers
+    __syncthreads();
+    const int per = (n + 64 * W - 1) / (64 * W);
+    if (per <= 1) pipe_pair<1>(sh, R, n, m, u, wv, l, out + job.first);
+    else if (per == 2) pipe_pair<2>(sh, R, n, m, u, wv, l, out + job.first);
+    else pipe_pair<4>(sh, R, n, m, u, wv, l, out + job.first);
+    // (pipe_pair ends at a barrier: the next job may reuse the buffers.)
   }
 }
 
@@ -979,11 +913,21 @@ __device__ uint32_t block_exclusive_scan(uint32_t* a, int n, uint32_t* red) {
   return total;
 }
 
-// Several-wave schedule of a pair of s 64-row strips over a row of b blocks
-// (runBatched's pipe_blocks: a lag of kLag blocks between strips).
-__device__ __forceinline__ int64_t pipe_blocks(int64_t s, int64_t b, int waves) {
+// What a pair of n rows and m columns keeps its wave busy for, in VALU
+// instructions per 16-step block: on one wave (64-lane strips of four rows per
+// lane, the last of two or one) and over several (edr_pipe_kernel's schedule,
+// with a lag of kLag blocks between strips and a barrier per block).
+// Grid::runBatched applies the same rule on the host.
+__device__ __forceinline__ int64_t one_wave_cost(int n, int m) {
+  const int rows = (n + 63) / 64, rest = rows & 3;
+  return int64_t((m + 63 + 15) / 16) * (19 * (rows / 4) + (rest >= 2 ? 11 : 0) + ((rest & 1) ? 7 : 0));
+}
+__device__ __forceinline__ int64_t pipe_cost(int n, int m, int waves) {
+  const int per = (n + 64 * waves - 1) / (64 * waves);
+  const int k = per <= 1 ? 1 : per == 2 ? 2 : 4;
+  const int64_t strips = (n + 64 * k - 1) / (64 * k), b = (m + 63 + 15) / 16;
   const int64_t P = b > int64_t(waves) * kLag ? b : int64_t(waves) * kLag;
-  return ((s - 1) / waves) * P + ((s - 1) % waves) * kLag + b;
+  return (((strips - 1) / waves) * P + ((strips - 1) % waves) * kLag + b) * (k == 1 ? 9 : k == 2 ? 13 : 21);
 }
 
 struct JobRules {
@@ -1010,8 +954,7 @@ struct JobShape {
 __device__ __forceinline__ uint32_t job_key(int n, int m, const JobRules& rules, const JobShape& sh,
                                             int64_t critical) {
   int bucket = m <= rules.split ? 0 : m <= sh.mid ? 1 : 2;
-  if (bucket == 2 && sh.multi && (rules.every_long || int64_t((n + 63) / 64) * ((m + 63 + 15) / 16) > critical))
-    bucket = 3;
+  if (bucket == 2 && sh.multi && (rules.every_long || one_wave_cost(n, m) > critical)) bucket = 3;
   const int strips = (n + 15) / 16;
   const int top = bucket == 0 ? rules.split : bucket == 1 ? sh.mid : GAT_MAX_TRAJ_LEN;
   const int step = max(1, (top + kLenSteps - 1) / kLenSteps);
@@ -1055,7 +998,7 @@ __global__ __launch_bounds__(kJobThreads) void edr_jobs_kernel(const int2* __res
     nm[i] = make_int2(n, m);
     my_cells += (unsigned long long)(n) * (unsigned long long)(m);
     if (multi && m > mid) {
-      const int64_t c = pipe_blocks((n + 63) / 64, (m + 63 + 15) / 16, rules.waves);
+      const int64_t c = pipe_cost(n, m, rules.waves);
       if (c > my_crit) my_crit = c;
     }
   }
@@ -1148,8 +1091,7 @@ __global__ __launch_bounds__(kJobsBlock) void edr_jobs_lengths_kernel(
     nm[i] = make_int2(n, m);
     my_cells += (unsigned long long)(n) * (unsigned long long)(m);
     if (sh.multi && m > sh.mid) {
-      const unsigned long long c =
-          (unsigned long long)pipe_blocks((n + 63) / 64, (m + 63 + 15) / 16, rules.waves);
+      const unsigned long long c = (unsigned long long)pipe_cost(n, m, rules.waves);
       my_crit = c > my_crit ? c : my_crit;
     }
   }

@@ -67,6 +67,21 @@ int upload_vec(DeviceBuffer& d, const std::vector<T>& v, void* s, const char* wh
 
 int strips_of(int n) { return (n + 15) / 16; }
 
+// What a pair keeps its wave busy for on one wave and over several, in VALU
+// instructions per 16-step block (gat_edr_jobs applies the same rule on the
+// device).
+int64_t one_wave_cost(int n, int m) {
+  const int rows = (n + 63) / 64, rest = rows & 3;
+  return int64_t((m + 63 + 15) / 16) * (19 * (rows / 4) + (rest >= 2 ? 11 : 0) + ((rest & 1) ? 7 : 0));
+}
+int64_t pipe_cost(int n, int m, int waves) {
+  const int per = (n + 64 * waves - 1) / (64 * waves);
+  const int k = per <= 1 ? 1 : per == 2 ? 2 : 4;
+  const int64_t strips = (n + 64 * k - 1) / (64 * k), b = (m + 63 + 15) / 16;
+  const int64_t P = std::max<int64_t>(b, int64_t(waves) * 6);
+  return (((strips - 1) / waves) * P + ((strips - 1) % waves) * 6 + b) * (k == 1 ? 9 : k == 2 ? 13 : 21);
+}
+
 }  // namespace
 
 int Grid::uploadTrajectories(const TrajectoryView& db) {
@@ -418,24 +433,17 @@ int Grid::runBatched(std::vector<int32_t>& pairs, int queryNum, std::vector<int3
     }
   }
   // In a one-round batch with several waves per long pair, only the pairs
-  // that would outlast the batch's longest pair on one wave take several:
-  // a pair of s 64-row strips over a b-block row takes s * b blocks on one
-  // wave and pipe_blocks(s, b) over `waves` waves (the workgroup's schedule,
-  // with the lag of 6 blocks between strips), and the batch cannot end before
-  // its longest pair's pipelined schedule does.  The rest run one pair per
-  // wave, beside it; several waves on a pair of fewer strips than waves leave
-  // the surplus waves idle at every barrier.
-  auto pipe_blocks = [&](int64_t s, int64_t b) {
-    const int64_t P = std::max<int64_t>(b, int64_t(waves) * 6);
-    return ((s - 1) / waves) * P + ((s - 1) % waves) * 6 + b;
-  };
+  // that would outlast the batch's longest pair on one wave take several: the
+  // batch cannot end before its longest pair's pipelined schedule does.  The
+  // rest run one pair per wave, beside it; several waves on a pair of fewer
+  // strips than waves leave the surplus waves idle at every barrier.
   const bool multiWave = latencyBound && waves > 1;
   int64_t critical = 0;
   if (multiWave)
     for (int64_t i = 0; i < np; ++i) {
       const int a = queryLenHost_[pairs[2 * i]], b = trajLenHost_[pairs[2 * i + 1]];
       const int n = std::min(a, b), m = std::max(a, b);
-      if (m > mid) critical = std::max(critical, pipe_blocks((n + 63) / 64, (m + 63 + 15) / 16));
+      if (m > mid) critical = std::max(critical, pipe_cost(n, m, waves));
     }
   std::vector<int32_t> key(static_cast<size_t>(np));
   int64_t cells = 0;
@@ -446,7 +454,7 @@ int Grid::runBatched(std::vector<int32_t>& pairs, int queryNum, std::vector<int3
     cells += int64_t(n) * m;
     int bucket = m <= split ? 0 : m <= mid ? 1 : 2;
     if (bucket == 2 && multiWave &&
-        (edrWavesEveryLongPair || int64_t((n + 63) / 64) * ((m + 63 + 15) / 16) > critical))
+        (edrWavesEveryLongPair || one_wave_cost(n, m) > critical))
       bucket = 3;
     maxlen[bucket] = std::max(maxlen[bucket], std::min(m, GAT_MAX_TRAJ_LEN));
     key[i] = (bucket * kS + (kS - 1 - strips_of(n))) * kM + (kM - 1 - m);
