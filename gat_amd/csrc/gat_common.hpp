@@ -72,6 +72,27 @@ __device__ __forceinline__ void store_pair2(int2* dst, const int4& v) {
   __builtin_nontemporal_store(w, reinterpret_cast<v4i*>(dst));
 }
 
+// Pairs at and at + 1 (at + 1 < end): one 16-byte load when kWide (16-byte
+// aligned pairs, even at), else two; a lone last pair (at + 1 == end) with
+// zeros beside it, since the next may lie past the buffer.
+template <bool kWide>
+__device__ __forceinline__ int4 load_pair2(const int2* pairs, uint64_t at, uint64_t end) {
+  int4 v = make_int4(0, 0, 0, 0);
+  if (at + 1 < end) {
+    if constexpr (kWide) {
+      v = *reinterpret_cast<const int4*>(pairs + at);
+    } else {
+      const int2 p = pairs[at], q = pairs[at + 1];
+      v = make_int4(p.x, p.y, q.x, q.y);
+    }
+  } else if (at < end) {
+    const int2 p = pairs[at];
+    v.x = p.x;
+    v.y = p.y;
+  }
+  return v;
+}
+
 // Order-independent digest of a (tid, pid) pair: a 64-bit mix (the splitmix64
 // finaliser) of tid in the high and pid in the low half.  A query's digest is
 // the wrapping sum over its pairs.

@@ -1333,26 +1333,77 @@ __global__ __launch_bounds__(256) void run_counts_kernel(const Item* __restrict_
   }
 }
 
-// Per-query digest of run-indexed pairs: one wave per run adds the run's
-// wrapping sum of pair mixes to its query's entry (out must start at zero).
-__global__ __launch_bounds__(256) void runs_digest_kernel(const int2* __restrict__ pairs, uint64_t npairs,
-                                                          const Run* __restrict__ runs, uint64_t nruns,
-                                                          uint32_t nqueries, unsigned long long* __restrict__ out) {
-  const uint32_t lane = threadIdx.x & (kWave - 1);
-  const uint64_t nw = uint64_t(gridDim.x) * (blockDim.x / kWave);
-  for (uint64_t r = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave; r < nruns; r += nw) {
-    const Run run = runs[r];
-    if (run.q >= nqueries || run.first > npairs || run.count > npairs - run.first) continue;
+// Per-query digest of run-indexed pairs: each 16-lane row of a wave takes one
+// run, 16 bytes (two pairs) per lane and load, up to 128 pairs in flight, and
+// adds the run's wrapping sum of pair mixes to its query's entry (out must
+// start at zero).  Bound by the read of the pairs (8 B each) and by the mix (two
+// 64-bit multiplies, about 0.6 of the read's time at full issue).  A wave per
+// run read a median run of 110 pairs in two half-empty 8-byte loads and spent
+// as long on its 64-lane reduction and atomic.  Each workgroup's runs are
+// consecutive, and the entries of the first lds_q queries are summed in LDS
+// first.
+constexpr int kDigBlock = 512;
+constexpr uint32_t kDigLds = 4096;  // 32 KB of 64-bit sums: four workgroups per CU
+
+// v added over the 16 lanes of a DPP row, in every lane.
+__device__ __forceinline__ uint64_t row16_sum(uint64_t v) {
+#define GAT_ROW_ADD(CTRL)                                                                                          \
+  v += uint64_t(uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(v)), CTRL, 0xf, 0xf, false))) |               \
+       (uint64_t(uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(v >> 32)), CTRL, 0xf, 0xf, false))) << 32)
+  GAT_ROW_ADD(0x128);  // row_ror by 8, 4, 2, 1
+  GAT_ROW_ADD(0x124);
+  GAT_ROW_ADD(0x122);
+  GAT_ROW_ADD(0x121);
+#undef GAT_ROW_ADD
+  return v;
+}
+
+template <bool kWide>
+__global__ __launch_bounds__(kDigBlock) void runs_digest_kernel(const int2* __restrict__ pairs, uint64_t npairs,
+                                                                const Run* __restrict__ runs, uint64_t nruns,
+                                                                uint32_t nqueries, uint32_t lds_q,
+                                                                unsigned long long* __restrict__ out) {
+  extern __shared__ unsigned long long dig[];
+  for (uint32_t q = threadIdx.x; q < lds_q; q += kDigBlock) dig[q] = 0;
+  __syncthreads();
+  constexpr uint32_t kRowsPer = kDigBlock / 16;
+  const uint32_t l = threadIdx.x & 15;
+  const uint64_t per = (nruns + gridDim.x - 1) / gridDim.x;
+  const uint64_t lo = uint64_t(blockIdx.x) * per;
+  const uint64_t hi = lo + per < nruns ? lo + per : nruns;
+  uint64_t r = lo + threadIdx.x / 16;
+  Run next = r < hi ? runs[r] : Run{0, 0, 0};
+  for (; r < hi; r += kRowsPer) {
+    const Run run = next;
+    if (r + kRowsPer < hi) next = runs[r + kRowsPer];
+    // Uniform over the row, so its lanes stay together for the sum.
+    if (run.count == 0 || run.q >= nqueries || run.first > npairs || run.count > npairs - run.first) continue;
+    const uint64_t end = run.first + run.count;
     uint64_t sum = 0;
-    for (uint64_t i = lane; i < run.count; i += kWave) sum += gat::pair_mix(pairs[run.first + i]);
+    // Lane l's pairs i, i + 1 from the even pair at or below the run's first.
+    for (uint64_t i = (run.first & ~uint64_t(1)) + 2 * l; i < end; i += 128) {
+      int4 v[4];
 #pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) {
-      const uint32_t lo = uint32_t(__shfl_xor(int(uint32_t(sum)), d, kWave));
-      const uint32_t hi = uint32_t(__shfl_xor(int(uint32_t(sum >> 32)), d, kWave));
-      sum += uint64_t(lo) | (uint64_t(hi) << 32);
+      for (int k = 0; k < 4; ++k) {
+        v[k] = gat::load_pair2<kWide>(pairs, i + 32 * k, end);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint64_t at = i + 32 * k;
+        if (at >= run.first && at < end) sum += gat::pair_mix(make_int2(v[k].x, v[k].y));
+        if (at + 1 < end) sum += gat::pair_mix(make_int2(v[k].z, v[k].w));
+      }
     }
-    if (lane == 0) atomicAdd(out + run.q, (unsigned long long)sum);
+    // Lanes that ran out early wait here with the rest of their row.
+    sum = row16_sum(sum);
+    if (l == 0) {
+      if (run.q < lds_q) atomicAdd(dig + run.q, (unsigned long long)sum);
+      else atomicAdd(out + run.q, (unsigned long long)sum);
+    }
   }
+  __syncthreads();
+  for (uint32_t q = threadIdx.x; q < lds_q; q += kDigBlock)
+    if (dig[q]) atomicAdd(out + q, dig[q]);
 }
 
 // Sum of n uint32 values into *out (which must start at zero).
@@ -1696,10 +1747,17 @@ int gat_runs_digest(const int32_t* pairs, int64_t npairs, const gat_range_run* r
   GAT_REQUIRE(out && (nruns == 0 || (pairs && runs)), "gat_runs_digest: null pointer");
   if (int rc = gat_fill_u32(reinterpret_cast<uint32_t*>(out), 0u, 2 * nqueries, stream)) return rc;
   if (nruns == 0) return GAT_OK;
-  runs_digest_kernel<<<dim3{uint32_t(grid_for(uint64_t(nruns) * kWave, 256, 16))}, dim3{256}, 0,
-                       gat::as_stream(stream)>>>(reinterpret_cast<const int2*>(pairs), uint64_t(npairs),
-                                                 reinterpret_cast<const Run*>(runs), uint64_t(nruns),
-                                                 uint32_t(nqueries), reinterpret_cast<unsigned long long*>(out));
+  const uint32_t lds_q = uint64_t(nqueries) < kDigLds ? uint32_t(nqueries) : kDigLds;
+  const dim3 grid{uint32_t(grid_for(uint64_t(nruns) * 16, kDigBlock, 4))}, block{kDigBlock};
+  const auto* P = reinterpret_cast<const int2*>(pairs);
+  const auto* R = reinterpret_cast<const Run*>(runs);
+  auto* O = reinterpret_cast<unsigned long long*>(out);
+  if (reinterpret_cast<uintptr_t>(pairs) % 16 == 0)
+    runs_digest_kernel<true><<<grid, block, size_t(lds_q) * 8, gat::as_stream(stream)>>>(
+        P, uint64_t(npairs), R, uint64_t(nruns), uint32_t(nqueries), lds_q, O);
+  else
+    runs_digest_kernel<false><<<grid, block, size_t(lds_q) * 8, gat::as_stream(stream)>>>(
+        P, uint64_t(npairs), R, uint64_t(nruns), uint32_t(nqueries), lds_q, O);
   GAT_LAUNCH_CHECK("runs_digest_kernel");
   return GAT_OK;
 }

@@ -422,9 +422,8 @@ int RangeBatch::fetch(int32_t* out, int64_t capacityPairs) {
 
 int RangeBatch::digests(uint64_t* out) const {
   if (queryNum == 0) return GAT_OK;
-  DeviceBuffer d;
-  if (int rc = d.reserve(size_t(queryNum) * 8)) return rc;
-  return digestsInto(d.as<uint64_t>(), out);
+  if (int rc = digestDev_.reserve(size_t(queryNum) * 8)) return rc;
+  return digestsInto(digestDev_.as<uint64_t>(), out);
 }
 
 int RangeBatch::digestsInto(uint64_t* dev, uint64_t* out) const {

@@ -84,6 +84,9 @@ struct RangeBatch {
   // The same into a caller-owned device buffer of queryNum entries (no
   // allocation), copied to `out` when it is not null.
   int digestsInto(uint64_t* dev, uint64_t* out) const;
+
+ private:
+  mutable DeviceBuffer digestDev_;  // digests(): kept, since a free waits for the device
 };
 
 // Device copy of an index's tree for the batched form: gat_tree_node in
