@@ -367,6 +367,23 @@ int RangeBatch::fetchCompact(int32_t* out, int64_t capacityPairs) {
     gath_set_error("fetch: %lld pairs, room for %lld", (long long)pairTotal, (long long)capacityPairs);
     return GAT_ERR_CAPACITY;
   }
+  if (pairTotal == 0) return GAT_OK;
+  const size_t bytes = size_t(pairTotal) * 8;
+  if (bytes <= kGatherBytes) {
+    size_t room = size_t(1) << 16;
+    while (room < bytes) room *= 2;
+    if (int rc = gatherAt_.reserve(size_t(queryNum) * 8)) return rc;
+    if (int rc = gatherHost_.reserve(room)) return rc;
+    GATH_TRY(gat_gather_pairs(pairs.as<int32_t>(), int64_t(pairs.size() / 8),
+                              runIndexed ? nullptr : qbase.as<uint64_t>(),
+                              runIndexed ? runs.as<gat_range_run>() : nullptr, runIndexed ? runTotal : 0,
+                              qcount.as<uint32_t>(), queryNum, gatherAt_.as<uint64_t>(), gatherHost_.as<int32_t>(),
+                              pairTotal, stream),
+             "pair gather");
+    GATH_TRY(gat_stream_sync(stream), "pair gather");
+    std::memcpy(out, gatherHost_.get(), bytes);
+    return GAT_OK;
+  }
   std::vector<int64_t> at(size_t(queryNum) + 1, 0);
   for (int q = 0; q < queryNum; ++q) at[size_t(q) + 1] = at[size_t(q)] + count[size_t(q)];
   if (runIndexed) {
@@ -576,77 +593,82 @@ int RangeEngine::reserveBatched(const DeviceTree& tree, int maxQueries, int64_t 
   if (int rc = lqRank_.reserve(size_t(lqCap_) * 4)) return rc;
   if (int rc = qlist_.reserve(size_t(qlistCap_) * 4)) return rc;
   if (int rc = items_.reserve(size_t(itemsCap_) * 16)) return rc;
-  if (int rc = directTasks_.reserve(size_t(lqCap_) * sizeof(gat_range_task))) return rc;
   if (int rc = out.runs.reserve(size_t(qlistCap_) * sizeof(gat_range_run))) return rc;
   if (int rc = itemBase_.reserve(size_t(itemsCap_) * 8)) return rc;
   if (int rc = itemTiles_.reserve(size_t(gat_scan_tiles(itemsCap_)) * 8)) return rc;
   return out.pairs.reserve(size_t(pairsCap_) * 8);
 }
 
-// Direct form: selection without per-node counts, then one refine task per
-// selected (leaf, rectangle).  Boxes are already on the device.
-int RangeEngine::runDirect(const DeviceTree& tree, int nq, RangeBatch& out) {
+// Direct form: selection without per-node counts, then one refine entry per
+// selected (leaf, rectangle), queued as one chain with the capacities at hand
+// and one synchronisation at its end; a batch that outgrew a capacity (the
+// device keeps inside them) grows it and runs again.
+int RangeEngine::runDirect(const DeviceTree& tree, const MBB* bounds, int nq, RangeBatch& out) {
   void* s = stream_.get();
-  const int64_t N = tree.nnodes;
+  const double t0 = now_ms();
+  if (clockKhz_ == 0) GATH_TRY(gat_wall_clock_khz(&clockKhz_), "device clock");
+  size_t bytes = 0;
+  if (int rc = stageBoxes(&tree, bounds, nq, &bytes)) return rc;
+  if (int rc = directHost_.reserve(size_t(gat_direct_words(nq)) * 4)) return rc;
   uint32_t* ctr = counters_.as<uint32_t>();
-  const uint32_t* ch = countersHost_.as<uint32_t>();
+  const uint32_t* ch = directHost_.as<uint32_t>();
   auto u64 = [&](int w) { return uint64_t(ch[w]) | (uint64_t(ch[w + 1]) << 32); };
+  if (pairsCap_ == 0) pairsCap_ = 1 << 16;
+  const bool clearCand = selectAddsCandidates(tree);
   for (int attempt = 0;; ++attempt) {
-    if (int rc = selTimer_.start(s)) return rc;
-    GATH_TRY(gat_fill_u32(out.qcount.as<uint32_t>(), 0, nq, s), "batch reset");
-    GATH_TRY(gat_fill_u32(ctr, 0, 16, s), "batch reset");
-    if (int rc = enqueueTreeSelect(tree, nq, nullptr)) return rc;
-    GATH_TRY(gat_scan_u64(cand_.as<uint64_t>(), nq, out.qbase.as<uint64_t>(), reinterpret_cast<uint64_t*>(ctr + 2),
-                          tiles_.as<uint64_t>(), s),
+    if (int rc = out.pairs.reserve(size_t(pairsCap_) * 8)) return rc;
+    uint32_t* const spans[2] = {ctr, cand_.as<uint32_t>()};
+    const int64_t lens[2] = {12, clearCand ? int64_t(nq) * 2 : 0};
+    GATH_TRY(gat_stage_in(devBoxes_.get(), hostStage_.get(), int64_t(bytes), 2, spans, lens, ctr + 12, s),
+             "box upload");
+    if (int rc = enqueueTreeSelect(tree, nq, nullptr, clearCand, walkTasks_)) return rc;
+    GATH_TRY(gat_direct_regions(cand_.as<uint64_t>(), nq, out.qbase.as<uint64_t>(), out.qcount.as<uint32_t>(), ctr, s),
              "region scan");
-    if (int rc = selTimer_.stop(s)) return rc;
-    GATH_TRY(gat_memcpy_d2h(countersHost_.get(), counters_.get(), 64, s), "counter readback");
+    GATH_TRY(gat_direct_refine(&store_, lq_.as<uint32_t>(), reinterpret_cast<const uint64_t*>(ctr), lqCap_,
+                               directExpected_ > 0 ? directExpected_ : int64_t(nq) * 64,
+                               tree.nodes.as<gat_tree_node>(), tree.nnodes, devBoxes_.as<float>(), nq,
+                               out.qbase.as<uint64_t>(), out.qcount.as<uint32_t>(), out.pairs.as<int32_t>(), pairsCap_,
+                               s),
+             "range refine");
+    GATH_TRY(gat_direct_finish(ctr, out.qcount.as<uint32_t>(), out.qbase.as<uint64_t>(), nq,
+                               directHost_.as<uint32_t>(), s),
+             "count readback");
     if (int rc = stream_.sync()) return rc;
     if (ch[4] & GAT_STATUS_STACK) {
       gath_set_error("batched range: traversal stack exceeded");
       return GAT_ERR_STATE;
     }
-    if (u64(0) <= uint64_t(lqCap_)) break;
-    if (attempt > 0 || u64(0) >= uint64_t(UINT32_MAX)) {
+    const bool entriesFit = u64(0) <= uint64_t(lqCap_);
+    if (entriesFit && u64(2) <= uint64_t(pairsCap_)) break;
+    if (attempt > 1 || u64(0) >= uint64_t(UINT32_MAX)) {
       gath_set_error("batched range: %llu (leaf, query) entries do not fit", (unsigned long long)u64(0));
       return GAT_ERR_CAPACITY;
     }
-    lqCap_ = int64_t(u64(0) + u64(0) / 4 + 1024);
-    if (int rc = lq_.reserve(size_t(lqCap_) * 8)) return rc;
+    if (!entriesFit) {
+      lqCap_ = int64_t(u64(0) + u64(0) / 4 + 1024);
+      if (int rc = lq_.reserve(size_t(lqCap_) * 8)) return rc;
+    }
+    // The candidate total covers the entries past the list's end too.
+    if (u64(2) > uint64_t(pairsCap_)) pairsCap_ = int64_t(u64(2) + u64(2) / 4 + 1024);
   }
-  float selMs = 0;
-  if (int rc = selTimer_.elapsed(&selMs)) return rc;
-  const int64_t ntasks = int64_t(u64(0));
-  const int64_t cand = int64_t(u64(2));
-  if (pairsCap_ < cand || pairsCap_ == 0) pairsCap_ = cand + cand / 4 + 1024;
-  if (int rc = out.pairs.reserve(size_t(pairsCap_) * 8)) return rc;
-  if (int rc = directTasks_.reserve(size_t(std::max<int64_t>(lqCap_, 1)) * sizeof(gat_range_task))) return rc;
-  if (int rc = timer_.start(s)) return rc;
-  GATH_TRY(gat_leaf_tasks(lq_.as<uint32_t>(), reinterpret_cast<const uint64_t*>(ctr), lqCap_,
-                          tree.nodes.as<gat_tree_node>(), N, directTasks_.as<gat_range_task>(), s),
-           "leaf tasks");
-  GATH_TRY(gat_range_refine_pairs(&store_, directTasks_.as<gat_range_task>(), ntasks, devBoxes_.as<float>(), nq,
-                                  out.qbase.as<uint64_t>(), out.qcount.as<uint32_t>(), out.pairs.as<int32_t>(),
-                                  pairsCap_, s),
-           "range refine");
-  if (int rc = timer_.stop(s)) return rc;
   out.count.resize(size_t(nq));
   out.base.resize(size_t(nq));
-  GATH_TRY(gat_memcpy_d2h(out.count.data(), out.qcount.get(), size_t(nq) * 4, s), "count readback");
-  GATH_TRY(gat_memcpy_d2h(out.base.data(), out.qbase.get(), size_t(nq) * 8, s), "region readback");
-  if (int rc = stream_.sync()) return rc;
-  if (int rc = timer_.elapsed(&out.kernelMs)) return rc;
-  out.selectMs = selMs;
+  std::memcpy(out.count.data(), ch + 32, size_t(nq) * 4);
+  std::memcpy(out.base.data(), ch + 32 + ((nq + 1) & ~1), size_t(nq) * 8);
+  directExpected_ = int64_t(u64(0));
+  out.selectMs = double(u64(14) - u64(12)) / clockKhz_;
+  out.kernelMs = float(double(u64(16) - u64(14)) / clockKhz_);
   out.refineMs = out.kernelMs;
   out.hostStale = false;
   out.runIndexed = false;
   out.runTotal = 0;
-  out.leafQueries = ntasks;
-  out.taskNum = ntasks;
-  out.candidates = cand;
+  out.leafQueries = int64_t(u64(0));
+  out.taskNum = out.leafQueries;
+  out.candidates = int64_t(u64(2));
   out.workItems = 0;
   out.pairTotal = 0;
   for (int q = 0; q < nq; ++q) out.pairTotal += out.count[size_t(q)];
+  out.uploadMs = now_ms() - t0;
   return GAT_OK;
 }
 
@@ -708,6 +730,14 @@ static float clamped_area(const MBB& b) {
 // any blocks past its chunks.  Rectangles under four blocks of area are not
 // looked at (a thin one among them keeps one task: slower, never wrong).
 int RangeEngine::uploadBoxes(const DeviceTree* tree, const MBB* bounds, int nq) {
+  size_t bytes = 0;
+  if (int rc = stageBoxes(tree, bounds, nq, &bytes)) return rc;
+  GATH_TRY(gat_memcpy_h2d(devBoxes_.get(), hostStage_.get(), bytes, stream_.get()), "box upload");
+  return GAT_OK;
+}
+
+// The host side of the upload: the layout in pinned memory and its used size.
+int RangeEngine::stageBoxes(const DeviceTree* tree, const MBB* bounds, int nq, size_t* used) {
   static_assert(sizeof(MBB) == 16, "MBB must be four packed floats");
   const BoxLayout lay = boxLayout(nq);
   const size_t bytes = lay.bytes;
@@ -731,6 +761,7 @@ int RangeEngine::uploadBoxes(const DeviceTree* tree, const MBB* bounds, int nq) 
   for (int b = 0; b < 256; ++b) start[b + 1] += start[b];
   for (int q = 0; q < nq; ++q) order[start[key[q]]++] = uint32_t(q);
   size_t upload = lay.order + size_t(nq) * 4;
+  walkTasks_ = 0;
   if (tree && tree->startLevel > 0) {
     auto* counts = reinterpret_cast<uint32_t*>(h + lay.ntasks);
     auto* tasks = reinterpret_cast<uint32_t*>(h + lay.tasks);
@@ -761,12 +792,14 @@ int RangeEngine::uploadBoxes(const DeviceTree* tree, const MBB* bounds, int nq) 
     counts[0] = uint32_t(n);  // tasks
     counts[1] = uint32_t(i);  // the order entries they cover
     upload = lay.tasks + n * 8;
+    walkTasks_ = int64_t(n);
   }
-  GATH_TRY(gat_memcpy_h2d(devBoxes_.get(), h, upload, stream_.get()), "box upload");
+  *used = upload;
   return GAT_OK;
 }
 
-int RangeEngine::enqueueTreeSelect(const DeviceTree& tree, int nq, uint32_t* nodeCount, bool candCleared) {
+int RangeEngine::enqueueTreeSelect(const DeviceTree& tree, int nq, uint32_t* nodeCount, bool candCleared,
+                                   int64_t walkTasks) {
   void* s = stream_.get();
   uint32_t* ctr = counters_.as<uint32_t>();
   auto* total = reinterpret_cast<uint64_t*>(ctr);
@@ -793,7 +826,7 @@ int RangeEngine::enqueueTreeSelect(const DeviceTree& tree, int nq, uint32_t* nod
                                tree.startBlock,
                                reinterpret_cast<const uint32_t*>(d + lay.tasks),
                                reinterpret_cast<const uint32_t*>(d + lay.ntasks),
-                               int64_t(lay.tasksCap)};
+                               walkTasks >= 0 ? walkTasks : int64_t(lay.tasksCap)};
     // Several tasks add to one rectangle's candidate count.
     if (tree.startLevel > 0 && !candCleared)
       GATH_TRY(gat_fill_u32(cand_.as<uint32_t>(), 0, int64_t(nq) * 2, s), "batch reset");
@@ -965,11 +998,9 @@ int RangeEngine::runTree(const DeviceTree& tree, const MBB* bounds, int nq, Rang
   out.kernelMs = out.refineMs = 0;
   if (nq == 0) return GAT_OK;
   const double t0 = now_ms();
-  if (int rc = uploadBoxes(&tree, bounds, nq)) return rc;
   const int64_t N = tree.nnodes;
   if (nq <= directMaxQueries) {
     // Direct form: workspace sized by the batch only.
-    if (int rc = tiles_.reserve(size_t(gat_scan_tiles(nq)) * 8)) return rc;
     if (int rc = cand_.reserve(size_t(nq) * 8)) return rc;
     if (int rc = out.qbase.reserve(size_t(nq) * 8)) return rc;
     if (int rc = out.qcount.reserve(size_t(nq) * 4)) return rc;
@@ -979,10 +1010,9 @@ int RangeEngine::runTree(const DeviceTree& tree, const MBB* bounds, int nq, Rang
       lqCap_ = std::max<int64_t>(int64_t(nq) * 16, 1 << 16);
       if (int rc = lq_.reserve(size_t(lqCap_) * 8)) return rc;
     }
-    const int rc = runDirect(tree, nq, out);
-    out.uploadMs = now_ms() - t0;
-    return rc;
+    return runDirect(tree, bounds, nq, out);
   }
+  if (int rc = uploadBoxes(&tree, bounds, nq)) return rc;
   out.runIndexed = runIndexed;
   const size_t tileBytes = size_t(std::max(2 * gat_scan_tiles(N) * 4, gat_scan_tiles(nq) * 8));
   if (nodeCount_.size() < size_t(N) * 4 || tiles_.size() < tileBytes || cand_.size() < size_t(nq) * 8 ||

@@ -87,6 +87,12 @@ struct RangeBatch {
 
  private:
   mutable DeviceBuffer digestDev_;  // digests(): kept, since a free waits for the device
+  // fetchCompact of up to kGatherBytes of pairs: gathered on the device into
+  // pinned memory in one launch pair.  Larger ones go by a copy per query (or
+  // per batch): the gather would hold as much pinned memory as the result.
+  static constexpr size_t kGatherBytes = size_t(32) << 20;
+  DeviceBuffer gatherAt_;
+  PinnedBuffer gatherHost_;
 };
 
 // Device copy of an index's tree for the batched form: gat_tree_node in
@@ -241,6 +247,7 @@ class RangeEngine {
     size_t order = 0, ntasks = 0, tasks = 0, bytes = 0, tasksCap = 0;
   };
   static BoxLayout boxLayout(int nq);
+  int stageBoxes(const DeviceTree* tree, const MBB* bounds, int nq, size_t* bytes);
   int uploadBoxes(const DeviceTree* tree, const MBB* bounds, int nq);
   int enqueueSelect(const DeviceTree& tree, int nq, RangeBatch& out);
   // The selection kernel for the tree's kind (nodeCount may be null).  The
@@ -249,12 +256,15 @@ class RangeEngine {
   static bool selectAddsCandidates(const DeviceTree& tree) {
     return !tree.flat() && !tree.implicit() && tree.startLevel > 0;
   }
-  int enqueueTreeSelect(const DeviceTree& tree, int nq, uint32_t* nodeCount, bool candCleared = false);
+  // walkTasks: the walk tasks staged for this batch, or -1 for as many as the
+  // buffer holds (a captured launch serves batches with other numbers).
+  int enqueueTreeSelect(const DeviceTree& tree, int nq, uint32_t* nodeCount, bool candCleared = false,
+                        int64_t walkTasks = -1);
   int enqueueJoin(const DeviceTree& tree, int nq, RangeBatch& out);
   int readCounters(int nq, RangeBatch& out);
   bool countersFit() const;
   int finishCounters(RangeBatch& out, bool replay);
-  int runDirect(const DeviceTree& tree, int nq, RangeBatch& out);
+  int runDirect(const DeviceTree& tree, const MBB* bounds, int nq, RangeBatch& out);
   void dropGraph();
 
   DeviceBuffer xy_, id_, pid_;
@@ -267,10 +277,14 @@ class RangeEngine {
 
   // Batched-form workspace.  counters_ (uint32 words): [0,1] selected entries,
   // [2,3] candidate total, [4] status, [5] list total, [6] work items,
-  // [8,9] result pairs, [10,11] run-indexed region total.
-  DeviceBuffer nodeCount_, lqRank_, nodeOff_, tiles_, cand_, lq_, qlist_, items_, counters_, directTasks_;
+  // [8,9] result pairs, [10,11] run-indexed region total; direct form: [12,13]
+  // and [14,15] the clock at the batch's start and after its selection.
+  DeviceBuffer nodeCount_, lqRank_, nodeOff_, tiles_, cand_, lq_, qlist_, items_, counters_;
   DeviceBuffer itemBase_, itemTiles_;  // run-indexed refine: item regions and their scan scratch
-  PinnedBuffer countersHost_;
+  PinnedBuffer countersHost_, directHost_;
+  int64_t walkTasks_ = 0;       // walk tasks stageBoxes last laid out
+  int64_t directExpected_ = 0;  // entries of the last direct batch
+  int32_t clockKhz_ = 0;
   int64_t lqCap_ = 0, qlistCap_ = 0, itemsCap_ = 0, pairsCap_ = 0;
   EventTimer selTimer_, refineTimer_;
   bool timeRefine_ = false;

@@ -569,6 +569,55 @@ int gat_morton_select(const uint32_t* cell_words_dev, int32_t total_level, int64
 int gat_leaf_tasks(const uint32_t* leaf_query_dev, const uint64_t* lq_total_dev, int64_t lq_capacity,
                    const gat_tree_node* nodes_dev, int64_t nnodes, gat_range_task* tasks_dev, void* stream);
 
+/* A run of result pairs of the run-indexed refine: `count` pairs of query q
+ * at pairs[first ...]. */
+typedef struct gat_range_run {
+  uint32_t q;
+  uint32_t count;
+  uint64_t first;
+} gat_range_run;
+
+/* The direct form as one chain on the device (no reference counterpart), for
+ * callers whose batches are bound by launches: gat_stage_in, a selection
+ * (node_qcount and lq_rank null), gat_direct_regions, gat_direct_refine,
+ * gat_direct_finish.
+ *
+ * gat_stage_in copies `bytes` (a multiple of 4) from pinned host memory to dst,
+ * clears up to 4 spans of 32-bit words, and writes the device's wall clock to
+ * stamp_dev[0..1] (null: not).
+ * gat_direct_regions: qbase_dev = the exclusive sum of cand_dev, qcount_dev = 0,
+ * the total to counters_dev[2..3], the wall clock to counters_dev[14..15].
+ * gat_direct_refine: the pairs of every (leaf, rectangle) entry, rectangle q's
+ * filling its region from qbase_dev[q] on (at most `capacity` pairs in all),
+ * qcount_dev[q] of them; `expected` is the number of entries the grid is sized
+ * for, any number is refined.
+ * gat_direct_finish writes gat_direct_words(nq) words to pinned host memory:
+ * [0, 16) counters_dev, [16, 18) the wall clock, [32, 32 + nq) the counts, then
+ * from the next even word the regions (uint64 each).
+ * gat_wall_clock_khz: the rate of those clocks. */
+int gat_stage_in(void* dst_dev, const void* src_pinned, int64_t bytes, int32_t nspans, uint32_t* const* spans_dev,
+                 const int64_t* words, uint32_t* stamp_dev, void* stream);
+int gat_direct_regions(const uint64_t* cand_dev, int64_t nq, uint64_t* qbase_dev, uint32_t* qcount_dev,
+                       uint32_t* counters_dev, void* stream);
+int gat_direct_refine(const gat_point_store* store, const uint32_t* leaf_query_dev, const uint64_t* lq_total_dev,
+                      int64_t lq_capacity, int64_t expected, const gat_tree_node* nodes_dev, int64_t nnodes,
+                      const float* boxes_dev, int64_t nqueries, const uint64_t* qbase_dev, uint32_t* qcount_dev,
+                      int32_t* pairs_dev, int64_t capacity, void* stream);
+int64_t gat_direct_words(int64_t nq);
+int gat_direct_finish(const uint32_t* counters_dev, const uint32_t* qcount_dev, const uint64_t* qbase_dev, int64_t nq,
+                      uint32_t* out_pinned, void* stream);
+int gat_wall_clock_khz(int32_t* khz);
+
+/* A batch's pairs query after query in `out` (device or pinned host memory,
+ * `capacity` pairs; what lies past it is left out): from per-query regions
+ * (qbase_dev; runs_dev null) or run-indexed pairs (runs_dev, nruns of them;
+ * qbase_dev null), qcount_dev[q] pairs of query q, of the `npairs` that pairs_dev
+ * holds.  at_dev: nq entries of scratch.  Within a query the runs come in no
+ * order. */
+int gat_gather_pairs(const int32_t* pairs_dev, int64_t npairs, const uint64_t* qbase_dev,
+                     const gat_range_run* runs_dev, int64_t nruns, const uint32_t* qcount_dev, int64_t nq,
+                     uint64_t* at_dev, int32_t* out, int64_t capacity, void* stream);
+
 /* Groups the selected (leaf, query) entries by leaf.  Entry i, of leaf L and
  * rank r = lq_rank[i] (from the selection), puts the rectangle's id (one
  * uint32) at qlist[node_off[2*L] + r]; every qb-th rank starts a work item
@@ -580,14 +629,6 @@ int gat_leaf_scatter(const uint32_t* leaf_query_dev, const uint64_t* lq_total_de
                      const uint32_t* node_qcount_dev, const uint32_t* lq_rank_dev, int32_t qb, int64_t nqueries,
                      uint32_t* qlist_dev, int64_t qlist_capacity, uint32_t* items_dev, int64_t items_capacity,
                      void* stream);
-
-/* A run of result pairs of the run-indexed refine: `count` pairs of query q
- * at pairs[first ...]. */
-typedef struct gat_range_run {
-  uint32_t q;
-  uint32_t count;
-  uint64_t first;
-} gat_range_run;
 
 /* The leaf-major refine with the output laid out by work item (no reference
  * counterpart), in three calls on one stream:

@@ -1,0 +1,48 @@
+"""The direct form's device chain and the gathered readback: batches of every
+size around a wave's four entries and the regions kernel's 256 threads, a batch
+that outgrows the buffers' capacities, leaves of more points than one round
+takes, both id packings' store, rectangles that select nothing; counts, digests
+and pair sets against the plain path and inclusive brute force."""
+import numpy as np
+import pytest
+
+import oracle as O
+from gat_amd import api, workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _rects(rng, n):
+    c = rng.random((n, 2)).astype(np.float32)
+    s = np.exp(rng.uniform(np.log(1e-4), np.log(0.3), n)).astype(np.float32)
+    r = np.concatenate([c - s[:, None] / 2, c + s[:, None] / 2], 1).astype(np.float32)
+    if n > 2:
+        r[0] = [2, 2, 3, 3]  # outside the domain
+        r[1] = [0.5, 0.5, 0.4, 0.4]  # inverted
+    return r
+
+
+@pytest.mark.parametrize("nq", [1, 3, 4, 5, 255, 256, 257, 700])
+@pytest.mark.parametrize("leaf", [64, 700])  # one round of 256 points per entry, and three
+def test_direct_chain(gpu, nq, leaf):
+    rng = np.random.default_rng(nq)
+    db = api.synth_walks(5, api.synth_lengths(5, 1500, "uniform", 1, 90, 1, 90), step_sigma=4e-3)
+    rects = _rects(rng, nq)
+    want_c, want_d = O.brute_range(db, rects, "digest", nthreads=8)
+    for ix in (api.GridIndex(W.UNIT_BOX, 0.02, leaf), api.StigIndex(leaf), api.FsgIndex(W.UNIT_BOX, 0.05)):
+        ix.build(db).set_batch_params(32, 1 << 20)
+        plain = ix.range_pairs(rects)
+        pc, pd, pp = plain.counts(), plain.digests(), plain.per_query()
+        if not isinstance(ix, api.GridIndex):  # the GT-quadtree's touching test is strict
+            assert (pc == want_c).all() and (pd == want_d).all()
+        for _ in range(2):  # the first call grows the buffers, the second finds them
+            res = ix.range_batched(rects)
+            assert res.pairs_total == plain.pairs_total and res.candidates == plain.candidates
+            assert (res.counts() == pc).all() and (res.digests() == pd).all()
+            for a, b in zip(res.per_query(), pp):
+                assert sorted(map(tuple, a.tolist())) == sorted(map(tuple, b.tolist()))
+        # Leaf-major batches read back through their runs.
+        res = ix.set_batch_params(8, 0).range_batched(rects)
+        assert (res.counts() == pc).all()
+        for a, b in zip(res.per_query(), pp):
+            assert sorted(map(tuple, a.tolist())) == sorted(map(tuple, b.tolist()))
