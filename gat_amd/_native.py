@@ -83,6 +83,12 @@ HIP_FUNCS = {
     "gat_edr_survivor_lists": (INT, [P, P, P, I64, I32, P, P, P, P, P]),
     "gat_edr_filter": (INT, [P, I32, P, I32, F64, P, I64, P, P]),
     "gat_edr_filter_grid": (INT, [P, I32, P, I32, P, F64, P, I64, P, P]),
+    "gat_edr_filter_grid_add": (INT, [P, I32, P, I32, P, F64, P, I64, P, P, P]),
+    "gat_edr_stage_queries": (INT, [P, I64, P, P, P, I32, I64, P, P, I64, P, P, P, I64, P, P]),
+    "gat_edr_bucket": (INT, [P, I64, P, I64, P, P, P, P, P, I32, P, P, P, I32, I32, F64, I32, I32, P, P, P]),
+    "gat_edr_pairs": (INT, [P, P, I64, P, P, P, P, I32, P, P, P, I32, I32, F64, I32, P, P, P, P]),
+    "gat_edr_length_table": (INT, [P, I32, P, P]),
+    "gat_edr_merge": (INT, [P, I32, P, I32, P, I32, P, P, P, P, I64, I32, I32, P, P, P, P, P, P]),
     "gat_edr_mismatch_table": (INT, [I32, P, P]),
     "gat_edr_pack_trajectories": (INT, [P, P, P, P, I32, I64, P, P, P]),
     "gat_edr_topk": (INT, [P, I32, P, I32, P, I32, P, P, P, P, P, I32, I32, P, P, P, P]),

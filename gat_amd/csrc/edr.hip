@@ -21,13 +21,13 @@ constexpr int kMaxLen = GAT_MAX_TRAJ_LEN;
 
 // The handler's stores carry no padding and its lengths are known on the
 // device only, so every column load is checked and the row buffer is sized
-// for the longest trajectory (4.4 KB of LDS: 32 waves per CU).
+// for the longest trajectory (8.8 KB of LDS: 16 waves per CU).
 __global__ __launch_bounds__(64, 4) void edr_plain_kernel(
     int ntasks, const gat_edr_task* __restrict__ tasks, const float2* __restrict__ qxy, const int32_t* __restrict__ qoff,
     const int32_t* __restrict__ qlen, const float2* __restrict__ cxy, const int64_t* __restrict__ coff,
     const int32_t* __restrict__ clen, float u, int32_t* __restrict__ result) {
-  constexpr int kOff = 64;
-  __shared__ int16_t above[kMaxLen + 2 * 64 + edr::kBlk][1];
+  // Columns from -63 on, the first a feed reads (column 1) 16-byte aligned.
+  __shared__ __align__(16) int32_t above[edr::kOff64 + kMaxLen + 64 + edr::kBlk][1];
   const int t = blockIdx.x;
   const int l = threadIdx.x;
   if (t >= ntasks) return;
@@ -48,7 +48,7 @@ __global__ __launch_bounds__(64, 4) void edr_plain_kernel(
   }
   const float2* R = query_rows ? qxy + qoff[task.qid] : cxy + coff[t];
   const float2* C = query_rows ? cxy + coff[t] : qxy + qoff[task.qid];
-  for (int i = l; i < m + 2 * 64 + edr::kBlk; i += 64) above[i][0] = int16_t(i - kOff);
+  for (int i = l; i < m + edr::kOff64 + 64 + edr::kBlk; i += 64) above[i][0] = i - edr::kOff64;
   const int ns[1] = {n}, ms[1] = {m};
   bool mine = false;
   const int res = edr::sweep_pairs<64, true>(R, n, C, m, n, m, ns, ms, u, above, 0, l, &mine);

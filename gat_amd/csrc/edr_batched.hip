@@ -42,6 +42,12 @@ __device__ __forceinline__ int32_t take_window(const int32_t* window, int32_t& n
 }
 
 
+__device__ __forceinline__ int64_t uniform64(int64_t v) {
+  const uint32_t lo = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(v))));
+  const uint32_t hi = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(v) >> 32))));
+  return int64_t(uint64_t(lo) | (uint64_t(hi) << 32));
+}
+
 // Issue priority of a wave by the length of its job's schedule in steps:
 // the longest pairs of a batch set its end, so their waves go first.
 __device__ __forceinline__ void job_priority(int64_t steps) {
@@ -49,6 +55,26 @@ __device__ __forceinline__ void job_priority(int64_t steps) {
   else if (steps >= 8192) __builtin_amdgcn_s_setprio(2);
   else if (steps >= 4096) __builtin_amdgcn_s_setprio(1);
   else __builtin_amdgcn_s_setprio(0);
+}
+
+// Without a job list (jobs null) a launch runs pairs 0 .. *live - 1 one per job,
+// in the order given, or none when *live exceeds the npairs the array holds;
+// *cells gets their cell count and *stamp the time the launch began.
+struct RawPairs {
+  const unsigned long long* live;
+  unsigned long long* cells;
+  uint32_t* stamp;
+};
+
+__device__ __forceinline__ int32_t raw_jobs(const RawPairs& raw, int64_t npairs) {
+  const unsigned long long n = *raw.live;
+  return n > (unsigned long long)npairs ? 0 : int32_t(n);
+}
+
+__device__ __forceinline__ void store_clock(uint32_t* p) {
+  const uint64_t t = wall_clock64();
+  p[0] = uint32_t(t);
+  p[1] = uint32_t(t >> 32);
 }
 
 // SEG lanes per pair: 16 (four pairs per wave) or 64 (one pair per wave, a
@@ -65,27 +91,30 @@ __global__ __launch_bounds__(64, (MAXM >= 2048 && SEG == 16) ? 2 : 4) void edr_w
                                                       const int32_t* __restrict__ qlen, const float2* __restrict__ cxy,
                                                       const int64_t* __restrict__ coff,
                                                       const int32_t* __restrict__ clen, float u,
-                                                      int32_t* __restrict__ out) {
+                                                      int32_t* __restrict__ out, RawPairs raw) {
   constexpr int kSeg = SEG;        // lanes per pair
   constexpr int kSegs = 64 / SEG;  // pairs per wave
   // Row above the current strip, E[r0][c] = D[r0][c] - r0, at [c + kOff][segment]
   // for columns 2 - SEG .. MAXM + SEG + kBlk - 1 (the lanes' look-behind, the
   // columns, and the last blocks' overrun).  Segments interleave, so one
   // segment's consecutive columns are 2 * kSegs bytes apart and each step's
-  // feed is a load of its own.
-  constexpr int kOff = SEG;
-  constexpr int kRows = MAXM + 2 * SEG + kBlk;
-  __shared__ int16_t above[kRows][kSegs];
+  // feed is a load of its own; a 64-lane pair's are 32 bits each, read four at
+  // a time.
+  constexpr int kOff = edr::kRowOff<SEG>;
+  constexpr int kRows = kOff + MAXM + SEG + kBlk;
+  __shared__ __align__(16) edr::RowValue<SEG> above[kRows][kSegs];
   const int lane = threadIdx.x;
   const int seg = lane / kSeg;
   const int l = lane & (kSeg - 1);
-  jobs += take_window(window, njobs);
+  if (jobs) jobs += take_window(window, njobs);
+  else njobs = raw_jobs(raw, npairs);
+  if (raw.stamp && blockIdx.x == 0 && lane == 0) store_clock(raw.stamp);
   for (;;) {
     int ji = 0;
     if (lane == 0) ji = atomicAdd(counter, 1);
     ji = __builtin_amdgcn_readfirstlane(ji);
     if (ji < 0 || ji >= njobs) break;  // a counter that was not cleared hands out nothing
-    const Job job = jobs[ji];
+    const Job job = jobs ? jobs[ji] : Job{ji, 1};
     // Jobs and pairs that point outside their arrays are skipped.
     const bool live = seg < job.count && job.first >= 0 && int64_t(job.first) + seg < npairs;
     int n = 0, m = 0;
@@ -94,7 +123,8 @@ __global__ __launch_bounds__(64, (MAXM >= 2048 && SEG == 16) ? 2 : 4) void edr_w
     // (loads further back than the padding are replaced by NaN, below).
     const float2* R = cxy;
     const float2* C = cxy + kPad;
-    bool valid = false;
+    int64_t row_off = 0, col_off = kPad;
+    bool valid = false, query_rows = false;
     if (live) {
       const int2 pr = pairs[job.first + seg];
       const bool ids_ok = pr.x >= 0 && pr.x < nqueries && pr.y >= 0 && pr.y < ncands;
@@ -104,17 +134,28 @@ __global__ __launch_bounds__(64, (MAXM >= 2048 && SEG == 16) ? 2 : 4) void edr_w
       if (valid) {
         // Rows are the shorter trajectory; on equal lengths the query
         // (Grid.cpp:1234-1247).
-        if (nc >= nq) {
-          R = qxy + qoff[pr.x]; n = nq; C = cxy + coff[pr.y]; m = nc;
-        } else {
-          R = cxy + coff[pr.y]; n = nc; C = qxy + qoff[pr.x]; m = nq;
-        }
+        query_rows = nc >= nq;
+        row_off = query_rows ? qoff[pr.x] : coff[pr.y];
+        col_off = query_rows ? coff[pr.y] : qoff[pr.x];
+        R = (query_rows ? qxy : cxy) + row_off;
+        C = (query_rows ? cxy : qxy) + col_off;
+        n = query_rows ? nq : nc;
+        m = query_rows ? nc : nq;
       }
+    }
+    if constexpr (kSegs == 1) {
+      // One pair for the whole wave: its pointers and lengths are scalars.
+      n = __builtin_amdgcn_readfirstlane(n);
+      m = __builtin_amdgcn_readfirstlane(m);
+      const bool q_rows = __builtin_amdgcn_readfirstlane(query_rows ? 1 : 0) != 0;
+      R = (q_rows ? qxy : cxy) + uniform64(row_off);
+      C = (q_rows || !valid ? cxy : qxy) + uniform64(col_off);
     }
     // Wave-uniform extents: the largest column count and strip count of the job.
     const int m0 = __builtin_amdgcn_readlane(m, 0), m1 = __builtin_amdgcn_readlane(m, 16);
     const int m2 = __builtin_amdgcn_readlane(m, 32), m3 = __builtin_amdgcn_readlane(m, 48);
     const int mmax = max(max(m0, m1), max(m2, m3));
+    if (raw.cells && l == 0 && valid) atomicAdd(raw.cells, (unsigned long long)n * (unsigned long long)m);
     const int n0 = __builtin_amdgcn_readlane(n, 0), n1 = __builtin_amdgcn_readlane(n, 16);
     const int n2 = __builtin_amdgcn_readlane(n, 32), n3 = __builtin_amdgcn_readlane(n, 48);
     const int nmax = max(max(n0, n1), max(n2, n3));
@@ -122,9 +163,9 @@ __global__ __launch_bounds__(64, (MAXM >= 2048 && SEG == 16) ? 2 : 4) void edr_w
     job_priority(int64_t(strips) * (mmax + kSeg - 1) * 2);
     // Row 0: E[0][c] = c, as far as the job's last block reads.  (Kept rolled:
     // unrolled, its length grows with MAXM and so does the register count.)
-    const int used = min(kRows, mmax + 2 * SEG + kBlk);
+    const int used = min(kRows, kOff + mmax + SEG + kBlk);
 #pragma unroll 2
-    for (int i = l; i < used; i += kSeg) above[i][seg] = int16_t(i - kOff);
+    for (int i = l; i < used; i += kSeg) above[i][seg] = edr::RowValue<SEG>(i - kOff);
     int ns[kSegs], ms[kSegs];
     if constexpr (kSegs == 4) {
       ns[0] = n0; ns[1] = n1; ns[2] = n2; ns[3] = n3;
@@ -194,7 +235,7 @@ __device__ __forceinline__ void pipe_pair(PipeShared<MAXM, W>& sh, const float2*
   // previous strip.
   const int P = max(nblocks, W * kLag);
   const int kend = ((strips - 1) / W) * P + ((strips - 1) % W) * kLag + nblocks;
-  job_priority(int64_t(kend) * kBlk * 2);
+  __builtin_amdgcn_s_setprio(3);  // these pairs set the batch's end
   edr::LaneRows<K> rows;
   rows.start();
   int s = wv, start = wv * kLag;
@@ -213,7 +254,7 @@ __device__ __forceinline__ void pipe_pair(PipeShared<MAXM, W>& sh, const float2*
   int16_t* own = sh.rows[wv];
   auto begin_strip = [&]() __attribute__((always_inline)) {
     rows.start();
-    const float4 box = edr::segment_box<64>(rows.load(R, n, s * kRows + l * K));
+    const float4 box = edr::segment_box<64>(rows.template load<true>(R, n, s * kRows + l * K));
     auto touches = [&](int c) __attribute__((always_inline)) -> uint64_t {
       return __ballot(c < nchunks && edr::may_touch(box, sh.chunk[min(c, S::kChunks - 1)], u));
     };
@@ -322,46 +363,54 @@ __global__ __launch_bounds__(64 * W) void edr_pipe_kernel(const int2* __restrict
                                                           const float2* __restrict__ cxy,
                                                           const int64_t* __restrict__ coff,
                                                           const int32_t* __restrict__ clen, float u,
-                                                          int32_t* __restrict__ out) {
+                                                          int32_t* __restrict__ out, RawPairs raw) {
   using S = PipeShared<MAXM, W>;
   __shared__ S sh;
   const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / 64);
   const int l = threadIdx.x & 63;
-  jobs += take_window(window, njobs);
+  if (jobs) jobs += take_window(window, njobs);
+  else njobs = raw_jobs(raw, npairs);
+  if (raw.stamp && blockIdx.x == 0 && threadIdx.x == 0) store_clock(raw.stamp);
   for (int i = threadIdx.x; i < S::kLen; i += 64 * W) sh.rows[W][i] = int16_t(i - S::kOff);
   for (;;) {
     if (threadIdx.x == 0) sh.job_slot = atomicAdd(counter, 1);
     __syncthreads();
-    const int ji = sh.job_slot;
+    const int ji = __builtin_amdgcn_readfirstlane(sh.job_slot);
     __syncthreads();  // every wave has read the slot before the next job overwrites it
     if (ji < 0 || ji >= njobs) break;  // a counter that was not cleared hands out nothing
-    const Job job = jobs[ji];
+    const Job job = jobs ? jobs[ji] : Job{ji, 1};
     // One pair per job; everything below is uniform across the workgroup.
     const bool live = job.count >= 1 && job.first >= 0 && int64_t(job.first) < npairs;
     int n = 0, m = 0;
-    const float2* R = cxy;
-    const float2* C = cxy;
-    bool valid = false;
+    int64_t row_off = 0, col_off = 0;
+    bool valid = false, query_rows = false;
     if (live) {
       const int2 pr = pairs[job.first];
       const bool ids_ok = pr.x >= 0 && pr.x < nqueries && pr.y >= 0 && pr.y < ncands;
       const int nq = ids_ok ? qlen[pr.x] : 0, nc = ids_ok ? clen[pr.y] : 0;
       valid = nq >= 1 && nc >= 1 && nq <= MAXM && nc <= MAXM;
       if (valid) {
-        if (nc >= nq) {
-          R = qxy + qoff[pr.x]; n = nq; C = cxy + coff[pr.y]; m = nc;
-        } else {
-          R = cxy + coff[pr.y]; n = nc; C = qxy + qoff[pr.x]; m = nq;
-        }
+        query_rows = nc >= nq;
+        row_off = query_rows ? qoff[pr.x] : coff[pr.y];
+        col_off = query_rows ? coff[pr.y] : qoff[pr.x];
+        n = query_rows ? nq : nc;
+        m = query_rows ? nc : nq;
       }
     }
     if (!valid) {
       if (live && threadIdx.x == 0) out[job.first] = -1;
       continue;
     }
+    // One pair for the whole workgroup: its pointers and lengths are scalars.
+    n = __builtin_amdgcn_readfirstlane(n);
+    m = __builtin_amdgcn_readfirstlane(m);
+    const bool q_rows = __builtin_amdgcn_readfirstlane(query_rows ? 1 : 0) != 0;
+    const float2* R = (q_rows ? qxy : cxy) + uniform64(row_off);
+    const float2* C = (q_rows ? cxy : qxy) + uniform64(col_off);
+    if (raw.cells && threadIdx.x == 0) atomicAdd(raw.cells, (unsigned long long)n * (unsigned long long)m);
     // Stage the columns the blocks read, a box per chunk of 16.
     for (int i = int(threadIdx.x) - 64; i < m + 96; i += 64 * W) {
-      const float2 p = i >= 0 && i < m ? C[i] : edr::nan_point();
+      const float2 p = edr::point_or_nan(C, i, m);
       sh.cols[S::kColOff + i] = p;
       // 64 divides the stride and the start: a row of 16 lanes holds one chunk.
       const float4 box = edr::segment_box<16>(edr::grow(edr::empty_box(), p));
@@ -453,7 +502,9 @@ constexpr int kGridFilterWaves = 4;
 
 __global__ __launch_bounds__(64 * kGridFilterWaves) void edr_filter_grid_kernel(
     const float4* __restrict__ qbox, int32_t nq, const float4* __restrict__ cbox, int32_t nc, CandGrid gr, float u,
-    int2* __restrict__ out, uint64_t capacity, unsigned long long* __restrict__ count) {
+    int2* __restrict__ out, uint64_t capacity, unsigned long long* __restrict__ count,
+    uint32_t* __restrict__ stamp) {
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) store_clock(stamp);
   const int lane = threadIdx.x & 63;
   const int q = int(blockIdx.x) * kGridFilterWaves + int(threadIdx.x >> 6);
   if (q >= nq) return;  // the whole wave
@@ -584,16 +635,20 @@ constexpr int kTopkMax = 1024;
 constexpr int kLenBins = GAT_MAX_TRAJ_LEN + 1;     // lengths 0..GAT_MAX_TRAJ_LEN
 constexpr int kDistBins = 2 * GAT_MAX_TRAJ_LEN + 1;  // distances 0..n + m
 constexpr int kTopkBlock = 256;
+constexpr int kScanAhead = 8;                               // ids per thread in flight
+constexpr int kScanRound = kScanAhead * kTopkBlock;
+constexpr int kScanRounds = 16;
 
-// Index of c in the ascending sid[s0, s1), or -1.
-__device__ __forceinline__ int32_t survivor_index(const int32_t* __restrict__ sid, int32_t s0, int32_t s1, int32_t c) {
+// Index of c among the survivors s0 .. s1 - 1, or -1.
+template <class Survivors>
+__device__ __forceinline__ int32_t survivor_index(const Survivors& sv, int32_t s0, int32_t s1, int32_t c) {
   int32_t lo = s0, hi = s1;
   while (lo < hi) {
     const int32_t mid = lo + ((hi - lo) >> 1);
-    if (sid[mid] < c) lo = mid + 1;
+    if (sv.id(mid) < c) lo = mid + 1;
     else hi = mid;
   }
-  return (lo < s1 && sid[lo] == c) ? lo : -1;
+  return (lo < s1 && sv.id(lo) == c) ? lo : -1;
 }
 
 // Number of entries <= x in the ascending ids[0, n).
@@ -616,25 +671,53 @@ __device__ __forceinline__ int32_t topk_block_sum(int32_t v, int32_t* red) {
   return red[0] + red[1] + red[2] + red[3];
 }
 
-__global__ __launch_bounds__(kTopkBlock) void edr_topk_kernel(
-    const int32_t* __restrict__ ftable, int32_t w, const int32_t* __restrict__ qlen,
-    const int32_t* __restrict__ clen, int32_t nc, const int32_t* __restrict__ len_ids,
-    const int32_t* __restrict__ len_off, const int32_t* __restrict__ sstart, const int32_t* __restrict__ sid,
-    const int32_t* __restrict__ sdist, int32_t k, int32_t kk, int32_t* __restrict__ out_ids,
-    int32_t* __restrict__ out_dist, int32_t* __restrict__ status) {
-  __shared__ int32_t val[kLenBins];    // the query's all-mismatch value per candidate length
+// Survivors s0 .. s1 - 1 of a query, ascending by id: lists in global memory
+// (edr_lists_kernel), or gathered into LDS by edr_merge_kernel.
+struct GlobalSurvivors {
+  const int32_t* __restrict__ sid;
+  const int32_t* __restrict__ sdist;
+  static constexpr bool kInLds = false;
+  __device__ int32_t id(int32_t i) const { return sid[i]; }
+  __device__ int32_t dist(int32_t i) const { return sdist[i]; }
+};
+struct LdsSurvivors {
+  const unsigned long long* v;  // id << 32 | distance
+  static constexpr bool kInLds = true;
+  __device__ int32_t id(int32_t i) const { return int32_t(v[i] >> 32); }
+  __device__ int32_t dist(int32_t i) const { return int32_t(uint32_t(v[i])); }
+};
+
+// kByLength: ftable rows are indexed by the two lengths in either order
+// (gat_edr_length_table), so a query's values are one contiguous row.
+template <bool kByLength, class Survivors>
+__device__ __forceinline__ void topk_query(int q, const Survivors& sv, int32_t s0, int32_t s1,
+                                           const int32_t* __restrict__ ftable, int32_t w,
+                                           const int32_t* __restrict__ qlen, const int32_t* __restrict__ clen,
+                                           int32_t nc, const int32_t* __restrict__ len_ids,
+                                           const int32_t* __restrict__ len_off, int32_t k, int32_t kk,
+                                           int32_t* __restrict__ out_ids, int32_t* __restrict__ out_dist,
+                                           int32_t* __restrict__ status) {
+  // The query's all-mismatch value per candidate length (16 bits: four
+  // workgroups of the merge fit a CU); kNoValue for one outside 0..kDistBins - 1.
+  constexpr uint16_t kNoValue = 0xFFFF;
+  static_assert(kDistBins < kNoValue, "distances fit 16 bits");
+  __shared__ uint16_t val[kLenBins];
   __shared__ int32_t hist[kDistBins];  // candidates per distance
   __shared__ int32_t out_d[kTopkMax], out_i[kTopkMax];
   __shared__ int32_t red[kTopkBlock / 64];
-  __shared__ int32_t n_out, sh_T, sh_below, sh_nt;
-  const int q = blockIdx.x;
+  __shared__ int32_t n_out, sh_T, sh_below, sh_at, sh_nt, sh_ng;
+  __shared__ int32_t part_at[kScanAhead][kTopkBlock / 64];
   const int tid = threadIdx.x;
   const int a = qlen[q];
   if (a < 1 || a > GAT_MAX_TRAJ_LEN) {
     if (tid == 0) atomicOr(status, 4);
     return;
   }
-  for (int L = tid; L < kLenBins; L += kTopkBlock) val[L] = L >= 1 ? ftable[int64_t(min(a, L)) * w + max(a, L)] : 0;
+#pragma unroll 9
+  for (int L = tid; L < kLenBins; L += kTopkBlock) {
+    const int32_t v = kByLength ? ftable[int64_t(a) * w + L] : ftable[int64_t(min(a, L)) * w + max(a, L)];
+    val[L] = L < 1 ? 0 : v < 0 || v >= kDistBins ? kNoValue : uint16_t(v);
+  }
   for (int b = tid; b < kDistBins; b += kTopkBlock) hist[b] = 0;
   if (tid == 0) {
     n_out = 0;
@@ -642,19 +725,19 @@ __global__ __launch_bounds__(kTopkBlock) void edr_topk_kernel(
     sh_below = 0;
   }
   __syncthreads();
+#pragma unroll 8
   for (int L = 1 + tid; L < kLenBins; L += kTopkBlock) {
     const int32_t cnt = len_off[L + 1] - len_off[L];
     const int32_t v = val[L];
     if (cnt > 0) {
-      if (v < 0 || v >= kDistBins) atomicOr(status, 1);
+      if (v >= kDistBins) atomicOr(status, 1);
       else atomicAdd(&hist[v], cnt);
     }
   }
-  const int32_t s0 = sstart[q], s1 = sstart[q + 1];
   for (int32_t i = s0 + tid; i < s1; i += kTopkBlock) {
-    const int32_t c = sid[i];
+    const int32_t c = sv.id(i);
     const int32_t L = (c >= 0 && c < nc) ? clen[c] : 0;
-    const int32_t d = sdist[i];
+    const int32_t d = sv.dist(i);
     if (L < 1 || L > GAT_MAX_TRAJ_LEN || d < 0 || d >= kDistBins || val[L] >= kDistBins) {
       atomicOr(status, 1);
       continue;
@@ -688,6 +771,7 @@ __global__ __launch_bounds__(kTopkBlock) void edr_topk_kernel(
       if (acc + hist[b] >= kk) {
         sh_T = b;
         sh_below = acc;
+        sh_at = hist[b];
         break;
       }
       acc += hist[b];
@@ -700,141 +784,257 @@ __global__ __launch_bounds__(kTopkBlock) void edr_topk_kernel(
     if (tid == 0) atomicOr(status, 2);
     return;
   }
-  // The distance histogram is done with: its space now holds the lengths
-  // valued T (when they fit) and this query's survivor ids, ascending (when
-  // they fit), so survivor lookups stay in LDS.
-  constexpr int32_t kTlMax = 2048, kStMax = kDistBins - kTlMax;
-  int32_t* tl = hist;             // lengths whose value is T
-  int32_t* st = hist + kTlMax;    // staged survivor ids
+  // The distance histogram is done with; its space now holds the lists of the
+  // lengths valued T or less (their lengths, and where their entries start in
+  // the order below), the gathered ids, and this query's survivor ids where
+  // those lie in global memory.
   const int32_t ns = s1 - s0;
-  const bool staged = ns <= kStMax;
+  const int32_t pre = r + ns;
+  constexpr int32_t kLists = 1024, kGather = Survivors::kInLds ? kDistBins - 2 * kLists : 1024;
+  constexpr int32_t kStage = Survivors::kInLds ? 0 : kDistBins - 2 * kLists - kGather;
+  constexpr int32_t kEntriesMax = 64 * kTopkBlock;
+  int32_t* tl = hist;
+  int32_t* first = hist + kLists;
+  int32_t* g = hist + 2 * kLists;
+  int32_t* st = g + kGather;
+  const bool staged = ns <= kStage;
   if (tid == 0) sh_nt = 0;
   __syncthreads();
   if (staged)
-    for (int32_t i = tid; i < ns; i += kTopkBlock) st[i] = sid[s0 + i];
-  for (int L = 1 + tid; L < kLenBins; L += kTopkBlock)
-    if (val[L] == T && len_off[L + 1] > len_off[L]) {
-      const int32_t at = atomicAdd(&sh_nt, 1);
-      if (at < kTlMax) tl[at] = L;
-    }
+    for (int32_t i = tid; i < ns; i += kTopkBlock) st[i] = sv.id(s0 + i);
   __syncthreads();
-  const int32_t nt = sh_nt;
-  auto is_survivor = [&](int32_t c) -> bool {
-    if (ns == 0) return false;
-    if (!staged) return survivor_index(sid, s0, s1, c) >= 0;
+  // The survivor list's index of c, or -1.
+  auto survivor = [&](int32_t c) -> int32_t {
+    if (ns == 0) return -1;
+    if (!staged) return survivor_index(sv, s0, s1, c);
     int32_t lo = 0, hi = ns;
     while (lo < hi) {
       const int32_t mid = lo + ((hi - lo) >> 1);
-      if (hist[kTlMax + mid] < c) lo = mid + 1;
+      if (st[mid] < c) lo = mid + 1;
       else hi = mid;
     }
-    return lo < ns && hist[kTlMax + lo] == c;
+    return lo < ns && st[lo] == c ? s0 + lo : -1;
   };
-  // Every candidate below T: non-survivors by length, survivors by DP distance.
-  for (int L = 1 + tid; L < kLenBins; L += kTopkBlock) {
-    if (val[L] >= T) continue;
-    for (int32_t i = len_off[L], e = len_off[L + 1]; i < e; ++i) {
-      const int32_t c = len_ids[i];
-      if (is_survivor(c)) continue;
-      const int32_t pos = atomicAdd(&n_out, 1);
-      if (pos < kTopkMax) {
-        out_d[pos] = val[L];
-        out_i[pos] = c;
+  auto take = [&](int32_t d, int32_t c) {
+    const int32_t pos = atomicAdd(&n_out, 1);
+    if (pos < kTopkMax) {
+      out_d[pos] = d;
+      out_i[pos] = c;
+    }
+  };
+  // The r smallest ids at T.  Where T is common they lie among the first ids:
+  // about r * nc / (candidates at T) of them, read in order, 2,048 at a time,
+  // until r are found.  (Of 200,000 candidates a median of 20,000 lie at T: 500
+  // ids for 50 results, where the lists of T's lengths hold 3,300 entries to
+  // look through.)  Ids ordered by length can hide them further back; then the
+  // lists below take over.
+  bool scanned = false;
+  if (int64_t(r) * nc <= int64_t(kScanRound) * (kScanRounds / 4) * sh_at) {
+    int32_t have = 0;
+    const int32_t kept = n_out;
+    for (int32_t base = 0, round = 0; base < nc && have < r && round < kScanRounds; base += kScanRound, ++round) {
+      int32_t len[kScanAhead];
+#pragma unroll
+      for (int j = 0; j < kScanAhead; ++j) {
+        const int64_t c = int64_t(base) + j * kTopkBlock + tid;
+        len[j] = c < nc ? clen[c] : 0;
       }
+      uint64_t at[kScanAhead];
+#pragma unroll
+      for (int j = 0; j < kScanAhead; ++j) {
+        bool is = false;
+        if (len[j] >= 1 && len[j] <= GAT_MAX_TRAJ_LEN) {
+          const int32_t i = survivor(base + j * kTopkBlock + tid);
+          is = (i >= 0 ? sv.dist(i) : int32_t(val[len[j]])) == T;
+        }
+        at[j] = __ballot(is);
+        if (lane == 0) part_at[j][wv] = __popcll(at[j]);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kScanAhead; ++j)
+#pragma unroll
+        for (int x = 0; x < kTopkBlock / 64; ++x) {
+          if (x == wv && (at[j] >> lane & 1u)) {
+            const int32_t before = have + int32_t(__builtin_amdgcn_mbcnt_hi(
+                                              uint32_t(at[j] >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(at[j]), 0u)));
+            if (before < r) take(T, base + j * kTopkBlock + tid);
+          }
+          have += part_at[j][x];
+        }
+      __syncthreads();  // part_at is read
+    }
+    scanned = have >= r;
+    if (!scanned) {
+      if (tid == 0) n_out = kept;
+      __syncthreads();
     }
   }
+#pragma unroll 8
+  for (int L = 1 + tid; L < kLenBins; L += kTopkBlock)
+    if (val[L] <= (scanned ? T - 1 : T) && len_off[L + 1] > len_off[L]) {
+      const int32_t at = atomicAdd(&sh_nt, 1);
+      if (at < kLists) tl[at] = L;
+    }
+  __syncthreads();
+  const int32_t nt = sh_nt;
+  auto is_survivor = [&](int32_t c) -> bool { return survivor(c) >= 0; };
+  // Survivors below T.
   for (int32_t i = s0 + tid; i < s1; i += kTopkBlock) {
-    const int32_t c = sid[i];
+    const int32_t c = sv.id(i);
     const int32_t L = (c >= 0 && c < nc) ? clen[c] : 0;
     if (L < 1 || L > GAT_MAX_TRAJ_LEN) continue;
-    if (sdist[i] < T) {
-      const int32_t pos = atomicAdd(&n_out, 1);
-      if (pos < kTopkMax) {
-        out_d[pos] = sdist[i];
-        out_i[pos] = c;
-      }
-    }
+    if (sv.dist(i) < T) take(sv.dist(i), c);
   }
-  // The r smallest ids at T: the least id X with r candidates at T at or
-  // below it, by a binary search over ids.  Each length valued T holds its ids
-  // ascending and at most ns of them are survivors (counted at their DP
-  // distance), so a list of at least r + ns ids has r non-survivors at or
-  // below its (r + ns)-th id: the least such id over those lists bounds X
-  // from above, and below that bound every list's count of ids <= X lies in
-  // its first r + ns ids.  The search then runs over that short range with
-  // short binary searches per list.
-  const int32_t pre = r + ns;
+  // The r smallest ids at T by lists: the least id X with r candidates at T at
+  // or below it.  Each length valued T holds its ids ascending and at most ns of them
+  // are survivors (counted at their DP distance), so a list of at least r + ns
+  // ids has r non-survivors at or below its (r + ns)-th id: the least such id
+  // over those lists bounds X from above, and below that bound every list's
+  // count of ids <= X lies in its first r + ns ids.
   int32_t bound = nc > 0 ? nc - 1 : 0;
-  for (int32_t t = tid; t < nt && nt <= kTlMax; t += kTopkBlock) {
-    const int L = tl[t];
-    if (len_off[L + 1] - len_off[L] >= pre) bound = min(bound, len_ids[len_off[L] + pre - 1]);
+  auto bound_by = [&](int L) {
+    const int32_t o = len_off[L];
+    if (val[L] == T && len_off[L + 1] - o >= pre) bound = min(bound, len_ids[o + pre - 1]);
+  };
+  if (scanned) {
+    bound = 0;
+  } else if (nt <= kLists) {
+    for (int32_t t = tid; t < nt; t += kTopkBlock) bound_by(tl[t]);
+  } else {
+    for (int L = 1 + tid; L < kLenBins; L += kTopkBlock) bound_by(L);
   }
-  if (nt > kTlMax)
-    for (int L = 1 + tid; L < kLenBins; L += kTopkBlock)
-      if (val[L] == T && len_off[L + 1] - len_off[L] >= pre) bound = min(bound, len_ids[len_off[L] + pre - 1]);
   for (int o = 32; o > 0; o >>= 1) bound = min(bound, __shfl_xor(bound, o));
   if ((tid & 63) == 0) red[tid >> 6] = bound;
   __syncthreads();
   bound = min(min(red[0], red[1]), min(red[2], red[3]));
-  __syncthreads();  // every thread has read red before ties_le reuses it
-  auto list_le = [&](int L, int32_t X) -> int32_t {
-    const int32_t size = len_off[L + 1] - len_off[L];
-    return count_le(len_ids + len_off[L], size < pre ? size : pre, X);
-  };
-  auto ties_le = [&](int32_t X) -> int32_t {
-    int32_t part = 0;
-    if (nt <= kTlMax) {
-      for (int32_t t = tid; t < nt; t += kTopkBlock) part += list_le(tl[t], X);
-    } else {
+  __syncthreads();  // every thread has read red before it is written again
+  // The entries that matter, each list's in full below T and the first r + ns
+  // at T, one per thread: a list per thread read its ids one after another, a
+  // microsecond each, and so did every step of a search over them.  The
+  // non-survivors below T go out, those at
+  // T and up to the bound are gathered, and X is searched among the gathered.
+  int32_t entries = kEntriesMax + 1;
+  if (nt <= kLists) {
+    constexpr int kPerList = kLists / kTopkBlock;
+    int32_t cnt[kPerList], sum = 0;
+#pragma unroll
+    for (int j = 0; j < kPerList; ++j) {
+      const int32_t t = tid * kPerList + j;
+      cnt[j] = 0;
+      if (t < nt) {
+        const int L = tl[t];
+        const int32_t size = len_off[L + 1] - len_off[L];
+        // (Saturated: more than kEntriesMax takes the other way.)
+        cnt[j] = min(val[L] < T ? size : min(size, pre), kEntriesMax + 1);
+      }
+      sum += cnt[j];
+    }
+    int32_t upto = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int32_t y = __shfl_up(upto, o);
+      if (lane >= o) upto += y;
+    }
+    if (lane == 63) red[wv] = upto;
+    __syncthreads();
+    int32_t at = upto - sum;
+    for (int j = 0; j < wv; ++j) at += red[j];
+    entries = red[0] + red[1] + red[2] + red[3];
+#pragma unroll
+    for (int j = 0; j < kPerList; ++j) {
+      const int32_t t = tid * kPerList + j;
+      if (t < nt) first[t] = at;
+      at += cnt[j];
+    }
+  }
+  if (tid == 0) sh_ng = 0;
+  __syncthreads();  // first, sh_ng, and red read
+  if (entries <= kEntriesMax) {
+    for (int32_t e = tid; e < entries; e += kTopkBlock) {
+      int32_t lo = 0, hi = nt - 1;  // the last list starting at or before e
+      while (lo < hi) {
+        const int32_t mid = (lo + hi + 1) >> 1;
+        if (first[mid] <= e) lo = mid;
+        else hi = mid - 1;
+      }
+      const int L = tl[lo];
+      const int32_t c = len_ids[len_off[L] + (e - first[lo])];
+      const bool below = val[L] < T;
+      if ((!below && c > bound) || is_survivor(c)) continue;
+      if (below) {
+        take(val[L], c);
+      } else {
+        const int32_t pos = atomicAdd(&sh_ng, 1);
+        if (pos < kGather) g[pos] = c;
+      }
+    }
+    for (int32_t i = s0 + tid; i < s1 && !scanned; i += kTopkBlock) {
+      const int32_t c = sv.id(i);
+      if (sv.dist(i) != T || c > bound || c < 0 || c >= nc || clen[c] < 1 || clen[c] > GAT_MAX_TRAJ_LEN) continue;
+      const int32_t pos = atomicAdd(&sh_ng, 1);
+      if (pos < kGather) g[pos] = c;
+    }
+  } else {
+    for (int L = 1 + tid; L < kLenBins; L += kTopkBlock) {
+      if (val[L] >= T) continue;
+      for (int32_t i = len_off[L], e = len_off[L + 1]; i < e; ++i)
+        if (!is_survivor(len_ids[i])) take(val[L], len_ids[i]);
+    }
+  }
+  __syncthreads();
+  const int32_t ng = sh_ng;
+  if (scanned) {
+    // (The candidates at T are out already.)
+  } else if (entries <= kEntriesMax && ng <= kGather) {
+    int32_t lo = 0, hi = bound;
+    while (lo < hi) {
+      const int32_t mid = lo + ((hi - lo) >> 1);
+      int32_t part = 0;
+      for (int32_t i = tid; i < ng; i += kTopkBlock) part += g[i] <= mid ? 1 : 0;
+      if (topk_block_sum(part, red) >= r) hi = mid;
+      else lo = mid + 1;
+    }
+    for (int32_t i = tid; i < ng; i += kTopkBlock)
+      if (g[i] <= lo) take(T, g[i]);
+  } else {
+    // More than fits: X by a binary search over ids with a search per list.
+    auto list_le = [&](int L, int32_t X) -> int32_t {
+      const int32_t size = len_off[L + 1] - len_off[L];
+      return count_le(len_ids + len_off[L], size < pre ? size : pre, X);
+    };
+    auto ties_le = [&](int32_t X) -> int32_t {
+      int32_t part = 0;
       for (int L = 1 + tid; L < kLenBins; L += kTopkBlock)
         if (val[L] == T) part += list_le(L, X);
+      for (int32_t i = s0 + tid; i < s1; i += kTopkBlock) {
+        const int32_t c = sv.id(i);
+        if (c > X || c < 0 || c >= nc) continue;
+        const int32_t L = clen[c];
+        if (L < 1 || L > GAT_MAX_TRAJ_LEN) continue;
+        part += (sv.dist(i) == T ? 1 : 0) - (val[L] == T ? 1 : 0);
+      }
+      return topk_block_sum(part, red);
+    };
+    int32_t lo = 0, hi = bound;
+    while (lo < hi) {
+      const int32_t mid = lo + ((hi - lo) >> 1);
+      if (ties_le(mid) >= r) hi = mid;
+      else lo = mid + 1;
+    }
+    const int32_t X = lo;
+    for (int L = 1 + tid; L < kLenBins; L += kTopkBlock) {
+      if (val[L] != T) continue;
+      const int32_t* ids = len_ids + len_off[L];
+      const int32_t u = list_le(L, X);
+      for (int32_t i = 0; i < u; ++i)
+        if (!is_survivor(ids[i])) take(T, ids[i]);
     }
     for (int32_t i = s0 + tid; i < s1; i += kTopkBlock) {
-      const int32_t c = sid[i];
+      const int32_t c = sv.id(i);
       if (c > X || c < 0 || c >= nc) continue;
       const int32_t L = clen[c];
       if (L < 1 || L > GAT_MAX_TRAJ_LEN) continue;
-      part += (sdist[i] == T ? 1 : 0) - (val[L] == T ? 1 : 0);
-    }
-    return topk_block_sum(part, red);
-  };
-  int32_t lo = 0, hi = bound;
-  while (lo < hi) {
-    const int32_t mid = lo + ((hi - lo) >> 1);
-    if (ties_le(mid) >= r) hi = mid;
-    else lo = mid + 1;
-  }
-  const int32_t X = lo;
-  auto collect = [&](int L) {
-    const int32_t* ids = len_ids + len_off[L];
-    const int32_t u = list_le(L, X);
-    for (int32_t i = 0; i < u; ++i) {
-      const int32_t c = ids[i];
-      if (is_survivor(c)) continue;  // counted at its DP distance
-      const int32_t pos = atomicAdd(&n_out, 1);
-      if (pos < kTopkMax) {
-        out_d[pos] = T;
-        out_i[pos] = c;
-      }
-    }
-  };
-  if (nt <= kTlMax) {
-    for (int32_t t = tid; t < nt; t += kTopkBlock) collect(tl[t]);
-  } else {
-    for (int L = 1 + tid; L < kLenBins; L += kTopkBlock)
-      if (val[L] == T) collect(L);
-  }
-  for (int32_t i = s0 + tid; i < s1; i += kTopkBlock) {
-    const int32_t c = sid[i];
-    if (c > X || c < 0 || c >= nc) continue;
-    const int32_t L = clen[c];
-    if (L < 1 || L > GAT_MAX_TRAJ_LEN) continue;
-    if (sdist[i] == T) {
-      const int32_t pos = atomicAdd(&n_out, 1);
-      if (pos < kTopkMax) {
-        out_d[pos] = T;
-        out_i[pos] = c;
-      }
+      if (sv.dist(i) == T) take(T, c);
     }
   }
   __syncthreads();
@@ -843,13 +1043,133 @@ __global__ __launch_bounds__(kTopkBlock) void edr_topk_kernel(
     if (tid == 0) atomicOr(status, 2);
     return;
   }
+  // In rank order through LDS: the results may be host memory, which takes
+  // whole lines, not one word at a time.
+  int32_t* rd = hist;
+  int32_t* ri = hist + kTopkMax;
   for (int i = tid; i < n; i += kTopkBlock) {
     const int32_t d = out_d[i], c = out_i[i];
     int32_t rank = 0;
     for (int j = 0; j < n; ++j) rank += (out_d[j] < d || (out_d[j] == d && out_i[j] < c)) ? 1 : 0;
-    out_dist[int64_t(q) * k + rank] = d;
-    out_ids[int64_t(q) * k + rank] = c + 1;
+    rd[rank] = d;
+    ri[rank] = c + 1;
   }
+  __syncthreads();
+  for (int i = tid; i < n; i += kTopkBlock) {
+    out_dist[int64_t(q) * k + i] = rd[i];
+    out_ids[int64_t(q) * k + i] = ri[i];
+  }
+}
+
+__global__ __launch_bounds__(kTopkBlock) void edr_topk_kernel(
+    const int32_t* __restrict__ ftable, int32_t w, const int32_t* __restrict__ qlen,
+    const int32_t* __restrict__ clen, int32_t nc, const int32_t* __restrict__ len_ids,
+    const int32_t* __restrict__ len_off, const int32_t* __restrict__ sstart, const int32_t* __restrict__ sid,
+    const int32_t* __restrict__ sdist, int32_t k, int32_t kk, int32_t* __restrict__ out_ids,
+    int32_t* __restrict__ out_dist, int32_t* __restrict__ status) {
+  const int q = blockIdx.x;
+  topk_query<false>(q, GlobalSurvivors{sid, sdist}, sstart[q], sstart[q + 1], ftable, w, qlen, clen, nc, len_ids,
+                    len_off, k, kk, out_ids, out_dist, status);
+}
+
+// A batch's control words (gat_edr_merge): device memory, cleared at its start.
+constexpr int kCtlCount = 0, kCtlLists = 2, kCtlStatus = 3, kCtlTicket = 7, kCtlWords = 32;
+constexpr int kMergeMax = 1024;  // survivors of a query gathered in LDS
+
+// The merge straight from the DP's pairs and distances, one workgroup per query
+// (no reference counterpart): the query's survivors are picked out of all the
+// batch's pairs, sorted by id in LDS and merged as edr_topk_kernel does, where
+// separate launches built lists, sorted them and merged.  Reading every pair
+// in every workgroup suits batches of few pairs.  The results may go to pinned
+// host memory; the last workgroup to end writes the control words and the time
+// after them.
+__global__ __launch_bounds__(kTopkBlock) void edr_merge_kernel(
+    const int32_t* __restrict__ ftable, int32_t w, const int32_t* __restrict__ qlen, int32_t nq,
+    const int32_t* __restrict__ clen, int32_t nc, const int32_t* __restrict__ len_ids,
+    const int32_t* __restrict__ len_off, const int2* __restrict__ pairs, const int32_t* __restrict__ dist,
+    uint32_t cap, int32_t k, int32_t kk, int32_t* __restrict__ out_ids, int32_t* __restrict__ out_dist,
+    uint32_t* __restrict__ ctl, uint32_t* __restrict__ ctl_out, uint32_t* __restrict__ stamp) {
+  __shared__ unsigned long long v[kMergeMax];
+  __shared__ int32_t found, wrong;
+  const int q = blockIdx.x, t = threadIdx.x;
+  if (stamp && q == 0 && t == 0) store_clock(stamp);
+  const unsigned long long total = *reinterpret_cast<const unsigned long long*>(ctl + kCtlCount);
+  const uint32_t np = total > cap ? 0u : uint32_t(total);
+  if (t == 0) found = wrong = 0;
+  __syncthreads();
+  constexpr uint32_t kAhead = 8;  // pairs per thread in flight
+  for (uint32_t i = t; i < np; i += kTopkBlock * kAhead) {
+    int2 p[kAhead];
+#pragma unroll
+    for (uint32_t j = 0; j < kAhead; ++j) p[j] = pairs[min(i + j * kTopkBlock, np - 1)];
+#pragma unroll
+    for (uint32_t j = 0; j < kAhead; ++j) {
+      const uint32_t k0 = i + j * kTopkBlock;
+      if (k0 >= np || p[j].x != q) continue;
+      const int32_t at = atomicAdd(&found, 1);
+      if (at < kMergeMax) v[at] = ((unsigned long long)(uint32_t(p[j].y)) << 32) | uint32_t(dist[k0]);
+    }
+  }
+  __syncthreads();
+  const int32_t m = found;
+  if (total <= cap && m <= kMergeMax) {
+    if (m > 1) {  // bitonic sort by id (distinct within a query)
+      int P = 2;
+      while (P < m) P <<= 1;
+      for (int i = m + t; i < P; i += kTopkBlock) v[i] = ~0ull;
+      __syncthreads();
+      for (int a = 2; a <= P; a <<= 1)
+        for (int b = a >> 1; b > 0; b >>= 1) {
+          for (int i = t; i < P; i += kTopkBlock) {
+            const int o = i ^ b;
+            if (o > i) {
+              const bool up = (i & a) == 0;
+              const unsigned long long x = v[i], y = v[o];
+              if ((x > y) == up) {
+                v[i] = y;
+                v[o] = x;
+              }
+            }
+          }
+          __syncthreads();
+        }
+    }
+    topk_query<true>(q, LdsSurvivors{v}, 0, m, ftable, w, qlen, clen, nc, len_ids, len_off, k, kk, out_ids, out_dist,
+                     &wrong);
+  }
+  __syncthreads();
+  if (t >= 64) return;
+  uint32_t ticket = 0;
+  if (t == 0) {
+    // The statuses are in before the ticket, which depends on what their
+    // atomics return: a fence would write the whole L2 back, once per workgroup.
+    uint32_t before = 0;
+    if (m > kMergeMax) before |= atomicOr(ctl + kCtlLists, 2u);
+    if (wrong) before |= atomicOr(ctl + kCtlStatus, uint32_t(wrong));
+    ticket = atomicAdd(ctl + kCtlTicket, before == ~0u ? 2u : 1u);  // (never 2: statuses are small)
+  }
+  if (uint32_t(__builtin_amdgcn_readfirstlane(int(ticket))) == uint32_t(nq) - 1u) {
+    if (t < kCtlWords) ctl_out[t] = atomicOr(ctl + t, 0u);
+    if (t == 0) store_clock(ctl_out + kCtlWords);
+  }
+}
+
+// out[a * w + L] = the all-mismatch value of lengths a and L in either order.
+__global__ __launch_bounds__(256) void edr_length_table_kernel(const int32_t* __restrict__ table, int32_t w,
+                                                               int32_t* __restrict__ out) {
+  // 16 x 16 tiles on and above the diagonal, each written to both sides.
+  __shared__ int32_t tile[16][17];
+  const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
+  const int c0 = int(blockIdx.x) * 16, r0 = int(blockIdx.y) * 16;
+  if (c0 < r0) return;
+  const int r = r0 + y, c = c0 + x;
+  int32_t v = 0;
+  if (r < w && c < w) v = table[int64_t(min(r, c)) * w + max(r, c)];
+  tile[y][x] = v;
+  if (r < w && c < w) out[int64_t(r) * w + c] = v;
+  __syncthreads();
+  const int rr = c0 + y, cc = r0 + x;
+  if (c0 != r0 && rr < w && cc < w) out[int64_t(rr) * w + cc] = tile[x][y];
 }
 
 // ---------------------------------------------------------------- device jobs
@@ -914,10 +1234,14 @@ __device__ uint32_t block_exclusive_scan(uint32_t* a, int n, uint32_t* red) {
 }
 
 // What a pair of n rows and m columns keeps its wave busy for, in VALU
-// instructions per 16-step block: on one wave (64-lane strips of four rows per
-// lane, the last of two or one) and over several (edr_pipe_kernel's schedule,
-// with a lag of kLag blocks between strips and a barrier per block).
-// Grid::runBatched applies the same rule on the host.
+// instructions per 16-step block: in a 16-lane segment, on one wave (64-lane
+// strips of four rows per lane, the last of two or one) and over several
+// (edr_pipe_kernel's schedule, with a lag of kLag blocks between strips and a
+// barrier per block).  Grid::runBatched applies the same rules on the host.
+__device__ __forceinline__ int64_t segment_cost(int n, int m) {
+  const int rows = (n + 15) / 16, rest = rows & 3;
+  return int64_t((m + 15 + 15) / 16) * (19 * (rows / 4) + (rest >= 2 ? 11 : 0) + ((rest & 1) ? 7 : 0));
+}
 __device__ __forceinline__ int64_t one_wave_cost(int n, int m) {
   const int rows = (n + 63) / 64, rest = rows & 3;
   return int64_t((m + 63 + 15) / 16) * (19 * (rows / 4) + (rest >= 2 ? 11 : 0) + ((rest & 1) ? 7 : 0));
@@ -934,27 +1258,46 @@ struct JobRules {
   int32_t split, waves, every_long, cus;
 };
 
-// The bucket rules of a batch of np pairs: in a batch of fewer than 64 jobs
-// per CU (one round of waves) long means longer than `split`, otherwise
-// longer than max(split, 1024); with several waves per pair such a batch
-// sends some long pairs to the several-wave bucket.
+// The bucket rules of a batch of np pairs.  A batch of 64 jobs per CU and more
+// keeps every SIMD busy whatever its pairs: long means longer than max(split,
+// 1024).  A smaller one (one round of waves) ends when its longest pair does:
+// its `critical` length is the longest pair's schedule over several waves (or
+// on one, when it may take no more), but not under twice the time all pairs
+// would take spread evenly in 16-lane segments.  A pair then takes the
+// cheapest form that ends in time: a 16-lane segment (a quarter of the
+// instructions, up to four times the length, and four waves share a SIMD) up
+// to half of critical and `split` columns, one wave up to all of it, several
+// beyond.
 struct JobShape {
   int mid;
-  bool multi;
+  bool latency, multi;
   __device__ JobShape(const JobRules& r, uint32_t np) {
-    const bool latency_bound = (int64_t(np) + 3) / 4 < int64_t(r.cus) * 16;
-    mid = latency_bound ? r.split : max(r.split, 1024);
-    multi = latency_bound && r.waves > 1;
+    latency = (int64_t(np) + 3) / 4 < int64_t(r.cus) * 16;
+    mid = latency ? r.split : max(r.split, 1024);
+    multi = latency && r.waves > 1;
   }
 };
 
+// A pair's share of critical: the longest schedule, and the spread work.
+__device__ __forceinline__ int64_t critical_share(int n, int m, const JobRules& r, const JobShape& sh) {
+  if (!sh.latency || n < 1) return 0;
+  return sh.multi ? pipe_cost(n, m, r.waves) : one_wave_cost(n, m);
+}
+__device__ __forceinline__ int64_t critical_of(int64_t longest, int64_t work, const JobRules& r) {
+  const int64_t spread = work / (4 * 4 * int64_t(r.cus)) / 2;  // four pairs a wave, four SIMDs a CU
+  return longest > spread ? longest : spread;
+}
+
 // Sort key of a pair of shorter length n and longer m: (bucket, strips
 // descending, longer length descending in sixteen steps of the bucket's
-// range); critical is the batch's longest several-wave schedule.
+// range).
 __device__ __forceinline__ uint32_t job_key(int n, int m, const JobRules& rules, const JobShape& sh,
                                             int64_t critical) {
   int bucket = m <= rules.split ? 0 : m <= sh.mid ? 1 : 2;
-  if (bucket == 2 && sh.multi && (rules.every_long || one_wave_cost(n, m) > critical)) bucket = 3;
+  if (sh.latency && n >= 1) {
+    if (bucket == 0 && 2 * segment_cost(n, m) > critical) bucket = 2;
+    if (bucket == 2 && sh.multi && (rules.every_long ? m > rules.split : one_wave_cost(n, m) > critical)) bucket = 3;
+  }
   const int strips = (n + 15) / 16;
   const int top = bucket == 0 ? rules.split : bucket == 1 ? sh.mid : GAT_MAX_TRAJ_LEN;
   const int step = max(1, (top + kLenSteps - 1) / kLenSteps);
@@ -978,18 +1321,16 @@ __global__ __launch_bounds__(kJobThreads) void edr_jobs_kernel(const int2* __res
   __shared__ unsigned long long red64[kJobThreads / 64];
   const int t = threadIdx.x;
   const unsigned long long total = *count;
+  if (t == 0) *status = total > cap ? 1 : 0;
   if (total > cap) {  // uniform: nothing to run; the caller grows the buffers
     if (t < 8) windows[t] = 0;
-    if (t == 0) atomicOr(status, 1);
     return;
   }
   const uint32_t np = uint32_t(total);
   // Lengths, the cell count and the several-wave threshold.
-  const JobShape sh0(rules, np);
-  const int mid = sh0.mid;
-  const bool multi = sh0.multi;
+  const JobShape shape(rules, np);
   unsigned long long my_cells = 0;
-  int64_t my_crit = 0;
+  int64_t my_crit = 0, my_work = 0;
   for (uint32_t i = t; i < np; i += kJobThreads) {
     const int2 p = pairs[i];
     const bool ok = p.x >= 0 && p.x < nq && p.y >= 0 && p.y < nc;
@@ -997,31 +1338,35 @@ __global__ __launch_bounds__(kJobThreads) void edr_jobs_kernel(const int2* __res
     const int n = min(a, b), m = max(a, b);
     nm[i] = make_int2(n, m);
     my_cells += (unsigned long long)(n) * (unsigned long long)(m);
-    if (multi && m > mid) {
-      const int64_t c = pipe_cost(n, m, rules.waves);
-      if (c > my_crit) my_crit = c;
-    }
+    const int64_t c = critical_share(n, m, rules, shape);
+    if (c > my_crit) my_crit = c;
+    if (n >= 1) my_work += segment_cost(n, m);
   }
   for (int off = 32; off > 0; off >>= 1) {
     my_cells += __shfl_xor(my_cells, off);
+    my_work += __shfl_xor(my_work, off);
     const int64_t o = __shfl_xor(my_crit, off);
     if (o > my_crit) my_crit = o;
   }
-  __shared__ int64_t crit_w[kJobThreads / 64];
+  __shared__ int64_t crit_w[kJobThreads / 64], work_w[kJobThreads / 64];
   if ((t & 63) == 0) {
     red64[t / 64] = my_cells;
     crit_w[t / 64] = my_crit;
+    work_w[t / 64] = my_work;
   }
   for (int i = t; i < kSortBins; i += kJobThreads) bins[i] = 0;
   __syncthreads();
-  int64_t critical = 0;
-  for (int w = 0; w < kJobThreads / 64; ++w) critical = crit_w[w] > critical ? crit_w[w] : critical;
+  int64_t longest = 0, work = 0;
+  for (int w = 0; w < kJobThreads / 64; ++w) {
+    longest = crit_w[w] > longest ? crit_w[w] : longest;
+    work += work_w[w];
+  }
+  const int64_t critical = critical_of(longest, work, rules);
   if (t == 0) {
     unsigned long long c = 0;
     for (int w = 0; w < kJobThreads / 64; ++w) c += red64[w];
     *cells = c;
   }
-  const JobShape shape(rules, np);
   auto key_of = [&](int2 v) { return job_key(v.x, v.y, rules, shape, critical); };
   for (uint32_t i = t; i < np; i += kJobThreads) atomicAdd(&bins[key_of(nm[i])], 1u);
   __syncthreads();
@@ -1082,7 +1427,7 @@ __global__ __launch_bounds__(kJobsBlock) void edr_jobs_lengths_kernel(
   uint32_t np;
   if (jobs_overflow(count, cap, &np)) return;
   const JobShape sh(rules, np);
-  unsigned long long my_cells = 0, my_crit = 0;
+  unsigned long long my_cells = 0, my_crit = 0, my_work = 0;
   for (uint32_t i = blockIdx.x * kJobsBlock + threadIdx.x; i < np; i += gridDim.x * kJobsBlock) {
     const int2 p = pairs[i];
     const bool ok = p.x >= 0 && p.x < nq && p.y >= 0 && p.y < nc;
@@ -1090,19 +1435,20 @@ __global__ __launch_bounds__(kJobsBlock) void edr_jobs_lengths_kernel(
     const int n = min(a, b), m = max(a, b);
     nm[i] = make_int2(n, m);
     my_cells += (unsigned long long)(n) * (unsigned long long)(m);
-    if (sh.multi && m > sh.mid) {
-      const unsigned long long c = (unsigned long long)pipe_cost(n, m, rules.waves);
-      my_crit = c > my_crit ? c : my_crit;
-    }
+    const unsigned long long c = (unsigned long long)critical_share(n, m, rules, sh);
+    my_crit = c > my_crit ? c : my_crit;
+    if (sh.latency && n >= 1) my_work += (unsigned long long)segment_cost(n, m);
   }
   for (int off = 32; off > 0; off >>= 1) {
     my_cells += __shfl_xor(my_cells, off);
     const unsigned long long o = __shfl_xor(my_crit, off);
     my_crit = o > my_crit ? o : my_crit;
+    my_work += __shfl_xor(my_work, off);
   }
   if ((threadIdx.x & 63) == 0) {
     if (my_cells) atomicAdd(cells, my_cells);
     if (my_crit) atomicMax(crit, my_crit);
+    if (my_work) atomicAdd(crit + 1, my_work);
   }
 }
 
@@ -1121,7 +1467,7 @@ __global__ __launch_bounds__(kJobsBlock) void edr_jobs_hist_kernel(const unsigne
   uint32_t np;
   if (jobs_overflow(count, cap, &np)) return;
   const JobShape sh(rules, np);
-  const int64_t critical = int64_t(*crit);
+  const int64_t critical = critical_of(int64_t(crit[0]), int64_t(crit[1]), rules);
   for (int b = threadIdx.x; b < kSortBins; b += kJobsBlock) h[b] = 0;
   __syncthreads();
   uint32_t lo, hi;
@@ -1187,7 +1533,7 @@ __global__ __launch_bounds__(kJobsBlock) void edr_jobs_scatter_kernel(
   uint32_t np;
   if (jobs_overflow(count, cap, &np)) return;
   const JobShape sh(rules, np);
-  const int64_t critical = int64_t(*crit);
+  const int64_t critical = critical_of(int64_t(crit[0]), int64_t(crit[1]), rules);
   for (int b = threadIdx.x; b < kSortBins; b += kJobsBlock) h[b] = 0;
   __syncthreads();
   uint32_t lo, hi;
@@ -1358,9 +1704,9 @@ extern "C" int gat_edr_filter(const float* qbox, int32_t nq, const float* cbox, 
   return GAT_OK;
 }
 
-extern "C" int gat_edr_filter_grid(const float* qbox, int32_t nq, const float* cbox, int32_t nc,
-                                   const gat_edr_cand_grid* grid, double eps, int32_t* pairs_out, int64_t capacity,
-                                   uint64_t* count, void* stream) {
+extern "C" int gat_edr_filter_grid_add(const float* qbox, int32_t nq, const float* cbox, int32_t nc,
+                                       const gat_edr_cand_grid* grid, double eps, int32_t* pairs_out,
+                                       int64_t capacity, uint64_t* count, uint32_t* stamp, void* stream) {
   GAT_REQUIRE(nq >= 0 && nc >= 0 && capacity >= 0, "EDR grid filter: bad sizes");
   GAT_REQUIRE(count && grid, "EDR grid filter: null count or grid");
   GAT_REQUIRE(grid->cells_per_side >= 1 && grid->cells_per_side <= 4096 && grid->nalways >= 0 &&
@@ -1368,8 +1714,6 @@ extern "C" int gat_edr_filter_grid(const float* qbox, int32_t nq, const float* c
                   std::isfinite(grid->y0) && std::isfinite(grid->inv_x) && std::isfinite(grid->inv_y) &&
                   grid->inv_x >= 0.0f && grid->inv_y >= 0.0f,
               "EDR grid filter: bad grid");
-  hipStream_t s = gat::as_stream(stream);
-  if (int rc = gat_fill_u32(reinterpret_cast<uint32_t*>(count), 0u, 2, stream)) return rc;
   if (nq == 0 || nc == 0) return GAT_OK;
   GAT_REQUIRE(qbox && cbox && (pairs_out || capacity == 0), "EDR grid filter: null pointer");
   GAT_REQUIRE(eps > 0, "EDR grid filter: eps must be positive");
@@ -1384,12 +1728,21 @@ extern "C" int gat_edr_filter_grid(const float* qbox, int32_t nq, const float* c
                     grid->always_dev,
                     grid->nalways};
   edr_filter_grid_kernel<<<dim3(uint32_t((nq + kGridFilterWaves - 1) / kGridFilterWaves)),
-                           dim3(64 * kGridFilterWaves), 0, s>>>(
+                           dim3(64 * kGridFilterWaves), 0, gat::as_stream(stream)>>>(
       reinterpret_cast<const float4*>(qbox), nq, reinterpret_cast<const float4*>(cbox), nc, gr,
       gat_eps_threshold(eps), reinterpret_cast<int2*>(pairs_out), uint64_t(capacity),
-      reinterpret_cast<unsigned long long*>(count));
+      reinterpret_cast<unsigned long long*>(count), stamp);
   GAT_LAUNCH_CHECK("edr_filter_grid_kernel");
   return GAT_OK;
+}
+
+extern "C" int gat_edr_filter_grid(const float* qbox, int32_t nq, const float* cbox, int32_t nc,
+                                   const gat_edr_cand_grid* grid, double eps, int32_t* pairs_out, int64_t capacity,
+                                   uint64_t* count, void* stream) {
+  GAT_REQUIRE(nq >= 0 && nc >= 0 && capacity >= 0, "EDR grid filter: bad sizes");
+  GAT_REQUIRE(count && grid, "EDR grid filter: null count or grid");
+  if (int rc = gat_fill_u32(reinterpret_cast<uint32_t*>(count), 0u, 2, stream)) return rc;
+  return gat_edr_filter_grid_add(qbox, nq, cbox, nc, grid, eps, pairs_out, capacity, count, nullptr, stream);
 }
 
 extern "C" int gat_edr_topk(const int32_t* ftable, int32_t w, const int32_t* qlen, int32_t nq, const int32_t* clen,
@@ -1445,7 +1798,106 @@ __global__ __launch_bounds__(64) void edr_pack_kernel(const float* __restrict__ 
   }
 }
 
+// A small batch's queries from pinned host memory in one launch: the metadata
+// (source offsets, padded offsets as 64 and 32 bits, lengths) copied as it is,
+// the padded store written whole (points, NaN elsewhere), the boxes, and a
+// batch's control words cleared.  One wave per trajectory, which also writes
+// the padding before it; the store's end is shared by all.  Two copies, a fill
+// and the packing kernel took 25 us for one 128-point query.
+__global__ __launch_bounds__(256) void edr_stage_queries_kernel(
+    const uint32_t* __restrict__ meta, uint32_t meta_words, uint32_t* __restrict__ up, const int64_t* __restrict__ src,
+    const int64_t* __restrict__ dst, int32_t ntraj, int64_t npoints, const float* __restrict__ lon,
+    const float* __restrict__ lat, int64_t total, float2* __restrict__ xy, float4* __restrict__ box,
+    uint32_t* __restrict__ ctl, uint32_t ctl_words, uint32_t* __restrict__ stamp) {
+  const int64_t i0 = int64_t(blockIdx.x) * 256 + threadIdx.x, stride = int64_t(gridDim.x) * 256;
+  for (int64_t i = i0; i < ctl_words; i += stride) ctl[i] = 0u;
+  if (stamp && i0 == 0) store_clock(stamp);
+  for (int64_t i = i0; i < meta_words; i += stride) up[i] = meta[i];
+  const float2 nan2 = edr::nan_point();
+  // Points end at: the last trajectory's end (the store's start when empty).
+  const int64_t end = ntraj > 0 ? dst[ntraj - 1] + (npoints - src[ntraj - 1]) : 0;
+  for (int64_t i = end + i0; i < total; i += stride) xy[i] = nan2;
+  const int lane = threadIdx.x & 63;
+  for (int64_t t = i0 / 64; t < ntraj; t += stride / 64) {
+    const int64_t b = src[t], n = src[t + 1] - b, d = dst[t];
+    for (int64_t i = d - kPad + lane; i < d; i += 64)
+      if (i >= 0 && i < total) xy[i] = nan2;
+    float4 bb = edr::empty_box();
+    // Eight points per lane in flight: a read of host memory takes microseconds.
+    constexpr int kAhead = 8;
+    for (int64_t i = lane; i < n; i += 64 * kAhead) {
+      float2 p[kAhead];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const int64_t at = b + min(i + 64 * k, n - 1);
+        p[k] = make_float2(lon[at], lat[at]);
+      }
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const int64_t at = i + 64 * k;
+        if (at < n && d + at >= 0 && d + at < total) xy[d + at] = p[k];
+        bb = edr::grow(bb, p[k]);  // (a repeated last point changes no box)
+      }
+    }
+    bb = edr::segment_box<64>(bb);
+    if (lane == 0) box[t] = bb;
+  }
+}
+
 }  // namespace
+
+extern "C" int gat_edr_stage_queries(const void* meta_pinned, int64_t meta_bytes, void* up, const int64_t* src_pinned,
+                                     const int64_t* dst_pinned, int32_t ntraj, int64_t npoints,
+                                     const float* lon_pinned, const float* lat_pinned, int64_t total, float* xy,
+                                     float* box, uint32_t* ctl, int64_t ctl_words, uint32_t* stamp, void* stream) {
+  GAT_REQUIRE(meta_bytes >= 0 && meta_bytes % 4 == 0 && meta_bytes / 4 <= int64_t(UINT32_MAX) && ntraj >= 0 &&
+                  npoints >= 0 && total >= 0 && ctl_words >= 0 && ctl_words <= int64_t(UINT32_MAX),
+              "EDR stage queries: bad sizes");
+  GAT_REQUIRE((meta_bytes == 0 || (meta_pinned && up)) && (total == 0 || xy) && (ctl_words == 0 || ctl),
+              "EDR stage queries: null pointer");
+  GAT_REQUIRE(ntraj == 0 || (src_pinned && dst_pinned && box && (npoints == 0 || (lon_pinned && lat_pinned))),
+              "EDR stage queries: null queries");
+  int64_t blocks = (int64_t(ntraj) + 3) / 4;
+  const int64_t fill = (total - npoints + 255) / 256;
+  if (blocks < fill) blocks = fill;
+  const int64_t most = int64_t(gat::cu_count()) * 8;
+  blocks = blocks < 1 ? 1 : blocks > most ? most : blocks;
+  edr_stage_queries_kernel<<<dim3(uint32_t(blocks)), dim3(256), 0, gat::as_stream(stream)>>>(
+      static_cast<const uint32_t*>(meta_pinned), uint32_t(meta_bytes / 4), static_cast<uint32_t*>(up), src_pinned,
+      dst_pinned, ntraj, npoints, lon_pinned, lat_pinned, total, reinterpret_cast<float2*>(xy),
+      reinterpret_cast<float4*>(box), ctl, uint32_t(ctl_words), stamp);
+  GAT_LAUNCH_CHECK("edr_stage_queries_kernel");
+  return GAT_OK;
+}
+
+extern "C" int gat_edr_length_table(const int32_t* table, int32_t w, int32_t* out, void* stream) {
+  GAT_REQUIRE(w >= 0 && w <= GAT_MAX_TRAJ_LEN + 1, "EDR length table: width outside 0..%d", GAT_MAX_TRAJ_LEN + 1);
+  if (w == 0) return GAT_OK;
+  GAT_REQUIRE(table && out, "EDR length table: null pointer");
+  const uint32_t tiles = uint32_t((w + 15) / 16);
+  edr_length_table_kernel<<<dim3(tiles, tiles), dim3(256), 0, gat::as_stream(stream)>>>(table, w, out);
+  GAT_LAUNCH_CHECK("edr_length_table_kernel");
+  return GAT_OK;
+}
+
+extern "C" int gat_edr_merge(const int32_t* length_table, int32_t w, const int32_t* qlen, int32_t nq,
+                             const int32_t* clen, int32_t nc, const int32_t* len_ids, const int32_t* len_off,
+                             const int32_t* pairs, const int32_t* dist, int64_t capacity, int32_t k, int32_t kk,
+                             int32_t* out_ids, int32_t* out_dist, uint32_t* ctl, uint32_t* ctl_out, uint32_t* stamp,
+                             void* stream) {
+  GAT_REQUIRE(w == GAT_MAX_TRAJ_LEN + 1, "EDR merge: the length table must be %d wide", GAT_MAX_TRAJ_LEN + 1);
+  GAT_REQUIRE(nq >= 1 && nc >= 0 && capacity >= 0 && capacity <= int64_t(INT32_MAX), "EDR merge: bad sizes");
+  GAT_REQUIRE(k >= 1 && k <= kTopkMax && kk >= 0 && kk <= k && kk <= nc,
+              "EDR merge: k outside 1..%d or kk outside 0..min(k, candidates)", kTopkMax);
+  GAT_REQUIRE(length_table && qlen && clen && len_ids && len_off && pairs && dist && out_ids && out_dist && ctl &&
+                  ctl_out,
+              "EDR merge: null pointer");
+  edr_merge_kernel<<<dim3(uint32_t(nq)), dim3(kTopkBlock), 0, gat::as_stream(stream)>>>(
+      length_table, w, qlen, nq, clen, nc, len_ids, len_off, reinterpret_cast<const int2*>(pairs), dist,
+      uint32_t(capacity), k, kk, out_ids, out_dist, ctl, ctl_out, stamp);
+  GAT_LAUNCH_CHECK("edr_merge_kernel");
+  return GAT_OK;
+}
 
 extern "C" int gat_edr_pack_trajectories(const float* lon, const float* lat, const int64_t* src_off,
                                          const int64_t* dst_off, int32_t ntraj, int64_t total, float* xy, float* box,
@@ -1472,30 +1924,14 @@ extern "C" int gat_edr_mismatch_table(int32_t maxlen, int32_t* out, void* stream
   return GAT_OK;
 }
 
-extern "C" int gat_edr_batched(const int32_t* pairs, int64_t npairs, const gat_edr_job* jobs, int64_t njobs,
-                               const int32_t* window, int32_t* counter, const float* qxy, const int64_t* qoff, const int32_t* qlen,
-                               int32_t nqueries, const float* cxy, const int64_t* coff, const int32_t* clen,
-                               int32_t ncands, int32_t maxlen, double eps, int32_t per_cu, int32_t lanes_per_pair,
-                               int32_t* out, void* stream) {
-  GAT_REQUIRE(npairs >= 0 && njobs >= 0 && njobs <= INT32_MAX && nqueries >= 0 && ncands >= 0,
-              "EDR batched: bad sizes");
-  GAT_REQUIRE(lanes_per_pair == 16 || lanes_per_pair == 64 || lanes_per_pair == 128 || lanes_per_pair == 256 ||
-                  lanes_per_pair == 512,
-              "EDR batched: lanes_per_pair must be 16, 64, 128, 256 or 512");
-  if (njobs == 0) return GAT_OK;
-  GAT_REQUIRE(pairs && jobs && counter && qxy && qoff && qlen && cxy && coff && clen && out,
-              "EDR batched: null pointer");
-  GAT_REQUIRE(maxlen >= 1 && maxlen <= GAT_MAX_TRAJ_LEN, "EDR batched: maxlen outside 1..%d", GAT_MAX_TRAJ_LEN);
-  GAT_REQUIRE(eps > 0, "EDR batched: eps must be positive");
-  GAT_REQUIRE(per_cu >= 0 && per_cu <= 64, "EDR batched: per_cu outside 0..64");
-  hipStream_t s = gat::as_stream(stream);
-  // The job counter is cleared by a kernel, so the launch can be captured in a graph.
-  if (int rc = gat_fill_u32(reinterpret_cast<uint32_t*>(counter), 0u, 1, stream)) return rc;
-  const float u = gat_eps_threshold(eps);
-  const auto* P = reinterpret_cast<const int2*>(pairs);
-  const auto* J = reinterpret_cast<const Job*>(jobs);
-  const auto* Q = reinterpret_cast<const float2*>(qxy);
-  const auto* Cs = reinterpret_cast<const float2*>(cxy);
+namespace {
+
+// The launches of gat_edr_batched and gat_edr_pairs (jobs null, raw set); the
+// job counter is cleared already.
+int launch_edr(const int2* P, int64_t npairs, const Job* J, int64_t njobs, const int32_t* window, int32_t* counter,
+               const float2* Q, const int64_t* qoff, const int32_t* qlen, int32_t nqueries, const float2* Cs,
+               const int64_t* coff, const int32_t* clen, int32_t ncands, int32_t maxlen, float u, int32_t per_cu,
+               int32_t lanes_per_pair, int32_t* out, const RawPairs& raw, hipStream_t s) {
   // LDS class: the smallest row buffer that holds maxlen columns (64-lane
   // pairs: 1024 or 2048).  Persistent grid: per_cu single-wave workgroups per
   // CU (default by class), capped by the work.
@@ -1511,7 +1947,7 @@ extern "C" int gat_edr_batched(const int32_t* pairs, int64_t npairs, const gat_e
     const dim3 wblock{uint32_t(64 * waves)};
 #define GAT_EDR_PIPE(M, W)                                                                                       \
   edr_pipe_kernel<M, W><<<grid, wblock, 0, s>>>(P, npairs, J, int32_t(njobs), window, counter, nqueries, ncands, Q, \
-                                                qoff, qlen, Cs, coff, clen, u, out)
+                                                qoff, qlen, Cs, coff, clen, u, out, raw)
     if (cls == 1024) {
       if (waves == 2) GAT_EDR_PIPE(1024, 2);
       else if (waves == 4) GAT_EDR_PIPE(1024, 4);
@@ -1527,7 +1963,7 @@ extern "C" int gat_edr_batched(const int32_t* pairs, int64_t npairs, const gat_e
   }
 #define GAT_EDR_LAUNCH(M, SEG)                                                                                  \
   edr_wave_kernel<M, SEG><<<grid, block, 0, s>>>(P, npairs, J, int32_t(njobs), window, counter, nqueries, ncands, Q, \
-                                                 qoff, qlen, Cs, coff, clen, u, out)
+                                                 qoff, qlen, Cs, coff, clen, u, out, raw)
   if (wide) {
     if (cls == 1024)
       GAT_EDR_LAUNCH(1024, 64);
@@ -1546,6 +1982,73 @@ extern "C" int gat_edr_batched(const int32_t* pairs, int64_t npairs, const gat_e
   return GAT_OK;
 }
 
+}  // namespace
+
+static int run_bucket(const int32_t* pairs, int64_t npairs, const gat_edr_job* jobs, int64_t njobs,
+                      const int32_t* window, int32_t* counter, bool clear, const float* qxy, const int64_t* qoff,
+                      const int32_t* qlen, int32_t nqueries, const float* cxy, const int64_t* coff,
+                      const int32_t* clen, int32_t ncands, int32_t maxlen, double eps, int32_t per_cu,
+                      int32_t lanes_per_pair, uint32_t* stamp, int32_t* out, void* stream) {
+  GAT_REQUIRE(npairs >= 0 && njobs >= 0 && njobs <= INT32_MAX && nqueries >= 0 && ncands >= 0,
+              "EDR batched: bad sizes");
+  GAT_REQUIRE(lanes_per_pair == 16 || lanes_per_pair == 64 || lanes_per_pair == 128 || lanes_per_pair == 256 ||
+                  lanes_per_pair == 512,
+              "EDR batched: lanes_per_pair must be 16, 64, 128, 256 or 512");
+  if (njobs == 0) return GAT_OK;
+  GAT_REQUIRE(pairs && jobs && counter && qxy && qoff && qlen && cxy && coff && clen && out,
+              "EDR batched: null pointer");
+  GAT_REQUIRE(maxlen >= 1 && maxlen <= GAT_MAX_TRAJ_LEN, "EDR batched: maxlen outside 1..%d", GAT_MAX_TRAJ_LEN);
+  GAT_REQUIRE(eps > 0, "EDR batched: eps must be positive");
+  GAT_REQUIRE(per_cu >= 0 && per_cu <= 64, "EDR batched: per_cu outside 0..64");
+  // The job counter is cleared by a kernel, so the launch can be captured in a graph.
+  if (clear)
+    if (int rc = gat_fill_u32(reinterpret_cast<uint32_t*>(counter), 0u, 1, stream)) return rc;
+  return launch_edr(reinterpret_cast<const int2*>(pairs), npairs, reinterpret_cast<const Job*>(jobs), njobs, window,
+                    counter, reinterpret_cast<const float2*>(qxy), qoff, qlen, nqueries,
+                    reinterpret_cast<const float2*>(cxy), coff, clen, ncands, maxlen, gat_eps_threshold(eps), per_cu,
+                    lanes_per_pair, out, RawPairs{nullptr, nullptr, stamp}, gat::as_stream(stream));
+}
+
+extern "C" int gat_edr_bucket(const int32_t* pairs, int64_t npairs, const gat_edr_job* jobs, int64_t njobs,
+                              const int32_t* window, int32_t* counter, const float* qxy, const int64_t* qoff,
+                              const int32_t* qlen, int32_t nqueries, const float* cxy, const int64_t* coff,
+                              const int32_t* clen, int32_t ncands, int32_t maxlen, double eps, int32_t per_cu,
+                              int32_t lanes_per_pair, uint32_t* stamp, int32_t* out, void* stream) {
+  return run_bucket(pairs, npairs, jobs, njobs, window, counter, false, qxy, qoff, qlen, nqueries, cxy, coff, clen,
+                    ncands, maxlen, eps, per_cu, lanes_per_pair, stamp, out, stream);
+}
+
+extern "C" int gat_edr_batched(const int32_t* pairs, int64_t npairs, const gat_edr_job* jobs, int64_t njobs,
+                               const int32_t* window, int32_t* counter, const float* qxy, const int64_t* qoff, const int32_t* qlen,
+                               int32_t nqueries, const float* cxy, const int64_t* coff, const int32_t* clen,
+                               int32_t ncands, int32_t maxlen, double eps, int32_t per_cu, int32_t lanes_per_pair,
+                               int32_t* out, void* stream) {
+  return run_bucket(pairs, npairs, jobs, njobs, window, counter, true, qxy, qoff, qlen, nqueries, cxy, coff, clen,
+                    ncands, maxlen, eps, per_cu, lanes_per_pair, nullptr, out, stream);
+}
+
+extern "C" int gat_edr_pairs(const int32_t* pairs, const uint64_t* live, int64_t capacity, int32_t* counter,
+                             const float* qxy, const int64_t* qoff, const int32_t* qlen, int32_t nqueries,
+                             const float* cxy, const int64_t* coff, const int32_t* clen, int32_t ncands,
+                             int32_t maxlen, double eps, int32_t lanes_per_pair, uint64_t* cells, uint32_t* stamp,
+                             int32_t* out, void* stream) {
+  GAT_REQUIRE(capacity >= 0 && capacity <= int64_t(INT32_MAX) - 8 && nqueries >= 0 && ncands >= 0,
+              "EDR pairs: bad sizes");
+  GAT_REQUIRE(lanes_per_pair == 64 || lanes_per_pair == 128 || lanes_per_pair == 256 || lanes_per_pair == 512,
+              "EDR pairs: lanes_per_pair must be 64, 128, 256 or 512");
+  if (capacity == 0) return GAT_OK;
+  GAT_REQUIRE(pairs && live && counter && qxy && qoff && qlen && cxy && coff && clen && out && cells,
+              "EDR pairs: null pointer");
+  GAT_REQUIRE(maxlen >= 1 && maxlen <= GAT_MAX_TRAJ_LEN, "EDR pairs: maxlen outside 1..%d", GAT_MAX_TRAJ_LEN);
+  GAT_REQUIRE(eps > 0, "EDR pairs: eps must be positive");
+  return launch_edr(reinterpret_cast<const int2*>(pairs), capacity, nullptr, capacity, nullptr, counter,
+                    reinterpret_cast<const float2*>(qxy), qoff, qlen, nqueries, reinterpret_cast<const float2*>(cxy),
+                    coff, clen, ncands, maxlen, gat_eps_threshold(eps), 0, lanes_per_pair, out,
+                    RawPairs{reinterpret_cast<const unsigned long long*>(live),
+                             reinterpret_cast<unsigned long long*>(cells), stamp},
+                    gat::as_stream(stream));
+}
+
 extern "C" int gat_edr_jobs(const int32_t* pairs, const uint64_t* count, int64_t capacity, const int32_t* qlen,
                             int32_t nq, const int32_t* clen, int32_t nc, int32_t split, int32_t waves,
                             int32_t every_long, int32_t* sorted, int32_t* origin, int32_t* scratch,
@@ -1555,7 +2058,6 @@ extern "C" int gat_edr_jobs(const int32_t* pairs, const uint64_t* count, int64_t
   GAT_REQUIRE(split >= 1 && split <= GAT_MAX_TRAJ_LEN && waves >= 1 && waves <= 8, "EDR jobs: bad rules");
   GAT_REQUIRE(pairs && count && qlen && clen && sorted && scratch && jobs && windows && status && cells,
               "EDR jobs: null pointer");
-  if (int rc = gat_fill_u32(reinterpret_cast<uint32_t*>(status), 0u, 1, stream)) return rc;
   const JobRules rules{split, waves, every_long ? 1 : 0, int32_t(gat::cu_count())};
   hipStream_t s = gat::as_stream(stream);
   const auto* P = reinterpret_cast<const int2*>(pairs);
@@ -1570,17 +2072,17 @@ extern "C" int gat_edr_jobs(const int32_t* pairs, const uint64_t* count, int64_t
     return GAT_OK;
   }
   // Scratch after the (n, m) pairs (8-byte aligned: 2 * capacity words): the
-  // several-wave threshold, bin totals, bin cursors, group starts, group job
+  // longest schedule and the spread work, bin totals, bin cursors, group starts, group job
   // offsets.
-  static_assert(2 + 2 * kSortBins + 2 * (kJobGroups + 1) <= kJobsScratchExtra, "job scratch");
+  static_assert(4 + 2 * kSortBins + 2 * (kJobGroups + 1) <= kJobsScratchExtra, "job scratch");
   auto* crit = reinterpret_cast<unsigned long long*>(scratch + 2 * capacity);
-  uint32_t* gbins = reinterpret_cast<uint32_t*>(scratch + 2 * capacity + 2);
+  uint32_t* gbins = reinterpret_cast<uint32_t*>(scratch + 2 * capacity + 4);
   uint32_t* gcur = gbins + kSortBins;
   uint32_t* gstart = gcur + kSortBins;
   uint32_t* gjobs = gstart + kJobGroups + 1;
-  if (int rc = gat_fill_u32(gbins, 0u, kSortBins, stream)) return rc;
+  if (int rc = gat_fill_u32(reinterpret_cast<uint32_t*>(crit), 0u, 4 + kSortBins, stream)) return rc;
+  if (int rc = gat_fill_u32(reinterpret_cast<uint32_t*>(status), 0u, 1, stream)) return rc;
   if (int rc = gat_fill_u32(reinterpret_cast<uint32_t*>(cells), 0u, 2, stream)) return rc;
-  if (int rc = gat_fill_u32(reinterpret_cast<uint32_t*>(crit), 0u, 2, stream)) return rc;
   int64_t blocks = (capacity + 4095) / 4096;
   const int64_t most = int64_t(gat::cu_count()) * 4;
   if (blocks > most) blocks = most;

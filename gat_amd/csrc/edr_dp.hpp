@@ -32,6 +32,11 @@ namespace edr {
 constexpr int kBlk = 16;    // steps per feed block
 constexpr int kPad = 16;    // NaN points before every trajectory of a padded store
 constexpr int kLaneRows = 4;  // most rows per lane
+// Where column 0 lies in a strip's row: columns back to 2 - SEG are stored, and
+// a 64-lane pair's blocks read from a multiple of four values on (column 1).
+constexpr int kOff64 = 67;
+template <int SEG>
+constexpr int kRowOff = SEG == 64 ? kOff64 : SEG;
 
 // Stores of different lanes to one LDS column come from different steps'
 // store instructions, and the row left behind is the last lane's only if those
@@ -54,6 +59,27 @@ __device__ __forceinline__ int shift_in(int old, int src) {
 }
 
 __device__ __forceinline__ float2 nan_point() { return make_float2(__builtin_nanf(""), __builtin_nanf("")); }
+
+// Point i of the n >= 1 points at P, one that matches nothing when i lies
+// outside them.  The load is unconditional (clamped): behind a branch its value
+// would be waited for at the branch's end, one memory latency per point.
+__device__ __forceinline__ float2 point_or_nan(const float2* P, int i, int n) {
+  // (The byte offset fits 32 bits, so a scalar P needs no 64-bit address.)
+  const uint32_t at = uint32_t(min(max(i, 0), n - 1)) * uint32_t(sizeof(float2));
+  const float2 v = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(P) + at);
+  return make_float2(uint32_t(i) < uint32_t(n) ? v.x : __builtin_nanf(""), v.y);
+}
+
+// The same for i >= 0; in a padded store (!kGuard) point n is a NaN point.
+template <bool kGuard>
+__device__ __forceinline__ float2 point_up_to(const float2* P, int i, int n) {
+  if constexpr (kGuard) {
+    return point_or_nan(P, i, n);
+  } else {
+    return *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(P) +
+                                            uint32_t(min(i, n)) * uint32_t(sizeof(float2)));
+  }
+}
 
 // Box tests of point sets by (xmin, ymin, xmax, ymax).  Float subtraction is
 // monotone, so for points a in box q and b in box c, fl(b.x - a.x) >=
@@ -91,6 +117,8 @@ __device__ __forceinline__ float4 segment_box(float4 b) {
 
 __device__ __forceinline__ float4 empty_box() { return make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY); }
 
+// (A point of NaN x and finite y may widen the box in y only, which tests more
+// and skips nothing that matches.)
 __device__ __forceinline__ float4 grow(const float4& b, const float2& p) {
   return make_float4(fminf(b.x, p.x), fminf(b.y, p.y), fmaxf(b.z, p.x), fmaxf(b.w, p.y));
 }
@@ -111,11 +139,12 @@ struct LaneRows {
     up = 0;
   }
   // Rows first .. first + K - 1 (0-based points) of the trajectory R of n points.
+  template <bool kGuard>
   __device__ __forceinline__ float4 load(const float2* R, int n, int first) {
     float4 b = empty_box();
 #pragma unroll
     for (int i = 0; i < K; ++i) {
-      const float2 p = first + i < n ? R[first + i] : nan_point();
+      const float2 p = point_up_to<kGuard>(R, first + i, n);
       rx[i] = p.x;
       ry[i] = p.y;
       b = grow(b, p);
@@ -153,9 +182,15 @@ struct LaneRows {
   }
 };
 
+// The type of a strip's row in LDS: 16 bits where four pairs share a wave; a
+// 64-lane pair's row is read in 16-byte pieces, and 32-bit values need no
+// unpacking (an instruction per step).
+template <int SEG>
+using RowValue = std::conditional_t<SEG == 64, int32_t, int16_t>;
+
 // One strip: rows row0 + 1 .. row0 + SEG * K of every segment's pair across
 // all its columns.  `above` holds E of the row above the strip by column
-// (interleaved across the wave's segments, [column + SEG][segment]); it is
+// (interleaved across the wave's segments, [column + kRowOff][segment]); it is
 // read once per step as a broadcast, lane 0 of a segment taking it as the
 // `old` operand of the shift, and every lane stores its bottom row's value
 // into it at its own column.  The last lane stores each column last, so the
@@ -173,14 +208,14 @@ struct LaneRows {
 template <int SEG, int K, bool kGuard>
 __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2* C, int m, int row0, int mmax,
                                             const int (&ns)[64 / SEG], const int (&ms)[64 / SEG], const float4& colbox,
-                                            float u, int16_t (*above)[64 / SEG], int seg, int l, int& res,
+                                            float u, RowValue<SEG> (*above)[64 / SEG], int seg, int l, int& res,
                                             bool& mine) {
   constexpr int kSegs = 64 / SEG;
-  constexpr int kOff = SEG;
+  constexpr int kOff = kRowOff<SEG>;
   constexpr uint32_t kWindow = SEG == 16 ? 0x3u : 0x1Fu;  // chunks a block's lanes reach back over
   LaneRows<K> rows;
   rows.start();
-  const float4 rowbox = segment_box<SEG>(rows.load(R, n, row0 + l * K));
+  const float4 rowbox = segment_box<SEG>(rows.template load<kGuard>(R, n, row0 + l * K));
   // Row n inside this strip: its lane, its row of the lane and the step its
   // last column comes at; the same per segment, wave-uniform.
   const int loc = n - 1 - row0;
@@ -198,10 +233,7 @@ __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2
   const float2* cp = C - l;  // column point of step t is cp[t]
   auto column = [&](int t) __attribute__((always_inline)) -> float2 {
     if constexpr (kGuard) {
-      const int i = t - l;
-      const bool in = uint32_t(i) < uint32_t(m);
-      const float2 v = C[in ? i : 0];
-      return in ? v : nan_point();
+      return point_or_nan(C, t - l, m);
     } else {
       return cp[t];
     }
@@ -209,11 +241,11 @@ __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2
   float2 src[kBlk];
   auto block = [&](auto near_c, auto cap_c, int t0) __attribute__((always_inline)) {
     constexpr bool kNear = decltype(near_c)::value, kCap = decltype(cap_c)::value;
-    const int16_t(*feed)[kSegs] = &above[kOff + t0 + 1];
+    const RowValue<SEG>(*feed)[kSegs] = &above[kOff + t0 + 1];
     int fv[kBlk];
 #pragma unroll
     for (int j = 0; j < kBlk; ++j) fv[j] = feed[j][seg];
-    int16_t(*own)[kSegs] = &above[kOff + t0 - l + 1];
+    RowValue<SEG>(*own)[kSegs] = &above[kOff + t0 - l + 1];
 #pragma unroll
     for (int j = 0; j < kBlk; ++j) {
       const int u0 = shift_in<SEG>(fv[j], rows.e[K - 1]);
@@ -225,7 +257,7 @@ __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2
 #pragma unroll
         for (int i = 0; i < K; ++i) res = (t0 + j == tcap && i == ic) ? rows.e[i] : res;
       }
-      own[j][seg] = int16_t(rows.e[K - 1]);
+      own[j][seg] = RowValue<SEG>(rows.e[K - 1]);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -240,7 +272,7 @@ __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2
       rows.template step<true>(u0, p, u);
 #pragma unroll
       for (int i = 0; i < K; ++i) res = (t == tcap && i == ic) ? rows.e[i] : res;
-      above[kOff + t - l + 1][seg] = int16_t(rows.e[K - 1]);
+      above[kOff + t - l + 1][seg] = RowValue<SEG>(rows.e[K - 1]);
     }
   };
   auto captures = [&](int t0) __attribute__((always_inline)) -> bool {
@@ -263,8 +295,7 @@ __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2
   }
   // Chunk b: columns 16 b .. 16 b + 15 of each segment, one per lane of a row.
   auto chunk = [&](int b) __attribute__((always_inline)) -> float2 {
-    const int i = b * kBlk + (l & 15);
-    return i < m ? C[i] : nan_point();
+    return point_up_to<kGuard>(C, b * kBlk + (l & 15), m);
   };
   auto touches = [&](const float2& p) __attribute__((always_inline)) -> uint32_t {
     const float4 cb = segment_box<16>(grow(empty_box(), p));
@@ -310,7 +341,7 @@ __device__ __forceinline__ float4 columns_box(const float2* C, int m, int l) {
 template <int SEG, bool kGuard>
 __device__ __forceinline__ int sweep_pairs(const float2* R, int n, const float2* C, int m, int nmax, int mmax,
                                            const int (&ns)[64 / SEG], const int (&ms)[64 / SEG], float u,
-                                           int16_t (*above)[64 / SEG], int seg, int l, bool* mine) {
+                                           RowValue<SEG> (*above)[64 / SEG], int seg, int l, bool* mine) {
   const float4 colbox = columns_box<SEG>(C, m, l);
   int res = 0;
   bool got = false;

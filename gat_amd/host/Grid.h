@@ -184,7 +184,13 @@ class Grid {
 
  private:
   int buildNode(int level, int id);
-  int ensureQueryStore(const TrajectoryView& queries);
+  // Queues the queries' upload on the engine's stream (the staging memory is
+  // in use until that stream is next waited for); ctlWords > 0 also clears as
+  // many control words of topCtl_ and records the time there.
+  int ensureQueryStore(const TrajectoryView& queries, int64_t ctlWords = 0);
+  int waitQueries();
+  // The all-mismatch table and its by-length form on the device.
+  int ensureDeviceTables();
   int checkTrajLengths(const char* what) const;
   int runBatched(std::vector<int32_t>& pairs, int queryNum, std::vector<int32_t>& dist, EdrBatchStats* stats);
   // Pinned arena bytes runBatched takes for np pairs (its callers begin() it).
@@ -198,8 +204,18 @@ class Grid {
   // take the host-built path instead (a query with more survivors than the
   // device's per-query sort holds).
   int similarityOnDevice(int nq, int kValue, std::vector<TopK>& out, EdrBatchStats* st, bool* done);
-  // The DP launches over a device-built job list (windows in win).
-  int launchDeviceBuckets(int64_t cap, int nq, const int32_t* win);
+  // The same for batches of few queries, whose time is their launches and the
+  // longest pair: no job list (every survivor takes several waves), the merge
+  // straight from the pairs, results written to pinned memory.  *done is
+  // false when more pairs survive than it is for.
+  int similaritySmall(const TrajectoryView& queries, int kValue, std::vector<TopK>& out, EdrBatchStats* st,
+                      bool* done);
+  static constexpr int64_t kUploadPart = 1 << 17;  // points of a part of the queries' upload
+  static constexpr int kSmallTopkQueries = 32;
+  static constexpr int64_t kSmallTopkPairs = 2048;
+  // The DP launches over a device-built job list (windows in win, a cleared job
+  // counter per bucket; the first launch records the time in stamp).
+  int launchDeviceBuckets(int64_t cap, int nq, const int32_t* win, int32_t* counters, uint32_t* stamp);
   // Batched EDR with the job list built on the device (pairsHost null: every
   // query x trajectory pair); dist in the pairs' order.
   int runBatchedOnDevice(const int32_t* pairsHost, int64_t np, int queryNum, std::vector<int32_t>& dist,
@@ -237,7 +253,15 @@ class Grid {
   // windows + status + cell count, and the DP's job counters.
   DeviceBuffer sortedDev_, nmDev_, windowsDev_, dpCounterDev_, originDev_, unsortDev_;
   int64_t deviceTopkCap_ = 0;  // survivor capacity of the device path, grown on overflow
-  EventTimer edrTimer_, filterTimer_, mergeTimer_;
+  // similaritySmall: control words on the device, the results and the control
+  // words in pinned memory; the survivors per query of the last batches.
+  DeviceBuffer topCtl_, lenTableDev_;
+  PinnedBuffer topHost_;
+  double survivorsPerQuery_ = 0;
+  bool queryPending_ = false;
+  int32_t clockKhz_ = 0;
+  int maxTrajLen_ = 1;
+  EventTimer edrTimer_, mergeTimer_;
   SideStream edrSide_;  // the longest EDR bucket runs here, beside the others
   SideStream edrSide2_;  // one-wave long pairs of a batch whose longest run over several waves
   std::vector<int32_t> trajLenHost_, queryLenHost_;

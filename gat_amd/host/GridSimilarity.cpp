@@ -67,9 +67,13 @@ int upload_vec(DeviceBuffer& d, const std::vector<T>& v, void* s, const char* wh
 
 int strips_of(int n) { return (n + 15) / 16; }
 
-// What a pair keeps its wave busy for on one wave and over several, in VALU
-// instructions per 16-step block (gat_edr_jobs applies the same rule on the
-// device).
+// What a pair keeps its wave busy for in a 16-lane segment, on one wave and
+// over several, in VALU instructions per 16-step block (gat_edr_jobs applies
+// the same rules on the device).
+int64_t segment_cost(int n, int m) {
+  const int rows = (n + 15) / 16, rest = rows & 3;
+  return int64_t((m + 15 + 15) / 16) * (19 * (rows / 4) + (rest >= 2 ? 11 : 0) + ((rest & 1) ? 7 : 0));
+}
 int64_t one_wave_cost(int n, int m) {
   const int rows = (n + 63) / 64, rest = rows & 3;
   return int64_t((m + 63 + 15) / 16) * (19 * (rows / 4) + (rest >= 2 ? 11 : 0) + ((rest & 1) ? 7 : 0));
@@ -89,6 +93,8 @@ int Grid::uploadTrajectories(const TrajectoryView& db) {
   Padded p = pad_store(db);
   trajLenHost_ = p.lengths;
   badTrajLen_ = 0;
+  maxTrajLen_ = 1;
+  for (int t = 0; t < T; ++t) maxTrajLen_ = std::max(maxTrajLen_, trajLenHost_[t]);
   for (int t = 0; t < T && badTrajLen_ == 0; ++t)
     if (trajLenHost_[t] < 1 || trajLenHost_[t] > GAT_MAX_TRAJ_LEN) badTrajLen_ = t + 1;
   std::vector<gat_edr_task> tasks(static_cast<size_t>(T));
@@ -228,7 +234,13 @@ int Grid::filterPairs(int nq, int64_t cap, void* stream) {
   return GAT_OK;
 }
 
-int Grid::ensureQueryStore(const TrajectoryView& q) {
+int Grid::waitQueries() {
+  if (queryPending_) GATH_TRY(gat_stream_sync(engine_.stream()), "query upload");
+  queryPending_ = false;
+  return GAT_OK;
+}
+
+int Grid::ensureQueryStore(const TrajectoryView& q, int64_t ctlWords) {
   for (int i = 0; i < q.trajNum; ++i) {
     const int64_t len = q.offsets[i + 1] - q.offsets[i];
     if (len < 1 || len > GAT_MAX_TRAJ_LEN) {
@@ -236,11 +248,11 @@ int Grid::ensureQueryStore(const TrajectoryView& q) {
       return GAT_ERR_ARG;
     }
   }
-  // The offsets, then the raw coordinates, go up from pinned memory in two
-  // DMAs (the second, of the latitudes, copied on the host while the first
-  // runs), and the device packs the padded store and the boxes
-  // (gat_edr_pack_trajectories).  The offsets and lengths the kernels read
-  // are views into the same device buffer.
+  // Everything is laid out in pinned memory, from where one kernel
+  // (gat_edr_stage_queries) writes the device's copies, the padded store and
+  // the boxes.  The offsets and lengths the kernels read are views into one
+  // device buffer.
+  if (int rc = waitQueries()) return rc;
   const int T = q.trajNum;
   const int64_t o0 = T > 0 ? q.offsets[0] : 0;
   const int64_t n = T > 0 ? q.offsets[T] - o0 : 0;
@@ -270,26 +282,37 @@ int Grid::ensureQueryStore(const TrajectoryView& q) {
   }
   src[T] = n;
   void* s = engine_.stream();
-  if (int rc = queryUp_.reserve(std::max<size_t>(meta + 2 * braw, 16))) return rc;
+  if (int rc = queryUp_.reserve(std::max<size_t>(meta, 16))) return rc;
   char* dev = queryUp_.as<char>();
-  if (n > 0) std::memcpy(lon, q.lon + o0, size_t(n) * 4);
-  GATH_TRY(gat_memcpy_h2d(dev, base, meta + braw, s), "query upload");
-  if (n > 0) {
-    std::memcpy(lat, q.lat + o0, size_t(n) * 4);
-    GATH_TRY(gat_memcpy_h2d(dev + meta + braw, lat, braw, s), "query upload");
-  }
   querySrcOffDev_ = reinterpret_cast<const int64_t*>(dev);
   queryOff64Dev_ = reinterpret_cast<const int64_t*>(dev + bsrc);
   queryOffDev_ = reinterpret_cast<const int32_t*>(dev + bsrc + b64);
   queryLenDev_ = reinterpret_cast<const int32_t*>(dev + bsrc + b64 + b32);
   if (int rc = queryXY_.reserve(size_t(total) * 8)) return rc;
   if (int rc = queryBox_.reserve(std::max<size_t>(size_t(T) * 16, 16))) return rc;
-  const float* rlon = reinterpret_cast<const float*>(dev + meta);
-  const float* rlat = reinterpret_cast<const float*>(dev + meta + braw);
-  GATH_TRY(gat_edr_pack_trajectories(rlon, rlat, querySrcOffDev_, queryOff64Dev_, T, total, queryXY_.as<float>(),
-                                     queryBox_.as<float>(), s),
-           "query packing");
-  GATH_TRY(gat_stream_sync(s), "query upload");
+  if (ctlWords > 0)
+    if (int rc = topCtl_.reserve(size_t(ctlWords) * 4 + 8)) return rc;
+  queryPending_ = true;
+  // In parts, each on its way to the device while the host copies the next: of
+  // 1,024 queries of 4.2 MB the upload takes 84 us and the copying twice that.
+  int t0 = 0;
+  do {
+    int t1 = t0;
+    while (t1 < T && src[t1] - src[t0] < kUploadPart) ++t1;
+    const int64_t p0 = src[t0], p1 = src[t1];
+    if (p1 > p0) {
+      std::memcpy(lon + p0, q.lon + o0 + p0, size_t(p1 - p0) * 4);
+      std::memcpy(lat + p0, q.lat + o0 + p0, size_t(p1 - p0) * 4);
+    }
+    const bool first = t0 == 0, last = t1 == T;
+    uint32_t* ctl = first && ctlWords > 0 ? topCtl_.as<uint32_t>() : nullptr;
+    GATH_TRY(gat_edr_stage_queries(base, first ? int64_t(meta) : 0, dev, src + t0, off64 + t0, t1 - t0, p1, lon, lat,
+                                   last ? total : off64[t1] - GAT_EDR_PAD, queryXY_.as<float>(),
+                                   queryBox_.as<float>() + 4 * size_t(t0), ctl, ctl ? ctlWords : 0,
+                                   ctl ? ctl + ctlWords : nullptr, s),
+             "query upload");
+    t0 = t1;
+  } while (t0 < T);
   return GAT_OK;
 }
 
@@ -375,13 +398,26 @@ int Grid::edrAll(const float* qlon, const float* qlat, int qlen, int32_t* dist) 
 
 // ------------------------------------------------------------------ batched
 
+int Grid::ensureDeviceTables() {
+  if (lenTableDev_.size() > 0) return GAT_OK;
+  const size_t w = GAT_MAX_TRAJ_LEN + 1;
+  void* s = engine_.stream();
+  DeviceBuffer byLength;
+  if (int rc = ftableDev_.reserve(w * w * 4)) return rc;
+  if (int rc = byLength.reserve(w * w * 4)) return rc;
+  GATH_TRY(gat_edr_mismatch_table(GAT_MAX_TRAJ_LEN, ftableDev_.as<int32_t>(), s), "mismatch table");
+  GATH_TRY(gat_edr_length_table(ftableDev_.as<int32_t>(), int32_t(w), byLength.as<int32_t>(), s), "length table");
+  lenTableDev_ = std::move(byLength);
+  return GAT_OK;
+}
+
 const std::vector<int32_t>& Grid::mismatchTable() {
   if (!ftable_.empty()) return ftable_;
   const size_t w = GAT_MAX_TRAJ_LEN + 1;
   void* s = engine_.stream();
   std::vector<int32_t> t(w * w);
-  if (ftableDev_.reserve(w * w * 4) == GAT_OK && gat_edr_mismatch_table(GAT_MAX_TRAJ_LEN, ftableDev_.as<int32_t>(), s) == GAT_OK &&
-      gat_memcpy_d2h(t.data(), ftableDev_.get(), w * w * 4, s) == GAT_OK && gat_stream_sync(s) == GAT_OK)
+  if (ensureDeviceTables() == GAT_OK && gat_memcpy_d2h(t.data(), ftableDev_.get(), w * w * 4, s) == GAT_OK &&
+      gat_stream_sync(s) == GAT_OK)
     ftable_.swap(t);
   else
     gath_fail_hip(GAT_ERR_HIP, "mismatch table");
@@ -432,19 +468,21 @@ int Grid::runBatched(std::vector<int32_t>& pairs, int queryNum, std::vector<int3
       return GAT_ERR_ARG;
     }
   }
-  // In a one-round batch with several waves per long pair, only the pairs
-  // that would outlast the batch's longest pair on one wave take several: the
-  // batch cannot end before its longest pair's pipelined schedule does.  The
-  // rest run one pair per wave, beside it; several waves on a pair of fewer
-  // strips than waves leave the surplus waves idle at every barrier.
+  // A one-round batch cannot end before its longest pair's schedule does, nor
+  // before its work spread over all SIMDs: each pair takes the cheapest form
+  // (16-lane segment, one wave, several) that ends within `critical`, the
+  // rules of gat_edr_jobs.
   const bool multiWave = latencyBound && waves > 1;
-  int64_t critical = 0;
-  if (multiWave)
+  int64_t schedule = 0, work = 0;
+  if (latencyBound)
     for (int64_t i = 0; i < np; ++i) {
       const int a = queryLenHost_[pairs[2 * i]], b = trajLenHost_[pairs[2 * i + 1]];
       const int n = std::min(a, b), m = std::max(a, b);
-      if (m > mid) critical = std::max(critical, pipe_cost(n, m, waves));
+      if (n < 1) continue;
+      schedule = std::max(schedule, multiWave ? pipe_cost(n, m, waves) : one_wave_cost(n, m));
+      work += segment_cost(n, m);
     }
+  const int64_t critical = std::max(schedule, work / (4 * 4 * cus) / 2);
   std::vector<int32_t> key(static_cast<size_t>(np));
   int64_t cells = 0;
   int maxlen[kBuckets] = {1, 1, 1, 1};
@@ -453,9 +491,10 @@ int Grid::runBatched(std::vector<int32_t>& pairs, int queryNum, std::vector<int3
     const int n = std::min(a, b), m = std::max(a, b);
     cells += int64_t(n) * m;
     int bucket = m <= split ? 0 : m <= mid ? 1 : 2;
-    if (bucket == 2 && multiWave &&
-        (edrWavesEveryLongPair || one_wave_cost(n, m) > critical))
-      bucket = 3;
+    if (latencyBound && n >= 1) {
+      if (bucket == 0 && 2 * segment_cost(n, m) > critical) bucket = 2;
+      if (bucket == 2 && multiWave && (edrWavesEveryLongPair ? m > split : one_wave_cost(n, m) > critical)) bucket = 3;
+    }
     maxlen[bucket] = std::max(maxlen[bucket], std::min(m, GAT_MAX_TRAJ_LEN));
     key[i] = (bucket * kS + (kS - 1 - strips_of(n))) * kM + (kM - 1 - m);
   }
@@ -656,19 +695,19 @@ int Grid::deviceTopk(const std::vector<int32_t>& pairs, const std::vector<int32_
 // the windows in win): one launch per bucket reading its window on the
 // device, buckets 3 (several waves per pair) and 2 (one pair per wave) on side
 // streams beside the short buckets, as runBatched launches them.
-int Grid::launchDeviceBuckets(int64_t cap, int nq, const int32_t* win) {
+int Grid::launchDeviceBuckets(int64_t cap, int nq, const int32_t* win, int32_t* counters, uint32_t* stamp) {
   void* s = engine_.stream();
   const int split = std::max(1, std::min(edrSplit, GAT_MAX_TRAJ_LEN));
   const int waves = (edrWavesPerPair == 2 || edrWavesPerPair == 4 || edrWavesPerPair == 8) ? edrWavesPerPair : 1;
   auto launch = [&](int bucket, void* stream) -> int {
     const int maxlen = bucket == 0 ? split : bucket == 1 ? std::max(split, 1024) : GAT_MAX_TRAJ_LEN;
-    GATH_TRY(gat_edr_batched(sortedDev_.as<int32_t>(), cap, jobsDev_.as<gat_edr_job>(), cap + 4, win + 2 * bucket,
-                             dpCounterDev_.as<int32_t>() + bucket, queryXY_.as<float>(), queryOff64Dev_,
-                             queryLenDev_, nq, trajXY_.as<float>(), trajOff_.as<int64_t>(),
-                             trajLen_.as<int32_t>(), trajNum, maxlen, epsilon,
-                             bucket == 0 ? edrPerCuShort : bucket == 1 ? edrPerCuLong : 0,
-                             bucket == 3 ? 64 * waves : bucket == 2 ? 64 : 16, outDev_.as<int32_t>(), stream),
+    GATH_TRY(gat_edr_bucket(sortedDev_.as<int32_t>(), cap, jobsDev_.as<gat_edr_job>(), cap + 4, win + 2 * bucket,
+                            counters + bucket, queryXY_.as<float>(), queryOff64Dev_, queryLenDev_, nq,
+                            trajXY_.as<float>(), trajOff_.as<int64_t>(), trajLen_.as<int32_t>(), trajNum, maxlen,
+                            epsilon, bucket == 0 ? edrPerCuShort : bucket == 1 ? edrPerCuLong : 0,
+                            bucket == 3 ? 64 * waves : bucket == 2 ? 64 : 16, stamp, outDev_.as<int32_t>(), stream),
              "batched EDR");
+    stamp = nullptr;  // the first launch records the start
     return GAT_OK;
   };
   if (int rc = edrSide_.fork(s)) return rc;
@@ -740,7 +779,8 @@ int Grid::runBatchedOnDevice(const int32_t* pairsHost, int64_t np, int queryNum,
            "device jobs");
   const double h1 = now_ms();
   if (int rc = edrTimer_.start(s)) return rc;
-  if (int rc = launchDeviceBuckets(np, queryNum, win)) return rc;
+  GATH_TRY(gat_fill_u32(dpCounterDev_.as<uint32_t>(), 0u, 4, s), "batched EDR");
+  if (int rc = launchDeviceBuckets(np, queryNum, win, dpCounterDev_.as<int32_t>(), nullptr)) return rc;
   if (int rc = edrTimer_.stop(s)) return rc;
   GATH_TRY(gat_edr_unsort(originDev_.as<int32_t>(), outDev_.as<int32_t>(), count, np, unsortDev_.as<int32_t>(), s),
            "distance order");
@@ -772,15 +812,33 @@ int Grid::runBatchedOnDevice(const int32_t* pairsHost, int64_t np, int queryNum,
   return GAT_OK;
 }
 
+// A batch's control words (topCtl_, cleared by the upload; the merge or a copy
+// brings them back): [0, 1] survivors, [2] lists and [3] merge status (as
+// gat_edr_merge's), [4, 5] cells, [6] the job counter of gat_edr_pairs, [7]
+// ticket, [8] job list status, [10, 16) the clock at the filter, the DP and the
+// merge, [16, 24) the buckets' windows, [24, 28) their job counters; after them
+// the clock at the upload (device) or at the end (host).
+namespace {
+constexpr int kCtlWords = 32;
+uint64_t ctl64(const uint32_t* c, int w) { return uint64_t(c[w]) | (uint64_t(c[w + 1]) << 32); }
+}  // namespace
+
 // The batch chained on the device: the filter writes the survivors,
 // gat_edr_jobs groups them into the DP's length buckets and jobs, the DP
-// launches read their job windows on the device, gat_edr_survivor_lists builds
-// each query's list and gat_edr_topk merges; one readback at the end carries
-// the results and the statuses.  A survivor count above the capacity empties
-// every window: the capacity grows and the batch runs again.
+// launches read their job windows on the device, and gat_edr_merge merges; the
+// results and the statuses are in pinned memory at the end.  Every workgroup of
+// that merge reads every pair, which is the cheaper way up to about 2^25 reads
+// in all: gat_edr_survivor_lists (one workgroup) and gat_edr_topk took 113 us
+// for 1,024 queries with 9,000 pairs, the merge takes 56.  A larger batch, and
+// one whose queries have more survivors than the merge sorts in LDS, takes
+// those two.  A survivor count above the capacity empties every window: the
+// capacity grows and the batch runs again.
 int Grid::similarityOnDevice(int nq, int kValue, std::vector<TopK>& out, EdrBatchStats* st, bool* done) {
-  *done = false;
+  *done = nq == 0;
+  out.clear();
+  if (nq == 0) return GAT_OK;
   void* s = engine_.stream();
+  if (clockKhz_ == 0) GATH_TRY(gat_wall_clock_khz(&clockKhz_), "device clock");
   int64_t eligible = 0;
   for (int L = 1; L <= GAT_MAX_TRAJ_LEN; ++L) eligible += int64_t(lengthIds_[L].size());
   const int kk = int(std::min<int64_t>(kValue, eligible));
@@ -788,92 +846,103 @@ int Grid::similarityOnDevice(int nq, int kValue, std::vector<TopK>& out, EdrBatc
   const int waves = (edrWavesPerPair == 2 || edrWavesPerPair == 4 || edrWavesPerPair == 8) ? edrWavesPerPair : 1;
   const size_t cells = size_t(nq) * size_t(kValue);
   int64_t cap = std::max<int64_t>({deviceTopkCap_, int64_t(nq) * 64, 1024});
-  for (int attempt = 0; attempt < 2; ++attempt) {
+  bool merge = kk > 0 && double(nq) * nq * std::max(survivorsPerQuery_, 8.0) <= double(1 << 25);
+  for (int attempt = 0; attempt < 3; ++attempt) {
     const size_t ns = size_t(nq) + 1;
     if (int rc = pairsDev_.reserve(size_t(cap) * 8)) return rc;
     if (int rc = sortedDev_.reserve(size_t(cap) * 8)) return rc;
     if (int rc = nmDev_.reserve((size_t(cap) * 2 + GAT_EDR_JOBS_SCRATCH_EXTRA) * 4)) return rc;
     if (int rc = jobsDev_.reserve((size_t(cap) + 4) * sizeof(gat_edr_job))) return rc;
     if (int rc = outDev_.reserve(size_t(cap) * 4)) return rc;
-    if (int rc = survDev_.reserve((ns + 2 * size_t(cap)) * 4)) return rc;
-    if (int rc = topDev_.reserve((2 * cells + 1) * 4)) return rc;
-    if (int rc = counterDev_.reserve(16)) return rc;
-    if (int rc = windowsDev_.reserve(64)) return rc;
-    if (int rc = dpCounterDev_.reserve(16)) return rc;
-    // windows: [0..7] bucket windows, [8] status, [10..11] cell count.
-    int32_t* win = windowsDev_.as<int32_t>();
-    auto* cellCount = reinterpret_cast<uint64_t*>(win + 10);
-    if (int rc = filterTimer_.start(s)) return rc;
-    if (int rc = filterPairs(nq, cap, s)) return rc;
-    if (int rc = filterTimer_.stop(s)) return rc;
-    GATH_TRY(gat_edr_jobs(pairsDev_.as<int32_t>(), counterDev_.as<uint64_t>(), cap, queryLenDev_, nq,
-                          trajLen_.as<int32_t>(), trajNum, split, waves, edrWavesEveryLongPair ? 1 : 0,
-                          sortedDev_.as<int32_t>(), nullptr, nmDev_.as<int32_t>(), jobsDev_.as<gat_edr_job>(), win,
-                          win + 8, cellCount, s),
+    if (int rc = topHost_.reserve((2 * cells + kCtlWords + 2) * 4)) return rc;
+    uint32_t* ctl = topCtl_.as<uint32_t>();
+    auto* count = reinterpret_cast<uint64_t*>(ctl);
+    int32_t* win = reinterpret_cast<int32_t*>(ctl + 16);
+    if (attempt > 0) GATH_TRY(gat_fill_u32(ctl, 0u, kCtlWords, s), "control words");
+    GATH_TRY(gat_edr_filter_grid_add(queryBox_.as<float>(), nq, trajBox_.as<float>(), trajNum, &candGrid_, epsilon,
+                                     pairsDev_.as<int32_t>(), cap, count, ctl + 10, s),
+             "candidate filter");
+    GATH_TRY(gat_edr_jobs(pairsDev_.as<int32_t>(), count, cap, queryLenDev_, nq, trajLen_.as<int32_t>(), trajNum,
+                          split, waves, edrWavesEveryLongPair ? 1 : 0, sortedDev_.as<int32_t>(), nullptr,
+                          nmDev_.as<int32_t>(), jobsDev_.as<gat_edr_job>(), win, reinterpret_cast<int32_t*>(ctl + 8),
+                          reinterpret_cast<uint64_t*>(ctl + 4), s),
              "device jobs");
-    if (int rc = edrTimer_.start(s)) return rc;
-    if (int rc = launchDeviceBuckets(cap, nq, win)) return rc;
-    if (int rc = edrTimer_.stop(s)) return rc;
-    if (int rc = mergeTimer_.start(s)) return rc;
-    int32_t* sv = survDev_.as<int32_t>();
-    GATH_TRY(gat_edr_survivor_lists(sortedDev_.as<int32_t>(), outDev_.as<int32_t>(), counterDev_.as<uint64_t>(), cap,
-                                    nq, sv, sv + ns, sv + ns + cap, win + 8, s),
-             "survivor lists");
-    int32_t* top = topDev_.as<int32_t>();
-    GATH_TRY(gat_edr_topk(ftableDev_.as<int32_t>(), GAT_MAX_TRAJ_LEN + 1, queryLenDev_, nq,
-                          trajLen_.as<int32_t>(), trajNum, lenIdsDev_.as<int32_t>(), lenOffDev_.as<int32_t>(), sv,
-                          sv + ns, sv + ns + cap, kValue, kk, top, top + cells, top + 2 * cells, s),
-             "top-k merge");
-    if (int rc = mergeTimer_.stop(s)) return rc;
-    if (int rc = stage_.begin((2 * cells + 1) * 4 + 2 * 256, s)) return rc;
-    int32_t* down = stage_.take_as<int32_t>(2 * cells + 1);
-    int32_t* ctl = stage_.take_as<int32_t>(16);
-    if (!down || !ctl) {
-      gath_set_error("device top-k: transfer arena too small");
-      return GAT_ERR_STATE;
+    if (!merge)
+      if (int rc = edrTimer_.start(s)) return rc;
+    if (int rc = launchDeviceBuckets(cap, nq, win, reinterpret_cast<int32_t*>(ctl + 24), ctl + 12)) return rc;
+    if (!merge)
+      if (int rc = edrTimer_.stop(s)) return rc;
+    int32_t* top = topHost_.as<int32_t>();
+    uint32_t* c = reinterpret_cast<uint32_t*>(top + 2 * cells);
+    if (merge) {
+      GATH_TRY(gat_edr_merge(lenTableDev_.as<int32_t>(), GAT_MAX_TRAJ_LEN + 1, queryLenDev_, nq,
+                             trajLen_.as<int32_t>(), trajNum, lenIdsDev_.as<int32_t>(), lenOffDev_.as<int32_t>(),
+                             sortedDev_.as<int32_t>(), outDev_.as<int32_t>(), cap, kValue, kk, top, top + cells, ctl,
+                             c, ctl + 14, s),
+               "top-k merge");
+    } else {
+      if (int rc = survDev_.reserve((ns + 2 * size_t(cap)) * 4)) return rc;
+      if (int rc = topDev_.reserve((2 * cells + 1) * 4)) return rc;
+      if (int rc = mergeTimer_.start(s)) return rc;
+      int32_t* sv = survDev_.as<int32_t>();
+      GATH_TRY(gat_edr_survivor_lists(sortedDev_.as<int32_t>(), outDev_.as<int32_t>(), count, cap, nq, sv, sv + ns,
+                                      sv + ns + cap, reinterpret_cast<int32_t*>(ctl + 2), s),
+               "survivor lists");
+      int32_t* dev = topDev_.as<int32_t>();
+      GATH_TRY(gat_edr_topk(lenTableDev_.as<int32_t>(), GAT_MAX_TRAJ_LEN + 1, queryLenDev_, nq,
+                            trajLen_.as<int32_t>(), trajNum, lenIdsDev_.as<int32_t>(), lenOffDev_.as<int32_t>(), sv,
+                            sv + ns, sv + ns + cap, kValue, kk, dev, dev + cells, dev + 2 * cells, s),
+               "top-k merge");
+      if (int rc = mergeTimer_.stop(s)) return rc;
+      GATH_TRY(gat_memcpy_d2h(top, dev, 2 * cells * 4, s), "top-k readback");
+      GATH_TRY(gat_memcpy_d2h(c, ctl, kCtlWords * 4, s), "top-k readback");
+      GATH_TRY(gat_memcpy_d2h(c + 3, dev + 2 * cells, 4, s), "top-k readback");
     }
-    GATH_TRY(gat_memcpy_d2h(down, topDev_.get(), (2 * cells + 1) * 4, s), "top-k readback");
-    GATH_TRY(gat_memcpy_d2h(ctl, windowsDev_.get(), 48, s), "top-k readback");
-    GATH_TRY(gat_memcpy_d2h(ctl + 12, counterDev_.get(), 8, s), "top-k readback");
     GATH_TRY(gat_stream_sync(s), "top-k readback");
-    uint64_t count = 0;
-    std::memcpy(&count, ctl + 12, 8);
-    const int32_t status = ctl[8];
-    if (status & 1) {  // more survivors than the capacity: grow and run again
-      if (count > uint64_t(INT32_MAX) - 8) {
+    queryPending_ = false;
+    const uint64_t found = ctl64(c, 0);
+    survivorsPerQuery_ = std::max(0.75 * survivorsPerQuery_, double(found) / nq);
+    if (c[8] & 1) {  // more survivors than the capacity: grow and run again
+      if (found > uint64_t(INT32_MAX) - 8) {
         gath_set_error("similarityBatched: %llu candidate pairs pass the filter (at most %d per call; split the "
                        "queries into smaller batches)",
-                       (unsigned long long)count, INT32_MAX - 8);
+                       (unsigned long long)found, INT32_MAX - 8);
         return GAT_ERR_CAPACITY;
       }
-      cap = std::min<int64_t>(int64_t(count) + int64_t(count) / 4 + 1024, INT32_MAX - 8);
+      cap = std::min<int64_t>(int64_t(found) + int64_t(found) / 4 + 1024, INT32_MAX - 8);
       deviceTopkCap_ = cap;
       continue;
     }
-    if (status & 2) return GAT_OK;  // a query's list exceeds the device sort: the host-built path
-    if (down[2 * cells] != 0) {
-      gath_set_error("top-k merge: inconsistent inputs (status %d)", down[2 * cells]);
+    if (c[2] & 2) {  // a query's survivors exceed the merge's sort, or the lists'
+      if (!merge) return GAT_OK;  // the host-built path
+      merge = false;
+      continue;
+    }
+    if (c[3] != 0) {
+      gath_set_error("top-k merge: inconsistent inputs (status %u)", c[3]);
       return GAT_ERR_HIP;
     }
     out.assign(size_t(nq), TopK{});
     for (int q = 0; q < nq; ++q) {
-      out[size_t(q)].ids.assign(down + int64_t(q) * kValue, down + int64_t(q) * kValue + kk);
-      out[size_t(q)].dist.assign(down + cells + int64_t(q) * kValue, down + cells + int64_t(q) * kValue + kk);
+      out[size_t(q)].ids.assign(top + int64_t(q) * kValue, top + int64_t(q) * kValue + kk);
+      out[size_t(q)].dist.assign(top + cells + int64_t(q) * kValue, top + cells + int64_t(q) * kValue + kk);
     }
     if (st) {
-      float fms = 0, dms = 0, mms = 0;
-      if (int rc = filterTimer_.elapsed(&fms)) return rc;
-      if (int rc = edrTimer_.elapsed(&dms)) return rc;
-      if (int rc = mergeTimer_.elapsed(&mms)) return rc;
-      uint64_t c = 0;
-      std::memcpy(&c, ctl + 10, 8);
-      st->pairs += int64_t(count);
-      st->cells += int64_t(c);
-      st->jobs += int64_t(ctl[1]) + ctl[3] + ctl[5] + ctl[7];
-      st->pruned += int64_t(nq) * trajNum - int64_t(count);
-      st->filterMs += fms;
-      st->kernelMs += dms;
-      st->mergeMs += mms;
+      st->pairs += int64_t(found);
+      st->cells += int64_t(ctl64(c, 4));
+      st->jobs += int64_t(c[17]) + c[19] + c[21] + c[23];
+      st->pruned += int64_t(nq) * trajNum - int64_t(found);
+      if (trajNum > 0) st->filterMs += double(ctl64(c, 12) - ctl64(c, 10)) / clockKhz_;
+      if (merge) {
+        st->kernelMs += double(ctl64(c, 14) - ctl64(c, 12)) / clockKhz_;
+        st->mergeMs += double(ctl64(c, kCtlWords) - ctl64(c, 14)) / clockKhz_;
+      } else {
+        float ms = 0;
+        if (int rc = mergeTimer_.elapsed(&ms)) return rc;
+        st->mergeMs += ms;
+        if (int rc = edrTimer_.elapsed(&ms)) return rc;
+        st->kernelMs += ms;
+      }
     }
     *done = true;
     return GAT_OK;
@@ -881,18 +950,89 @@ int Grid::similarityOnDevice(int nq, int kValue, std::vector<TopK>& out, EdrBatc
   return GAT_OK;  // still over capacity after growing once: the host-built path
 }
 
+int Grid::similaritySmall(const TrajectoryView& queries, int kValue, std::vector<TopK>& out, EdrBatchStats* st,
+                          bool* done) {
+  *done = false;
+  const int nq = queries.trajNum;
+  int64_t eligible = 0;
+  for (int L = 1; L <= GAT_MAX_TRAJ_LEN; ++L) eligible += int64_t(lengthIds_[L].size());
+  const int kk = int(std::min<int64_t>(kValue, eligible));
+  if (kk == 0) return GAT_OK;
+  void* s = engine_.stream();
+  const double u0 = now_ms();
+  if (clockKhz_ == 0) GATH_TRY(gat_wall_clock_khz(&clockKhz_), "device clock");
+  if (int rc = ensureQueryStore(queries, kCtlWords)) return rc;
+  if (st) st->uploadMs += now_ms() - u0;
+  if (int rc = ensureDeviceTables()) return rc;
+  const int64_t cap = kSmallTopkPairs;
+  const size_t cells = size_t(nq) * size_t(kValue);
+  if (int rc = pairsDev_.reserve(size_t(cap) * 8)) return rc;
+  if (int rc = outDev_.reserve(size_t(cap) * 4)) return rc;
+  if (int rc = topHost_.reserve((2 * cells + kCtlWords + 2) * 4)) return rc;
+  uint32_t* ctl = topCtl_.as<uint32_t>();
+  auto* count = reinterpret_cast<uint64_t*>(ctl);
+  int longest = maxTrajLen_;
+  for (int q = 0; q < nq; ++q) longest = std::max(longest, queryLenHost_[size_t(q)]);
+  const int waves = (edrWavesPerPair == 2 || edrWavesPerPair == 4 || edrWavesPerPair == 8) ? edrWavesPerPair : 1;
+  GATH_TRY(gat_edr_filter_grid_add(queryBox_.as<float>(), nq, trajBox_.as<float>(), trajNum, &candGrid_, epsilon,
+                                   pairsDev_.as<int32_t>(), cap, count, ctl + 10, s),
+           "candidate filter");
+  GATH_TRY(gat_edr_pairs(pairsDev_.as<int32_t>(), count, cap, reinterpret_cast<int32_t*>(ctl + 6),
+                         queryXY_.as<float>(), queryOff64Dev_, queryLenDev_, nq, trajXY_.as<float>(),
+                         trajOff_.as<int64_t>(), trajLen_.as<int32_t>(), trajNum, longest, epsilon, 64 * waves,
+                         reinterpret_cast<uint64_t*>(ctl + 4), ctl + 12, outDev_.as<int32_t>(), s),
+           "batched EDR");
+  int32_t* top = topHost_.as<int32_t>();
+  GATH_TRY(gat_edr_merge(lenTableDev_.as<int32_t>(), GAT_MAX_TRAJ_LEN + 1, queryLenDev_, nq, trajLen_.as<int32_t>(),
+                         trajNum, lenIdsDev_.as<int32_t>(), lenOffDev_.as<int32_t>(), pairsDev_.as<int32_t>(),
+                         outDev_.as<int32_t>(), cap, kValue, kk, top, top + cells, ctl,
+                         reinterpret_cast<uint32_t*>(top + 2 * cells), ctl + 14, s),
+           "top-k merge");
+  GATH_TRY(gat_stream_sync(s), "top-k readback");
+  queryPending_ = false;
+  const uint32_t* c = reinterpret_cast<const uint32_t*>(top + 2 * cells);
+  const uint64_t found = ctl64(c, 0);
+  survivorsPerQuery_ = std::max(0.75 * survivorsPerQuery_, double(found) / nq);
+  if (found > uint64_t(cap) || c[2] != 0) return GAT_OK;
+  if (c[3] != 0) {
+    gath_set_error("top-k merge: inconsistent inputs (status %u)", c[3]);
+    return GAT_ERR_HIP;
+  }
+  out.assign(size_t(nq), TopK{});
+  for (int q = 0; q < nq; ++q) {
+    out[size_t(q)].ids.assign(top + int64_t(q) * kValue, top + int64_t(q) * kValue + kk);
+    out[size_t(q)].dist.assign(top + cells + int64_t(q) * kValue, top + cells + int64_t(q) * kValue + kk);
+  }
+  if (st) {
+    st->pairs += int64_t(found);
+    st->cells += int64_t(ctl64(c, 4));
+    st->jobs += int64_t(found);
+    st->pruned += int64_t(nq) * trajNum - int64_t(found);
+    st->filterMs += double(ctl64(c, 12) - ctl64(c, 10)) / clockKhz_;
+    st->kernelMs += double(ctl64(c, 14) - ctl64(c, 12)) / clockKhz_;
+    st->mergeMs += double(ctl64(c, kCtlWords) - ctl64(c, 14)) / clockKhz_;
+  }
+  *done = true;
+  return GAT_OK;
+}
+
 int Grid::similarityBatched(const TrajectoryView& queries, int kValue, std::vector<TopK>& out, EdrBatchStats* st) {
   if (int rc = checkTrajLengths("similarityBatched")) return rc;
-  const double u0 = now_ms();
-  if (int rc = ensureQueryStore(queries)) return rc;
-  if (st) st->uploadMs += now_ms() - u0;
   const int nq = queries.trajNum;
+  if (deviceChain && kValue >= 1 && kValue <= kDeviceTopkMax && nq >= 1 && nq <= kSmallTopkQueries && trajNum >= 1 &&
+      survivorsPerQuery_ * nq * 1.5 <= kSmallTopkPairs) {
+    bool done = false;
+    if (int rc = similaritySmall(queries, kValue, out, st, &done)) return rc;
+    if (done) return GAT_OK;
+  }
+  const double u0 = now_ms();
+  if (int rc = ensureQueryStore(queries, kCtlWords)) return rc;
+  if (st) st->uploadMs += now_ms() - u0;
   if (nq > 65535) {
     gath_set_error("similarityBatched: at most 65535 queries per call");
     return GAT_ERR_ARG;
   }
-  const std::vector<int32_t>& F = mismatchTable();
-  if (F.empty()) return GAT_ERR_HIP;
+  if (int rc = ensureDeviceTables()) return rc;
   if (deviceChain && kValue >= 1 && kValue <= kDeviceTopkMax && nq <= kDeviceListQueries) {
     bool done = false;
     if (int rc = similarityOnDevice(nq, kValue, out, st, &done)) return rc;
@@ -950,6 +1090,8 @@ int Grid::similarityBatched(const TrajectoryView& queries, int kValue, std::vect
   }
   // Per query: the survivors with their exact distances, and every other
   // trajectory at the all-mismatch value of its length, merged by (distance, id).
+  const std::vector<int32_t>& F = mismatchTable();
+  if (F.empty()) return GAT_ERR_HIP;
   std::vector<int64_t> start(size_t(nq) + 1, 0);
   for (size_t i = 0; i < count; ++i) ++start[size_t(pairs[2 * i]) + 1];
   for (int q = 0; q < nq; ++q) start[q + 1] += start[q];

@@ -381,6 +381,55 @@ int gat_edr_filter_grid(const float* query_box_dev, int32_t nq, const float* can
                         const gat_edr_cand_grid* grid, double eps, int32_t* pairs_out_dev, int64_t capacity,
                         uint64_t* count_dev, void* stream);
 
+/* gat_edr_filter_grid adding to *count_dev, which the caller has cleared, and
+ * recording the device's wall clock in stamp_dev[0..1] (null: not). */
+int gat_edr_filter_grid_add(const float* qbox_dev, int32_t nq, const float* cbox_dev, int32_t nc,
+                            const gat_edr_cand_grid* grid, double eps, int32_t* pairs_dev, int64_t capacity,
+                            uint64_t* count_dev, uint32_t* stamp_dev, void* stream);
+
+/* A small top-k batch's stages without a job list (no reference counterpart).
+ *
+ * gat_edr_stage_queries: the queries from pinned host memory: meta_bytes (a
+ * multiple of 4) copied to up_dev, the padded store of `total` points written
+ * (trajectory t's points [src[t], src[t + 1]) at dst[t], NaN elsewhere), its
+ * boxes, ctl_words of ctl_dev cleared and the wall clock in stamp_dev (null:
+ * not).  GAT_EDR_PAD points lie before every trajectory.  A part of a set
+ * (src, dst, box from its first trajectory on, npoints = src[ntraj], total =
+ * the end of its last trajectory) is written as the set is.
+ * gat_edr_bucket: gat_edr_batched with *counter_dev cleared by the caller, and
+ * the wall clock at its start in stamp_dev (null: not).
+ * gat_edr_pairs: gat_edr_batched over pairs 0 .. *live_dev - 1 (none when that
+ * exceeds `capacity`) in the order given, one pair per wave or workgroup
+ * (lanes_per_pair 64, 128, 256 or 512); counter_dev is cleared by the caller,
+ * *cells_dev grows by the pairs' cells.
+ * gat_edr_length_table: out_dev[a * w + L] = table_dev[min(a, L) * w + max(a, L)].
+ * gat_edr_merge: gat_edr_topk from the pairs and their distances, with the
+ * length table; the results may be pinned host memory.  ctl_dev (32 words):
+ * [0, 1] the number of pairs, [2] gets 2 when a query has over 1,024 of them
+ * (its results are left out), [3] as gat_edr_topk's status, [7] zero before the
+ * call; ctl_out receives the words and the wall clock after them.  Nothing is
+ * merged when the pairs exceed `capacity`. */
+int gat_edr_stage_queries(const void* meta_pinned, int64_t meta_bytes, void* up_dev, const int64_t* src_pinned,
+                          const int64_t* dst_pinned, int32_t ntraj, int64_t npoints, const float* lon_pinned,
+                          const float* lat_pinned, int64_t total, float* xy_dev, float* box_dev, uint32_t* ctl_dev,
+                          int64_t ctl_words, uint32_t* stamp_dev, void* stream);
+int gat_edr_bucket(const int32_t* pairs_dev, int64_t npairs, const gat_edr_job* jobs_dev, int64_t njobs,
+                   const int32_t* window_dev, int32_t* counter_dev, const float* qxy_dev, const int64_t* qoff_dev,
+                   const int32_t* qlen_dev, int32_t nqueries, const float* cxy_dev, const int64_t* coff_dev,
+                   const int32_t* clen_dev, int32_t ncands, int32_t maxlen, double eps, int32_t per_cu,
+                   int32_t lanes_per_pair, uint32_t* stamp_dev, int32_t* out_dev, void* stream);
+int gat_edr_pairs(const int32_t* pairs_dev, const uint64_t* live_dev, int64_t capacity, int32_t* counter_dev,
+                  const float* qxy_dev, const int64_t* qoff_dev, const int32_t* qlen_dev, int32_t nqueries,
+                  const float* cxy_dev, const int64_t* coff_dev, const int32_t* clen_dev, int32_t ncands,
+                  int32_t maxlen, double eps, int32_t lanes_per_pair, uint64_t* cells_dev, uint32_t* stamp_dev,
+                  int32_t* out_dev, void* stream);
+int gat_edr_length_table(const int32_t* table_dev, int32_t w, int32_t* out_dev, void* stream);
+int gat_edr_merge(const int32_t* length_table_dev, int32_t w, const int32_t* qlen_dev, int32_t nq,
+                  const int32_t* clen_dev, int32_t nc, const int32_t* len_ids_dev, const int32_t* len_off_dev,
+                  const int32_t* pairs_dev, const int32_t* dist_dev, int64_t capacity, int32_t k, int32_t kk,
+                  int32_t* out_ids, int32_t* out_dist, uint32_t* ctl_dev, uint32_t* ctl_out, uint32_t* stamp_dev,
+                  void* stream);
+
 /* Exact top-k merge on the device (no reference counterpart: the reference
  * keeps a k-entry priority queue per query on the host, Grid.cpp:1600-1729,
  * fed in its frequency-distance order).  For
