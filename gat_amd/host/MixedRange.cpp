@@ -7,6 +7,8 @@ namespace {
 double now_ms() {
   return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
+// The largest rectangles' index first: the others run beside its long kernels.
+constexpr int kQueueOrder[3] = {2, 1, 0};
 }  // namespace
 
 MixedRange::~MixedRange() {
@@ -28,14 +30,18 @@ const DeviceTree& MixedRange::tree(int i) {
 int MixedRange::capture(const int nq[3]) {
   if (graph_) gat_graph_destroy(graph_);
   graph_ = nullptr;
+  for (int i = 0; i < 3; ++i)
+    if (nq[i] > 0)
+      if (int rc = engine(i).reserveResults(nq[i], batch_[i])) return rc;
   void* c = coord_.get();
   GATH_TRY(gat_graph_begin(c), "mixed capture");
   int rc = gat_event_record(fork_, c);
-  for (int i = 0; i < 3 && rc == GAT_OK; ++i) {
-    if (nq[i] == 0) continue;
+  for (int i : kQueueOrder) {
+    if (rc != GAT_OK || nq[i] == 0) continue;
     void* s = engine(i).stream();
     rc = gat_stream_wait_event(s, fork_);
     if (rc == GAT_OK) rc = engine(i).enqueueBatch(tree(i), nq[i], batch_[i]);
+    if (rc == GAT_OK) rc = engine(i).enqueueResults(nq[i], batch_[i]);
     if (rc == GAT_OK) rc = gat_event_record(join_[i], s);
     if (rc == GAT_OK) rc = gat_stream_wait_event(c, join_[i]);
   }
@@ -45,14 +51,20 @@ int MixedRange::capture(const int nq[3]) {
   GATH_TRY(rc_end, "mixed capture");
   graph_ = g;
   std::copy(nq, nq + 3, shape_);
-  for (int i = 0; i < 3; ++i) keys_[i] = engine(i).layoutKey(tree(i), nq[i], batch_[i]);
+  for (int i = 0; i < 3; ++i) {
+    keys_[i] = engine(i).layoutKey(tree(i), nq[i], batch_[i]);
+    results_[i][0] = batch_[i].digestDev_.get();
+    results_[i][1] = engine(i).resultsHost();
+  }
   ++captures;
   return GAT_OK;
 }
 
 bool MixedRange::keysMatch(const int nq[3]) {
   for (int i = 0; i < 3; ++i)
-    if (nq[i] > 0 && engine(i).layoutKey(tree(i), nq[i], batch_[i]) != keys_[i]) return false;
+    if (nq[i] > 0 && (engine(i).layoutKey(tree(i), nq[i], batch_[i]) != keys_[i] ||
+                      batch_[i].digestDev_.get() != results_[i][0] || engine(i).resultsHost() != results_[i][1]))
+      return false;
   return true;
 }
 
@@ -106,30 +118,72 @@ int MixedRange::run(const MBB* bounds, int n, const MixedConfig& cfg, MixedResul
       for (int k = 0; k < nq[i]; ++k) boxes[i].push_back(bounds[list[i][b + size_t(k)]]);
     }
     bool done = false;
-    if (cfg.graph && graph_ && std::equal(nq, nq + 3, shape_)) {
-      // Replay: stage every index's rectangles, launch the one graph, check capacities.
+    const uint64_t* digests[3] = {nullptr, nullptr, nullptr};
+    // Both quick ways below leave counts and digests in pinned memory.
+    auto wait = [&](bool replay) -> int {
+      int rc = replay ? coord_.sync() : GAT_OK;
+      for (int i = 0; i < 3; ++i)
+        if (nq[i] > 0 && !replay) {
+          const int r = gat_stream_sync(engine(i).stream());
+          if (rc == GAT_OK) rc = r;
+        }
+      bool fits = true;
+      for (int i = 0; i < 3 && rc == GAT_OK; ++i) {
+        bool f = true;
+        if (nq[i] > 0) rc = engine(i).finishResults(nq[i], batch_[i], replay, &f, &digests[i]);
+        fits = fits && f;
+      }
+      done = rc == GAT_OK && fits;
+      return rc;
+    };
+    const bool captured = cfg.graph && graph_ && std::equal(nq, nq + 3, shape_);
+    if (captured) {
+      // Replay: stage every index's rectangles, launch the one graph behind
+      // them, check capacities.
       int rc = GAT_OK;
       for (int i = 0; i < 3 && rc == GAT_OK; ++i)
-        if (nq[i] > 0) rc = engine(i).stageBatch(tree(i), boxes[i].data(), nq[i]);
-      for (int i = 0; i < 3 && rc == GAT_OK; ++i)
-        if (nq[i] > 0) rc = gat_stream_sync(engine(i).stream());
+        if (nq[i] > 0) {
+          rc = engine(i).stageBatch(tree(i), boxes[i].data(), nq[i]);
+          if (rc == GAT_OK) rc = gat_event_record(join_[i], engine(i).stream());
+          if (rc == GAT_OK) rc = gat_stream_wait_event(coord_.get(), join_[i]);
+        }
       // A workspace that moved since the capture: the graph's kernels would
       // read freed memory, so this group runs step by step and is recaptured.
       const bool current = rc == GAT_OK && keysMatch(nq);
-      if (rc == GAT_OK && current) rc = gat_graph_launch(graph_, coord_.get());
-      if (rc == GAT_OK) rc = coord_.sync();
-      bool fits = current;
-      for (int i = 0; i < 3 && rc == GAT_OK && current; ++i) {
-        bool f = true;
-        if (nq[i] > 0) rc = engine(i).finishBatch(nq[i], batch_[i], &f);
-        fits = fits && f;
-      }
+      if (current) rc = gat_graph_launch(graph_, coord_.get());
+      if (rc == GAT_OK && current) rc = wait(true);
+      else if (const int r = coord_.sync(); rc == GAT_OK) rc = r;
       if (rc != GAT_OK) {
         restore();
         return gath_fail_hip(rc, "mixed replay");
       }
-      done = fits;
       if (done) ++out->replays;
+    } else if (graph_ || !cfg.graph || gi + 2 >= groups) {
+      // A group of another shape than the captured one, or one not to be captured:
+      // the three pipelines queued on their own streams with one wait, where
+      // earlier batches have sized the workspaces (step by step they took a
+      // wait per pipeline half and several per index's results, and ran one
+      // index after another).
+      int rc = GAT_OK;
+      bool all = true;
+      for (int i : kQueueOrder) {
+        if (rc != GAT_OK || !all || nq[i] == 0) continue;
+        rc = engine(i).reserveResults(nq[i], batch_[i]);
+        if (rc == GAT_OK) rc = engine(i).queueBatch(tree(i), boxes[i].data(), nq[i], batch_[i], &all);
+      }
+      if (rc == GAT_OK && all) {
+        rc = wait(false);
+      } else {
+        for (int i = 0; i < 3; ++i)
+          if (nq[i] > 0) {
+            const int r = gat_stream_sync(engine(i).stream());
+            if (rc == GAT_OK) rc = r;
+          }
+      }
+      if (rc != GAT_OK) {
+        restore();
+        return gath_fail_hip(rc, "mixed batch");
+      }
     }
     if (!done) {
       // Step by step (sizes every workspace, which may move its buffers, so
@@ -153,9 +207,12 @@ int MixedRange::run(const MBB* bounds, int n, const MixedConfig& cfg, MixedResul
       if (nq[i] == 0) continue;
       RangeBatch& b = batch_[i];
       int rc = b.syncHost();
-      if (rc == GAT_OK) rc = digests_[i].reserve(size_t(nq[i]) * 8);
-      dig.resize(size_t(nq[i]));
-      if (rc == GAT_OK) rc = b.digestsInto(digests_[i].as<uint64_t>(), dig.data());
+      const uint64_t* d = digests[i];
+      if (rc == GAT_OK && !done) {
+        dig.resize(size_t(nq[i]));
+        rc = b.digests(dig.data());
+        d = dig.data();
+      }
       if (rc != GAT_OK) {
         restore();
         return rc;
@@ -164,7 +221,7 @@ int MixedRange::run(const MBB* bounds, int n, const MixedConfig& cfg, MixedResul
       for (int k = 0; k < nq[i]; ++k) {
         const int q = list[i][base + size_t(k)];
         out->count[size_t(q)] = b.count[size_t(k)];
-        out->digest[size_t(q)] = dig[size_t(k)];
+        out->digest[size_t(q)] = d[k];
       }
       out->pairs += b.pairTotal;
       out->candidates += b.candidates;

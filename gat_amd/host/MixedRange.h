@@ -56,7 +56,6 @@ class MixedRange {
   STIG& stig_;
   FSG& fsg_;
   RangeBatch batch_[3];
-  DeviceBuffer digests_[3];
   Stream coord_;
   void* fork_ = nullptr;
   void* join_[3] = {nullptr, nullptr, nullptr};
@@ -66,6 +65,7 @@ class MixedRange {
   // three still hold (an engine's own range_batched, tune or reserve call can
   // grow and so reallocate its workspace between two runs).
   RangeEngine::GraphKey keys_[3];
+  const void* results_[3][2] = {};  // and its digests' and results' buffers
   bool keysMatch(const int nq[3]);
  public:
   int captures = 0;  // graphs captured over this object's life

@@ -839,7 +839,7 @@ int RangeEngine::enqueueTreeSelect(const DeviceTree& tree, int nq, uint32_t* nod
   return GAT_OK;
 }
 
-int RangeEngine::enqueueSelect(const DeviceTree& tree, int nq, RangeBatch& out) {
+int RangeEngine::enqueueSelect(const DeviceTree& tree, int nq, RangeBatch& out, bool cleared) {
   void* s = stream_.get();
   const int64_t N = tree.nnodes;
   uint32_t* ctr = counters_.as<uint32_t>();
@@ -848,7 +848,7 @@ int RangeEngine::enqueueSelect(const DeviceTree& tree, int nq, RangeBatch& out) 
   const bool clearCand = selectAddsCandidates(tree);
   uint32_t* const spans[4] = {nodeCount_.as<uint32_t>(), out.qcount.as<uint32_t>(), ctr, cand_.as<uint32_t>()};
   const int64_t lens[4] = {N, nq, 16, clearCand ? int64_t(nq) * 2 : 0};
-  GATH_TRY(gat_fill_u32_spans(4, spans, lens, 0, s), "batch reset");
+  if (!cleared) GATH_TRY(gat_fill_u32_spans(4, spans, lens, 0, s), "batch reset");
   if (int rc = enqueueTreeSelect(tree, nq, nodeCount_.as<uint32_t>(), clearCand)) return rc;
   // The run-indexed join places its output by work item: it needs the
   // candidate total but no per-query regions.  (The walk adding the total
@@ -979,6 +979,75 @@ int RangeEngine::finishBatch(int nq, RangeBatch& out, bool* fits) {
   return *fits ? finishCounters(out, true) : GAT_OK;
 }
 
+// Whether the workspace and `out` hold everything the leaf-major pipeline of nq
+// rectangles touches at the capacities at hand.
+bool RangeEngine::sizedFor(const DeviceTree& tree, int nq, const RangeBatch& out) const {
+  const int64_t N = tree.nnodes;
+  const size_t tileBytes = size_t(std::max(2 * gat_scan_tiles(N) * 4, gat_scan_tiles(nq) * 8));
+  auto holds = [](const DeviceBuffer& b, int64_t n, size_t size) { return n > 0 && b.size() >= size_t(n) * size; };
+  return holds(nodeCount_, N, 4) && holds(nodeOff_, N, 8) && tiles_.size() >= tileBytes && holds(cand_, nq, 8) &&
+         holds(out.qbase, nq, 8) && holds(out.qcount, nq, 4) && holds(counters_, 1, 256) && holds(lq_, lqCap_, 8) &&
+         holds(lqRank_, lqCap_, 4) && holds(qlist_, qlistCap_, 4) && holds(items_, itemsCap_, 16) &&
+         holds(out.pairs, pairsCap_, 8) && holds(out.runs, qlistCap_, sizeof(gat_range_run)) &&
+         holds(itemBase_, itemsCap_, 8) && holds(itemTiles_, gat_scan_tiles(itemsCap_), 8);
+}
+
+int RangeEngine::reserveResults(int nq, RangeBatch& out) {
+  if (int rc = countersHost_.reserve(256)) return rc;
+  if (int rc = out.digestDev_.reserve(size_t(std::max(nq, 1)) * 8)) return rc;
+  return resultHost_.reserve(size_t(gat_direct_words(std::max(nq, 1))) * 4);
+}
+
+int RangeEngine::queueBatch(const DeviceTree& tree, const MBB* bounds, int nq, RangeBatch& out, bool* queued) {
+  *queued = false;
+  if (nq < 1 || !sizedFor(tree, nq, out)) return GAT_OK;
+  size_t bytes = 0;
+  if (int rc = stageBoxes(&tree, bounds, nq, &bytes)) return rc;
+  uint32_t* const spans[4] = {nodeCount_.as<uint32_t>(), out.qcount.as<uint32_t>(), counters_.as<uint32_t>(),
+                              cand_.as<uint32_t>()};
+  const int64_t lens[4] = {tree.nnodes, nq, 16, selectAddsCandidates(tree) ? int64_t(nq) * 2 : 0};
+  GATH_TRY(gat_stage_in(devBoxes_.get(), hostStage_.get(), int64_t(bytes), 4, spans, lens, nullptr, stream_.get()),
+           "box upload");
+  *queued = true;
+  if (int rc = enqueueSelect(tree, nq, out, true)) return rc;
+  if (int rc = enqueueJoin(tree, nq, out)) return rc;
+  return enqueueResults(nq, out);
+}
+
+int RangeEngine::enqueueResults(int nq, RangeBatch& out) {
+  void* s = stream_.get();
+  uint32_t* ctr = counters_.as<uint32_t>();
+  uint64_t* dig = out.digestDev_.as<uint64_t>();
+  if (runIndexed)
+    GATH_TRY(gat_runs_digest_live(out.pairs.as<int32_t>(), pairsCap_, out.runs.as<gat_range_run>(), qlistCap_, ctr + 5,
+                                  nq, dig, s),
+             "run digest");
+  else
+    GATH_TRY(gat_pairs_digest(out.pairs.as<int32_t>(), out.qbase.as<uint64_t>(), out.qcount.as<uint32_t>(), nq,
+                              pairsCap_, dig, s),
+             "pair digest");
+  GATH_TRY(gat_direct_finish(ctr, out.qcount.as<uint32_t>(), dig, nq, resultHost_.as<uint32_t>(), s),
+           "batch readback");
+  return GAT_OK;
+}
+
+int RangeEngine::finishResults(int nq, RangeBatch& out, bool replay, bool* fits, const uint64_t** digests) {
+  const uint32_t* w = resultHost_.as<uint32_t>();
+  std::memcpy(countersHost_.get(), w, 64);
+  *fits = countersFit();
+  if (!*fits) return GAT_OK;
+  out.queryNum = nq;
+  out.stream = stream_.get();
+  out.taskNum = 0;
+  out.selectMs = out.uploadMs = 0;
+  out.kernelMs = out.refineMs = 0;
+  out.count.assign(w + 32, w + 32 + nq);
+  out.base.assign(size_t(nq), 0);
+  out.hostStale = !out.runIndexed;  // regions
+  *digests = reinterpret_cast<const uint64_t*>(w + 32 + (nq + 1) / 2 * 2);
+  return finishCounters(out, replay);
+}
+
 int RangeEngine::runTree(const DeviceTree& tree, const MBB* bounds, int nq, RangeBatch& out, bool graph) {
   if (int rc = stream_.create()) return rc;
   if (tree.nnodes <= 0 || nq < 0 || (nq > 0 && !bounds) || queriesPerItem < 1 || queriesPerItem > 64) {
@@ -1047,50 +1116,67 @@ int RangeEngine::runTree(const DeviceTree& tree, const MBB* bounds, int nq, Rang
       // The batch outgrew the captured capacities: run it step by step below.
     }
   }
-  // Selection, then capacities from its totals, then the join.
-  if (lqCap_ < int64_t(nq) * 16) lqCap_ = std::max<int64_t>(int64_t(nq) * 16, 1 << 16);
-  if (int rc = lq_.reserve(size_t(lqCap_) * 8)) return rc;
-  if (int rc = lqRank_.reserve(size_t(lqCap_) * 4)) return rc;
-  for (int attempt = 0;; ++attempt) {
+  // Selection and join, the join at once where earlier batches have sized the
+  // workspace (the device keeps inside the capacities), and after it a look at
+  // the counters; a batch that did not fit, and a first one, runs step by step.
+  auto join = [&]() -> int {
+    if (int rc = timer_.start(stream_.get())) return rc;
+    timeRefine_ = true;
+    const int rc_join = enqueueJoin(tree, nq, out);
+    timeRefine_ = false;
+    if (rc_join) return rc_join;
+    return timer_.stop(stream_.get());
+  };
+  bool done = false;
+  if (sizedFor(tree, nq, out)) {
     if (int rc = selTimer_.start(stream_.get())) return rc;
     if (int rc = enqueueSelect(tree, nq, out)) return rc;
     if (int rc = selTimer_.stop(stream_.get())) return rc;
-    GATH_TRY(gat_memcpy_d2h(countersHost_.get(), counters_.get(), 64, stream_.get()), "counter readback");
-    if (int rc = stream_.sync()) return rc;
-    if (u64(0) <= uint64_t(lqCap_)) break;
-    if (attempt > 0 || u64(0) >= uint64_t(UINT32_MAX)) {
-      gath_set_error("batched range: %llu (leaf, query) entries do not fit", (unsigned long long)u64(0));
-      return GAT_ERR_CAPACITY;
-    }
-    lqCap_ = int64_t(u64(0) + u64(0) / 4 + 1024);
-    if (int rc = lq_.reserve(size_t(lqCap_) * 8)) return rc;
-    if (int rc = lqRank_.reserve(size_t(lqCap_) * 4)) return rc;
+    if (int rc = join()) return rc;
+    if (int rc = readCounters(nq, out)) return rc;
+    done = fits() || (ch[4] & GAT_STATUS_STACK);
   }
   float selMs = 0;
+  if (!done) {
+    // Selection, then capacities from its totals, then the join.
+    if (lqCap_ < int64_t(nq) * 16) lqCap_ = std::max<int64_t>(int64_t(nq) * 16, 1 << 16);
+    if (int rc = lq_.reserve(size_t(lqCap_) * 8)) return rc;
+    if (int rc = lqRank_.reserve(size_t(lqCap_) * 4)) return rc;
+    for (int attempt = 0;; ++attempt) {
+      if (int rc = selTimer_.start(stream_.get())) return rc;
+      if (int rc = enqueueSelect(tree, nq, out)) return rc;
+      if (int rc = selTimer_.stop(stream_.get())) return rc;
+      GATH_TRY(gat_memcpy_d2h(countersHost_.get(), counters_.get(), 64, stream_.get()), "counter readback");
+      if (int rc = stream_.sync()) return rc;
+      if (u64(0) <= uint64_t(lqCap_)) break;
+      if (attempt > 0 || u64(0) >= uint64_t(UINT32_MAX)) {
+        gath_set_error("batched range: %llu (leaf, query) entries do not fit", (unsigned long long)u64(0));
+        return GAT_ERR_CAPACITY;
+      }
+      lqCap_ = int64_t(u64(0) + u64(0) / 4 + 1024);
+      if (int rc = lq_.reserve(size_t(lqCap_) * 8)) return rc;
+      if (int rc = lqRank_.reserve(size_t(lqCap_) * 4)) return rc;
+    }
+    if (ch[4] & GAT_STATUS_STACK) return finish(false);
+    // Room with a quarter to spare, so a captured pipeline serves similar batches.
+    auto grow = [](int64_t need, int64_t& cap) {
+      if (need > cap || cap == 0) cap = need + need / 4 + 1024;
+    };
+    grow(int64_t(ch[5]), qlistCap_);
+    grow(int64_t(ch[6]), itemsCap_);
+    // Run-indexed regions round each work item up to a line: 15 pairs each at most.
+    grow(int64_t(u64(2)) + (runIndexed ? 16 * int64_t(ch[6]) : 0), pairsCap_);
+    if (int rc = qlist_.reserve(size_t(qlistCap_) * 4)) return rc;
+    if (int rc = items_.reserve(size_t(itemsCap_) * 16)) return rc;
+    if (int rc = out.pairs.reserve(size_t(pairsCap_) * 8)) return rc;
+    if (int rc = out.runs.reserve(size_t(qlistCap_) * sizeof(gat_range_run))) return rc;
+    if (int rc = itemBase_.reserve(size_t(itemsCap_) * 8)) return rc;
+    if (int rc = itemTiles_.reserve(size_t(gat_scan_tiles(itemsCap_)) * 8)) return rc;
+    if (int rc = join()) return rc;
+    if (int rc = readCounters(nq, out)) return rc;
+  }
   if (int rc = selTimer_.elapsed(&selMs)) return rc;
   out.selectMs = selMs;
-  if (ch[4] & GAT_STATUS_STACK) return finish(false);
-  // Room with a quarter to spare, so a captured pipeline serves similar batches.
-  auto grow = [](int64_t need, int64_t& cap) {
-    if (need > cap || cap == 0) cap = need + need / 4 + 1024;
-  };
-  grow(int64_t(ch[5]), qlistCap_);
-  grow(int64_t(ch[6]), itemsCap_);
-  // Run-indexed regions round each work item up to a line: 15 pairs each at most.
-  grow(int64_t(u64(2)) + (runIndexed ? 16 * int64_t(ch[6]) : 0), pairsCap_);
-  if (int rc = qlist_.reserve(size_t(qlistCap_) * 4)) return rc;
-  if (int rc = items_.reserve(size_t(itemsCap_) * 16)) return rc;
-  if (int rc = out.pairs.reserve(size_t(pairsCap_) * 8)) return rc;
-  if (int rc = out.runs.reserve(size_t(qlistCap_) * sizeof(gat_range_run))) return rc;
-  if (int rc = itemBase_.reserve(size_t(itemsCap_) * 8)) return rc;
-  if (int rc = itemTiles_.reserve(size_t(gat_scan_tiles(itemsCap_)) * 8)) return rc;
-  if (int rc = timer_.start(stream_.get())) return rc;
-  timeRefine_ = true;
-  const int rc_join = enqueueJoin(tree, nq, out);
-  timeRefine_ = false;
-  if (rc_join) return rc_join;
-  if (int rc = timer_.stop(stream_.get())) return rc;
-  if (int rc = readCounters(nq, out)) return rc;
   if (int rc = timer_.elapsed(&out.kernelMs)) return rc;
   if (int rc = refineTimer_.elapsed(&out.refineMs)) return rc;
   out.uploadMs = now_ms() - t0;

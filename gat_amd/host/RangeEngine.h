@@ -84,9 +84,9 @@ struct RangeBatch {
   // The same into a caller-owned device buffer of queryNum entries (no
   // allocation), copied to `out` when it is not null.
   int digestsInto(uint64_t* dev, uint64_t* out) const;
+  mutable DeviceBuffer digestDev_;  // digests(): kept, since a free waits for the device
 
  private:
-  mutable DeviceBuffer digestDev_;  // digests(): kept, since a free waits for the device
   // fetchCompact of up to kGatherBytes of pairs: gathered on the device into
   // pinned memory in one launch pair.  Larger ones go by a copy per query (or
   // per batch): the gather would hold as much pinned memory as the result.
@@ -204,6 +204,17 @@ class RangeEngine {
   int stageBatch(const DeviceTree& tree, const MBB* bounds, int nq);
   int enqueueBatch(const DeviceTree& tree, int nq, RangeBatch& out);
   int finishBatch(int nq, RangeBatch& out, bool* fits);
+  // The whole batch, counts and digests included, queued without a wait, when
+  // earlier batches have sized the workspace for it (*queued, else nothing is):
+  // reserveResults before, then either queueBatch (upload and pipeline) or, to
+  // be captured, enqueueBatch and enqueueResults; once the stream has been waited for
+  // finishResults, as finishBatch, with the digests in *digests (pinned, valid
+  // until the next batch).
+  int reserveResults(int nq, RangeBatch& out);
+  int queueBatch(const DeviceTree& tree, const MBB* bounds, int nq, RangeBatch& out, bool* queued);
+  int enqueueResults(int nq, RangeBatch& out);
+  int finishResults(int nq, RangeBatch& out, bool replay, bool* fits, const uint64_t** digests);
+  const void* resultsHost() const { return resultHost_.get(); }
 
   // Everything a captured batch pipeline has baked into its kernel arguments:
   // every device buffer it reads or writes, the capacities it was sized with,
@@ -249,7 +260,8 @@ class RangeEngine {
   static BoxLayout boxLayout(int nq);
   int stageBoxes(const DeviceTree* tree, const MBB* bounds, int nq, size_t* bytes);
   int uploadBoxes(const DeviceTree* tree, const MBB* bounds, int nq);
-  int enqueueSelect(const DeviceTree& tree, int nq, RangeBatch& out);
+  int enqueueSelect(const DeviceTree& tree, int nq, RangeBatch& out, bool cleared = false);
+  bool sizedFor(const DeviceTree& tree, int nq, const RangeBatch& out) const;
   // The selection kernel for the tree's kind (nodeCount may be null).  The
   // start-table walk adds to the candidate counts, which it clears first
   // unless the caller already has (candCleared).
@@ -281,7 +293,7 @@ class RangeEngine {
   // and [14,15] the clock at the batch's start and after its selection.
   DeviceBuffer nodeCount_, lqRank_, nodeOff_, tiles_, cand_, lq_, qlist_, items_, counters_;
   DeviceBuffer itemBase_, itemTiles_;  // run-indexed refine: item regions and their scan scratch
-  PinnedBuffer countersHost_, directHost_;
+  PinnedBuffer countersHost_, directHost_, resultHost_;
   int64_t walkTasks_ = 0;       // walk tasks stageBoxes last laid out
   int64_t directExpected_ = 0;  // entries of the last direct batch
   int32_t clockKhz_ = 0;

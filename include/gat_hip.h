@@ -642,7 +642,7 @@ typedef struct gat_range_run {
  * for, any number is refined.
  * gat_direct_finish writes gat_direct_words(nq) words to pinned host memory:
  * [0, 16) counters_dev, [16, 18) the wall clock, [32, 32 + nq) the counts, then
- * from the next even word the regions (uint64 each).
+ * from the next even word the regions (uint64 each; any nq values serve).
  * gat_wall_clock_khz: the rate of those clocks. */
 int gat_stage_in(void* dst_dev, const void* src_pinned, int64_t bytes, int32_t nspans, uint32_t* const* spans_dev,
                  const int64_t* words, uint32_t* stamp_dev, void* stream);
@@ -717,6 +717,11 @@ int gat_run_counts(const gat_point_store* store, const uint32_t* items_dev, cons
  * out_dev first.  Asynchronous. */
 int gat_runs_digest(const int32_t* pairs_dev, int64_t npairs, const gat_range_run* runs_dev, int64_t nruns,
                     int64_t nqueries, uint64_t* out_dev, void* stream);
+
+/* gat_runs_digest of the first min(nruns, *live_dev) runs (null: all of them),
+ * for a chain whose host does not know their number yet. */
+int gat_runs_digest_live(const int32_t* pairs_dev, int64_t npairs, const gat_range_run* runs_dev, int64_t nruns,
+                         const uint32_t* live_dev, int64_t nqueries, uint64_t* out_dev, void* stream);
 
 /* The leaf-major refine: per work item the leaf's points and ids are loaded
  * once and tested against each of the item's rectangles; hits go to query q's
