@@ -102,6 +102,8 @@ HIP_FUNCS = {
     "gat_stage_in": (INT, [P, P, I64, I32, P, P, P, P]),
     "gat_direct_regions": (INT, [P, I64, P, P, P, P]),
     "gat_direct_refine": (INT, [P, P, P, I64, I64, P, I64, P, I64, P, P, P, I64, P]),
+    "gat_direct_bitmap": (INT, [P, P, P, I64, I64, P, I64, P, I64, P, I64, P]),
+    "gat_bitmap_finish": (INT, [P, P, I64, P, P]),
     "gat_direct_words": (I64, [I64]),
     "gat_direct_finish": (INT, [P, P, P, I64, P, P]),
     "gat_wall_clock_khz": (INT, [P]),

@@ -672,6 +672,87 @@ int RangeEngine::runDirect(const DeviceTree& tree, const MBB* bounds, int nq, Ra
   return GAT_OK;
 }
 
+namespace {
+// The eight bytes (0 or 1) of eight bits, lowest first.
+struct BitBytes {
+  uint64_t at[256];
+  BitBytes() {
+    for (int v = 0; v < 256; ++v) {
+      at[v] = 0;
+      for (int b = 0; b < 8; ++b) at[v] |= uint64_t((v >> b) & 1) << (8 * b);
+    }
+  }
+};
+
+// out[i] = bit i, i < n.
+void expand_bits(const uint32_t* bits, int64_t n, uint8_t* out) {
+  static const BitBytes table;
+  const uint8_t* b = reinterpret_cast<const uint8_t*>(bits);
+  int64_t i = 0;
+  for (; i + 8 <= n; i += 8) std::memcpy(out + i, &table.at[b[i / 8]], 8);
+  for (; i < n; ++i) out[i] = (b[i / 8] >> (i % 8)) & 1;
+}
+}  // namespace
+
+int RangeEngine::runBitmapDirect(const DeviceTree& tree, const MBB* bounds, int nq, int64_t stride, uint8_t* out) {
+  if (int rc = stream_.create()) return rc;
+  if (tree.nnodes <= 0 || nq < 0 || stride < 1 || (nq > 0 && (!bounds || !out))) {
+    gath_set_error("range bitmap: bad arguments");
+    return GAT_ERR_ARG;
+  }
+  void* s = stream_.get();
+  const int most = int(std::max<int64_t>(std::min(kBitmapQueries, kBitmapBytes / stride), 1));
+  for (int q0 = 0; q0 < nq; q0 += most) {
+    const int n = std::min(most, nq - q0);
+    const int64_t bytes = (int64_t(n) * stride + 31) / 32 * 32;
+    size_t staged = 0;
+    if (int rc = cand_.reserve(size_t(n) * 8)) return rc;
+    if (int rc = counters_.reserve(256)) return rc;
+    if (int rc = bitmapDev_.reserve(size_t(bytes))) return rc;
+    if (int rc = bitmapHost_.reserve(size_t(bytes) / 8 + 32 * 4)) return rc;
+    if (lqCap_ < int64_t(n) * 16) {
+      lqCap_ = std::max<int64_t>(int64_t(n) * 16, 1 << 16);
+      dropGraph();
+    }
+    if (int rc = lq_.reserve(size_t(lqCap_) * 8)) return rc;
+    if (int rc = stageBoxes(&tree, bounds + q0, n, &staged)) return rc;
+    uint32_t* ctr = counters_.as<uint32_t>();
+    const uint32_t* ch = bitmapHost_.as<uint32_t>();
+    const bool clearCand = selectAddsCandidates(tree);
+    for (int attempt = 0;; ++attempt) {
+      uint32_t* const spans[3] = {ctr, cand_.as<uint32_t>(), bitmapDev_.as<uint32_t>()};
+      const int64_t lens[3] = {16, clearCand ? int64_t(n) * 2 : 0, bytes / 4};
+      GATH_TRY(gat_stage_in(devBoxes_.get(), hostStage_.get(), int64_t(staged), 3, spans, lens, nullptr, s),
+               "box upload");
+      if (int rc = enqueueTreeSelect(tree, n, nullptr, clearCand, walkTasks_)) return rc;
+      GATH_TRY(gat_direct_bitmap(&store_, lq_.as<uint32_t>(), reinterpret_cast<const uint64_t*>(ctr), lqCap_,
+                                 bitmapExpected_ > 0 ? bitmapExpected_ : int64_t(n) * 64,
+                                 tree.nodes.as<gat_tree_node>(), tree.nnodes, devBoxes_.as<float>(), n,
+                                 bitmapDev_.as<uint8_t>(), stride, s),
+               "range bitmap");
+      GATH_TRY(gat_bitmap_finish(ctr, bitmapDev_.as<uint8_t>(), bytes, bitmapHost_.as<uint32_t>(), s),
+               "bitmap readback");
+      if (int rc = stream_.sync()) return rc;
+      if (ch[4] & GAT_STATUS_STACK) {
+        gath_set_error("batched range: traversal stack exceeded");
+        return GAT_ERR_STATE;
+      }
+      const uint64_t entries = uint64_t(ch[0]) | (uint64_t(ch[1]) << 32);
+      bitmapExpected_ = int64_t(entries);
+      if (entries <= uint64_t(lqCap_)) break;
+      if (attempt > 0 || entries >= uint64_t(UINT32_MAX)) {
+        gath_set_error("batched range: %llu (leaf, query) entries do not fit", (unsigned long long)entries);
+        return GAT_ERR_CAPACITY;
+      }
+      lqCap_ = int64_t(entries + entries / 4 + 1024);
+      dropGraph();
+      if (int rc = lq_.reserve(size_t(lqCap_) * 8)) return rc;
+    }
+    expand_bits(ch + 32, int64_t(n) * stride, out + int64_t(q0) * stride);
+  }
+  return GAT_OK;
+}
+
 RangeEngine::GraphKey RangeEngine::layoutKey(const DeviceTree& tree, int nq, const RangeBatch& out) const {
   GraphKey key;
   const void* p[GraphKey::kPtrs] = {tree.nodes.get(), tree.cellWords.get(), devBoxes_.get(), out.pairs.get(),

@@ -175,6 +175,11 @@ class RangeEngine {
   // reference-signature handler (synchronous, host result).
   int runBitmap(const MBB* bounds, int nq, const Selector& select, int threads, int maxTrajNum,
                 uint8_t* resultHost, bool stigHandler);
+  // The same trajectory bitmap, out[q * stride + tid] in {0, 1}, by the direct
+  // form's chain: device selection, a byte per trajectory on the device, bits to
+  // pinned memory and bytes from there, for as many rectangles at a time as
+  // kBitmapBytes of bitmap hold.
+  int runBitmapDirect(const DeviceTree& tree, const MBB* bounds, int nq, int64_t stride, uint8_t* out);
   // Batched form: device selection against `tree`, grouping by leaf and the
   // leaf-major refine, for the whole batch.  With graph=true the device
   // pipeline is captured once per buffer layout and replayed while the batch
@@ -292,6 +297,10 @@ class RangeEngine {
   // [8,9] result pairs, [10,11] run-indexed region total; direct form: [12,13]
   // and [14,15] the clock at the batch's start and after its selection.
   DeviceBuffer nodeCount_, lqRank_, nodeOff_, tiles_, cand_, lq_, qlist_, items_, counters_;
+  static constexpr int64_t kBitmapBytes = int64_t(64) << 20, kBitmapQueries = 1024;
+  DeviceBuffer bitmapDev_;
+  PinnedBuffer bitmapHost_;
+  int64_t bitmapExpected_ = 0;  // entries of the last bitmap batch
   DeviceBuffer itemBase_, itemTiles_;  // run-indexed refine: item regions and their scan scratch
   PinnedBuffer countersHost_, directHost_, resultHost_;
   int64_t walkTasks_ = 0;       // walk tasks stageBoxes last laid out

@@ -185,6 +185,11 @@ int64_t gath_index_select(void* p, const float* boxes, int nq, uint32_t* tasks_o
 int gath_index_range_bitmap(void* p, const float* boxes, int nq, uint8_t* out) {
   Index* ix = as_index(p);
   if (!ix || nq < 0 || (nq > 0 && (!boxes || !out))) return bad("gath_index_range_bitmap: bad arguments");
+  // The index's own device tree selects; an index without one (built without
+  // upload) takes the handlers, which report that.
+  const DeviceTree& tree = ix->grid ? ix->grid->deviceTree() : ix->fsg ? ix->fsg->deviceTree() : ix->stig->deviceTree();
+  RangeEngine& engine = ix->grid ? ix->grid->engine() : ix->fsg ? ix->fsg->engine() : ix->stig->engine();
+  if (tree.nnodes > 0) return engine.runBitmapDirect(tree, as_boxes(boxes), nq, int64_t(ix->trajNum()) + 1, out);
   std::vector<CPURangeQueryResult> res(static_cast<size_t>(nq));
   int rc;
   if (ix->grid) rc = ix->grid->rangeQueryBatchGPU(as_boxes(boxes), nq, res.data(), nullptr);

@@ -643,6 +643,10 @@ typedef struct gat_range_run {
  * gat_direct_finish writes gat_direct_words(nq) words to pinned host memory:
  * [0, 16) counters_dev, [16, 18) the wall clock, [32, 32 + nq) the counts, then
  * from the next even word the regions (uint64 each; any nq values serve).
+ * gat_direct_bitmap in the place of regions and refine: bitmap_dev[q * stride
+ * + tid] = 1 for the trajectories with a point in rectangle q (tid < stride; the
+ * rest stays as it is), and gat_bitmap_finish, which writes [0, 16) counters_dev
+ * and from word 32 one bit per byte (0 or 1; bytes a multiple of 32) of it.
  * gat_wall_clock_khz: the rate of those clocks. */
 int gat_stage_in(void* dst_dev, const void* src_pinned, int64_t bytes, int32_t nspans, uint32_t* const* spans_dev,
                  const int64_t* words, uint32_t* stamp_dev, void* stream);
@@ -652,6 +656,11 @@ int gat_direct_refine(const gat_point_store* store, const uint32_t* leaf_query_d
                       int64_t lq_capacity, int64_t expected, const gat_tree_node* nodes_dev, int64_t nnodes,
                       const float* boxes_dev, int64_t nqueries, const uint64_t* qbase_dev, uint32_t* qcount_dev,
                       int32_t* pairs_dev, int64_t capacity, void* stream);
+int gat_direct_bitmap(const gat_point_store* store, const uint32_t* leaf_query_dev, const uint64_t* lq_total_dev,
+                      int64_t lq_capacity, int64_t expected, const gat_tree_node* nodes_dev, int64_t nnodes,
+                      const float* boxes_dev, int64_t nqueries, uint8_t* bitmap_dev, int64_t stride, void* stream);
+int gat_bitmap_finish(const uint32_t* counters_dev, const uint8_t* bitmap_dev, int64_t bytes, uint32_t* out_pinned,
+                      void* stream);
 int64_t gat_direct_words(int64_t nq);
 int gat_direct_finish(const uint32_t* counters_dev, const uint32_t* qcount_dev, const uint64_t* qbase_dev, int64_t nq,
                       uint32_t* out_pinned, void* stream);
