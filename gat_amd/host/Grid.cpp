@@ -71,13 +71,14 @@ int Grid::addDatasetToGrid(const TrajectoryView& db, bool upload) {
   if (upload && deviceBuild) {
     const gat_cell_grid g{1, cellNum_axis, cellNum_axis, range.xmin, range.ymax, cell_size};
     int64_t bad = -1;
-    if (int rc = engine_.buildStore(g, db, &cellStart, &bad)) return rc;
+    RangeEngine::DevicePoints points;
+    if (int rc = engine_.buildStore(g, db, &cellStart, &bad, &points)) return rc;
     if (bad >= 0) {
       gath_set_error("Grid: point %lld (%g, %g) lies outside the grid", (long long)bad, double(db.lon[bad]),
                      double(db.lat[bad]));
       return GAT_ERR_ARG;
     }
-    return finishBuild(db);
+    return finishBuild(db, &points);
   }
   // Split the trajectories into contiguous groups of about equal point count;
   // each thread owns one group, so the order within a cell stays the
@@ -164,7 +165,7 @@ int Grid::addDatasetToGrid(const TrajectoryView& db, bool upload) {
   if (int rc = engine_.upload(xy.data(), tp.data(), N)) return rc;
   xy = std::vector<float>();
   tp = std::vector<int32_t>();
-  return finishBuild(db);
+  return finishBuild(db, nullptr);
 }
 
 // The quadtree over the cell offsets, its device copy and the trajectory
@@ -182,7 +183,7 @@ int64_t Grid::leafNum() const {
   return n;
 }
 
-int Grid::finishBuild(const TrajectoryView& db) {
+int Grid::finishBuild(const TrajectoryView& db, const RangeEngine::DevicePoints* points) {
   if (int rc = buildHostTree()) return rc;
   int depth = 0;
   const std::vector<gat_tree_node> tn = treeNodes(&depth);
@@ -192,7 +193,7 @@ int Grid::finishBuild(const TrajectoryView& db) {
   const std::vector<uint32_t> owner = startTable(depth, &k, &block);
   if (!owner.empty())
     if (int rc = tree_.uploadStart(owner, k, range.xmin, range.ymax, block, engine_.stream())) return rc;
-  return uploadTrajectories(db);
+  return uploadTrajectories(db, points);
 }
 
 // The device walk starts at the owners of a level-k table, k = min(7, depth -

@@ -173,11 +173,11 @@ class Grid {
   // The host tree over cellStart, then (finishBuild) its device form and the
   // trajectory store.
   virtual int buildHostTree();
-  virtual int finishBuild(const TrajectoryView& db);
+  virtual int finishBuild(const TrajectoryView& db, const RangeEngine::DevicePoints* points);
   // Appends the store runs of the leaves `bound` selects, as query q.
   virtual void addLeafRuns(const MBB& bound, uint32_t q, TaskList& list) const;
   int threads() const;
-  int uploadTrajectories(const TrajectoryView& db);
+  int uploadTrajectories(const TrajectoryView& db, const RangeEngine::DevicePoints* points);
 
   RangeEngine engine_;
   DeviceTree tree_;

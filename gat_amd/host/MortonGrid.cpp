@@ -82,7 +82,7 @@ std::vector<gat_tree_node> MortonGrid::treeNodes(int* depth) const {
   return out;
 }
 
-int MortonGrid::finishBuild(const TrajectoryView& db) {
+int MortonGrid::finishBuild(const TrajectoryView& db, const RangeEngine::DevicePoints* points) {
   if (int rc = buildHostTree()) return rc;
   int depth = 0;
   const std::vector<gat_tree_node> recs = treeNodes(&depth);
@@ -96,7 +96,7 @@ int MortonGrid::finishBuild(const TrajectoryView& db) {
   }
   if (int rc = tree_.uploadImplicit(recs, words, totalLevel, range.xmin, range.ymax, cell_size, engine_.stream()))
     return rc;
-  return uploadTrajectories(db);
+  return uploadTrajectories(db, points);
 }
 
 void MortonGrid::addLeafRuns(const MBB& bound, uint32_t q, TaskList& list) const {

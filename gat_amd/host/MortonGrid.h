@@ -54,6 +54,6 @@ class MortonGrid : public Grid {
 
  protected:
   int buildHostTree() override;
-  int finishBuild(const TrajectoryView& db) override;
+  int finishBuild(const TrajectoryView& db, const RangeEngine::DevicePoints* points) override;
   void addLeafRuns(const MBB& bound, uint32_t q, TaskList& list) const override;
 };

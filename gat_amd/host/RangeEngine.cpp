@@ -169,7 +169,7 @@ int RangeEngine::stageBuild(const TrajectoryView& db, int pidBits, DeviceBuffer&
 }
 
 int RangeEngine::buildStore(const gat_cell_grid& grid, const TrajectoryView& db, std::vector<int64_t>* cellStart,
-                            int64_t* badPoint) {
+                            int64_t* badPoint, DevicePoints* points) {
   if (int rc = stream_.create()) return rc;
   *badPoint = -1;
   int pid_bits = 0;
@@ -177,7 +177,9 @@ int RangeEngine::buildStore(const gat_cell_grid& grid, const TrajectoryView& db,
   const int64_t n = db.pointNum();
   const uint64_t cellnum = uint64_t(grid.cells_x) * uint64_t(grid.cells_y);
   void* s = stream_.get();
-  DeviceBuffer lon, lat, off, starts;
+  DevicePoints own;
+  DevicePoints& in = points ? *points : own;
+  DeviceBuffer &lon = in.lon, &lat = in.lat, &off = in.off, starts;
   if (int rc = starts.reserve((cellnum + 1) * 8)) return rc;
   if (int rc = stageBuild(db, pid_bits, lon, lat, off)) return rc;
   GATH_TRY(gat_cell_store_build(&grid, lon.as<float>(), lat.as<float>(), off.as<int64_t>(), db.trajNum, n, pid_bits,

@@ -148,8 +148,12 @@ class RangeEngine {
   // the cells of `grid` (gat_cell_store_build), with the same id packing as
   // upload(); *cellStart receives the grid's cellnum + 1 store offsets and
   // *badPoint the first point off the grid (then no store is kept) or -1.
+  // `points` (when not null) keeps the trajectories' own device copy.
+  struct DevicePoints {
+    DeviceBuffer lon, lat, off;
+  };
   int buildStore(const gat_cell_grid& grid, const TrajectoryView& db, std::vector<int64_t>* cellStart,
-                 int64_t* badPoint);
+                 int64_t* badPoint, DevicePoints* points = nullptr);
   // Builds the store on the device in the order of a kd-tree of the given
   // shape (gat_kd_store_build), with the same id packing; *medians gets one
   // value per split node, *leafBoxes four per leaf.
