@@ -175,7 +175,7 @@ __global__ __launch_bounds__(64, (MAXM >= 2048 && SEG == 16) ? 2 : 4) void edr_w
       ms[0] = m0;
     }
     bool mine = false;
-    const int res = edr::sweep_pairs<SEG, SEG == 64>(R, n, C, m, nmax, mmax, ns, ms, u, above, seg, l, &mine);
+    const int res = edr::sweep_pairs<SEG, false>(R, n, C, m, nmax, mmax, ns, ms, u, above, seg, l, &mine);
     __syncthreads();  // the next job re-initialises `above`
     if (live && !valid && l == 0) out[job.first + seg] = -1;
     if (valid && mine) out[job.first + seg] = res + n;  // D = E + n
@@ -254,18 +254,30 @@ __device__ __forceinline__ void pipe_pair(PipeShared<MAXM, W>& sh, const float2*
   int16_t* own = sh.rows[wv];
   auto begin_strip = [&]() __attribute__((always_inline)) {
     rows.start();
-    const float4 box = edr::segment_box<64>(rows.template load<true>(R, n, s * kRows + l * K));
-    auto touches = [&](int c) __attribute__((always_inline)) -> uint64_t {
-      return __ballot(c < nchunks && edr::may_touch(box, sh.chunk[min(c, S::kChunks - 1)], u));
-    };
-    // A block's lanes reach back over the five chunks up to its own.
-    const uint64_t t0 = touches(l), t1 = touches(l + 64), t2 = touches(l + 128);
+    // Each 16-lane row of lanes against the columns it is at: row r, block b,
+    // the chunks b - r and b - r - 1 (as in sweep_strip).
+    const float4 own_box = edr::segment_box<16>(rows.template load<true>(R, n, s * kRows + l * K));
+    float4 cb[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int c = l + 64 * i;
+      cb[i] = c < nchunks ? sh.chunk[min(c, S::kChunks - 1)] : edr::empty_box();
+    }
     near0 = near1 = near2 = 0;
 #pragma unroll
-    for (int d = 0; d < 5; ++d) {
-      near0 |= t0 << d;
-      near1 |= t1 << d | (d ? t0 >> (64 - d) : 0);
-      near2 |= t2 << d | (d ? t1 >> (64 - d) : 0);
+    for (int r = 0; r < 4; ++r) {
+      const auto row = [&](float v) __attribute__((always_inline)) {
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16 * r));
+      };
+      const float4 box = make_float4(row(own_box.x), row(own_box.y), row(own_box.z), row(own_box.w));
+      const uint64_t t0 = __ballot(edr::may_touch(box, cb[0], u)), t1 = __ballot(edr::may_touch(box, cb[1], u)),
+                     t2 = __ballot(edr::may_touch(box, cb[2], u));
+#pragma unroll
+      for (int d = r; d < r + 2; ++d) {
+        near0 |= t0 << d;
+        near1 |= t1 << d | (d ? t0 >> (64 - d) : 0);
+        near2 |= t2 << d | (d ? t1 >> (64 - d) : 0);
+      }
     }
     loaded = false;
     const int loc = n - 1 - s * kRows;  // < kRows in the last strip only

@@ -70,14 +70,15 @@ __device__ __forceinline__ float2 point_or_nan(const float2* P, int i, int n) {
   return make_float2(uint32_t(i) < uint32_t(n) ? v.x : __builtin_nanf(""), v.y);
 }
 
-// The same for i >= 0; in a padded store (!kGuard) point n is a NaN point.
+// The same; in a padded store (!kGuard) point n is a NaN point, and one
+// unsigned minimum takes every i outside 0 .. n - 1 to it.
 template <bool kGuard>
-__device__ __forceinline__ float2 point_up_to(const float2* P, int i, int n) {
+__device__ __forceinline__ float2 point_in(const float2* P, int i, int n) {
   if constexpr (kGuard) {
     return point_or_nan(P, i, n);
   } else {
-    return *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(P) +
-                                            uint32_t(min(i, n)) * uint32_t(sizeof(float2)));
+    const uint32_t at = min(uint32_t(i) * uint32_t(sizeof(float2)), uint32_t(n) * uint32_t(sizeof(float2)));
+    return *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(P) + at);
   }
 }
 
@@ -144,7 +145,7 @@ struct LaneRows {
     float4 b = empty_box();
 #pragma unroll
     for (int i = 0; i < K; ++i) {
-      const float2 p = point_up_to<kGuard>(R, first + i, n);
+      const float2 p = point_in<kGuard>(R, first + i, n);
       rx[i] = p.x;
       ry[i] = p.y;
       b = grow(b, p);
@@ -203,8 +204,9 @@ using RowValue = std::conditional_t<SEG == 64, int32_t, int16_t>;
 // is taken by the lane that owns row n at the step it reaches column m; the
 // block it falls into is the only one that tests for it.
 //
-// kGuard: the store holds no padding around the columns, so every load is
-// checked against 0 .. m - 1 (NaN outside).
+// kGuard: the store holds no padding, so every load is checked against
+// 0 .. m - 1 (NaN outside).  Otherwise a NaN point follows every trajectory, and
+// the padding before it covers a 16-lane segment's look-behind.
 template <int SEG, int K, bool kGuard>
 __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2* C, int m, int row0, int mmax,
                                             const int (&ns)[64 / SEG], const int (&ms)[64 / SEG], const float4& colbox,
@@ -212,10 +214,18 @@ __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2
                                             bool& mine) {
   constexpr int kSegs = 64 / SEG;
   constexpr int kOff = kRowOff<SEG>;
-  constexpr uint32_t kWindow = SEG == 16 ? 0x3u : 0x1Fu;  // chunks a block's lanes reach back over
+  // hist: kSpread bits per block, the newest lowest; row r of a 64-lane segment
+  // is at the chunks of r and r + 1 blocks ago, a 16-lane segment at the last two.
+  constexpr int kSpread = SEG == 16 ? 1 : 4;
+  constexpr uint32_t kWindow =
+      SEG == 16 ? 0x3u : (1u << 0 | 1u << 4) | (1u << 5 | 1u << 9) | (1u << 10 | 1u << 14) | (1u << 15 | 1u << 19);
   LaneRows<K> rows;
   rows.start();
-  const float4 rowbox = segment_box<SEG>(rows.template load<kGuard>(R, n, row0 + l * K));
+  // The box of each 16-lane row's rows.  (A 64-lane segment's rows of lanes lie
+  // 16 columns apart: each is tested against the columns it is at.  One box of
+  // all 256 rows against the five chunks they cover called 0.30 of a top-k
+  // batch's blocks near, this 0.22.)
+  const float4 rowbox = segment_box<16>(rows.template load<kGuard>(R, n, row0 + l * K));
   // Row n inside this strip: its lane, its row of the lane and the step its
   // last column comes at; the same per segment, wave-uniform.
   const int loc = n - 1 - row0;
@@ -232,8 +242,8 @@ __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2
   const int steps = mmax + SEG - 1;
   const float2* cp = C - l;  // column point of step t is cp[t]
   auto column = [&](int t) __attribute__((always_inline)) -> float2 {
-    if constexpr (kGuard) {
-      return point_or_nan(C, t - l, m);
+    if constexpr (kGuard || SEG == 64) {
+      return point_in<kGuard>(C, t - l, m);
     } else {
       return cp[t];
     }
@@ -295,11 +305,14 @@ __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2
   }
   // Chunk b: columns 16 b .. 16 b + 15 of each segment, one per lane of a row.
   auto chunk = [&](int b) __attribute__((always_inline)) -> float2 {
-    return point_up_to<kGuard>(C, b * kBlk + (l & 15), m);
+    return point_in<kGuard>(C, b * kBlk + (l & 15), m);
   };
   auto touches = [&](const float2& p) __attribute__((always_inline)) -> uint32_t {
     const float4 cb = segment_box<16>(grow(empty_box(), p));
-    return __ballot(may_touch(rowbox, cb, u)) != 0 ? 1u : 0u;
+    const uint64_t t = __ballot(may_touch(rowbox, cb, u));
+    if constexpr (SEG == 16) return t != 0 ? 1u : 0u;
+    // (The same in all lanes of a row.)
+    return uint32_t(t & 1u) | uint32_t(t >> 15 & 2u) | uint32_t(t >> 30 & 4u) | uint32_t(t >> 45 & 8u);
   };
   uint32_t hist = touches(chunk(0));
   float2 ahead = chunk(1);
@@ -321,7 +334,7 @@ __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2
       if (cap) block(No{}, Yes{}, t0);
       else block(No{}, No{}, t0);
     }
-    hist = (hist << 1) | touches(pn);
+    hist = (hist << kSpread) | touches(pn);
   }
 }
 
