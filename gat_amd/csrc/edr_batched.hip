@@ -595,35 +595,93 @@ __global__ __launch_bounds__(64 * kGridFilterWaves) void edr_filter_grid_kernel(
 
 // The all-mismatch table: out[r * (maxlen + 1) + c] = D[r][c] of the recurrence
 // with every substitution costing 1, for 0 <= r, c <= maxlen.  A pair of
-// lengths n <= m with no matching point has distance out[n][m].  One
-// workgroup sweeps the anti-diagonals.
-__global__ __launch_bounds__(1024) void edr_mismatch_table_kernel(int32_t maxlen, int32_t* __restrict__ out) {
-  __shared__ int32_t dg[3][GAT_MAX_TRAJ_LEN + 2];
-  const int w = maxlen + 1;
-  int32_t* d2 = dg[0];
-  int32_t* d1 = dg[1];
-  int32_t* d0 = dg[2];
-  for (int d = 0; d <= 2 * maxlen; ++d) {
-    const int rlo = d - maxlen > 0 ? d - maxlen : 0;
-    const int rhi = d < maxlen ? d : maxlen;
-    for (int r = rlo + int(threadIdx.x); r <= rhi; r += 1024) {
-      const int c = d - r;
-      int v;
-      if (r == 0) v = c;
-      else if (c == 0) v = r;
-      else {
-        const int mm = d2[r - 1] + 1, uu = d1[r - 1] + 1, ll = d1[r] + 1;
-        const bool c1 = mm < uu && mm < ll, c2 = ll < uu && ll < mm;  // Grid.cpp:1297-1300
-        v = c1 ? mm : (c2 ? ll : uu);
+// lengths n <= m with no matching point has distance out[n][m].  A serial chain
+// of 2 * maxlen anti-diagonals: one workgroup with a barrier after each took
+// 2.32 ms, which an index's first top-k waited for.  In two launches: a
+// workgroup sweeps strips of 256 rows as the EDR kernels do (edr_dp.hpp), a
+// barrier per 16 columns, and keeps every 64th row; then a wave per 64 rows
+// sweeps them again from the row above and stores them all, 64 bytes per lane
+// (4.2M values stored by the one workgroup would take its CU 0.45 ms alone): 0.36
+// and 0.09 ms.
+constexpr int kTabWaves = 8, kTabRows = 256, kTabLag = 5;  // lane 63 is 62 columns behind: blocks b .. b + 4
+constexpr int kTabRing = 128;                             // a reader is at most 79 columns behind
+
+__global__ __launch_bounds__(64 * kTabWaves) void edr_mismatch_rows_kernel(int32_t maxlen, int32_t* __restrict__ out) {
+  __shared__ int32_t ring[kTabWaves][kTabRing];
+  static_assert(kTabWaves * kTabRows >= GAT_MAX_TRAJ_LEN, "the waves cover every row");
+  const int64_t w = maxlen + 1;
+  for (int64_t c = threadIdx.x; c < w; c += blockDim.x) {
+    out[c] = int32_t(c);
+    out[c * w] = int32_t(c);
+  }
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int nblocks = (maxlen + 63 + kBlk - 1) / kBlk;
+  const int kend = nblocks + (kTabWaves - 1) * kTabLag;
+  const int row = wv * kTabRows + (l + 1) * 4;  // the lane's last row
+  edr::LaneRows<4> rows;
+  rows.start();
+  for (int k = 0; k < kend; ++k) {
+    const int b = k - wv * kTabLag;
+    if (b >= 0 && b < nblocks && wv * kTabRows < maxlen) {
+      const int t0 = b * kBlk;
+      int bottom[kBlk];
+#pragma unroll
+      for (int j = 0; j < kBlk; ++j)
+        bottom[j] = wv == 0 ? t0 + j + 1 : ring[wv == 0 ? 0 : wv - 1][(t0 + j + 1) & (kTabRing - 1)];
+#pragma unroll
+      for (int j = 0; j < kBlk; ++j) {
+        const int u0 = edr::shift_in<64>(bottom[j], rows.e[3]);
+        rows.step<false>(u0, make_float2(0.0f, 0.0f), 0.0f);
+        bottom[j] = rows.e[3];
       }
-      d0[r] = v;
-      out[int64_t(r) * w + c] = v;
+      if ((l & 15) == 15) {
+#pragma unroll
+        for (int j = 0; j < kBlk; ++j) {
+          const int c = t0 + j - l + 1;
+          if (l == 63) ring[wv][c & (kTabRing - 1)] = bottom[j];
+          if (c >= 1 && c <= maxlen && row <= maxlen) out[row * w + c] = bottom[j] + row;
+        }
+      }
     }
     __syncthreads();
-    int32_t* t = d2;
-    d2 = d1;
-    d1 = d0;
-    d0 = t;
+  }
+}
+
+struct alignas(4) FourInts {
+  int32_t v[4];
+};
+
+__global__ __launch_bounds__(64) void edr_mismatch_fill_kernel(int32_t maxlen, int32_t* __restrict__ out) {
+  const int64_t w = maxlen + 1;
+  const int l = threadIdx.x;
+  const int r0 = int(blockIdx.x) * 64, row = r0 + l + 1;
+  const int steps = maxlen + 63;
+  const bool mine = row <= maxlen && l < 63;  // every 64th row is there already
+  edr::LaneRows<1> rows;
+  rows.start();
+  auto feed = [&](int t0) { return out[r0 * w + min(t0 + 1 + (l & 15), maxlen)] - r0; };
+  int ahead = feed(0);
+  for (int t0 = 0; t0 < steps; t0 += kBlk) {
+    const int above = ahead;
+    ahead = feed(t0 + kBlk);
+    int32_t v[kBlk];
+#pragma unroll
+    for (int j = 0; j < kBlk; ++j) {
+      const int u0 = edr::shift_in<64>(__builtin_amdgcn_readlane(above, j), rows.e[0]);
+      rows.step<false>(u0, make_float2(0.0f, 0.0f), 0.0f);
+      v[j] = rows.e[0] + row;
+    }
+    const int c0 = t0 - l + 1;
+    int32_t* dst = out + row * w + c0;
+    if (mine && c0 >= 1 && c0 + kBlk - 1 <= maxlen) {
+#pragma unroll
+      for (int j = 0; j < kBlk; j += 4)
+        *reinterpret_cast<FourInts*>(dst + j) = FourInts{{v[j], v[j + 1], v[j + 2], v[j + 3]}};
+    } else if (mine) {
+#pragma unroll
+      for (int j = 0; j < kBlk; ++j)
+        if (c0 + j >= 1 && c0 + j <= maxlen) dst[j] = v[j];
+    }
   }
 }
 
@@ -1931,8 +1989,12 @@ extern "C" int gat_edr_pack_trajectories(const float* lon, const float* lat, con
 extern "C" int gat_edr_mismatch_table(int32_t maxlen, int32_t* out, void* stream) {
   GAT_REQUIRE(maxlen >= 0 && maxlen <= GAT_MAX_TRAJ_LEN, "mismatch table: maxlen outside 0..%d", GAT_MAX_TRAJ_LEN);
   GAT_REQUIRE(out, "mismatch table: null output");
-  edr_mismatch_table_kernel<<<dim3(1), dim3(1024), 0, gat::as_stream(stream)>>>(maxlen, out);
-  GAT_LAUNCH_CHECK("edr_mismatch_table_kernel");
+  edr_mismatch_rows_kernel<<<dim3(1), dim3(64 * kTabWaves), 0, gat::as_stream(stream)>>>(maxlen, out);
+  GAT_LAUNCH_CHECK("edr_mismatch_rows_kernel");
+  if (maxlen > 0) {
+    edr_mismatch_fill_kernel<<<dim3(uint32_t((maxlen + 63) / 64)), dim3(64), 0, gat::as_stream(stream)>>>(maxlen, out);
+    GAT_LAUNCH_CHECK("edr_mismatch_fill_kernel");
+  }
   return GAT_OK;
 }
 
