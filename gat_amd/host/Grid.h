@@ -31,6 +31,17 @@ struct TopK {
   std::vector<int32_t> ids, dist;
 };
 
+// Where a batch's answers go: one TopK per query, or rows of `width` ids and
+// distances (what a row lacks: id 0, distance -1).
+struct TopKSink {
+  std::vector<TopK>* vec = nullptr;
+  int32_t* ids = nullptr;
+  int32_t* dists = nullptr;
+  // nq rows of `width` of which `have` are results.
+  void put(const int32_t* rowIds, const int32_t* rowDists, int nq, int width, int have);
+  void put(const std::vector<TopK>& rows, int width);
+};
+
 // Counters of one batched EDR call.
 struct EdrBatchStats {
   int64_t pairs = 0;       // pairs whose DP ran
@@ -114,6 +125,7 @@ class Grid {
   // value, the rest run the batched DP.
   int edrBatchedAll(const TrajectoryView& queries, std::vector<int32_t>& dist, EdrBatchStats* stats);
   int similarityBatched(const TrajectoryView& queries, int kValue, std::vector<TopK>& out, EdrBatchStats* stats);
+  int similarityBatched(const TrajectoryView& queries, int kValue, TopKSink out, EdrBatchStats* stats);
   // The all-mismatch table F[r][c], (GAT_MAX_TRAJ_LEN + 1)^2 entries, computed
   // on the device once.
   const std::vector<int32_t>& mismatchTable();
@@ -203,13 +215,14 @@ class Grid {
   // merge) with one readback at the end; *done is false when the batch must
   // take the host-built path instead (a query with more survivors than the
   // device's per-query sort holds).
-  int similarityOnDevice(int nq, int kValue, std::vector<TopK>& out, EdrBatchStats* st, bool* done);
+  int similarityOnDevice(int nq, int kValue, TopKSink& out, EdrBatchStats* st, bool* done);
   // The same for batches of few queries, whose time is their launches and the
   // longest pair: no job list (every survivor takes several waves), the merge
   // straight from the pairs, results written to pinned memory.  *done is
   // false when more pairs survive than it is for.
-  int similaritySmall(const TrajectoryView& queries, int kValue, std::vector<TopK>& out, EdrBatchStats* st,
-                      bool* done);
+  int similaritySmall(const TrajectoryView& queries, int kValue, TopKSink& out, EdrBatchStats* st, bool* done);
+  // The batch with its pairs, jobs and lists built on the host.
+  int similarityHost(int nq, int kValue, std::vector<TopK>& out, EdrBatchStats* st);
   static constexpr int64_t kUploadPart = 1 << 17;  // points of a part of the queries' upload
   static constexpr int kSmallTopkQueries = 32;
   static constexpr int64_t kSmallTopkPairs = 2048;

@@ -861,10 +861,12 @@ uint64_t ctl64(const uint32_t* c, int w) { return uint64_t(c[w]) | (uint64_t(c[w
 // one whose queries have more survivors than the merge sorts in LDS, takes
 // those two.  A survivor count above the capacity empties every window: the
 // capacity grows and the batch runs again.
-int Grid::similarityOnDevice(int nq, int kValue, std::vector<TopK>& out, EdrBatchStats* st, bool* done) {
+int Grid::similarityOnDevice(int nq, int kValue, TopKSink& out, EdrBatchStats* st, bool* done) {
   *done = nq == 0;
-  out.clear();
-  if (nq == 0) return GAT_OK;
+  if (nq == 0) {
+    out.put(nullptr, nullptr, 0, kValue, 0);
+    return GAT_OK;
+  }
   void* s = engine_.stream();
   if (clockKhz_ == 0) GATH_TRY(gat_wall_clock_khz(&clockKhz_), "device clock");
   int64_t eligible = 0;
@@ -950,11 +952,7 @@ int Grid::similarityOnDevice(int nq, int kValue, std::vector<TopK>& out, EdrBatc
       gath_set_error("top-k merge: inconsistent inputs (status %u)", c[3]);
       return GAT_ERR_HIP;
     }
-    out.assign(size_t(nq), TopK{});
-    for (int q = 0; q < nq; ++q) {
-      out[size_t(q)].ids.assign(top + int64_t(q) * kValue, top + int64_t(q) * kValue + kk);
-      out[size_t(q)].dist.assign(top + cells + int64_t(q) * kValue, top + cells + int64_t(q) * kValue + kk);
-    }
+    out.put(top, top + cells, nq, kValue, kk);
     if (st) {
       st->pairs += int64_t(found);
       st->cells += int64_t(ctl64(c, 4));
@@ -978,8 +976,7 @@ int Grid::similarityOnDevice(int nq, int kValue, std::vector<TopK>& out, EdrBatc
   return GAT_OK;  // still over capacity after growing once: the host-built path
 }
 
-int Grid::similaritySmall(const TrajectoryView& queries, int kValue, std::vector<TopK>& out, EdrBatchStats* st,
-                          bool* done) {
+int Grid::similaritySmall(const TrajectoryView& queries, int kValue, TopKSink& out, EdrBatchStats* st, bool* done) {
   *done = false;
   const int nq = queries.trajNum;
   int64_t eligible = 0;
@@ -1026,11 +1023,7 @@ int Grid::similaritySmall(const TrajectoryView& queries, int kValue, std::vector
     gath_set_error("top-k merge: inconsistent inputs (status %u)", c[3]);
     return GAT_ERR_HIP;
   }
-  out.assign(size_t(nq), TopK{});
-  for (int q = 0; q < nq; ++q) {
-    out[size_t(q)].ids.assign(top + int64_t(q) * kValue, top + int64_t(q) * kValue + kk);
-    out[size_t(q)].dist.assign(top + cells + int64_t(q) * kValue, top + cells + int64_t(q) * kValue + kk);
-  }
+  out.put(top, top + cells, nq, kValue, kk);
   if (st) {
     st->pairs += int64_t(found);
     st->cells += int64_t(ctl64(c, 4));
@@ -1044,7 +1037,47 @@ int Grid::similaritySmall(const TrajectoryView& queries, int kValue, std::vector
   return GAT_OK;
 }
 
+void TopKSink::put(const int32_t* rowIds, const int32_t* rowDists, int nq, int width, int have) {
+  if (vec) {
+    vec->assign(size_t(nq), TopK{});
+    for (int q = 0; q < nq; ++q) {
+      const int64_t at = int64_t(q) * width;
+      (*vec)[size_t(q)].ids.assign(rowIds + at, rowIds + at + have);
+      (*vec)[size_t(q)].dist.assign(rowDists + at, rowDists + at + have);
+    }
+    return;
+  }
+  const size_t n = size_t(nq) * size_t(std::max(width, 0));
+  if (n == 0) return;
+  if (have == width) {
+    std::memcpy(ids, rowIds, n * 4);
+    std::memcpy(dists, rowDists, n * 4);
+    return;
+  }
+  for (int q = 0; q < nq; ++q)
+    for (int j = 0; j < width; ++j) {
+      const int64_t at = int64_t(q) * width + j;
+      ids[at] = j < have ? rowIds[at] : 0;
+      dists[at] = j < have ? rowDists[at] : -1;
+    }
+}
+
+void TopKSink::put(const std::vector<TopK>& rows, int width) {
+  for (size_t q = 0; q < rows.size(); ++q)
+    for (int j = 0; j < width; ++j) {
+      const bool has = j < int(rows[q].ids.size());
+      ids[q * size_t(width) + size_t(j)] = has ? rows[q].ids[size_t(j)] : 0;
+      dists[q * size_t(width) + size_t(j)] = has ? rows[q].dist[size_t(j)] : -1;
+    }
+}
+
 int Grid::similarityBatched(const TrajectoryView& queries, int kValue, std::vector<TopK>& out, EdrBatchStats* st) {
+  TopKSink sink;
+  sink.vec = &out;
+  return similarityBatched(queries, kValue, sink, st);
+}
+
+int Grid::similarityBatched(const TrajectoryView& queries, int kValue, TopKSink out, EdrBatchStats* st) {
   if (int rc = checkTrajLengths("similarityBatched")) return rc;
   const int nq = queries.trajNum;
   if (deviceChain && kValue >= 1 && kValue <= kDeviceTopkMax && nq >= 1 && nq <= kSmallTopkQueries && trajNum >= 1 &&
@@ -1066,6 +1099,14 @@ int Grid::similarityBatched(const TrajectoryView& queries, int kValue, std::vect
     if (int rc = similarityOnDevice(nq, kValue, out, st, &done)) return rc;
     if (done) return GAT_OK;
   }
+  if (out.vec) return similarityHost(nq, kValue, *out.vec, st);
+  std::vector<TopK> rows;
+  if (int rc = similarityHost(nq, kValue, rows, st)) return rc;
+  out.put(rows, kValue);
+  return GAT_OK;
+}
+
+int Grid::similarityHost(int nq, int kValue, std::vector<TopK>& out, EdrBatchStats* st) {
   void* s = engine_.stream();
   // Candidate filter on the device; grow the survivor buffer until it fits.
   int64_t cap = std::max<int64_t>(int64_t(nq) * 64, 1024);

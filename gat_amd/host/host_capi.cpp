@@ -603,15 +603,11 @@ int gath_grid_similarity_batched(void* p, const int64_t* q_offsets, int nq, cons
   if (!ix || !ix->grid || nq < 0 || k < 0 || !q_offsets) return bad("gath_grid_similarity_batched: bad arguments");
   ix->grid->epsilon = eps;
   TrajectoryView q{q_offsets, nq, qlon, qlat};
-  std::vector<TopK> res;
+  TopKSink rows;
+  rows.ids = ids;
+  rows.dists = dists;
   EdrBatchStats st;
-  if (int rc = ix->grid->similarityBatched(q, k, res, &st)) return rc;
-  for (int i = 0; i < nq; ++i)
-    for (int j = 0; j < k; ++j) {
-      const bool have = j < int(res[i].ids.size());
-      ids[int64_t(i) * k + j] = have ? res[i].ids[j] : 0;
-      dists[int64_t(i) * k + j] = have ? res[i].dist[j] : -1;
-    }
+  if (int rc = ix->grid->similarityBatched(q, k, rows, &st)) return rc;
   put_stats(st, stats, ms);
   return GAT_OK;
 }
