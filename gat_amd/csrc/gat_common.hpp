@@ -93,6 +93,21 @@ __device__ __forceinline__ int4 load_pair2(const int2* pairs, uint64_t at, uint6
   return v;
 }
 
+// The same without a branch: of an end below or at an even capacity, the pair
+// group at min(at, the last one's).  (Behind a branch each load was waited for
+// before the next was issued.)
+template <bool kWide>
+__device__ __forceinline__ int4 load_pair2_in(const int2* pairs, uint64_t at, uint64_t end) {
+  const uint64_t last = (end - 1) & ~uint64_t(1);
+  at = at < last ? at : last;
+  if constexpr (kWide) {
+    return *reinterpret_cast<const int4*>(pairs + at);
+  } else {
+    const int2 p = pairs[at], q = pairs[at + 1];
+    return make_int4(p.x, p.y, q.x, q.y);
+  }
+}
+
 // Order-independent digest of a (tid, pid) pair: a 64-bit mix (the splitmix64
 // finaliser) of tid in the high and pid in the low half.  A query's digest is
 // the wrapping sum over its pairs.

@@ -219,19 +219,23 @@ __global__ __launch_bounds__(kBlock) void pairs_digest_kernel(const int2* __rest
     const uint64_t a = b & ~uint64_t(1), e = b + n;
     uint64_t acc = 0;
     if (a + uint64_t(blockIdx.y) * kDigestSpan >= e) continue;  // uniform: no pair of this split's
-    for (uint64_t s = a + uint64_t(blockIdx.y) * kDigestSpan; s < e; s += uint64_t(gridDim.y) * kDigestSpan) {
-      int4 v[4];
+    auto sweep = [&](auto load) __attribute__((always_inline)) {
+      for (uint64_t s = a + uint64_t(blockIdx.y) * kDigestSpan; s < e; s += uint64_t(gridDim.y) * kDigestSpan) {
+        int4 v[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        v[k] = gat::load_pair2<kWide>(pairs, s + 2 * threadIdx.x + uint64_t(k) * 2 * kBlock, e);
-      }
+        for (int k = 0; k < 4; ++k) v[k] = load(s + 2 * threadIdx.x + uint64_t(k) * 2 * kBlock);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint64_t i = s + 2 * threadIdx.x + uint64_t(k) * 2 * kBlock;
-        if (i >= b && i < e) acc += gat::pair_mix(make_int2(v[k].x, v[k].y));
-        if (i + 1 < e) acc += gat::pair_mix(make_int2(v[k].z, v[k].w));
+        for (int k = 0; k < 4; ++k) {
+          const uint64_t i = s + 2 * threadIdx.x + uint64_t(k) * 2 * kBlock;
+          if (i >= b && i < e) acc += gat::pair_mix(make_int2(v[k].x, v[k].y));
+          if (i + 1 < e) acc += gat::pair_mix(make_int2(v[k].z, v[k].w));
+        }
       }
-    }
+    };
+    if (e <= (capacity & ~uint64_t(1)))
+      sweep([&](uint64_t at) { return gat::load_pair2_in<kWide>(pairs, at, e); });
+    else  // the last pair of an odd number of them
+      sweep([&](uint64_t at) { return gat::load_pair2<kWide>(pairs, at, e); });
     for (int off = kWave / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
     if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = acc;
     __syncthreads();

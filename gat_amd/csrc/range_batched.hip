@@ -652,9 +652,14 @@ template <class L>
 __global__ __launch_bounds__(kScanBlock) void scan_tiles_kernel(L load, uint64_t n, typename L::T* __restrict__ tiles) {
   using T = typename L::T;
   const uint64_t b = uint64_t(blockIdx.x) * kScanTile + uint64_t(threadIdx.x) * kScanItems;
+  // (Loads clamped, not conditional: behind a branch each was waited for before
+  // the next.)
+  T v[kScanItems];
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) v[k] = load(b + k < n ? b + k : n - 1);
   T s = vzero(T{});
-  for (int k = 0; k < kScanItems; ++k)
-    if (b + k < n) s = vadd(s, load(b + k));
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) s = vadd(s, b + k < n ? v[k] : vzero(T{}));
   T all;
   block_exclusive(s, &all);
   if (threadIdx.x == 0) tiles[blockIdx.x] = all;
@@ -682,11 +687,11 @@ __global__ __launch_bounds__(kScanBlock) void scan_apply_kernel(L load, uint64_t
   }
   const uint64_t b = uint64_t(blockIdx.x) * kScanTile + uint64_t(threadIdx.x) * kScanItems;
   T v[kScanItems];
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) v[k] = load(b + k < n ? b + k : n - 1);
   T s = vzero(T{});
-  for (int k = 0; k < kScanItems; ++k) {
-    v[k] = b + k < n ? load(b + k) : vzero(T{});
-    s = vadd(s, v[k]);
-  }
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) s = vadd(s, b + k < n ? v[k] : vzero(T{}));
   T all;
   T run = vadd(carry, block_exclusive(s, &all));
   for (int k = 0; k < kScanItems; ++k)
@@ -729,9 +734,9 @@ struct LoadItemBounds {
   using T = uint64_t;
   __device__ T operator()(uint64_t i) const {
     const uint64_t total = *item_total;
-    if (i >= (total < cap ? total : cap)) return 0;
-    const Item it = items[i];
-    return (uint64_t(it.n) * it.count + 15) & ~uint64_t(15);
+    const Item it = items[i];  // i < cap: in the buffer, if not an item
+    const uint64_t bound = (uint64_t(it.n) * it.count + 15) & ~uint64_t(15);
+    return i < (total < cap ? total : cap) ? bound : 0;
   }
 };
 
@@ -955,18 +960,16 @@ static_assert(sizeof(Run) == sizeof(gat_range_run), "run record layout");
 template <int NS, bool kPacked>
 __device__ __forceinline__ void load_chunk(const Store& store, uint64_t at0, uint32_t left, uint32_t lane,
                                            float2 (&v)[NS], uint32_t (&id)[NS], uint32_t (&pid)[NS]) {
-  const float nan = __builtin_nanf("");
+  // (Clamped to the last point, not conditional; left >= 1.)
 #pragma unroll
   for (int k = 0; k < NS; ++k) {
     const uint32_t i = k * kWave + lane;
-    v[k] = make_float2(nan, 0.0f);
-    id[k] = 0;
+    const uint64_t at = at0 + (i < left ? i : left - 1);
+    v[k] = store.xy[at];
+    id[k] = store.id[at];
     pid[k] = 0;
-    if (i < left) {
-      v[k] = store.xy[at0 + i];
-      id[k] = store.id[at0 + i];
-      if constexpr (!kPacked) pid[k] = store.pid[at0 + i];
-    }
+    if constexpr (!kPacked) pid[k] = store.pid[at];
+    v[k].x = i < left ? v[k].x : __builtin_nanf("");
   }
 }
 
@@ -1339,9 +1342,10 @@ __global__ __launch_bounds__(256) void run_counts_kernel(const Item* __restrict_
 // start at zero).  Bound by the read of the pairs (8 B each) and by the mix (two
 // 64-bit multiplies, about 0.6 of the read's time at full issue).  A wave per
 // run read a median run of 110 pairs in two half-empty 8-byte loads and spent
-// as long on its 64-lane reduction and atomic.  Each workgroup's runs are
-// consecutive, and the entries of the first lds_q queries are summed in LDS
-// first.
+// as long on its 64-lane reduction and atomic.  The loads are clamped, not
+// conditional (load_pair2_in): 5.6 GB of pairs in 1,069 us, 5.2 TB/s, where loads
+// behind branches were waited for one by one and took 1,268 us (nontemporal
+// ones: 1,109).  The entries of the first lds_q queries are summed in LDS first.
 constexpr int kDigBlock = 512;
 constexpr uint32_t kDigLds = 4096;  // 32 KB of 64-bit sums: four workgroups per CU
 
@@ -1370,31 +1374,32 @@ __global__ __launch_bounds__(kDigBlock) void runs_digest_kernel(const int2* __re
   __syncthreads();
   constexpr uint32_t kRowsPer = kDigBlock / 16;
   const uint32_t l = threadIdx.x & 15;
-  const uint64_t per = (nruns + gridDim.x - 1) / gridDim.x;
-  const uint64_t lo = uint64_t(blockIdx.x) * per;
-  const uint64_t hi = lo + per < nruns ? lo + per : nruns;
-  uint64_t r = lo + threadIdx.x / 16;
-  Run next = r < hi ? runs[r] : Run{0, 0, 0};
-  for (; r < hi; r += kRowsPer) {
+  const uint64_t step = uint64_t(gridDim.x) * kRowsPer;
+  uint64_t r = uint64_t(blockIdx.x) * kRowsPer + threadIdx.x / 16;
+  Run next = r < nruns ? runs[r] : Run{0, 0, 0};
+  for (; r < nruns; r += step) {
     const Run run = next;
-    if (r + kRowsPer < hi) next = runs[r + kRowsPer];
+    if (r + step < nruns) next = runs[r + step];
     // Uniform over the row, so its lanes stay together for the sum.
     if (run.count == 0 || run.q >= nqueries || run.first > npairs || run.count > npairs - run.first) continue;
     const uint64_t end = run.first + run.count;
     uint64_t sum = 0;
     // Lane l's pairs i, i + 1 from the even pair at or below the run's first.
-    for (uint64_t i = (run.first & ~uint64_t(1)) + 2 * l; i < end; i += 128) {
-      int4 v[4];
+    auto add = [&](const int4& v, uint64_t at) __attribute__((always_inline)) {
+      if (at >= run.first && at < end) sum += gat::pair_mix(make_int2(v.x, v.y));
+      if (at + 1 < end) sum += gat::pair_mix(make_int2(v.z, v.w));
+    };
+    if (end <= (npairs & ~uint64_t(1))) {
+      for (uint64_t i = (run.first & ~uint64_t(1)) + 2 * l; i < end; i += 128) {
+        int4 v[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        v[k] = gat::load_pair2<kWide>(pairs, i + 32 * k, end);
-      }
+        for (int k = 0; k < 4; ++k) v[k] = gat::load_pair2_in<kWide>(pairs, i + 32 * k, end);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint64_t at = i + 32 * k;
-        if (at >= run.first && at < end) sum += gat::pair_mix(make_int2(v[k].x, v[k].y));
-        if (at + 1 < end) sum += gat::pair_mix(make_int2(v[k].z, v[k].w));
+        for (int k = 0; k < 4; ++k) add(v[k], i + 32 * k);
       }
+    } else {  // the last pair of an odd number of them
+      for (uint64_t i = (run.first & ~uint64_t(1)) + 2 * l; i < end; i += 32)
+        add(gat::load_pair2<kWide>(pairs, i, end), i);
     }
     // Lanes that ran out early wait here with the rest of their row.
     sum = row16_sum(sum);
