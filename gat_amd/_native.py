@@ -116,7 +116,7 @@ HIP_FUNCS = {
     "gat_leaf_item_regions": (INT, [P, P, I64, P, P, P, P]),
     "gat_leaf_refine_runs": (INT, [P, P, P, I64, P, I64, P, I64, P, I64, P, I64, P, P]),
     "gat_run_counts": (INT, [P, P, P, I64, I64, P, I64, I64, P, P, P]),
-    "gat_runs_digest_live": (INT, [P, I64, P, I64, P, I64, P, P]),
+    "gat_runs_digest_live": (INT, [P, I64, P, I64, P, I64, P, P, P]),
     "gat_runs_digest": (INT, [P, I64, P, I64, I64, P, P]),
     "gat_graph_begin": (INT, [P]),
     "gat_graph_end": (INT, [P, P]),

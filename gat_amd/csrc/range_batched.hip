@@ -1367,8 +1367,14 @@ __global__ __launch_bounds__(kDigBlock) void runs_digest_kernel(const int2* __re
                                                                 const Run* __restrict__ runs, uint64_t nruns,
                                                                 const uint32_t* __restrict__ live,
                                                                 uint32_t nqueries, uint32_t lds_q,
-                                                                unsigned long long* __restrict__ out) {
+                                                                unsigned long long* __restrict__ out,
+                                                                uint32_t* __restrict__ stamp) {
   extern __shared__ unsigned long long dig[];
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) {
+    const uint64_t t = wall_clock64();
+    stamp[0] = uint32_t(t);
+    stamp[1] = uint32_t(t >> 32);
+  }
   if (live) nruns = min(nruns, uint64_t(*live));
   for (uint32_t q = threadIdx.x; q < lds_q; q += kDigBlock) dig[q] = 0;
   __syncthreads();
@@ -1747,7 +1753,7 @@ int gat_run_counts(const gat_point_store* sp, const uint32_t* items, const uint3
 }
 
 int gat_runs_digest_live(const int32_t* pairs, int64_t npairs, const gat_range_run* runs, int64_t nruns,
-                         const uint32_t* live, int64_t nqueries, uint64_t* out, void* stream) {
+                         const uint32_t* live, int64_t nqueries, uint64_t* out, uint32_t* stamp, void* stream) {
   GAT_REQUIRE(npairs >= 0 && nruns >= 0 && nqueries >= 0 && nqueries <= int64_t(UINT32_MAX),
               "gat_runs_digest: bad sizes");
   if (nqueries == 0) return GAT_OK;
@@ -1761,17 +1767,17 @@ int gat_runs_digest_live(const int32_t* pairs, int64_t npairs, const gat_range_r
   auto* O = reinterpret_cast<unsigned long long*>(out);
   if (reinterpret_cast<uintptr_t>(pairs) % 16 == 0)
     runs_digest_kernel<true><<<grid, block, size_t(lds_q) * 8, gat::as_stream(stream)>>>(
-        P, uint64_t(npairs), R, uint64_t(nruns), live, uint32_t(nqueries), lds_q, O);
+        P, uint64_t(npairs), R, uint64_t(nruns), live, uint32_t(nqueries), lds_q, O, stamp);
   else
     runs_digest_kernel<false><<<grid, block, size_t(lds_q) * 8, gat::as_stream(stream)>>>(
-        P, uint64_t(npairs), R, uint64_t(nruns), live, uint32_t(nqueries), lds_q, O);
+        P, uint64_t(npairs), R, uint64_t(nruns), live, uint32_t(nqueries), lds_q, O, stamp);
   GAT_LAUNCH_CHECK("runs_digest_kernel");
   return GAT_OK;
 }
 
 int gat_runs_digest(const int32_t* pairs, int64_t npairs, const gat_range_run* runs, int64_t nruns,
                     int64_t nqueries, uint64_t* out, void* stream) {
-  return gat_runs_digest_live(pairs, npairs, runs, nruns, nullptr, nqueries, out, stream);
+  return gat_runs_digest_live(pairs, npairs, runs, nruns, nullptr, nqueries, out, nullptr, stream);
 }
 
 int gat_graph_begin(void* stream) {

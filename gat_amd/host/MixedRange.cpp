@@ -119,6 +119,7 @@ int MixedRange::run(const MBB* bounds, int n, const MixedConfig& cfg, MixedResul
     }
     bool done = false;
     const uint64_t* digests[3] = {nullptr, nullptr, nullptr};
+    std::vector<std::pair<uint64_t, uint64_t>> digestSpans;  // device clock
     // Both quick ways below leave counts and digests in pinned memory.
     auto wait = [&](bool replay) -> int {
       int rc = replay ? coord_.sync() : GAT_OK;
@@ -129,8 +130,11 @@ int MixedRange::run(const MBB* bounds, int n, const MixedConfig& cfg, MixedResul
         }
       bool fits = true;
       for (int i = 0; i < 3 && rc == GAT_OK; ++i) {
+        if (nq[i] == 0) continue;
         bool f = true;
-        if (nq[i] > 0) rc = engine(i).finishResults(nq[i], batch_[i], replay, &f, &digests[i]);
+        uint64_t clock[2] = {0, 0};
+        rc = engine(i).finishResults(nq[i], batch_[i], replay, &f, &digests[i], clock);
+        if (f) digestSpans.emplace_back(clock[0], clock[1]);
         fits = fits && f;
       }
       done = rc == GAT_OK && fits;
@@ -227,6 +231,24 @@ int MixedRange::run(const MBB* bounds, int n, const MixedConfig& cfg, MixedResul
       out->candidates += b.candidates;
     }
     out->digestMs += now_ms() - d0;
+    if (done) {
+      // The time in which digests ran, beside each other or not.
+      if (clockKhz_ == 0) {
+        const int rc = gat_wall_clock_khz(&clockKhz_);
+        if (rc != GAT_OK) {
+          restore();
+          return gath_fail_hip(rc, "device clock");
+        }
+      }
+      std::sort(digestSpans.begin(), digestSpans.end());
+      uint64_t covered = 0, ticks = 0;
+      for (const auto& d : digestSpans) {
+        const uint64_t from = std::max(d.first, covered);
+        if (d.second > from) ticks += d.second - from;
+        covered = std::max(covered, d.second);
+      }
+      out->digestMs += double(ticks) / clockKhz_;
+    }
     ++out->groups;
   }
   restore();

@@ -67,6 +67,7 @@ class MixedRange {
   RangeEngine::GraphKey keys_[3];
   const void* results_[3][2] = {};  // and its digests' and results' buffers
   bool keysMatch(const int nq[3]);
+  int32_t clockKhz_ = 0;
  public:
   int captures = 0;  // graphs captured over this object's life
 };

@@ -1103,7 +1103,7 @@ int RangeEngine::enqueueResults(int nq, RangeBatch& out) {
   uint64_t* dig = out.digestDev_.as<uint64_t>();
   if (runIndexed)
     GATH_TRY(gat_runs_digest_live(out.pairs.as<int32_t>(), pairsCap_, out.runs.as<gat_range_run>(), qlistCap_, ctr + 5,
-                                  nq, dig, s),
+                                  nq, dig, ctr + 12, s),
              "run digest");
   else
     GATH_TRY(gat_pairs_digest(out.pairs.as<int32_t>(), out.qbase.as<uint64_t>(), out.qcount.as<uint32_t>(), nq,
@@ -1114,7 +1114,8 @@ int RangeEngine::enqueueResults(int nq, RangeBatch& out) {
   return GAT_OK;
 }
 
-int RangeEngine::finishResults(int nq, RangeBatch& out, bool replay, bool* fits, const uint64_t** digests) {
+int RangeEngine::finishResults(int nq, RangeBatch& out, bool replay, bool* fits, const uint64_t** digests,
+                               uint64_t digestClock[2]) {
   const uint32_t* w = resultHost_.as<uint32_t>();
   std::memcpy(countersHost_.get(), w, 64);
   *fits = countersFit();
@@ -1128,6 +1129,9 @@ int RangeEngine::finishResults(int nq, RangeBatch& out, bool replay, bool* fits,
   out.base.assign(size_t(nq), 0);
   out.hostStale = !out.runIndexed;  // regions
   *digests = reinterpret_cast<const uint64_t*>(w + 32 + (nq + 1) / 2 * 2);
+  digestClock[1] = uint64_t(w[16]) | (uint64_t(w[17]) << 32);
+  digestClock[0] = uint64_t(w[12]) | (uint64_t(w[13]) << 32);
+  if (digestClock[0] == 0) digestClock[0] = digestClock[1];  // no run: no digest ran
   return finishCounters(out, replay);
 }
 

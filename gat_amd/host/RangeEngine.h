@@ -218,11 +218,12 @@ class RangeEngine {
   // reserveResults before, then either queueBatch (upload and pipeline) or, to
   // be captured, enqueueBatch and enqueueResults; once the stream has been waited for
   // finishResults, as finishBatch, with the digests in *digests (pinned, valid
-  // until the next batch).
+  // until the next batch) and the device clock at their start and end.
   int reserveResults(int nq, RangeBatch& out);
   int queueBatch(const DeviceTree& tree, const MBB* bounds, int nq, RangeBatch& out, bool* queued);
   int enqueueResults(int nq, RangeBatch& out);
-  int finishResults(int nq, RangeBatch& out, bool replay, bool* fits, const uint64_t** digests);
+  int finishResults(int nq, RangeBatch& out, bool replay, bool* fits, const uint64_t** digests,
+                    uint64_t digestClock[2]);
   const void* resultsHost() const { return resultHost_.get(); }
 
   // Everything a captured batch pipeline has baked into its kernel arguments:
@@ -299,7 +300,8 @@ class RangeEngine {
   // Batched-form workspace.  counters_ (uint32 words): [0,1] selected entries,
   // [2,3] candidate total, [4] status, [5] list total, [6] work items,
   // [8,9] result pairs, [10,11] run-indexed region total; direct form: [12,13]
-  // and [14,15] the clock at the batch's start and after its selection.
+  // and [14,15] the clock at the batch's start and after its selection; chained
+  // digests: [12,13] the clock at their start.
   DeviceBuffer nodeCount_, lqRank_, nodeOff_, tiles_, cand_, lq_, qlist_, items_, counters_;
   static constexpr int64_t kBitmapBytes = int64_t(64) << 20, kBitmapQueries = 1024;
   DeviceBuffer bitmapDev_;

@@ -728,9 +728,11 @@ int gat_runs_digest(const int32_t* pairs_dev, int64_t npairs, const gat_range_ru
                     int64_t nqueries, uint64_t* out_dev, void* stream);
 
 /* gat_runs_digest of the first min(nruns, *live_dev) runs (null: all of them),
- * for a chain whose host does not know their number yet. */
+ * for a chain whose host does not know their number yet; the wall clock at its
+ * start in stamp_dev (null, or no run: not). */
 int gat_runs_digest_live(const int32_t* pairs_dev, int64_t npairs, const gat_range_run* runs_dev, int64_t nruns,
-                         const uint32_t* live_dev, int64_t nqueries, uint64_t* out_dev, void* stream);
+                         const uint32_t* live_dev, int64_t nqueries, uint64_t* out_dev, uint32_t* stamp_dev,
+                         void* stream);
 
 /* The leaf-major refine: per work item the leaf's points and ids are loaded
  * once and tested against each of the item's rectangles; hits go to query q's
