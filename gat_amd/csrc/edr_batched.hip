@@ -696,11 +696,10 @@ __global__ __launch_bounds__(64) void edr_mismatch_fill_kernel(int32_t maxlen, i
 // its DP distance, and the cut T is the smallest distance whose running count
 // reaches kk.  Every candidate below T is taken (fewer than kk: the
 // non-survivors of the lengths whose value is below T, the survivors whose DP
-// distance is), then the r smallest ids at distance T, found by a binary
-// search for the id bound X over the ascending id lists of the lengths whose
-// value is T (their survivors left out) and the survivors at T; the search
-// range and each list's part of it are cut to the lists' first r + (number of
-// survivors) ids.  The kk results are ranked by (distance, id).
+// distance is), then the r smallest ids at distance T, found among the first ids
+// where T is common, else among the first r + (number of survivors) ids of the
+// lists of the lengths whose value is T (their survivors left out) and the
+// survivors at T.  The kk results are ranked by (distance, id).
 constexpr int kTopkMax = 1024;
 constexpr int kLenBins = GAT_MAX_TRAJ_LEN + 1;     // lengths 0..GAT_MAX_TRAJ_LEN
 constexpr int kDistBins = 2 * GAT_MAX_TRAJ_LEN + 1;  // distances 0..n + m
@@ -1244,8 +1243,7 @@ __global__ __launch_bounds__(256) void edr_length_table_kernel(const int32_t* __
 
 // ---------------------------------------------------------------- device jobs
 // The batch's job list built on the device from the filter's survivors, so a
-// top-k batch runs filter -> jobs -> DP -> survivor lists -> merge with no host
-// round trip.  One workgroup: per pair the shorter and longer length, the
+// top-k batch runs filter -> jobs -> DP -> merge with no host round trip.  One workgroup: per pair the shorter and longer length, the
 // length bucket (runBatched's rules: short up to `split`, long up to `mid`,
 // the rest one pair per wave, and in a batch of one round of waves the pairs
 // that would outlast the longest pair's several-wave schedule on one wave
@@ -1332,12 +1330,14 @@ struct JobRules {
 // keeps every SIMD busy whatever its pairs: long means longer than max(split,
 // 1024).  A smaller one (one round of waves) ends when its longest pair does:
 // its `critical` length is the longest pair's schedule over several waves (or
-// on one, when it may take no more), but not under twice the time all pairs
-// would take spread evenly in 16-lane segments.  A pair then takes the
-// cheapest form that ends in time: a 16-lane segment (a quarter of the
-// instructions, up to four times the length, and four waves share a SIMD) up
-// to half of critical and `split` columns, one wave up to all of it, several
-// beyond.
+// on one, when it may take no more), but not under half of what all pairs
+// would take spread evenly in 16-lane segments (a wave that shares its SIMD
+// waits out its steps' latency and issues about a quarter of the time: with
+// twice the spread work the longest pairs ran 1,040 us on one wave, the whole
+// DP 510 with half).  A pair then takes the cheapest form that ends in time: a
+// 16-lane segment (a quarter of the instructions, up to four times the length,
+// and four waves share a SIMD) up to half of critical and `split` columns, one
+// wave up to all of it, several beyond.
 struct JobShape {
   int mid;
   bool latency, multi;
