@@ -9,6 +9,7 @@
 #include <string>
 
 #include "gat_hip.h"
+#include "pair_region.hpp"
 
 namespace gat {
 
@@ -93,13 +94,12 @@ __device__ __forceinline__ int4 load_pair2(const int2* pairs, uint64_t at, uint6
   return v;
 }
 
-// The same without a branch: of an end below or at an even capacity, the pair
-// group at min(at, the last one's).  (Behind a branch each load was waited for
+// The same without a branch, for an end >= 1 that is below or at an even
+// capacity (whole_groups): the pair group at min(at, the last one's).  (Behind a branch each load was waited for
 // before the next was issued.)
 template <bool kWide>
 __device__ __forceinline__ int4 load_pair2_in(const int2* pairs, uint64_t at, uint64_t end) {
-  const uint64_t last = (end - 1) & ~uint64_t(1);
-  at = at < last ? at : last;
+  at = clamped_group(at, end);
   if constexpr (kWide) {
     return *reinterpret_cast<const int4*>(pairs + at);
   } else {

@@ -214,9 +214,8 @@ __global__ __launch_bounds__(kBlock) void pairs_digest_kernel(const int2* __rest
                                                              uint64_t capacity, unsigned long long* __restrict__ out) {
   __shared__ uint64_t part[kBlock / kWave];
   for (uint32_t q = blockIdx.x; q < nq; q += gridDim.x) {
-    const uint64_t b = qbase[q];
-    const uint64_t n = b < capacity ? (qcount[q] < capacity - b ? qcount[q] : capacity - b) : 0;
-    const uint64_t a = b & ~uint64_t(1), e = b + n;
+    const gat::PairRegion r = gat::pair_region(qbase[q], qcount[q], capacity);
+    const uint64_t a = r.first, b = r.begin, e = r.end;
     uint64_t acc = 0;
     if (a + uint64_t(blockIdx.y) * kDigestSpan >= e) continue;  // uniform: no pair of this split's
     auto sweep = [&](auto load) __attribute__((always_inline)) {
@@ -232,7 +231,7 @@ __global__ __launch_bounds__(kBlock) void pairs_digest_kernel(const int2* __rest
         }
       }
     };
-    if (e <= (capacity & ~uint64_t(1)))
+    if (gat::whole_groups(e, capacity))
       sweep([&](uint64_t at) { return gat::load_pair2_in<kWide>(pairs, at, e); });
     else  // the last pair of an odd number of them
       sweep([&](uint64_t at) { return gat::load_pair2<kWide>(pairs, at, e); });

@@ -1395,7 +1395,7 @@ __global__ __launch_bounds__(kDigBlock) void runs_digest_kernel(const int2* __re
       if (at >= run.first && at < end) sum += gat::pair_mix(make_int2(v.x, v.y));
       if (at + 1 < end) sum += gat::pair_mix(make_int2(v.z, v.w));
     };
-    if (end <= (npairs & ~uint64_t(1))) {
+    if (gat::whole_groups(end, npairs)) {
       for (uint64_t i = (run.first & ~uint64_t(1)) + 2 * l; i < end; i += 128) {
         int4 v[4];
 #pragma unroll

@@ -1,7 +1,8 @@
 """Digest kernels over per-query regions and over runs: odd starts and lengths
 around the 16-byte loads and a row's 128 pairs in flight, buffers that are only
 8-byte aligned, a region split over several workgroups, more queries than the
-LDS sums hold; against the same mix in numpy."""
+LDS sums hold, regions at, across and past the end of the pairs; against the
+same mix in numpy."""
 import ctypes as C
 
 import numpy as np
@@ -55,3 +56,27 @@ def test_digests(gpu, offset, nq):
     N.check_hip(N.hip().gat_runs_digest(ptr, total, drun.ptr, len(runs), nq, out.ptr, None))
     N.check_hip(N.hip().gat_device_sync())
     assert (out.get(np.uint64, nq) == want).all()
+
+
+@pytest.mark.parametrize("capacity", [0, 1, 2, 999, 1000])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_regions_past_the_pairs(gpu, capacity, offset):
+    """Regions as a batch leaves them that outgrew its pair buffer: every start
+    around the capacity, and far past it, inside a larger allocation."""
+    rng = np.random.default_rng(capacity)
+    room = 1 << 16
+    pairs = rng.integers(0, 2**31, (room, 2)).astype(np.int32)
+    dev = DevBuf.of(np.concatenate([np.zeros((offset, 2), np.int32), pairs]))
+    base = np.concatenate([np.arange(max(capacity - 40, 0), capacity + 41), np.arange(5000, 5003), [room - 1]])
+    base = np.repeat(base, 4).astype(np.uint64)
+    count = np.tile([0, 1, 33, 4096], len(base) // 4).astype(np.uint32)
+    m = _mix(pairs)
+    with np.errstate(over="ignore"):
+        want = np.array([m[b:min(b + c, capacity)].sum(dtype=np.uint64) if b < capacity else 0
+                         for b, c in zip(base.astype(int), count.astype(int))], np.uint64)
+    out = DevBuf.of(np.full(len(base), 7, np.uint64))
+    qbase, qcount = DevBuf.of(base), DevBuf.of(count)
+    N.check_hip(N.hip().gat_pairs_digest(C.c_void_p(dev.ptr.value + 8 * offset), qbase.ptr, qcount.ptr, len(base),
+                                         capacity, out.ptr, None))
+    N.check_hip(N.hip().gat_device_sync())
+    assert (out.get(np.uint64, len(base)) == want).all()

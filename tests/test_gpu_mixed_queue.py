@@ -2,7 +2,8 @@
 wait (another shape than the captured one, or too few groups to capture):
 answers against each index's own plain form, on a first run, on one whose
 workspaces earlier runs have sized, after small batches sized them for less, and
-with one index left out of a group; the same for the single index's batched form
+with one index left out of a group, in both result layouts (a queued or replayed
+group that outgrows its pair buffer has its digests queued behind it); the same for the single index's batched form
 without a graph, whose join follows its selection without a look between."""
 import numpy as np
 import pytest
@@ -35,9 +36,18 @@ def _expected(indexes, rects, route):
     return pick(0), pick(1)
 
 
+@pytest.fixture(params=[True, False], ids=["runs", "regions"])
+def layout(indexes, request):
+    for ix in indexes:
+        ix.set_result_layout(request.param)
+    yield request.param
+    for ix in indexes:
+        ix.set_result_layout(True)
+
+
 @pytest.mark.parametrize("graph", [True, False])
 @pytest.mark.parametrize("group", [300, 2000])  # several groups of two shapes, and one group
-def test_queued_groups(indexes, graph, group):
+def test_queued_groups(indexes, layout, graph, group):
     g, s, f = indexes
     rng = np.random.default_rng(group)
     m = api.MixedRange(g, s, f)
