@@ -1237,7 +1237,11 @@ __global__ __launch_bounds__(kRunsBlock, 8) void leaf_refine_runs_kernel(
         bj = boxes[q];
       }
     }
-    const uint64_t base = o.item_base[t];
+    // No further than the buffer's end: a batch that outgrew its entry list
+    // leaves items of earlier batches among its own, whose bounds may add up to
+    // anything, and positions counted from here must not wrap.
+    const uint64_t at0 = o.item_base[t];
+    const uint64_t base = at0 < capacity ? at0 : capacity;
     if (count <= uint32_t(kSpan)) {
       switch (slots_for(count)) {
         case 1:

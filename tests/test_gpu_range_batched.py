@@ -362,6 +362,30 @@ def test_run_indexed_abi_skips_malformed_items(gpu, nqueries):
                                   6, base.ptr, None) == 2
 
 
+@pytest.mark.parametrize("back", [0, 1, 2, 3, 16])
+def test_run_indexed_item_bases_do_not_wrap(gpu, back):
+    """Items whose region starts up to `back` pairs below 2^64, as the bounds of
+    items an outgrown batch did not write may sum to: nothing is stored, neither
+    before the pairs nor in them.  One chunk of points (staged writes) and
+    several (direct ones); the pairs lie inside a larger allocation."""
+    h = N.hip()
+    n = 400
+    xy = np.full((n, 2), 0.5, np.float32)
+    dxy, did = DevBuf.of(xy), DevBuf.of(np.arange(n, dtype=np.uint32) << 3)
+    store = N.PointStore(dxy.ptr, did.ptr, None, n, 3)
+    dboxes = DevBuf.of(np.array([[0, 0, 1, 1], [0, 0, 1, 1]], np.float32))
+    dq = DevBuf.of(np.array([0, 1, 0, 1], np.uint32))
+    ditems = DevBuf.of(np.array([[0, 100, 0, 2], [0, n, 2, 2]], np.uint32))
+    total = DevBuf.of(np.array([2], np.uint32))
+    base = DevBuf.of(np.full(2, (1 << 64) - back - 1, np.uint64) - np.uint64(back % 2 == 0))
+    room, lead, cap = 4096, 1024, 512
+    pairs = DevBuf.of(np.full((room, 2), 7, np.int32))
+    runs = DevBuf.of(np.zeros(4, api.RUN))
+    N.check_hip(h.gat_leaf_refine_runs(ctypes.byref(store), ditems.ptr, total.ptr, 2, dq.ptr, 4, dboxes.ptr, 2,
+                                       ctypes.c_void_p(pairs.ptr.value + 8 * lead), cap, runs.ptr, 4, base.ptr, None))
+    assert (pairs.get(np.int32, 2 * room) == 7).all()
+
+
 @pytest.mark.parametrize("n", [0, 1, 4095, 4096, 4097, 3 * 4096 + 5, 200_000])
 def test_scan_u64_over_tiles(gpu, n):
     """The exclusive scan the pipeline's regions and lists come from: tiles
