@@ -3,8 +3,8 @@ wait (another shape than the captured one, or too few groups to capture):
 answers against each index's own plain form, on a first run, on one whose
 workspaces earlier runs have sized, after small batches sized them for less, and
 with one index left out of a group, in both result layouts (a queued or replayed
-group that outgrows its pair buffer has its digests queued behind it); the same for the single index's batched form
-without a graph, whose join follows its selection without a look between."""
+group that outgrows its pair buffer has its digests queued behind it); and the
+single index's batched form without a graph over batches that grow and shrink."""
 import numpy as np
 import pytest
 
@@ -59,7 +59,7 @@ def test_queued_groups(indexes, layout, graph, group):
         assert st["pairs"] == int(c.astype(np.int64).sum())
 
 
-def test_batched_form_without_a_look_between(indexes):
+def test_batched_form_over_growing_batches(indexes):
     rng = np.random.default_rng(5)
     for ix in indexes:
         for lo, hi, n in ((1e-3, 2e-2, 400), (1e-3, 2e-2, 300), (1e-2, 5e-1, 700), (1e-3, 2e-2, 257)):
