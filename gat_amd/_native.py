@@ -171,6 +171,7 @@ HOST_FUNCS = {
     "gath_mixed_new": (P, [P, P, P]),
     "gath_mixed_free": (None, [P]),
     "gath_mixed_run": (INT, [P, P, INT, P, P, P, P, P]),
+    "gath_mixed_pipelines": (INT, [P, P]),
     "gath_grid_set_edr_params": (INT, [P, INT, INT, INT]),
     "gath_tune_range": (INT, [P, P, INT, INT, P]),
     "gath_tune_edr": (INT, [P, P, INT, P, P, F64, INT, P]),

@@ -680,6 +680,14 @@ class MixedRange:
         keys = ["pairs", "candidates", "groups", "replays", "ms", "digest_ms", "captures"]
         return counts[:n], digests[:n], route[:n], dict(zip(keys, st.tolist()))
 
+    def pipelines(self) -> dict:
+        """An index's part of a group, over all runs so far: pipelines queued,
+        parts run step by step, and queued or replayed ones that outgrew their
+        workspace and were run again."""
+        out = np.zeros(3, np.int64)
+        N.check_host(N.host().gath_mixed_pipelines(self.handle, _ptr(out)))
+        return dict(zip(["queued", "stepped", "discarded"], out.tolist()))
+
 
 class MortonGridIndex(GridIndex):
     """MortonGrid (MortonGrid.cpp): the GT-quadtree kept implicitly — leaf

@@ -117,29 +117,45 @@ int MixedRange::run(const MBB* bounds, int n, const MixedConfig& cfg, MixedResul
       boxes[i].clear();
       for (int k = 0; k < nq[i]; ++k) boxes[i].push_back(bounds[list[i][b + size_t(k)]]);
     }
-    bool done = false;
     const uint64_t* digests[3] = {nullptr, nullptr, nullptr};
     std::vector<std::pair<uint64_t, uint64_t>> digestSpans;  // device clock
-    // Both quick ways below leave counts and digests in pinned memory.
-    auto wait = [&](bool replay) -> int {
-      int rc = replay ? coord_.sync() : GAT_OK;
+    // Which indexes' answers are in: both quick ways below leave counts and
+    // digests in pinned memory.
+    bool done[3] = {nq[0] == 0, nq[1] == 0, nq[2] == 0};
+    auto waitAll = [&](int rc) -> int {
       for (int i = 0; i < 3; ++i)
-        if (nq[i] > 0 && !replay) {
+        if (nq[i] > 0) {
           const int r = gat_stream_sync(engine(i).stream());
           if (rc == GAT_OK) rc = r;
         }
-      bool fits = true;
-      for (int i = 0; i < 3 && rc == GAT_OK; ++i) {
-        if (nq[i] == 0) continue;
-        bool f = true;
-        uint64_t clock[2] = {0, 0};
-        rc = engine(i).finishResults(nq[i], batch_[i], replay, &f, &digests[i], clock);
-        if (f) digestSpans.emplace_back(clock[0], clock[1]);
-        fits = fits && f;
-      }
-      done = rc == GAT_OK && fits;
       return rc;
     };
+    // Once the work has been waited for: the answers of the indexes that ran.
+    auto collect = [&](bool replay, const bool ran[3]) -> int {
+      int rc = GAT_OK;
+      for (int i = 0; i < 3 && rc == GAT_OK; ++i) {
+        if (nq[i] == 0 || !ran[i]) continue;
+        uint64_t clock[2] = {0, 0};
+        rc = engine(i).finishResults(nq[i], batch_[i], replay, &done[i], &digests[i], clock);
+        if (done[i]) digestSpans.emplace_back(clock[0], clock[1]);
+        else ++pipelines.discarded;
+      }
+      return rc;
+    };
+    // Step by step: sizes the workspace, which may move its buffers, so the
+    // captured graph is dropped first.
+    bool stepped = false;
+    auto step = [&](int i) -> int {
+      if (graph_) gat_graph_destroy(graph_);
+      graph_ = nullptr;
+      std::fill(shape_, shape_ + 3, -1);
+      stepped = true;
+      ++pipelines.stepped;
+      return i == 0   ? fsg_.rangeQueryBatchedGPU(boxes[i].data(), nq[i], batch_[i], false)
+             : i == 1 ? grid_.rangeQueryBatchedGPU(boxes[i].data(), nq[i], batch_[i], false)
+                      : stig_.rangeQueryBatchedGPU(boxes[i].data(), nq[i], batch_[i], false);
+    };
+    bool byStep[3] = {false, false, false};
     const bool captured = cfg.graph && graph_ && std::equal(nq, nq + 3, shape_);
     if (captured) {
       // Replay: stage every index's rectangles, launch the one graph behind
@@ -155,56 +171,49 @@ int MixedRange::run(const MBB* bounds, int n, const MixedConfig& cfg, MixedResul
       // read freed memory, so this group runs step by step and is recaptured.
       const bool current = rc == GAT_OK && keysMatch(nq);
       if (current) rc = gat_graph_launch(graph_, coord_.get());
-      if (rc == GAT_OK && current) rc = wait(true);
-      else if (const int r = coord_.sync(); rc == GAT_OK) rc = r;
+      if (const int r = coord_.sync(); rc == GAT_OK) rc = r;
+      const bool all[3] = {true, true, true};
+      if (rc == GAT_OK && current) rc = collect(true, all);
       if (rc != GAT_OK) {
         restore();
         return gath_fail_hip(rc, "mixed replay");
       }
-      if (done) ++out->replays;
+      if (current && done[0] && done[1] && done[2]) ++out->replays;
     } else if (graph_ || !cfg.graph || gi + 2 >= groups) {
       // A group of another shape than the captured one, or one not to be captured:
-      // the three pipelines queued on their own streams with one wait, where
-      // earlier batches have sized the workspaces (step by step they took a
-      // wait per pipeline half and several per index's results, and ran one
-      // index after another).
+      // the pipelines of the indexes whose workspaces earlier batches have
+      // sized are queued on their own streams with one wait (step by step they
+      // took a wait per pipeline half and several per index's results, and ran
+      // one index after another).  An index whose workspace is too small runs
+      // step by step beside them, so nothing queued is thrown away for it.
       int rc = GAT_OK;
-      bool all = true;
+      bool queued[3] = {false, false, false};
       for (int i : kQueueOrder) {
-        if (rc != GAT_OK || !all || nq[i] == 0) continue;
-        rc = engine(i).reserveResults(nq[i], batch_[i]);
-        if (rc == GAT_OK) rc = engine(i).queueBatch(tree(i), boxes[i].data(), nq[i], batch_[i], &all);
+        if (rc != GAT_OK || nq[i] == 0) continue;
+        rc = engine(i).queueBatch(tree(i), boxes[i].data(), nq[i], batch_[i], &queued[i]);
+        if (queued[i]) ++pipelines.queued;
       }
-      if (rc == GAT_OK && all) {
-        rc = wait(false);
-      } else {
-        for (int i = 0; i < 3; ++i)
-          if (nq[i] > 0) {
-            const int r = gat_stream_sync(engine(i).stream());
-            if (rc == GAT_OK) rc = r;
-          }
-      }
+      for (int i = 0; i < 3 && rc == GAT_OK; ++i)
+        if (nq[i] > 0 && !queued[i]) {
+          rc = step(i);
+          byStep[i] = rc == GAT_OK;
+        }
+      rc = waitAll(rc);
+      if (rc == GAT_OK) rc = collect(false, queued);
       if (rc != GAT_OK) {
         restore();
         return gath_fail_hip(rc, "mixed batch");
       }
     }
-    if (!done) {
-      // Step by step (sizes every workspace, which may move its buffers, so
-      // the captured graph is dropped first), then capture this shape.
-      if (graph_) gat_graph_destroy(graph_);
-      graph_ = nullptr;
-      std::fill(shape_, shape_ + 3, -1);
-      int rc = GAT_OK;
-      if (rc == GAT_OK && nq[0] > 0) rc = fsg_.rangeQueryBatchedGPU(boxes[0].data(), nq[0], batch_[0], false);
-      if (rc == GAT_OK && nq[1] > 0) rc = grid_.rangeQueryBatchedGPU(boxes[1].data(), nq[1], batch_[1], false);
-      if (rc == GAT_OK && nq[2] > 0) rc = stig_.rangeQueryBatchedGPU(boxes[2].data(), nq[2], batch_[2], false);
-      // A shape met again (every group but the last) is worth a graph.
-      if (rc == GAT_OK && cfg.graph && gi + 2 < groups) rc = capture(nq);
-      if (rc != GAT_OK) {
-        restore();
-        return rc;
-      }
+    // What the quick ways did not take, or what outgrew its workspace there.
+    int rc_step = GAT_OK;
+    for (int i = 0; i < 3 && rc_step == GAT_OK; ++i)
+      if (!done[i] && !byStep[i]) rc_step = step(i);
+    // A group that sized its workspaces and is not among the last two is captured.
+    if (rc_step == GAT_OK && stepped && cfg.graph && gi + 2 < groups) rc_step = capture(nq);
+    if (rc_step != GAT_OK) {
+      restore();
+      return rc_step;
     }
     const double d0 = now_ms();
     for (int i = 0; i < 3; ++i) {
@@ -212,7 +221,7 @@ int MixedRange::run(const MBB* bounds, int n, const MixedConfig& cfg, MixedResul
       RangeBatch& b = batch_[i];
       int rc = b.syncHost();
       const uint64_t* d = digests[i];
-      if (rc == GAT_OK && !done) {
+      if (rc == GAT_OK && !done[i]) {
         dig.resize(size_t(nq[i]));
         rc = b.digests(dig.data());
         d = dig.data();
@@ -231,8 +240,8 @@ int MixedRange::run(const MBB* bounds, int n, const MixedConfig& cfg, MixedResul
       out->candidates += b.candidates;
     }
     out->digestMs += now_ms() - d0;
-    if (done) {
-      // The time in which digests ran, beside each other or not.
+    if (!digestSpans.empty()) {
+      // The time in which the quick ways' digests ran, beside each other or not.
       if (clockKhz_ == 0) {
         const int rc = gat_wall_clock_khz(&clockKhz_);
         if (rc != GAT_OK) {

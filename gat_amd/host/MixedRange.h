@@ -70,4 +70,10 @@ class MixedRange {
   int32_t clockKhz_ = 0;
  public:
   int captures = 0;  // graphs captured over this object's life
+  // An index's part of a group, over this object's life: pipelines queued,
+  // parts run step by step, and queued or replayed ones whose batch outgrew its
+  // workspace (run again step by step).
+  struct Pipelines {
+    int64_t queued = 0, stepped = 0, discarded = 0;
+  } pipelines;
 };

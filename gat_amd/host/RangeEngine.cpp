@@ -1049,19 +1049,6 @@ int RangeEngine::enqueueBatch(const DeviceTree& tree, int nq, RangeBatch& out) {
   return enqueueJoin(tree, nq, out);
 }
 
-int RangeEngine::finishBatch(int nq, RangeBatch& out, bool* fits) {
-  out.queryNum = nq;
-  out.count.assign(size_t(nq), 0);
-  out.base.assign(size_t(nq), 0);
-  out.stream = stream_.get();
-  out.taskNum = 0;
-  out.selectMs = out.uploadMs = 0;
-  out.kernelMs = out.refineMs = 0;
-  if (int rc = readCounters(nq, out)) return rc;
-  *fits = countersFit();
-  return *fits ? finishCounters(out, true) : GAT_OK;
-}
-
 // Whether the workspace and `out` hold everything the leaf-major pipeline of nq
 // rectangles touches at the capacities at hand.
 bool RangeEngine::sizedFor(const DeviceTree& tree, int nq, const RangeBatch& out) const {
@@ -1075,15 +1062,24 @@ bool RangeEngine::sizedFor(const DeviceTree& tree, int nq, const RangeBatch& out
          holds(itemBase_, itemsCap_, 8) && holds(itemTiles_, gat_scan_tiles(itemsCap_), 8);
 }
 
+// Pinned room for a batch's results, rounded up to a power of two of queries:
+// an allocation takes 0.1 ms and more, and batches grow by a few rectangles.
+static size_t result_bytes(int nq) {
+  int64_t n = 256;
+  while (n < nq) n *= 2;
+  return size_t(gat_direct_words(n)) * 4;
+}
+
 int RangeEngine::reserveResults(int nq, RangeBatch& out) {
   if (int rc = countersHost_.reserve(256)) return rc;
   if (int rc = out.digestDev_.reserve(size_t(std::max(nq, 1)) * 8)) return rc;
-  return resultHost_.reserve(size_t(gat_direct_words(std::max(nq, 1))) * 4);
+  return resultHost_.reserve(result_bytes(nq));
 }
 
 int RangeEngine::queueBatch(const DeviceTree& tree, const MBB* bounds, int nq, RangeBatch& out, bool* queued) {
   *queued = false;
   if (nq < 1 || !sizedFor(tree, nq, out)) return GAT_OK;
+  if (int rc = reserveResults(nq, out)) return rc;
   size_t bytes = 0;
   if (int rc = stageBoxes(&tree, bounds, nq, &bytes)) return rc;
   uint32_t* const spans[4] = {nodeCount_.as<uint32_t>(), out.qcount.as<uint32_t>(), counters_.as<uint32_t>(),

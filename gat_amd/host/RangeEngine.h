@@ -204,23 +204,23 @@ class RangeEngine {
   int uniqueCandidates(const DeviceTree& tree, int64_t* points);
   ~RangeEngine();
 
-  // Pieces of the batched form for a coordinator that captures several
-  // engines into one graph.  After a runTree of the same batch size has sized
-  // the workspace: stageBatch uploads the rectangles, enqueueBatch queues the
-  // whole device pipeline on this engine's stream (no host sync, capturable),
-  // finishBatch reads the counters back and reports in *fits whether the batch
-  // stayed inside the workspace (if not, rerun it with runTree).
+  // Pieces of the batched form, counts and digests included, for a coordinator
+  // of several engines, after a runTree of the same batch size has sized the
+  // workspace.  Nothing here waits for the device.
+  //
+  // queueBatch: the whole batch on this engine's stream, upload first, when the
+  // workspace holds it (*queued, else nothing is queued).
+  // To be captured: reserveResults, then enqueueBatch (the device pipeline) and
+  // enqueueResults (digests, and everything the host reads to pinned memory);
+  // before each launch of the graph stageBatch uploads the rectangles.
+  // Once the work has been waited for, finishResults: *fits tells whether the
+  // batch stayed inside the workspace (if not, rerun it with runTree), *digests
+  // points at the digests (pinned, valid until the next batch), digestClock
+  // gets the device clock at their start and end.
+  int queueBatch(const DeviceTree& tree, const MBB* bounds, int nq, RangeBatch& out, bool* queued);
+  int reserveResults(int nq, RangeBatch& out);
   int stageBatch(const DeviceTree& tree, const MBB* bounds, int nq);
   int enqueueBatch(const DeviceTree& tree, int nq, RangeBatch& out);
-  int finishBatch(int nq, RangeBatch& out, bool* fits);
-  // The whole batch, counts and digests included, queued without a wait, when
-  // earlier batches have sized the workspace for it (*queued, else nothing is):
-  // reserveResults before, then either queueBatch (upload and pipeline) or, to
-  // be captured, enqueueBatch and enqueueResults; once the stream has been waited for
-  // finishResults, as finishBatch, with the digests in *digests (pinned, valid
-  // until the next batch) and the device clock at their start and end.
-  int reserveResults(int nq, RangeBatch& out);
-  int queueBatch(const DeviceTree& tree, const MBB* bounds, int nq, RangeBatch& out, bool* queued);
   int enqueueResults(int nq, RangeBatch& out);
   int finishResults(int nq, RangeBatch& out, bool replay, bool* fits, const uint64_t** digests,
                     uint64_t digestClock[2]);

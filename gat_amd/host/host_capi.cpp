@@ -718,6 +718,15 @@ int gath_mixed_run(void* m, const float* boxes, int nq, const double* cfg, uint3
   return GAT_OK;
 }
 
+int gath_mixed_pipelines(void* m, int64_t* out) {
+  auto* mr = static_cast<MixedRange*>(m);
+  if (!mr || !out) return bad("gath_mixed_pipelines: bad arguments");
+  out[0] = mr->pipelines.queued;
+  out[1] = mr->pipelines.stepped;
+  out[2] = mr->pipelines.discarded;
+  return GAT_OK;
+}
+
 int gath_serve(void* p, const gath_request* reqs, int n, const float* qlon, const float* qlat, int64_t nqpoints,
                const double* cfg, gath_outcome* out, int32_t* topk_ids, int32_t* topk_dists, double* stats) {
   Index* ix = as_index(p);

@@ -231,6 +231,11 @@ void* gath_mixed_new(void* grid, void* stig, void* fsg);
 void gath_mixed_free(void* mixed);
 int gath_mixed_run(void* mixed, const float* boxes, int nq, const double* cfg, uint32_t* counts, uint64_t* digests,
                    int8_t* route, double* stats);
+/* out[0..2] = what this object's runs did with an index's part of a group so
+ * far: pipelines queued on the index's stream, parts run step by step, and
+ * queued or replayed pipelines whose batch outgrew its workspace (their parts
+ * are among the second too). */
+int gath_mixed_pipelines(void* mixed, int64_t* out);
 
 /* ---------------------------------------------------------------- serving
  * The serving loop over a Grid (no reference counterpart): requests arrive at

@@ -59,6 +59,36 @@ def test_queued_groups(indexes, layout, graph, group):
         assert st["pairs"] == int(c.astype(np.int64).sum())
 
 
+@pytest.mark.parametrize("kind", [0, 1, 2])  # FSG, the GT-quadtree, STIG
+def test_a_small_workspace_discards_no_other(gpu, layout, kind):
+    """One index's part of a group has one rectangle more than its workspace was
+    sized for: that index runs step by step and the others' queued pipelines
+    are used.  A part that outgrows a capacity is the only one run again."""
+    db = api.synth_walks(9, api.synth_lengths(9, 2500, "uniform", 1, 90, 1, 90), step_sigma=4e-3)
+    ix = (api.GridIndex(W.UNIT_BOX, 0.01, 64).build(db), api.StigIndex(64).build(db),
+          api.FsgIndex(W.UNIT_BOX, 0.01).build(db))
+    for i in ix:
+        i.set_result_layout(layout)
+    m = api.MixedRange(*ix)
+    rng = np.random.default_rng(kind)
+    sides = [(1e-4, 9e-4), (2e-3, 2e-2), (4e-2, 6e-2)]  # an index each
+
+    def run(counts, lo_hi):
+        rects = np.concatenate([_rects(rng, n, *s) for n, s in zip(counts, lo_hi)])
+        c, d, route, _ = m.run(rects, 1e-6, 1e-3)
+        assert (np.bincount(route, minlength=3) == counts).all()
+        want_c, want_d = _expected(ix, rects, route)
+        assert (c == want_c).all() and (d == want_d).all()
+        return np.array(list(m.pipelines().values()))
+
+    counts = np.array([300, 300, 300])
+    assert run(counts, sides).tolist() == [0, 3, 0]
+    counts[kind] += 1
+    assert run(counts, sides).tolist() == [2, 4, 0]
+    sides[2] = (0.4, 0.6)  # STIG's rectangles outgrow its lists
+    assert run(counts, sides).tolist() == [5, 5, 1]
+
+
 def test_batched_form_over_growing_batches(indexes):
     rng = np.random.default_rng(5)
     for ix in indexes:
