@@ -645,7 +645,9 @@ def serve(grid: "GridIndex", requests: np.ndarray, qlon: np.ndarray, qlat: np.nd
                                      out.ctypes.data, _ptr(ids), _ptr(dists), _ptr(st)))
     keys = ["range_batches", "topk_batches", "range_done", "topk_done", "wall_ms", "peak_range_bytes",
             "peak_topk_bytes", "range_budget", "topk_budget", "peak_topk_survivors", "device_allocs"]
-    return out[:n], ids[:n], dists[:n], dict(zip(keys, st.tolist()))
+    pinned = np.zeros(1, np.int64)
+    N.check_host(N.host().gath_serve_pinned_allocs(grid.handle, _ptr(pinned)))
+    return out[:n], ids[:n], dists[:n], dict(zip(keys, st.tolist()), pinned_allocs=int(pinned[0]))
 
 
 class MixedRange:

@@ -19,6 +19,8 @@ int gath_fail_hip(int rc, const char* what);
 // Device allocations DeviceBuffer::reserve has made in this process (each
 // growth is one); the serving loop reports how many happened while it served.
 int64_t gath_device_alloc_count();
+// The same of PinnedBuffer::reserve.
+int64_t gath_pinned_alloc_count();
 
 #define GATH_TRY(expr, what)                       \
   do {                                             \

@@ -563,6 +563,14 @@ int DeviceTree::uploadImplicit(const std::vector<gat_tree_node>& leaves, const s
 
 RangeEngine::~RangeEngine() { dropGraph(); }
 
+// Pinned room for a batch's results, rounded up to a power of two of queries:
+// an allocation takes 0.1 ms and more, and batches grow by a few rectangles.
+static size_t result_bytes(int nq) {
+  int64_t n = 256;
+  while (n < nq) n *= 2;
+  return size_t(gat_direct_words(n)) * 4;
+}
+
 int RangeEngine::attachStore(const RangeEngine& src) {
   if (int rc = stream_.create()) return rc;
   store_ = src.store_;
@@ -585,6 +593,7 @@ int RangeEngine::reserveBatched(const DeviceTree& tree, int maxQueries, int64_t 
   if (int rc = out.qcount.reserve(size_t(nq) * 4)) return rc;
   if (int rc = counters_.reserve(256)) return rc;
   if (int rc = countersHost_.reserve(256)) return rc;
+  if (int rc = directHost_.reserve(result_bytes(int(nq)))) return rc;
   // Leaves average well over 16 points, so candidates / 16 entries is ample.
   const int64_t entries = std::max<int64_t>(maxCandidates / 16 + nq * 64, 1 << 16);
   lqCap_ = std::max(lqCap_, entries);
@@ -611,7 +620,7 @@ int RangeEngine::runDirect(const DeviceTree& tree, const MBB* bounds, int nq, Ra
   if (clockKhz_ == 0) GATH_TRY(gat_wall_clock_khz(&clockKhz_), "device clock");
   size_t bytes = 0;
   if (int rc = stageBoxes(&tree, bounds, nq, &bytes)) return rc;
-  if (int rc = directHost_.reserve(size_t(gat_direct_words(nq)) * 4)) return rc;
+  if (int rc = directHost_.reserve(result_bytes(nq))) return rc;
   uint32_t* ctr = counters_.as<uint32_t>();
   const uint32_t* ch = directHost_.as<uint32_t>();
   auto u64 = [&](int w) { return uint64_t(ch[w]) | (uint64_t(ch[w + 1]) << 32); };
@@ -1060,14 +1069,6 @@ bool RangeEngine::sizedFor(const DeviceTree& tree, int nq, const RangeBatch& out
          holds(lqRank_, lqCap_, 4) && holds(qlist_, qlistCap_, 4) && holds(items_, itemsCap_, 16) &&
          holds(out.pairs, pairsCap_, 8) && holds(out.runs, qlistCap_, sizeof(gat_range_run)) &&
          holds(itemBase_, itemsCap_, 8) && holds(itemTiles_, gat_scan_tiles(itemsCap_), 8);
-}
-
-// Pinned room for a batch's results, rounded up to a power of two of queries:
-// an allocation takes 0.1 ms and more, and batches grow by a few rectangles.
-static size_t result_bytes(int nq) {
-  int64_t n = 256;
-  while (n < nq) n *= 2;
-  return size_t(gat_direct_words(n)) * 4;
 }
 
 int RangeEngine::reserveResults(int nq, RangeBatch& out) {

@@ -254,7 +254,7 @@ class RangeEngine {
   int attachStore(const RangeEngine& src);
   // Sizes the batched-form workspace for batches of up to maxQueries
   // rectangles and maxCandidates candidate points, so later batches within
-  // those bounds allocate nothing.
+  // those bounds allocate nothing, on the device or of pinned host memory.
   int reserveBatched(const DeviceTree& tree, int maxQueries, int64_t maxCandidates, RangeBatch& out);
 
   // Candidate selection only (host), exposed for tests of the host logic.

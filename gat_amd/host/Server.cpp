@@ -165,8 +165,9 @@ int Server::run(const gath_request* reqs, int n, const float* qlon, const float*
   }
 
   // Range slots: engines over the grid's resident store, each with its own
-  // stream and a workspace sized up front for its budget, so serving does no
-  // device allocation (a free would synchronise the whole device).
+  // stream and a workspace sized up front for its budget, so serving allocates
+  // neither device nor pinned memory (a free would synchronise the whole
+  // device).
   struct RangeSlot {
     RangeEngine engine;
     RangeBatch batch;
@@ -300,7 +301,7 @@ int Server::run(const gath_request* reqs, int n, const float* qlon, const float*
     survivorsPerQuery = double(es.pairs) / double(std::max<size_t>(first.size(), 1));
   }
   std::vector<std::thread> workers;
-  const int64_t allocs0 = gath_device_alloc_count();
+  const int64_t allocs0 = gath_device_alloc_count(), pinned0 = gath_pinned_alloc_count();
   t0 = Clock::now();
   for (auto& s : slots) workers.emplace_back(range_worker, s.get());
   if (anyTopk) workers.emplace_back(topk_worker);
@@ -327,6 +328,7 @@ int Server::run(const gath_request* reqs, int n, const float* qlon, const float*
   for (auto& w : workers) w.join();
   st.wallMs = ms_since(t0);
   st.deviceAllocs = gath_device_alloc_count() - allocs0;
+  st.pinnedAllocs = gath_pinned_alloc_count() - pinned0;
   if (sh.failed) {
     gath_set_error("%s", sh.error.c_str());
     return sh.rc;

@@ -43,6 +43,7 @@ struct ServeStats {
   double rangeBudgetBytes = 0, topkBudgetBytes = 0;  // budgets after the free-memory check
   int64_t peakTopkSurvivors = 0;  // most filter survivors of one top-k batch
   int64_t deviceAllocs = 0;       // device allocations while serving (buffers that grew)
+  int64_t pinnedAllocs = 0;       // and of pinned host memory
 };
 
 class Server {

@@ -23,6 +23,7 @@ struct Index {
   std::unique_ptr<FSG> fsg;
   std::unique_ptr<STIG> stig;
   RangeBatch last;
+  int64_t servePinnedAllocs = 0;  // of the last gath_serve
   int trajNum() const { return kind == kGrid ? grid->trajNum : kind == kFsg ? fsg->trajNum : stig->maxTid; }
 };
 
@@ -743,6 +744,7 @@ int gath_serve(void* p, const gath_request* reqs, int n, const float* qlon, cons
   ServeStats st;
   Server server(*ix->grid, c);
   if (int rc = server.run(reqs, n, qlon, qlat, nqpoints, out, topk_ids, topk_dists, &st)) return rc;
+  ix->servePinnedAllocs = st.pinnedAllocs;
   if (stats) {
     const double v[11] = {double(st.rangeBatches), double(st.topkBatches), double(st.rangeDone),
                           double(st.topkDone),     st.wallMs,           st.peakRangeBytes,
@@ -750,6 +752,13 @@ int gath_serve(void* p, const gath_request* reqs, int n, const float* qlon, cons
                           double(st.peakTopkSurvivors), double(st.deviceAllocs)};
     for (int i = 0; i < 11; ++i) stats[i] = v[i];
   }
+  return GAT_OK;
+}
+
+int gath_serve_pinned_allocs(void* p, int64_t* out) {
+  Index* ix = as_index(p);
+  if (!ix || !ix->grid || !out) return bad("gath_serve_pinned_allocs: bad arguments");
+  *out = ix->servePinnedAllocs;
   return GAT_OK;
 }
 

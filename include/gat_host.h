@@ -271,6 +271,9 @@ typedef struct gath_outcome {
  * serving (buffers that had to grow). */
 int gath_serve(void* grid, const gath_request* reqs, int n, const float* qlon, const float* qlat, int64_t nqpoints,
                const double* cfg, gath_outcome* out, int32_t* topk_ids, int32_t* topk_dists, double* stats);
+/* *out = the pinned host allocations made while the grid's last gath_serve
+ * was serving. */
+int gath_serve_pinned_allocs(void* grid, int64_t* out);
 
 #pragma GCC visibility pop
 

@@ -53,13 +53,14 @@ def test_range_admission_never_grows_buffers(served):
     """Range requests are charged an exact bound of their result and list
     buffers (from the leaves they select), so a range-only stream whose
     requests fit the budget is served with the workspaces reserved up front:
-    no device allocation while serving.  A request above the budget on its own
+    no device allocation and none of pinned host memory while serving, as batches
+    of every size come by.  A request above the budget on its own
     is still admitted, alone, and its buffers grow."""
     db, g, req, qlon, qlat, out, ids, dists, st = served
     rng = req[req["kind"] == api.REQ_RANGE].copy()
     want = out["count"][req["kind"] == api.REQ_RANGE]
     r_out, _, _, r_st = api.serve(g, rng, qlon, qlat, K, EPS, range_budget=4e9)
-    assert r_st["device_allocs"] == 0
+    assert r_st["device_allocs"] == 0 and r_st["pinned_allocs"] == 0
     assert r_st["range_done"] == len(rng) and (r_out["count"] == want).all()
     assert 0 < r_st["peak_range_bytes"] <= 4e9
     t_out, _, _, t_st = api.serve(g, rng, qlon, qlat, K, EPS, range_budget=1.0)
