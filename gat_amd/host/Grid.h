@@ -126,6 +126,10 @@ class Grid {
   int edrBatchedAll(const TrajectoryView& queries, std::vector<int32_t>& dist, EdrBatchStats* stats);
   int similarityBatched(const TrajectoryView& queries, int kValue, std::vector<TopK>& out, EdrBatchStats* stats);
   int similarityBatched(const TrajectoryView& queries, int kValue, TopKSink out, EdrBatchStats* stats);
+  // Runs a batch once through the job-list chain, answers discarded, where
+  // similarityBatched may take the short chain for it: a later batch as large
+  // then finds the buffers and streams of either.
+  int warmTopk(const TrajectoryView& queries, int kValue);
   // The all-mismatch table F[r][c], (GAT_MAX_TRAJ_LEN + 1)^2 entries, computed
   // on the device once.
   const std::vector<int32_t>& mismatchTable();

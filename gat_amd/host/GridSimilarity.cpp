@@ -1106,6 +1106,19 @@ int Grid::similarityBatched(const TrajectoryView& queries, int kValue, TopKSink 
   return GAT_OK;
 }
 
+int Grid::warmTopk(const TrajectoryView& queries, int kValue) {
+  const int nq = queries.trajNum;
+  if (!deviceChain || kValue < 1 || kValue > kDeviceTopkMax || nq < 1 || nq > kSmallTopkQueries) return GAT_OK;
+  if (int rc = checkTrajLengths("similarityBatched")) return rc;
+  if (int rc = ensureQueryStore(queries, kCtlWords)) return rc;
+  if (int rc = ensureDeviceTables()) return rc;
+  std::vector<TopK> rows;
+  TopKSink sink;
+  sink.vec = &rows;
+  bool done = false;
+  return similarityOnDevice(nq, kValue, sink, nullptr, &done);
+}
+
 int Grid::similarityHost(int nq, int kValue, std::vector<TopK>& out, EdrBatchStats* st) {
   void* s = engine_.stream();
   // Candidate filter on the device; grow the survivor buffer until it fits.

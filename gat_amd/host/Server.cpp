@@ -289,7 +289,8 @@ int Server::run(const gath_request* reqs, int n, const float* qlon, const float*
 
   if (anyTopk) {
     // Size the top-k buffers before the clock starts with one batch of the
-    // run's own queries (its answers are discarded).
+    // run's own queries (its answers are discarded), by either chain a later
+    // batch may take.
     std::vector<int> first;
     for (int i = 0; i < n && int(first.size()) < cfg_.maxTopkBatch; ++i)
       if (reqs[i].kind == GATH_REQ_TOPK) first.push_back(i);
@@ -297,6 +298,7 @@ int Server::run(const gath_request* reqs, int n, const float* qlon, const float*
     std::vector<TopK> res;
     gather_queries(first, qdb);
     EdrBatchStats es;
+    if (int rc = grid_.warmTopk(TrajectoryView::of(qdb), cfg_.k)) return rc;
     if (int rc = grid_.similarityBatched(TrajectoryView::of(qdb), cfg_.k, res, &es)) return rc;
     survivorsPerQuery = double(es.pairs) / double(std::max<size_t>(first.size(), 1));
   }

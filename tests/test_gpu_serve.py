@@ -67,6 +67,31 @@ def test_range_admission_never_grows_buffers(served):
     assert t_st["range_batches"] == len(rng) and (t_out["count"] == want).all()
 
 
+def test_topk_chains_are_sized_before_serving(gpu):
+    """Top-k batches of up to 32 queries take the short chain while few survivors
+    are expected and the job-list chain when more are: a run whose first batch
+    has none and whose later ones have 60 a query changes over while it
+    serves, and finds the second chain's buffers there."""
+    rng = np.random.default_rng(3)
+    n, m = 560, 20
+    at = rng.random((n, 2)) * 0.5
+    at[:60] = 0.2  # a crowd
+    walk = (at[:, None, :] + rng.normal(0, 2e-5, (n, m, 2))).astype(np.float32)
+    db = api.TrajSet(np.arange(n + 1, dtype=np.int64) * m, walk[:, :, 0].ravel().copy(), walk[:, :, 1].ravel().copy())
+    g = api.GridIndex(W.UNIT_BOX, 0.01, 64).build(db)
+    nq = 160
+    q = np.where(np.arange(nq)[:, None, None] < 32, 0.9, 0.2) + rng.normal(0, 2e-5, (nq, m, 2))
+    req = np.zeros(nq, api.REQUEST)
+    req["kind"], req["qlen"], req["qoff"] = api.REQ_TOPK, m, np.arange(nq) * m
+    lon, lat = q[:, :, 0].astype(np.float32).ravel(), q[:, :, 1].astype(np.float32).ravel()
+    out, ids, dists, st = api.serve(g, req, lon, lat, K, EPS, max_topk_batch=32)
+    assert st["topk_batches"] == 5 and st["peak_topk_survivors"] == 32 * 60
+    assert st["device_allocs"] == 0 and st["pinned_allocs"] == 0
+    qs = api.TrajSet(np.arange(nq + 1, dtype=np.int64) * m, lon, lat)
+    want_i, want_d, _ = g.set_topk_device_chain(False).similarity_batched(qs, K, EPS)
+    assert (ids == want_i).all() and (dists == want_d).all()
+
+
 def test_topk_in_the_mix_matches_oracle(served):
     db, g, req, qlon, qlat, out, ids, dists, st = served
     tid = np.arange(1, db.ntraj + 1, dtype=np.int32)
