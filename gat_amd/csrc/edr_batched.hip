@@ -1151,7 +1151,9 @@ constexpr int kMergeMax = 1024;  // survivors of a query gathered in LDS
 // separate launches built lists, sorted them and merged.  Reading every pair
 // in every workgroup suits batches of few pairs.  The results may go to pinned
 // host memory; the last workgroup to end writes the control words and the time
-// after them.
+// after them.  The start's time goes elsewhere (stamp): the last workgroup, on
+// another XCD as a rule, is ordered behind the atomics whose results its ticket
+// depends on, not behind the first one's plain stores.
 __global__ __launch_bounds__(kTopkBlock) void edr_merge_kernel(
     const int32_t* __restrict__ ftable, int32_t w, const int32_t* __restrict__ qlen, int32_t nq,
     const int32_t* __restrict__ clen, int32_t nc, const int32_t* __restrict__ len_ids,

@@ -843,11 +843,13 @@ int Grid::runBatchedOnDevice(const int32_t* pairsHost, int64_t np, int queryNum,
 // A batch's control words (topCtl_, cleared by the upload; the merge or a copy
 // brings them back): [0, 1] survivors, [2] lists and [3] merge status (as
 // gat_edr_merge's), [4, 5] cells, [6] the job counter of gat_edr_pairs, [7]
-// ticket, [8] job list status, [10, 16) the clock at the filter, the DP and the
-// merge, [16, 24) the buckets' windows, [24, 28) their job counters; after them
-// the clock at the upload (device) or at the end (host).
+// ticket, [8] job list status, [10, 14) the clock at the filter and the DP,
+// [16, 24) the buckets' windows, [24, 28) their job counters; after them the
+// clock at the upload (device), or at the merge's end and its start (host: the
+// merge writes both there itself, since its workgroup that brings the words
+// back is not ordered behind the one that starts first).
 namespace {
-constexpr int kCtlWords = 32;
+constexpr int kCtlWords = 32, kHostWords = kCtlWords + 4;
 uint64_t ctl64(const uint32_t* c, int w) { return uint64_t(c[w]) | (uint64_t(c[w + 1]) << 32); }
 }  // namespace
 
@@ -884,7 +886,7 @@ int Grid::similarityOnDevice(int nq, int kValue, TopKSink& out, EdrBatchStats* s
     if (int rc = nmDev_.reserve((size_t(cap) * 2 + GAT_EDR_JOBS_SCRATCH_EXTRA) * 4)) return rc;
     if (int rc = jobsDev_.reserve((size_t(cap) + 4) * sizeof(gat_edr_job))) return rc;
     if (int rc = outDev_.reserve(size_t(cap) * 4)) return rc;
-    if (int rc = topHost_.reserve((2 * cells + kCtlWords + 2) * 4)) return rc;
+    if (int rc = topHost_.reserve((2 * cells + kHostWords) * 4)) return rc;
     uint32_t* ctl = topCtl_.as<uint32_t>();
     auto* count = reinterpret_cast<uint64_t*>(ctl);
     int32_t* win = reinterpret_cast<int32_t*>(ctl + 16);
@@ -908,7 +910,7 @@ int Grid::similarityOnDevice(int nq, int kValue, TopKSink& out, EdrBatchStats* s
       GATH_TRY(gat_edr_merge(lenTableDev_.as<int32_t>(), GAT_MAX_TRAJ_LEN + 1, queryLenDev_, nq,
                              trajLen_.as<int32_t>(), trajNum, lenIdsDev_.as<int32_t>(), lenOffDev_.as<int32_t>(),
                              sortedDev_.as<int32_t>(), outDev_.as<int32_t>(), cap, kValue, kk, top, top + cells, ctl,
-                             c, ctl + 14, s),
+                             c, c + kCtlWords + 2, s),
                "top-k merge");
     } else {
       if (int rc = survDev_.reserve((ns + 2 * size_t(cap)) * 4)) return rc;
@@ -960,8 +962,8 @@ int Grid::similarityOnDevice(int nq, int kValue, TopKSink& out, EdrBatchStats* s
       st->pruned += int64_t(nq) * trajNum - int64_t(found);
       if (trajNum > 0) st->filterMs += double(ctl64(c, 12) - ctl64(c, 10)) / clockKhz_;
       if (merge) {
-        st->kernelMs += double(ctl64(c, 14) - ctl64(c, 12)) / clockKhz_;
-        st->mergeMs += double(ctl64(c, kCtlWords) - ctl64(c, 14)) / clockKhz_;
+        st->kernelMs += double(ctl64(c, kCtlWords + 2) - ctl64(c, 12)) / clockKhz_;
+        st->mergeMs += double(ctl64(c, kCtlWords) - ctl64(c, kCtlWords + 2)) / clockKhz_;
       } else {
         float ms = 0;
         if (int rc = mergeTimer_.elapsed(&ms)) return rc;
@@ -993,7 +995,7 @@ int Grid::similaritySmall(const TrajectoryView& queries, int kValue, TopKSink& o
   const size_t cells = size_t(nq) * size_t(kValue);
   if (int rc = pairsDev_.reserve(size_t(cap) * 8)) return rc;
   if (int rc = outDev_.reserve(size_t(cap) * 4)) return rc;
-  if (int rc = topHost_.reserve((2 * cells + kCtlWords + 2) * 4)) return rc;
+  if (int rc = topHost_.reserve((2 * cells + kHostWords) * 4)) return rc;
   uint32_t* ctl = topCtl_.as<uint32_t>();
   auto* count = reinterpret_cast<uint64_t*>(ctl);
   int longest = maxTrajLen_;
@@ -1011,7 +1013,8 @@ int Grid::similaritySmall(const TrajectoryView& queries, int kValue, TopKSink& o
   GATH_TRY(gat_edr_merge(lenTableDev_.as<int32_t>(), GAT_MAX_TRAJ_LEN + 1, queryLenDev_, nq, trajLen_.as<int32_t>(),
                          trajNum, lenIdsDev_.as<int32_t>(), lenOffDev_.as<int32_t>(), pairsDev_.as<int32_t>(),
                          outDev_.as<int32_t>(), cap, kValue, kk, top, top + cells, ctl,
-                         reinterpret_cast<uint32_t*>(top + 2 * cells), ctl + 14, s),
+                         reinterpret_cast<uint32_t*>(top + 2 * cells),
+                         reinterpret_cast<uint32_t*>(top + 2 * cells) + kCtlWords + 2, s),
            "top-k merge");
   GATH_TRY(gat_stream_sync(s), "top-k readback");
   queryPending_ = false;
@@ -1030,8 +1033,8 @@ int Grid::similaritySmall(const TrajectoryView& queries, int kValue, TopKSink& o
     st->jobs += int64_t(found);
     st->pruned += int64_t(nq) * trajNum - int64_t(found);
     st->filterMs += double(ctl64(c, 12) - ctl64(c, 10)) / clockKhz_;
-    st->kernelMs += double(ctl64(c, 14) - ctl64(c, 12)) / clockKhz_;
-    st->mergeMs += double(ctl64(c, kCtlWords) - ctl64(c, 14)) / clockKhz_;
+    st->kernelMs += double(ctl64(c, kCtlWords + 2) - ctl64(c, 12)) / clockKhz_;
+    st->mergeMs += double(ctl64(c, kCtlWords) - ctl64(c, kCtlWords + 2)) / clockKhz_;
   }
   *done = true;
   return GAT_OK;

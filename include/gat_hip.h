@@ -407,8 +407,11 @@ int gat_edr_filter_grid_add(const float* qbox_dev, int32_t nq, const float* cbox
  * length table; the results may be pinned host memory.  ctl_dev (32 words):
  * [0, 1] the number of pairs, [2] gets 2 when a query has over 1,024 of them
  * (its results are left out), [3] as gat_edr_topk's status, [7] zero before the
- * call; ctl_out receives the words and the wall clock after them.  Nothing is
- * merged when the pairs exceed `capacity`. */
+ * call; ctl_out receives the words and the wall clock after them, written by the
+ * workgroup that ends last.  The wall clock at the start goes to stamp (null:
+ * not), device or pinned memory; among ctl_dev's words it may come back stale in
+ * ctl_out, since the workgroup that reads those is not ordered behind it.
+ * Nothing is merged when the pairs exceed `capacity`. */
 int gat_edr_stage_queries(const void* meta_pinned, int64_t meta_bytes, void* up_dev, const int64_t* src_pinned,
                           const int64_t* dst_pinned, int32_t ntraj, int64_t npoints, const float* lon_pinned,
                           const float* lat_pinned, int64_t total, float* xy_dev, float* box_dev, uint32_t* ctl_dev,
@@ -427,7 +430,7 @@ int gat_edr_length_table(const int32_t* table_dev, int32_t w, int32_t* out_dev, 
 int gat_edr_merge(const int32_t* length_table_dev, int32_t w, const int32_t* qlen_dev, int32_t nq,
                   const int32_t* clen_dev, int32_t nc, const int32_t* len_ids_dev, const int32_t* len_off_dev,
                   const int32_t* pairs_dev, const int32_t* dist_dev, int64_t capacity, int32_t k, int32_t kk,
-                  int32_t* out_ids, int32_t* out_dist, uint32_t* ctl_dev, uint32_t* ctl_out, uint32_t* stamp_dev,
+                  int32_t* out_ids, int32_t* out_dist, uint32_t* ctl_dev, uint32_t* ctl_out, uint32_t* stamp,
                   void* stream);
 
 /* Exact top-k merge on the device (no reference counterpart: the reference

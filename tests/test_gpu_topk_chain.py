@@ -4,6 +4,8 @@ list and the same merge, and the lists a query with more survivors than that
 merge sorts falls back to; queries uploaded in one part and in several; no
 survivor at all, more results asked for than trajectories.  Answers of every
 route equal the host-built path's, and sampled rows the oracle's."""
+import time
+
 import numpy as np
 import pytest
 
@@ -161,3 +163,20 @@ def test_merge_routes(gpu, case, nsurv):
                                ldist.ptr, k, kk, out_i.ptr, out_d.ptr, status.ptr, None))
     assert status.get(np.int32, 1)[0] == 0
     assert (out_i.get(np.int32, kk) == order + 1).all() and (out_d.get(np.int32, kk) == d[order]).all()
+
+
+@pytest.mark.parametrize("nq", [13, 200])  # the short chain and the job-list chain
+def test_stage_times_add_up(gpu, nq):
+    """Each stage's device time is what it can be, batch after batch: the merge's
+    start is written by another workgroup than the one that brings the rest of
+    the clock readings back, and a stale reading would wrap around."""
+    db = api.synth_walks(3, api.synth_lengths(3, 4000, "lognormal", 64, 0.8, 8, 512))
+    g = api.GridIndex(W.UNIT_BOX, 0.01, 64).build(db)
+    q = api.synth_queries(5, api.synth_lengths(4, nq, "uniform", 16, 256, 16, 256), db, copy_mode=2)
+    g.similarity_batched(q, 20, EPS)
+    for _ in range(100):
+        t0 = time.perf_counter()
+        st = g.similarity_batched(q, 20, EPS)[2]
+        wall = (time.perf_counter() - t0) * 1e3
+        stages = [st["filter_ms"], st["kernel_ms"], st["merge_ms"]]
+        assert min(stages) > 0 and sum(stages) <= wall, (stages, wall)
