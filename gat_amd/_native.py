@@ -78,6 +78,7 @@ HIP_FUNCS = {
     "gatEDRDistanceBatchHandler": (INT, [INT, P, P, P, P, P, P, P, F64, P, P]),
     "gat_edr_batched": (INT, [P, I64, P, I64, P, P, P, P, P, I32, P, P, P, I32, I32, F64, I32, I32, P, P]),
     "gat_edr_jobs": (INT, [P, P, I64, P, I32, P, I32, I32, I32, I32, P, P, P, P, P, P, P, P]),
+    "gat_edr_jobs_stamped": (INT, [P, P, I64, P, I32, P, I32, I32, I32, I32, P, P, P, P, P, P, P, P, P]),
     "gat_edr_all_pairs": (INT, [I32, I32, P, P, P]),
     "gat_edr_unsort": (INT, [P, P, P, I64, P, P]),
     "gat_edr_survivor_lists": (INT, [P, P, P, I64, I32, P, P, P, P, P]),

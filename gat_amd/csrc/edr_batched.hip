@@ -1386,12 +1386,14 @@ __global__ __launch_bounds__(kJobThreads) void edr_jobs_kernel(const int2* __res
                                                                int2* __restrict__ nm, Job* __restrict__ jobs,
                                                                int32_t* __restrict__ windows,
                                                                int32_t* __restrict__ status,
-                                                               unsigned long long* __restrict__ cells) {
+                                                               unsigned long long* __restrict__ cells,
+                                                               uint32_t* __restrict__ stamp) {
   __shared__ uint32_t bins[kSortBins];
   __shared__ uint32_t gjobs[kJobGroups + 1];
   __shared__ uint32_t red[kJobThreads / 64 + 1];
   __shared__ unsigned long long red64[kJobThreads / 64];
   const int t = threadIdx.x;
+  if (stamp && t == 0) store_clock(stamp);
   const unsigned long long total = *count;
   if (t == 0) *status = total > cap ? 1 : 0;
   if (total > cap) {  // uniform: nothing to run; the caller grows the buffers
@@ -1495,7 +1497,9 @@ __device__ __forceinline__ bool jobs_overflow(const unsigned long long* count, u
 __global__ __launch_bounds__(kJobsBlock) void edr_jobs_lengths_kernel(
     const int2* __restrict__ pairs, const unsigned long long* __restrict__ count, uint32_t cap,
     const int32_t* __restrict__ qlen, int32_t nq, const int32_t* __restrict__ clen, int32_t nc, JobRules rules,
-    int2* __restrict__ nm, unsigned long long* __restrict__ cells, unsigned long long* __restrict__ crit) {
+    int2* __restrict__ nm, unsigned long long* __restrict__ cells, unsigned long long* __restrict__ crit,
+    uint32_t* __restrict__ stamp) {
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) store_clock(stamp);
   uint32_t np;
   if (jobs_overflow(count, cap, &np)) return;
   const JobShape sh(rules, np);
@@ -2125,10 +2129,11 @@ extern "C" int gat_edr_pairs(const int32_t* pairs, const uint64_t* live, int64_t
                     gat::as_stream(stream));
 }
 
-extern "C" int gat_edr_jobs(const int32_t* pairs, const uint64_t* count, int64_t capacity, const int32_t* qlen,
-                            int32_t nq, const int32_t* clen, int32_t nc, int32_t split, int32_t waves,
-                            int32_t every_long, int32_t* sorted, int32_t* origin, int32_t* scratch,
-                            gat_edr_job* jobs, int32_t* windows, int32_t* status, uint64_t* cells, void* stream) {
+extern "C" int gat_edr_jobs_stamped(const int32_t* pairs, const uint64_t* count, int64_t capacity, const int32_t* qlen,
+                                    int32_t nq, const int32_t* clen, int32_t nc, int32_t split, int32_t waves,
+                                    int32_t every_long, int32_t* sorted, int32_t* origin, int32_t* scratch,
+                                    gat_edr_job* jobs, int32_t* windows, int32_t* status, uint64_t* cells,
+                                    uint32_t* stamp, void* stream) {
   GAT_REQUIRE(capacity >= 0 && capacity <= int64_t(INT32_MAX) - 8 && nq >= 0 && nc >= 0,
               "EDR jobs: bad sizes");
   GAT_REQUIRE(split >= 1 && split <= GAT_MAX_TRAJ_LEN && waves >= 1 && waves <= 8, "EDR jobs: bad rules");
@@ -2143,7 +2148,8 @@ extern "C" int gat_edr_jobs(const int32_t* pairs, const uint64_t* count, int64_t
   if (capacity <= kJobsOneBlock) {
     edr_jobs_kernel<<<dim3(1), dim3(kJobThreads), 0, s>>>(P, C, uint32_t(capacity), qlen, nq, clen, nc, rules,
                                                           reinterpret_cast<int2*>(sorted), origin, NM,
-                                                          reinterpret_cast<Job*>(jobs), windows, status, cells_u);
+                                                          reinterpret_cast<Job*>(jobs), windows, status, cells_u,
+                                                          stamp);
     GAT_LAUNCH_CHECK("edr_jobs_kernel");
     return GAT_OK;
   }
@@ -2165,7 +2171,7 @@ extern "C" int gat_edr_jobs(const int32_t* pairs, const uint64_t* count, int64_t
   if (blocks < 1) blocks = 1;
   const dim3 grid{uint32_t(blocks)}, block{kJobsBlock};
   const uint32_t cap = uint32_t(capacity);
-  edr_jobs_lengths_kernel<<<grid, block, 0, s>>>(P, C, cap, qlen, nq, clen, nc, rules, NM, cells_u, crit);
+  edr_jobs_lengths_kernel<<<grid, block, 0, s>>>(P, C, cap, qlen, nq, clen, nc, rules, NM, cells_u, crit, stamp);
   GAT_LAUNCH_CHECK("edr_jobs_lengths_kernel");
   edr_jobs_hist_kernel<<<grid, block, 0, s>>>(C, cap, rules, NM, crit, gbins);
   GAT_LAUNCH_CHECK("edr_jobs_hist_kernel");
@@ -2177,6 +2183,14 @@ extern "C" int gat_edr_jobs(const int32_t* pairs, const uint64_t* count, int64_t
   edr_jobs_write_kernel<<<grid, block, 0, s>>>(C, cap, gstart, gjobs, reinterpret_cast<Job*>(jobs));
   GAT_LAUNCH_CHECK("edr_jobs_write_kernel");
   return GAT_OK;
+}
+
+extern "C" int gat_edr_jobs(const int32_t* pairs, const uint64_t* count, int64_t capacity, const int32_t* qlen,
+                            int32_t nq, const int32_t* clen, int32_t nc, int32_t split, int32_t waves,
+                            int32_t every_long, int32_t* sorted, int32_t* origin, int32_t* scratch,
+                            gat_edr_job* jobs, int32_t* windows, int32_t* status, uint64_t* cells, void* stream) {
+  return gat_edr_jobs_stamped(pairs, count, capacity, qlen, nq, clen, nc, split, waves, every_long, sorted, origin,
+                              scratch, jobs, windows, status, cells, nullptr, stream);
 }
 
 extern "C" int gat_edr_survivor_lists(const int32_t* sorted, const int32_t* dist, const uint64_t* count,

@@ -843,8 +843,8 @@ int Grid::runBatchedOnDevice(const int32_t* pairsHost, int64_t np, int queryNum,
 // A batch's control words (topCtl_, cleared by the upload; the merge or a copy
 // brings them back): [0, 1] survivors, [2] lists and [3] merge status (as
 // gat_edr_merge's), [4, 5] cells, [6] the job counter of gat_edr_pairs, [7]
-// ticket, [8] job list status, [10, 14) the clock at the filter and the DP,
-// [16, 24) the buckets' windows, [24, 28) their job counters; after them the
+// ticket, [8] job list status, [10, 16) the clock at the filter, the DP and the
+// job list (between the two), [16, 24) the buckets' windows, [24, 28) their job counters; after them the
 // clock at the upload (device), or at the merge's end and its start (host: the
 // merge writes both there itself, since its workgroup that brings the words
 // back is not ordered behind the one that starts first).
@@ -894,10 +894,11 @@ int Grid::similarityOnDevice(int nq, int kValue, TopKSink& out, EdrBatchStats* s
     GATH_TRY(gat_edr_filter_grid_add(queryBox_.as<float>(), nq, trajBox_.as<float>(), trajNum, &candGrid_, epsilon,
                                      pairsDev_.as<int32_t>(), cap, count, ctl + 10, s),
              "candidate filter");
-    GATH_TRY(gat_edr_jobs(pairsDev_.as<int32_t>(), count, cap, queryLenDev_, nq, trajLen_.as<int32_t>(), trajNum,
-                          split, waves, edrWavesEveryLongPair ? 1 : 0, sortedDev_.as<int32_t>(), nullptr,
-                          nmDev_.as<int32_t>(), jobsDev_.as<gat_edr_job>(), win, reinterpret_cast<int32_t*>(ctl + 8),
-                          reinterpret_cast<uint64_t*>(ctl + 4), s),
+    GATH_TRY(gat_edr_jobs_stamped(pairsDev_.as<int32_t>(), count, cap, queryLenDev_, nq, trajLen_.as<int32_t>(),
+                                  trajNum, split, waves, edrWavesEveryLongPair ? 1 : 0, sortedDev_.as<int32_t>(),
+                                  nullptr, nmDev_.as<int32_t>(), jobsDev_.as<gat_edr_job>(), win,
+                                  reinterpret_cast<int32_t*>(ctl + 8), reinterpret_cast<uint64_t*>(ctl + 4), ctl + 14,
+                                  s),
              "device jobs");
     if (!merge)
       if (int rc = edrTimer_.start(s)) return rc;
@@ -960,7 +961,7 @@ int Grid::similarityOnDevice(int nq, int kValue, TopKSink& out, EdrBatchStats* s
       st->cells += int64_t(ctl64(c, 4));
       st->jobs += int64_t(c[17]) + c[19] + c[21] + c[23];
       st->pruned += int64_t(nq) * trajNum - int64_t(found);
-      if (trajNum > 0) st->filterMs += double(ctl64(c, 12) - ctl64(c, 10)) / clockKhz_;
+      if (trajNum > 0) st->filterMs += double(ctl64(c, 14) - ctl64(c, 10)) / clockKhz_;
       if (merge) {
         st->kernelMs += double(ctl64(c, kCtlWords + 2) - ctl64(c, 12)) / clockKhz_;
         st->mergeMs += double(ctl64(c, kCtlWords) - ctl64(c, kCtlWords + 2)) / clockKhz_;

@@ -314,6 +314,12 @@ int gat_edr_jobs(const int32_t* pairs_dev, const uint64_t* count_dev, int64_t ca
                  int32_t every_long, int32_t* sorted_dev, int32_t* origin_dev, int32_t* scratch_dev,
                  gat_edr_job* jobs_dev, int32_t* windows_dev, int32_t* status_dev, uint64_t* cells_dev,
                  void* stream);
+/* gat_edr_jobs, with the wall clock at its start in stamp_dev (null: not). */
+int gat_edr_jobs_stamped(const int32_t* pairs_dev, const uint64_t* count_dev, int64_t capacity, const int32_t* query_length_dev,
+                         int32_t nqueries, const int32_t* cand_length_dev, int32_t ncands, int32_t split, int32_t waves,
+                         int32_t every_long, int32_t* sorted_dev, int32_t* origin_dev, int32_t* scratch_dev,
+                         gat_edr_job* jobs_dev, int32_t* windows_dev, int32_t* status_dev, uint64_t* cells_dev,
+                         uint32_t* stamp_dev, void* stream);
 
 /* Every (query, candidate) pair of nq x nc: pairs_dev[2i], [2i+1] = (i / nc,
  * i % nc); *count_dev = nq * nc (at most INT32_MAX).  For gat_edr_jobs over a

@@ -180,3 +180,19 @@ def test_stage_times_add_up(gpu, nq):
         wall = (time.perf_counter() - t0) * 1e3
         stages = [st["filter_ms"], st["kernel_ms"], st["merge_ms"]]
         assert min(stages) > 0 and sum(stages) <= wall, (stages, wall)
+
+
+def test_filter_time_leaves_out_the_job_list(gpu):
+    """filter_ms is the filter's on the device chain as on the host-built path,
+    where events bracket it: in a batch whose 90,000 survivors keep the one
+    workgroup of the job list busy several times as long."""
+    db = _near(21, 300, [40, 60], 1e-4)
+    g = api.GridIndex(W.UNIT_BOX, 0.01, 64).build(db)
+    q = _near(22, 300, [40, 60], 1e-4)
+    ms = {}
+    for chain in (True, False):
+        g.set_topk_device_chain(chain)
+        runs = [g.similarity_batched(q, 20, EPS)[2] for _ in range(6)]
+        assert runs[0]["pairs"] > 80_000
+        ms[chain] = min(r["filter_ms"] for r in runs[2:])
+    assert ms[True] <= 1.25 * ms[False] + 0.01, ms
