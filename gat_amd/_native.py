@@ -75,6 +75,7 @@ HIP_FUNCS = {
     "gat_range_refine_bitmap": (INT, [P, P, I64, P, I64, P, I64, P]),
     "gat_range_refine_pairs": (INT, [P, P, I64, P, I64, P, P, P, I64, P]),
     "gat_pairs_digest": (INT, [P, P, P, I64, I64, P, P]),
+    "gat_pairs_digest_stamped": (INT, [P, P, P, I64, I64, P, P, P]),
     "gatEDRDistanceBatchHandler": (INT, [INT, P, P, P, P, P, P, P, F64, P, P]),
     "gat_edr_batched": (INT, [P, I64, P, I64, P, P, P, P, P, I32, P, P, P, I32, I32, F64, I32, I32, P, P]),
     "gat_edr_jobs": (INT, [P, P, I64, P, I32, P, I32, I32, I32, I32, P, P, P, P, P, P, P, P]),

@@ -211,8 +211,14 @@ template <bool kWide>
 __global__ __launch_bounds__(kBlock) void pairs_digest_kernel(const int2* __restrict__ pairs,
                                                              const uint64_t* __restrict__ qbase,
                                                              const uint32_t* __restrict__ qcount, uint32_t nq,
-                                                             uint64_t capacity, unsigned long long* __restrict__ out) {
+                                                             uint64_t capacity, unsigned long long* __restrict__ out,
+                                                             uint32_t* __restrict__ stamp) {
   __shared__ uint64_t part[kBlock / kWave];
+  if (stamp && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    const uint64_t t = wall_clock64();
+    stamp[0] = uint32_t(t);
+    stamp[1] = uint32_t(t >> 32);
+  }
   for (uint32_t q = blockIdx.x; q < nq; q += gridDim.x) {
     const gat::PairRegion r = gat::pair_region(qbase[q], qcount[q], capacity);
     const uint64_t a = r.first, b = r.begin, e = r.end;
@@ -352,8 +358,8 @@ int gatRangeQueryTestHandlerNoAlloc(const gat_point_store* store, const gat_rang
   return rc;
 }
 
-int gat_pairs_digest(const int32_t* pairs, const uint64_t* qbase, const uint32_t* qcount, int64_t nq,
-                     int64_t pairs_capacity, uint64_t* digest, void* stream) {
+int gat_pairs_digest_stamped(const int32_t* pairs, const uint64_t* qbase, const uint32_t* qcount, int64_t nq,
+                             int64_t pairs_capacity, uint64_t* digest, uint32_t* stamp, void* stream) {
   GAT_REQUIRE(nq >= 0 && nq <= int64_t(UINT32_MAX), "pairs digest: bad query count");
   if (nq == 0) return GAT_OK;
   GAT_REQUIRE(pairs && qbase && qcount && digest && pairs_capacity >= 0, "pairs digest: bad argument");
@@ -366,12 +372,17 @@ int gat_pairs_digest(const int32_t* pairs, const uint64_t* qbase, const uint32_t
   auto* O = reinterpret_cast<unsigned long long*>(digest);
   if (reinterpret_cast<uintptr_t>(pairs) % 16 == 0)
     pairs_digest_kernel<true><<<grid, block, 0, gat::as_stream(stream)>>>(P, qbase, qcount, uint32_t(nq),
-                                                                          uint64_t(pairs_capacity), O);
+                                                                          uint64_t(pairs_capacity), O, stamp);
   else
     pairs_digest_kernel<false><<<grid, block, 0, gat::as_stream(stream)>>>(P, qbase, qcount, uint32_t(nq),
-                                                                           uint64_t(pairs_capacity), O);
+                                                                           uint64_t(pairs_capacity), O, stamp);
   GAT_LAUNCH_CHECK("pairs_digest_kernel");
   return GAT_OK;
+}
+
+int gat_pairs_digest(const int32_t* pairs, const uint64_t* qbase, const uint32_t* qcount, int64_t nq,
+                     int64_t pairs_capacity, uint64_t* digest, void* stream) {
+  return gat_pairs_digest_stamped(pairs, qbase, qcount, nq, pairs_capacity, digest, nullptr, stream);
 }
 
 }  // extern "C"

@@ -1103,8 +1103,8 @@ int RangeEngine::enqueueResults(int nq, RangeBatch& out) {
                                   nq, dig, ctr + 12, s),
              "run digest");
   else
-    GATH_TRY(gat_pairs_digest(out.pairs.as<int32_t>(), out.qbase.as<uint64_t>(), out.qcount.as<uint32_t>(), nq,
-                              pairsCap_, dig, s),
+    GATH_TRY(gat_pairs_digest_stamped(out.pairs.as<int32_t>(), out.qbase.as<uint64_t>(), out.qcount.as<uint32_t>(), nq,
+                                      pairsCap_, dig, ctr + 12, s),
              "pair digest");
   GATH_TRY(gat_direct_finish(ctr, out.qcount.as<uint32_t>(), dig, nq, resultHost_.as<uint32_t>(), s),
            "batch readback");

@@ -234,6 +234,10 @@ int gat_range_refine_pairs(const gat_point_store* store, const gat_range_task* t
  * SystemTest.cpp:79-89.) */
 int gat_pairs_digest(const int32_t* pairs_dev, const uint64_t* qbase_dev, const uint32_t* qcount_dev, int64_t nq,
                      int64_t pairs_capacity, uint64_t* digest_dev, void* stream);
+/* The same with the wall clock at its start in stamp_dev (null: not). */
+int gat_pairs_digest_stamped(const int32_t* pairs_dev, const uint64_t* qbase_dev, const uint32_t* qcount_dev,
+                             int64_t nq, int64_t pairs_capacity, uint64_t* digest_dev, uint32_t* stamp_dev,
+                             void* stream);
 
 /* ------------------------------------------------------------------ EDR */
 /* One (query, candidate) pair.  Replaces TaskInfoTableForSimilarity

@@ -89,6 +89,23 @@ def test_a_small_workspace_discards_no_other(gpu, layout, kind):
     assert run(counts, sides).tolist() == [5, 5, 1]
 
 
+@pytest.mark.parametrize("run_indexed", [True, False])
+def test_digest_time_is_the_digests(gpu, run_indexed):
+    """digest_ms of a queued group covers the digest kernels, which cannot read
+    the pairs faster than the memory's 8 TB/s."""
+    db = api.synth_walks(9, api.synth_lengths(9, 40_000, "uniform", 16, 256, 16, 256), step_sigma=4e-3)
+    ix = (api.GridIndex(W.UNIT_BOX, 0.01, 256).build(db, device=True), api.StigIndex(256).build(db, device=True),
+          api.FsgIndex(W.UNIT_BOX, 0.01).build(db, device=True))
+    for i in ix:
+        i.set_result_layout(run_indexed)
+    m = api.MixedRange(*ix)
+    rects = _rects(np.random.default_rng(1), 600, 0.24, 0.26)
+    for _ in range(2):
+        st = m.run(rects)[3]
+    assert m.pipelines() == {"queued": 1, "stepped": 1, "discarded": 0}
+    assert st["pairs"] > 1e8 and st["digest_ms"] * 1e-3 >= 8 * st["pairs"] / 8e12, st
+
+
 def test_batched_form_over_growing_batches(indexes):
     rng = np.random.default_rng(5)
     for ix in indexes:
