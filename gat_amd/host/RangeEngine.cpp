@@ -372,6 +372,7 @@ int RangeBatch::fetchCompact(int32_t* out, int64_t capacityPairs) {
   if (pairTotal == 0) return GAT_OK;
   const size_t bytes = size_t(pairTotal) * 8;
   if (bytes <= kGatherBytes) {
+    std::lock_guard<std::mutex> hold(lock_.m);
     size_t room = size_t(1) << 16;
     while (room < bytes) room *= 2;
     if (int rc = gatherAt_.reserve(size_t(queryNum) * 8)) return rc;
@@ -441,6 +442,7 @@ int RangeBatch::fetch(int32_t* out, int64_t capacityPairs) {
 
 int RangeBatch::digests(uint64_t* out) const {
   if (queryNum == 0) return GAT_OK;
+  std::lock_guard<std::mutex> hold(lock_.m);
   if (int rc = digestDev_.reserve(size_t(queryNum) * 8)) return rc;
   return digestsInto(digestDev_.as<uint64_t>(), out);
 }

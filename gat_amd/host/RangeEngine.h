@@ -12,6 +12,7 @@
 
 #include <cstdint>
 #include <functional>
+#include <mutex>
 #include <vector>
 
 #include "DeviceArena.h"
@@ -87,6 +88,15 @@ struct RangeBatch {
   mutable DeviceBuffer digestDev_;  // digests(): kept, since a free waits for the device
 
  private:
+  // Held by a readback that goes through the kept buffers, so that several
+  // threads may read one batch.  A moved batch gets a lock of its own.
+  struct Lock {
+    std::mutex m;
+    Lock() = default;
+    Lock(Lock&&) noexcept {}
+    Lock& operator=(Lock&&) noexcept { return *this; }
+  };
+  mutable Lock lock_;
   // fetchCompact of up to kGatherBytes of pairs: gathered on the device into
   // pinned memory in one launch pair.  Larger ones go by a copy per query (or
   // per batch): the gather would hold as much pinned memory as the result.

@@ -3,6 +3,8 @@ size around a wave's four entries and the regions kernel's 256 threads, a batch
 that outgrows the buffers' capacities, leaves of more points than one round
 takes, both id packings' store, rectangles that select nothing; counts, digests
 and pair sets against the plain path and inclusive brute force."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -46,3 +48,33 @@ def test_direct_chain(gpu, nq, leaf):
         assert (res.counts() == pc).all()
         for a, b in zip(res.per_query(), pp):
             assert sorted(map(tuple, a.tolist())) == sorted(map(tuple, b.tolist()))
+
+
+@pytest.mark.parametrize("direct", [256, 0])  # regions of the direct form, runs of the leaf-major one
+def test_a_batch_read_by_several_threads(gpu, direct):
+    """Digests and pairs of one batch asked for by several threads at once (a
+    reader's call leaves the interpreter while it waits for the device)."""
+    db = api.synth_walks(5, api.synth_lengths(5, 3000, "uniform", 1, 90, 1, 90), step_sigma=4e-3)
+    ix = api.GridIndex(W.UNIT_BOX, 0.02, 64).build(db).set_batch_params(32, direct)
+    res = ix.range_batched(_rects(np.random.default_rng(8), 200))
+    counts = np.concatenate([[0], np.cumsum(res.counts(), dtype=np.int64)])
+
+    def keys():
+        p = res.pairs().astype(np.int64)
+        key = np.repeat(np.arange(len(counts) - 1), np.diff(counts)) << 40 | p[:, 0] << 16 | p[:, 1]
+        return np.sort(key)
+
+    want_d, want_k = res.digests(), keys()
+    bad = []
+
+    def read(n):
+        for _ in range(n):
+            if not (res.digests() == want_d).all() or not (keys() == want_k).all():
+                bad.append(threading.get_ident())
+
+    threads = [threading.Thread(target=read, args=(40,)) for _ in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
