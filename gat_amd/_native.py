@@ -160,6 +160,7 @@ HOST_FUNCS = {
     "gath_index_select": (I64, [P, P, INT, P, I64, P]),
     "gath_index_cell_of": (I64, [P, F32, F32]),
     "gath_index_range_bitmap": (INT, [P, P, INT, P]),
+    "gath_index_range_handler": (INT, [P, P, INT, P, P]),
     "gath_index_range_pairs": (INT, [P, P, INT, P, P]),
     "gath_index_range_batched": (INT, [P, P, INT, INT, P, P]),
     "gath_index_tree_nodes": (I64, [P, P, I64, P]),

@@ -354,6 +354,16 @@ class _Index:
         N.check_host(N.host().gath_index_range_bitmap(self.handle, _ptr(b), len(b), _ptr(out)))
         return out
 
+    def range_handler(self, boxes: np.ndarray) -> tuple[np.ndarray, np.ndarray]:
+        """range_bitmap's answer by the index's reference-signature method (host
+        selection and the bitmap handler), and each rectangle's number of
+        trajectories."""
+        b = _req(boxes, np.float32).reshape(-1, 4)
+        out = np.empty((len(b), self.ntraj + 1), np.uint8)
+        sizes = np.zeros(max(len(b), 1), np.int32)
+        N.check_host(N.host().gath_index_range_handler(self.handle, _ptr(b), len(b), _ptr(out), _ptr(sizes)))
+        return out, sizes[:len(b)]
+
     def range_pairs(self, boxes: np.ndarray) -> RangeResult:
         b = _req(boxes, np.float32).reshape(-1, 4)
         stats = np.zeros(3, np.int64)

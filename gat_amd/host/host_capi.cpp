@@ -186,16 +186,22 @@ int64_t gath_index_select(void* p, const float* boxes, int nq, uint32_t* tasks_o
 int gath_index_range_bitmap(void* p, const float* boxes, int nq, uint8_t* out) {
   Index* ix = as_index(p);
   if (!ix || nq < 0 || (nq > 0 && (!boxes || !out))) return bad("gath_index_range_bitmap: bad arguments");
-  // The index's own device tree selects; an index without one (built without
-  // upload) takes the handlers, which report that.
+  // The index's own device tree selects; an index without one (no points, or
+  // built without upload) takes the handlers.
   const DeviceTree& tree = ix->grid ? ix->grid->deviceTree() : ix->fsg ? ix->fsg->deviceTree() : ix->stig->deviceTree();
   RangeEngine& engine = ix->grid ? ix->grid->engine() : ix->fsg ? ix->fsg->engine() : ix->stig->engine();
   if (tree.nnodes > 0) return engine.runBitmapDirect(tree, as_boxes(boxes), nq, int64_t(ix->trajNum()) + 1, out);
+  return gath_index_range_handler(p, boxes, nq, out, nullptr);
+}
+
+int gath_index_range_handler(void* p, const float* boxes, int nq, uint8_t* out, int32_t* set_sizes) {
+  Index* ix = as_index(p);
+  if (!ix || nq < 0 || (nq > 0 && (!boxes || !out))) return bad("gath_index_range_handler: bad arguments");
   std::vector<CPURangeQueryResult> res(static_cast<size_t>(nq));
   int rc;
-  if (ix->grid) rc = ix->grid->rangeQueryBatchGPU(as_boxes(boxes), nq, res.data(), nullptr);
-  else if (ix->fsg) rc = ix->fsg->rangeQueryBatchGPU(as_boxes(boxes), nq, res.data(), nullptr);
-  else rc = ix->stig->rangeQueryGPU(as_boxes(boxes), nq, res.data(), nullptr);
+  if (ix->grid) rc = ix->grid->rangeQueryBatchGPU(as_boxes(boxes), nq, res.data(), set_sizes);
+  else if (ix->fsg) rc = ix->fsg->rangeQueryBatchGPU(as_boxes(boxes), nq, res.data(), set_sizes);
+  else rc = ix->stig->rangeQueryGPU(as_boxes(boxes), nq, res.data(), set_sizes);
   if (rc) return rc;
   const size_t stride = size_t(ix->trajNum()) + 1;
   for (int q = 0; q < nq; ++q)

@@ -95,8 +95,14 @@ int64_t gath_index_select(void* index, const float* boxes, int nq, uint32_t* tas
                           uint64_t* candidates_out);
 /* Cell of a point (Grid: Morton id; FSG: row-major id; -1 outside). */
 int64_t gath_index_cell_of(void* index, float lon, float lat);
-/* The reference-signature path: trajectory bitmap (nq * (ntraj + 1) bytes). */
+/* The reference's result form: trajectory bitmap (nq * (ntraj + 1) bytes), by
+ * the direct form's chain on the device. */
 int gath_index_range_bitmap(void* index, const float* boxes, int nq, uint8_t* out);
+/* The same bitmap through the index's reference-signature method
+ * (Grid / FSG::rangeQueryBatchGPU, STIG::rangeQueryGPU: host selection, then
+ * the bitmap handler); set_sizes (null: not) gets each rectangle's number of
+ * trajectories. */
+int gath_index_range_handler(void* index, const float* boxes, int nq, uint8_t* out, int32_t* set_sizes);
 /* Compacted-pair path.  stats[0..2] = pairs, candidates, tasks; ms[0..2] =
  * host selection, task upload, refine kernel.  The result stays on the device
  * until the next call. */

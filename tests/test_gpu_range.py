@@ -31,6 +31,12 @@ def _check_pairs(res, want_sets, rects):
         assert s == w, f"query {q}: {len(s - w)} extra, {len(w - s)} missing"
 
 
+def _check_handler(ix, rects, bitmap):
+    """The index's reference-signature method gives the same bitmap."""
+    got, sizes = ix.range_handler(rects)
+    assert (got == bitmap).all() and (sizes == bitmap.sum(1)).all()
+
+
 @pytest.fixture(scope="module")
 def cfg1(gpu):
     db = W.CFG1.db()
@@ -48,7 +54,9 @@ def test_cfg1_grid_pairs_and_bitmap(cfg1):
     assert res.candidates >= res.pairs_total > 0
     counts, dig = og.range(rects, "digest")
     assert (res.digests() == dig).all()
-    assert (g.range_bitmap(rects) == og.range(rects, "bitmap")).all()
+    bm = og.range(rects, "bitmap")
+    assert (g.range_bitmap(rects) == bm).all()
+    _check_handler(g, rects, bm)
 
 
 def test_cfg1_fsg_and_stig(cfg1):
@@ -61,6 +69,10 @@ def test_cfg1_fsg_and_stig(cfg1):
     bm = O.brute_range(db, rects, "bitmap")
     assert (f.range_bitmap(rects) == bm).all()
     assert (s.range_bitmap(rects) == bm).all()
+    _check_handler(f, rects, bm)
+    _check_handler(s, rects, bm)
+    m = api.MortonGridIndex(W.UNIT_BOX, W.CFG1.grid_cell, W.CFG1.leaf).build(db)
+    _check_handler(m, rects, O.Grid(W.UNIT_BOX, W.CFG1.grid_cell, W.CFG1.leaf).add(db).range(rects, "bitmap"))
 
 
 def _edge_rects(db, cell, n, seed):
@@ -116,6 +128,9 @@ def test_empty_batches(gpu):
     res = g.range_pairs(far)
     assert res.pairs_total == 0 and res.candidates == 0
     assert g.range_bitmap(far).sum() == 0
+    _check_handler(g, far, np.zeros((1, 51), np.uint8))
+    with pytest.raises(GatError, match="null result buffer"):
+        g.range_handler(np.zeros((0, 4), np.float32))
 
 
 def test_repeated_batches_reuse_buffers(gpu, cfg1):
