@@ -186,11 +186,12 @@ int64_t gath_index_select(void* p, const float* boxes, int nq, uint32_t* tasks_o
 int gath_index_range_bitmap(void* p, const float* boxes, int nq, uint8_t* out) {
   Index* ix = as_index(p);
   if (!ix || nq < 0 || (nq > 0 && (!boxes || !out))) return bad("gath_index_range_bitmap: bad arguments");
-  // The index's own device tree selects; an index without one (no points, or
-  // built without upload) takes the handlers.
+  // The index's own device tree selects.  An index without one (no points, or
+  // built without upload) takes the handlers, and so does an empty batch, which
+  // they refuse.
   const DeviceTree& tree = ix->grid ? ix->grid->deviceTree() : ix->fsg ? ix->fsg->deviceTree() : ix->stig->deviceTree();
   RangeEngine& engine = ix->grid ? ix->grid->engine() : ix->fsg ? ix->fsg->engine() : ix->stig->engine();
-  if (tree.nnodes > 0) return engine.runBitmapDirect(tree, as_boxes(boxes), nq, int64_t(ix->trajNum()) + 1, out);
+  if (tree.nnodes > 0 && nq > 0) return engine.runBitmapDirect(tree, as_boxes(boxes), nq, int64_t(ix->trajNum()) + 1, out);
   return gath_index_range_handler(p, boxes, nq, out, nullptr);
 }
 

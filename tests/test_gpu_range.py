@@ -57,6 +57,7 @@ def test_cfg1_grid_pairs_and_bitmap(cfg1):
     bm = og.range(rects, "bitmap")
     assert (g.range_bitmap(rects) == bm).all()
     _check_handler(g, rects, bm)
+    _check_handler(api.MortonGridIndex(W.UNIT_BOX, W.CFG1.grid_cell, W.CFG1.leaf).build(db), rects, bm)
 
 
 def test_cfg1_fsg_and_stig(cfg1):
@@ -71,8 +72,6 @@ def test_cfg1_fsg_and_stig(cfg1):
     assert (s.range_bitmap(rects) == bm).all()
     _check_handler(f, rects, bm)
     _check_handler(s, rects, bm)
-    m = api.MortonGridIndex(W.UNIT_BOX, W.CFG1.grid_cell, W.CFG1.leaf).build(db)
-    _check_handler(m, rects, O.Grid(W.UNIT_BOX, W.CFG1.grid_cell, W.CFG1.leaf).add(db).range(rects, "bitmap"))
 
 
 def _edge_rects(db, cell, n, seed):
@@ -129,8 +128,9 @@ def test_empty_batches(gpu):
     assert res.pairs_total == 0 and res.candidates == 0
     assert g.range_bitmap(far).sum() == 0
     _check_handler(g, far, np.zeros((1, 51), np.uint8))
-    with pytest.raises(GatError, match="null result buffer"):
-        g.range_handler(np.zeros((0, 4), np.float32))
+    for call in (g.range_handler, g.range_bitmap):
+        with pytest.raises(GatError, match="null result buffer"):
+            call(np.zeros((0, 4), np.float32))
 
 
 def test_repeated_batches_reuse_buffers(gpu, cfg1):
