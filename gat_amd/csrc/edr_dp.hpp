@@ -38,17 +38,6 @@ constexpr int kOff64 = 67;
 template <int SEG>
 constexpr int kRowOff = SEG == 64 ? kOff64 : SEG;
 
-// Stores of different lanes to one LDS column come from different steps'
-// store instructions, and the row left behind is the last lane's only if those
-// instructions keep program order.  Per lane their addresses differ, so the
-// scheduler may reorder them; this barrier lets every other kind of
-// instruction (ALU, global loads, LDS reads) move across it, but not LDS
-// writes.
-__device__ __forceinline__ void keep_store_order() {
-  // 0x1 ALU, 0x2 VALU, 0x4 SALU, 0x10 VMEM, 0x20 VMEM read, 0x100 DS read.
-  __builtin_amdgcn_sched_barrier(0x1 | 0x2 | 0x4 | 0x10 | 0x20 | 0x100);
-}
-
 // Lane l of a segment takes src from lane l - 1; lane 0 keeps old.  Segments
 // of 16 lanes are DPP rows (row_shr:1); a 64-lane segment is the wave
 // (wave_shr:1).
@@ -268,6 +257,9 @@ __device__ __forceinline__ void sweep_strip(const float2* R, int n, const float2
         for (int i = 0; i < K; ++i) res = (t0 + j == tcap && i == ic) ? rows.e[i] : res;
       }
       own[j][seg] = RowValue<SEG>(rows.e[K - 1]);
+      // The stores of different lanes to one column come from different steps,
+      // and the last lane's must stay last; per lane their addresses differ, so
+      // without this the scheduler could reorder them.
       __builtin_amdgcn_sched_barrier(0);
     }
   };

@@ -252,10 +252,9 @@ class Grid {
   // pair whose boxes could hold a matching point pair.
   int filterPairs(int nq, int64_t cap, void* stream);
   DeviceBuffer queryXY_, queryBox_;
-  // The uploaded queries: offsets and lengths, then the raw coordinates
-  // (packed into queryXY_ on the device); the pointers below view it.
+  // The uploaded queries' offsets and lengths, which the pointers below view
+  // (their points are in queryXY_).
   DeviceBuffer queryUp_;
-  const int64_t* querySrcOffDev_ = nullptr;
   const int64_t* queryOff64Dev_ = nullptr;
   const int32_t* queryOffDev_ = nullptr;
   const int32_t* queryLenDev_ = nullptr;

@@ -278,8 +278,8 @@ int Grid::ensureQueryStore(const TrajectoryView& q, int64_t ctlWords) {
   }
   // Everything is laid out in pinned memory, from where one kernel
   // (gat_edr_stage_queries) writes the device's copies, the padded store and
-  // the boxes.  The offsets and lengths the kernels read are views into one
-  // device buffer.
+  // the boxes.  The offsets and lengths that later kernels read are views into
+  // one device buffer; the source offsets only that kernel reads.
   if (int rc = waitQueries()) return rc;
   const int T = q.trajNum;
   const int64_t o0 = T > 0 ? q.offsets[0] : 0;
@@ -288,7 +288,7 @@ int Grid::ensureQueryStore(const TrajectoryView& q, int64_t ctlWords) {
   auto up16 = [](size_t b) { return (b + 15) & ~size_t(15); };
   const size_t braw = up16(size_t(n) * 4), bsrc = up16((size_t(T) + 1) * 8), b64 = up16(size_t(T) * 8);
   const size_t b32 = up16(size_t(T) * 4);
-  const size_t meta = bsrc + b64 + 2 * b32;
+  const size_t up = b64 + 2 * b32, meta = bsrc + up;
   if (int rc = queryStage_.reserve(meta + 2 * braw)) return rc;
   char* base = queryStage_.as<char>();
   int64_t* src = reinterpret_cast<int64_t*>(base);
@@ -310,12 +310,11 @@ int Grid::ensureQueryStore(const TrajectoryView& q, int64_t ctlWords) {
   }
   src[T] = n;
   void* s = engine_.stream();
-  if (int rc = queryUp_.reserve(std::max<size_t>(meta, 16))) return rc;
+  if (int rc = queryUp_.reserve(std::max<size_t>(up, 16))) return rc;
   char* dev = queryUp_.as<char>();
-  querySrcOffDev_ = reinterpret_cast<const int64_t*>(dev);
-  queryOff64Dev_ = reinterpret_cast<const int64_t*>(dev + bsrc);
-  queryOffDev_ = reinterpret_cast<const int32_t*>(dev + bsrc + b64);
-  queryLenDev_ = reinterpret_cast<const int32_t*>(dev + bsrc + b64 + b32);
+  queryOff64Dev_ = reinterpret_cast<const int64_t*>(dev);
+  queryOffDev_ = reinterpret_cast<const int32_t*>(dev + b64);
+  queryLenDev_ = reinterpret_cast<const int32_t*>(dev + b64 + b32);
   if (int rc = queryXY_.reserve(size_t(total) * 8)) return rc;
   if (int rc = queryBox_.reserve(std::max<size_t>(size_t(T) * 16, 16))) return rc;
   if (ctlWords > 0)
@@ -334,7 +333,7 @@ int Grid::ensureQueryStore(const TrajectoryView& q, int64_t ctlWords) {
     }
     const bool first = t0 == 0, last = t1 == T;
     uint32_t* ctl = first && ctlWords > 0 ? topCtl_.as<uint32_t>() : nullptr;
-    GATH_TRY(gat_edr_stage_queries(base, first ? int64_t(meta) : 0, dev, src + t0, off64 + t0, t1 - t0, p1, lon, lat,
+    GATH_TRY(gat_edr_stage_queries(base + bsrc, first ? int64_t(up) : 0, dev, src + t0, off64 + t0, t1 - t0, p1, lon, lat,
                                    last ? total : off64[t1] - GAT_EDR_PAD, queryXY_.as<float>(),
                                    queryBox_.as<float>() + 4 * size_t(t0), ctl, ctl ? ctlWords : 0,
                                    ctl ? ctl + ctlWords : nullptr, s),

@@ -425,3 +425,37 @@ def test_edr_jobs_overflow_empties_the_windows(gpu, capacity):
             assert (got == np.arange(capacity)).all()  # every pair placed once
             n, m = np.minimum(qlen[pairs[:, 0]], clen[pairs[:, 1]]), np.maximum(qlen[pairs[:, 0]], clen[pairs[:, 1]])
             assert int(cells.get(np.uint64, 1)[0]) == int((n.astype(np.int64) * m).sum())
+
+
+@pytest.mark.parametrize("lens", [[], [1], [0, 5, 0], [64, 65, 1, 2048, 63]])
+def test_pack_and_staged_stores_agree(gpu, lens):
+    """gat_edr_pack_trajectories (points already on the device) writes the
+    padded store and boxes that gat_edr_stage_queries writes from pinned memory:
+    the points at their offsets, NaN elsewhere, an empty trajectory's box
+    empty."""
+    h = N.hip()
+    n, pad, tail = len(lens), 16, api.MAX_TRAJ_LEN + 64
+    rng = np.random.default_rng(n)
+    src = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    m = int(src[-1])
+    dst = (src[:-1] + pad * (1 + np.arange(n))).astype(np.int64)
+    lon, lat = rng.random(m).astype(np.float32), rng.random(m).astype(np.float32)
+    total = m + pad * (n + 1) + tail
+    want = np.full((total, 2), np.nan, np.float32)
+    boxes = np.zeros((n, 4), np.float32)
+    for t in range(n):
+        p = np.stack([lon[src[t]:src[t + 1]], lat[src[t]:src[t + 1]]], 1)
+        want[dst[t]:dst[t] + len(p)] = p
+        boxes[t] = np.concatenate([p.min(0), p.max(0)]) if len(p) else [np.inf, np.inf, -np.inf, -np.inf]
+    dlon, dlat, dsrc, ddst = DevBuf.of(lon), DevBuf.of(lat), DevBuf.of(src), DevBuf.of(dst)
+    for staged in (False, True):
+        xy, box = DevBuf.of(np.zeros((total, 2), np.float32)), DevBuf.of(np.zeros((max(n, 1), 4), np.float32))
+        if staged:
+            N.check_hip(h.gat_edr_stage_queries(None, 0, None, dsrc.ptr, ddst.ptr, n, m, dlon.ptr, dlat.ptr, total,
+                                                xy.ptr, box.ptr, None, 0, None, None))
+        else:
+            N.check_hip(h.gat_edr_pack_trajectories(dlon.ptr, dlat.ptr, dsrc.ptr, ddst.ptr, n, total, xy.ptr, box.ptr,
+                                                    None))
+        got = xy.get(np.float32, 2 * total).reshape(-1, 2)
+        assert (np.isnan(got) == np.isnan(want)).all() and (got == want)[~np.isnan(want)].all()
+        assert (box.get(np.float32, 4 * n).reshape(n, 4) == boxes).all()

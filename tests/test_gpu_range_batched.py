@@ -418,3 +418,23 @@ def test_fill_spans(gpu):
         got = b.get(np.uint32, m + 2)
         assert got[0] == 7 and got[-1] == 7 and (got[1:-1] == 0xABCD).all()
     assert h.gat_fill_u32_spans(5, ptrs, n, 0, None) == 2
+
+
+@pytest.mark.parametrize("n,capacity", [(0, 4), (1, 4), (300, 300), (300, 256)])
+def test_leaf_tasks(gpu, n, capacity):
+    """gat_leaf_tasks, for callers that refine by gat_range_refine_pairs: each
+    listed (leaf, rectangle) entry inside the capacity becomes the leaf's store
+    run, an entry naming no leaf an empty one."""
+    h = N.hip()
+    rng = np.random.default_rng(n)
+    nodes = np.zeros(40, api.TREE_NODE)
+    nodes["start"], nodes["count"] = rng.integers(0, 1000, 40), rng.integers(1, 90, 40)
+    lq = np.stack([rng.integers(0, 44, max(n, 1)), rng.integers(0, 7, max(n, 1))], 1).astype(np.uint32)
+    dn, dq, total = DevBuf.of(nodes), DevBuf.of(lq), DevBuf.of(np.array([n], np.uint64))
+    tasks = DevBuf.of(np.full((capacity + 1, 3), 9, np.uint32))
+    N.check_hip(h.gat_leaf_tasks(dq.ptr, total.ptr, capacity, dn.ptr, 40, tasks.ptr, None))
+    got, m = tasks.get(np.uint32, 3 * (capacity + 1)).reshape(-1, 3), min(n, capacity)
+    leaf = np.minimum(lq[:m, 0], 39)
+    ok = lq[:m, 0] < 40
+    want = np.stack([np.where(ok, nodes["start"][leaf], 0), np.where(ok, nodes["count"][leaf], 0), lq[:m, 1]], 1)
+    assert (got[:m] == want).all() and (got[m:] == 9).all()
