@@ -108,7 +108,9 @@ def test_device_built_indexes_answer_like_the_oracle(gpu):
 
 def test_unpacked_ids(gpu):
     """More than 2^21 trajectories and 2048-point ones: trajectory and point ids
-    do not share 32 bits, so point ids go to the 16-bit array."""
+    do not share 32 bits, so point ids go to the 16-bit array.  Range batches
+    over such a store (direct, leaf-major, both layouts) and its bitmaps against
+    brute force."""
     n = (1 << 21) + 2
     lens = np.ones(n, np.int64)
     lens[-1] = 2048
@@ -125,6 +127,22 @@ def test_unpacked_ids(gpu):
     assert bits == 0 and hbits == 0
     assert (ids == hids).all() and (pid == hpid).all() and (xy.view(np.uint32) == hxy.view(np.uint32)).all()
     assert pid.max() == 2047
+    rects = np.array([[0.1, 0.2, 0.1037, 0.2041], [0.3, 0.3, 0.3, 0.3], [0.61, 0.62, 0.6601, 0.6703]], np.float32)
+    tid = np.repeat(np.arange(1, n + 1), lens)
+    at = np.arange(m) - np.repeat(offsets[:-1], lens)
+    want = []
+    for x0, y0, x1, y1 in rects:
+        i = np.nonzero((db.lon >= x0) & (db.lon <= x1) & (db.lat >= y0) & (db.lat <= y1))[0]
+        want.append(set(zip(tid[i].tolist(), at[i].tolist())))
+    assert len(want[0]) > 10 and len(want[2]) > 1000
+    for direct, runs in ((256, True), (0, True), (0, False)):
+        dev.set_batch_params(32, direct).set_result_layout(runs)
+        res = dev.range_batched(rects)
+        assert [set(map(tuple, p.tolist())) for p in res.per_query()] == want
+        assert (res.digests() == dev.range_pairs(rects).digests()).all()
+    bitmap = dev.range_bitmap(rects)
+    for row, w in zip(bitmap, want):
+        assert set(np.nonzero(row)[0].tolist()) == {t for t, _ in w} and row.max(initial=0) <= 1
 
 
 def test_points_off_the_grid_are_rejected(gpu):

@@ -1,8 +1,9 @@
 """The direct form's device chain and the gathered readback: batches of every
-size around a wave's four entries and the regions kernel's 256 threads, a batch
-that outgrows the buffers' capacities, leaves of more points than one round
-takes, both id packings' store, rectangles that select nothing; counts, digests
-and pair sets against the plain path and inclusive brute force."""
+size around a wave's four entries and the regions kernel's 256 threads, batches
+that outgrow the pairs and the selection's list, leaves of more points than one
+round takes, rectangles that select nothing; counts, digests and pair sets
+against the plain path and inclusive brute force.  (Stores of unpacked ids:
+test_unpacked_ids of test_gpu_build.py.)"""
 import threading
 
 import numpy as np
@@ -48,6 +49,24 @@ def test_direct_chain(gpu, nq, leaf):
         assert (res.counts() == pc).all()
         for a, b in zip(res.per_query(), pp):
             assert sorted(map(tuple, a.tolist())) == sorted(map(tuple, b.tolist()))
+
+
+def test_direct_outgrows_the_list(gpu):
+    """More (leaf, rectangle) entries than the list's first 65,536: it grows and
+    the batch runs again, and the next one of its size fits."""
+    db = api.synth_walks(6, np.full(3000, 60, np.int32), step_sigma=4e-3)
+    ix = api.GridIndex(W.UNIT_BOX, 0.005, 16).build(db)
+    rects = np.tile(np.array([[0.0, 0.0, 1.0, 1.0]], np.float32), (40, 1))
+    rects[1::2] = [0.25, 0.25, 0.75, 0.75]
+    plain = ix.range_pairs(rects)
+    pc, pd = plain.counts(), plain.digests()
+    # The leaf-major form counts the entries.
+    assert ix.set_batch_params(32, 0).range_batched(rects).leaf_queries > 1 << 16
+    fresh = api.GridIndex(W.UNIT_BOX, 0.005, 16).build(db)
+    for _ in range(2):
+        res = fresh.range_batched(rects)
+        assert res.leaf_queries > 1 << 16
+        assert (res.counts() == pc).all() and (res.digests() == pd).all()
 
 
 @pytest.mark.parametrize("direct", [256, 0])  # regions of the direct form, runs of the leaf-major one
