@@ -697,13 +697,21 @@ struct BitBytes {
   }
 };
 
-// out[i] = bit i, i < n.
+// out[i] = bit i, i < n.  A word at a time: with eight bits per turn the loop's
+// own instructions set its pace, and where it happened to lie in the code
+// decided between 50 and 90 us for 2 MB.
 void expand_bits(const uint32_t* bits, int64_t n, uint8_t* out) {
   static const BitBytes table;
-  const uint8_t* b = reinterpret_cast<const uint8_t*>(bits);
-  int64_t i = 0;
-  for (; i + 8 <= n; i += 8) std::memcpy(out + i, &table.at[b[i / 8]], 8);
-  for (; i < n; ++i) out[i] = (b[i / 8] >> (i % 8)) & 1;
+  const uint64_t* at = table.at;
+  const int64_t words = n / 32;
+  for (int64_t w = 0; w < words; ++w, out += 32) {
+    const uint32_t v = bits[w];
+    std::memcpy(out, at + (v & 255), 8);
+    std::memcpy(out + 8, at + (v >> 8 & 255), 8);
+    std::memcpy(out + 16, at + (v >> 16 & 255), 8);
+    std::memcpy(out + 24, at + (v >> 24), 8);
+  }
+  for (int64_t i = 0; i < n % 32; ++i) out[i] = (bits[words] >> i) & 1;
 }
 }  // namespace
 
