@@ -664,7 +664,8 @@ class MixedRange:
     """One batch over the three indexes of a data set: each rectangle routed by
     area (FSG below fsg_max_area, GT-quadtree below grid_max_area, STIG above),
     in groups of group_size per index; the three device pipelines of a group run
-    as one captured graph.  Results: per-rectangle counts and digests."""
+    together, queued on the indexes' streams or replayed as one captured graph.
+    Results: per-rectangle counts and digests."""
 
     def __init__(self, grid: "GridIndex", stig: "StigIndex", fsg: "FsgIndex"):
         self._keep = (grid, stig, fsg)

@@ -1245,14 +1245,13 @@ __global__ __launch_bounds__(256) void edr_length_table_kernel(const int32_t* __
 
 // ---------------------------------------------------------------- device jobs
 // The batch's job list built on the device from the filter's survivors, so a
-// top-k batch runs filter -> jobs -> DP -> merge with no host round trip.  One workgroup: per pair the shorter and longer length, the
-// length bucket (runBatched's rules: short up to `split`, long up to `mid`,
-// the rest one pair per wave, and in a batch of one round of waves the pairs
-// that would outlast the longest pair's several-wave schedule on one wave
-// take several), then a counting sort in LDS by (bucket, strips descending,
+// top-k batch runs filter -> jobs -> DP -> merge with no host round trip.  One
+// workgroup: per pair the shorter and longer length and the length bucket
+// (JobShape below), then a counting sort in LDS by (bucket, strips descending,
 // longer length descending in sixteen steps of the bucket's length range) and
-// jobs of up to four pairs of one strip count (one pair in the long buckets).  Pairs of equal sort key
-// keep no particular order: it only changes which pairs share a job.
+// jobs of up to four pairs of one strip count (one pair in the long buckets).
+// Pairs of equal sort key keep no particular order: it only changes which pairs
+// share a job.
 constexpr int kJobThreads = 1024;
 constexpr int64_t kJobsOneBlock = 131072;  // larger batches take the whole device
 constexpr int kJobsScratchExtra = GAT_EDR_JOBS_SCRATCH_EXTRA;

@@ -766,9 +766,9 @@ __global__ void leaf_scatter_kernel(const uint2* __restrict__ lq, const unsigned
   }
 }
 
-// Direct form for small batches: each selected (leaf, query) entry becomes a
-// refine task of the per-task kernel (range.hip), so nothing sized by the
-// tree is touched.
+// Each selected (leaf, query) entry as a task of the per-task refine kernel
+// (range.hip), for callers that refine that way.  (The library's own small
+// batches refine the entries as they are, range_direct.hip.)
 __global__ void leaf_tasks_kernel(const uint2* __restrict__ lq, const unsigned long long* __restrict__ lq_total,
                                   uint64_t lq_cap, const Node* __restrict__ nodes, uint32_t nnodes,
                                   gat_range_task* __restrict__ tasks) {

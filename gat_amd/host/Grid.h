@@ -215,10 +215,10 @@ class Grid {
   static constexpr int kDeviceTopkMax = 1024;
   int deviceTopk(const std::vector<int32_t>& pairs, const std::vector<int32_t>& dist, int nq, int kValue,
                  std::vector<TopK>& out);
-  // The whole top-k batch on the device (filter, jobs, DP, survivor lists,
-  // merge) with one readback at the end; *done is false when the batch must
-  // take the host-built path instead (a query with more survivors than the
-  // device's per-query sort holds).
+  // The whole top-k batch on the device (filter, jobs, DP, merge) with one wait
+  // at the end; *done is false when the batch must take the host-built path
+  // instead (a query with more survivors than the device's per-query sort
+  // holds).
   int similarityOnDevice(int nq, int kValue, TopKSink& out, EdrBatchStats* st, bool* done);
   // The same for batches of few queries, whose time is their launches and the
   // longest pair: no job list (every survivor takes several waves), the merge
@@ -228,6 +228,15 @@ class Grid {
   // The batch with its pairs, jobs and lists built on the host.
   int similarityHost(int nq, int kValue, std::vector<TopK>& out, EdrBatchStats* st);
   static constexpr int64_t kUploadPart = 1 << 17;  // points of a part of the queries' upload
+  // Where the short chain gives way to the job list's.  Measured on 300,000
+  // trajectories (lengths lognormal, median 64; k = 20), short chain against job
+  // list: 120 and 199 us for 8 queries, 163 and 268 for 32, 167 and 340 for 64,
+  // 231 and 407 for 256 (1,884 pairs); 16 queries in crowds: 125 and 187 us with
+  // 1,024 pairs, 164 and 287 with 2,048, 253 and 352 with 4,096, 419 and 443 with
+  // 8,192.  So both lines lie on the near side of where the two meet: they bound
+  // the pairs that go several waves each whatever their lengths (the job list
+  // gives a pair the cheapest form that ends in time), and every workgroup of the
+  // merge reads every pair.
   static constexpr int kSmallTopkQueries = 32;
   static constexpr int64_t kSmallTopkPairs = 2048;
   // The DP launches over a device-built job list (windows in win, a cleared job

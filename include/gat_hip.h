@@ -299,12 +299,17 @@ int gat_edr_batched(const int32_t* pairs_dev, int64_t npairs, const gat_edr_job*
  * counterpart), so that filter, DP and merge run without a host round trip.
  * Reads the *count_dev pairs (query, candidate) of pairs_dev (the filter's
  * output; at most capacity); writes them to sorted_dev grouped by length
- * bucket (longer length up to `split`; up to max(split, 1024), or `split` in a
- * batch of fewer than 64 jobs per CU; longer; and, in such a batch with waves
- * > 1, the long pairs that would outlast the batch's longest several-wave
- * pair, or every long pair when every_long) and within a bucket by strip count
- * and longer length (in sixteen steps of the bucket's range), descending; jobs_dev (capacity + 4 entries) gets jobs of
- * up to four pairs of one strip count (one pair in the two long buckets) and
+ * bucket (0: longer length up to `split`, four pairs per wave; 1: up to
+ * max(split, 1024), likewise; 2: one pair per wave; 3: several waves per pair,
+ * with waves > 1) and within a bucket by strip count and longer length (in
+ * sixteen steps of the bucket's range), descending.  A batch of 64 jobs per CU
+ * and more uses buckets 0 to 2 by length.  A smaller one, a single round of
+ * waves, has a critical length (its longest pair's schedule, over several waves
+ * where it may take them, but at least half of what its pairs take spread
+ * evenly over the SIMDs): a pair stays in bucket 0 up to `split` and while twice
+ * its cost there fits, goes to bucket 2 while its cost on one wave fits, else to
+ * bucket 3 (with every_long, every pair longer than `split` does, and one up to
+ * it never).  jobs_dev (capacity + 4 entries) gets jobs of up to four pairs of one strip count (one pair in the two long buckets) and
  * windows_dev[2b], [2b+1] the first job and job count of bucket b (four
  * buckets), for gat_edr_batched's windows; origin_dev (may be null; capacity
  * entries) gets each sorted pair's index in pairs_dev.  scratch_dev: capacity * 2
@@ -625,9 +630,10 @@ int gat_morton_select(const uint32_t* cell_words_dev, int32_t total_level, int64
                       uint32_t* node_qcount_dev, uint64_t* cand_dev, uint32_t* leaf_query_dev, uint32_t* lq_rank_dev,
                       int64_t lq_capacity, uint64_t* lq_total_dev, uint32_t* status_dev, void* stream);
 
-/* The direct form for small batches: entry i of the (leaf, query) list becomes
- * tasks_dev[i] = {leaf start, leaf count, query} for gat_range_refine_pairs, so
- * no per-node array is touched.  tasks_dev holds lq_capacity tasks. */
+/* Entry i of the (leaf, query) list as tasks_dev[i] = {leaf start, leaf count,
+ * query} for gat_range_refine_pairs, a direct form that touches no per-node
+ * array (gat_direct_refine below refines the entries themselves).  tasks_dev
+ * holds lq_capacity tasks. */
 int gat_leaf_tasks(const uint32_t* leaf_query_dev, const uint64_t* lq_total_dev, int64_t lq_capacity,
                    const gat_tree_node* nodes_dev, int64_t nnodes, gat_range_task* tasks_dev, void* stream);
 

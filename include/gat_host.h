@@ -226,8 +226,9 @@ int gath_tune_edr(void* grid, const int64_t* q_offsets, int nq, const float* qlo
 /* ---------------------------------------------------------------- mixed
  * One batch of rectangles over the three indexes of a data set: each goes to
  * FSG (area < cfg[0]), the GT-quadtree (area < cfg[1]) or STIG, in groups of
- * cfg[2] rectangles per index, the three device pipelines of a group captured
- * as one graph and replayed (cfg[3] != 0).  Per rectangle: counts, digests
+ * cfg[2] rectangles per index, the three device pipelines of a group running
+ * together: queued on the indexes' streams, or, where a group has the sizes of
+ * one captured before, replayed as one graph (cfg[3] != 0).  Per rectangle: counts, digests
  * (as gat_pairs_digest), route (0 FSG, 1 GT-quadtree, 2 STIG); stats[0..6] =
  * pairs, candidates, groups, graph replays, wall ms, of which digest ms, and
  * the graphs this object has captured so far (a group whose engines' buffers
