@@ -195,8 +195,12 @@ int MixedRange::run(const MBB* bounds, int n, const MixedConfig& cfg, MixedResul
       }
       for (int i = 0; i < 3 && rc == GAT_OK; ++i)
         if (nq[i] > 0 && !queued[i]) {
-          rc = step(i);
-          byStep[i] = rc == GAT_OK;
+          if (const int r = step(i)) {  // it has said what failed
+            waitAll(r);
+            restore();
+            return r;
+          }
+          byStep[i] = true;
         }
       rc = waitAll(rc);
       if (rc == GAT_OK) rc = collect(false, queued);
