@@ -79,13 +79,13 @@ def test_topk_chains_are_sized_before_serving(gpu):
     walk = (at[:, None, :] + rng.normal(0, 2e-5, (n, m, 2))).astype(np.float32)
     db = api.TrajSet(np.arange(n + 1, dtype=np.int64) * m, walk[:, :, 0].ravel().copy(), walk[:, :, 1].ravel().copy())
     g = api.GridIndex(W.UNIT_BOX, 0.01, 64).build(db)
-    nq = 160
+    nq = 416  # (the worker starts as they arrive, so its first batches may be small)
     q = np.where(np.arange(nq)[:, None, None] < 32, 0.9, 0.2) + rng.normal(0, 2e-5, (nq, m, 2))
     req = np.zeros(nq, api.REQUEST)
     req["kind"], req["qlen"], req["qoff"] = api.REQ_TOPK, m, np.arange(nq) * m
     lon, lat = q[:, :, 0].astype(np.float32).ravel(), q[:, :, 1].astype(np.float32).ravel()
     out, ids, dists, st = api.serve(g, req, lon, lat, K, EPS, max_topk_batch=32)
-    assert st["topk_batches"] == 5 and st["peak_topk_survivors"] == 32 * 60
+    assert st["topk_batches"] >= 13 and st["peak_topk_survivors"] == 32 * 60
     assert st["device_allocs"] == 0 and st["pinned_allocs"] == 0
     qs = api.TrajSet(np.arange(nq + 1, dtype=np.int64) * m, lon, lat)
     want_i, want_d, _ = g.set_topk_device_chain(False).similarity_batched(qs, K, EPS)
