@@ -843,10 +843,10 @@ int Grid::runBatchedOnDevice(const int32_t* pairsHost, int64_t np, int queryNum,
 // brings them back): [0, 1] survivors, [2] lists and [3] merge status (as
 // gat_edr_merge's), [4, 5] cells, [6] the job counter of gat_edr_pairs, [7]
 // ticket, [8] job list status, [10, 16) the clock at the filter, the DP and the
-// job list (between the two), [16, 24) the buckets' windows, [24, 28) their job counters; after them the
-// clock at the upload (device), or at the merge's end and its start (host: the
-// merge writes both there itself, since its workgroup that brings the words
-// back is not ordered behind the one that starts first).
+// job list (between the two), [16, 24) the buckets' windows, [24, 28) their job
+// counters; after them the clock at the upload (device), or at the merge's end
+// and its start (host: the merge writes both there itself, since its workgroup
+// that brings the words back is not ordered behind the one that starts first).
 namespace {
 constexpr int kCtlWords = 32, kHostWords = kCtlWords + 4;
 uint64_t ctl64(const uint32_t* c, int w) { return uint64_t(c[w]) | (uint64_t(c[w + 1]) << 32); }

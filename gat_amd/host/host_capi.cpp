@@ -191,7 +191,8 @@ int gath_index_range_bitmap(void* p, const float* boxes, int nq, uint8_t* out) {
   // they refuse.
   const DeviceTree& tree = ix->grid ? ix->grid->deviceTree() : ix->fsg ? ix->fsg->deviceTree() : ix->stig->deviceTree();
   RangeEngine& engine = ix->grid ? ix->grid->engine() : ix->fsg ? ix->fsg->engine() : ix->stig->engine();
-  if (tree.nnodes > 0 && nq > 0) return engine.runBitmapDirect(tree, as_boxes(boxes), nq, int64_t(ix->trajNum()) + 1, out);
+  if (tree.nnodes > 0 && nq > 0)
+    return engine.runBitmapDirect(tree, as_boxes(boxes), nq, int64_t(ix->trajNum()) + 1, out);
   return gath_index_range_handler(p, boxes, nq, out, nullptr);
 }
 
